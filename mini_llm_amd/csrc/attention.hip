@@ -880,13 +880,13 @@ MLLM_API int mllm_attention_prefill_supported(int head_size, int page_size) {
 
 MLLM_API int mllm_attention_prefill(const void* q, int q_stride, const void* k_pages, const void* v_pages, void* out,
                                     int out_stride, const int* q_starts, const int* context_lens,
-                                    const int* block_tables, int max_blocks, int n_requests, int max_q_len,
+                                    const int* block_tables, int max_blocks, int n_requests, int rows, int max_q_len,
                                     int max_len, int n_heads, int n_kv_heads, int head_size, int page_size, int window,
                                     float scale, int dtype, float softcap, const float* sinks, int chunk, int keep, int wide_out, hipStream_t stream) {
     const ScoreOptions options = {softcap, sinks, chunk, keep, wide_out};
-    // max_len: the longest sequence after this step, or a bound on it (0 or less: what the block tables can hold); it only
+    // rows: the rows of all portions in sum, or more (padding rows count); max_len: the longest sequence after this step, or a bound on it (0 or less: what the block tables can hold); it only
     // decides how many waves share a block's keys
-    MLLM_REQUIRE(n_requests >= 0 && max_q_len >= 0 && n_heads > 0 && n_kv_heads > 0 && max_blocks > 0, "attention_prefill: bad sizes");
+    MLLM_REQUIRE(n_requests >= 0 && rows >= 0 && max_q_len >= 0 && n_heads > 0 && n_kv_heads > 0 && max_blocks > 0, "attention_prefill: bad sizes");
     MLLM_REQUIRE(n_heads % n_kv_heads == 0, "attention_prefill: %d heads do not divide into %d key/value heads", n_heads, n_kv_heads);
     MLLM_REQUIRE(mllm_attention_prefill_supported(head_size, page_size),
                  "attention_prefill: head size %d is not a multiple of 16 in 16..128, or page size %d is no power of two", head_size, page_size);
@@ -905,7 +905,7 @@ MLLM_API int mllm_attention_prefill(const void* q, int q_stride, const void* k_p
     const int reach = (int)(max_len > 0 && max_len < table_reach ? max_len : (table_reach < (1 << 30) ? table_reach : (1 << 30)));
 #define MLLM_STREAM_CASE(T, HD)                                                                                            \
     prefill_stream::launch<T, HD>(q, q_stride, k_pages, v_pages, out, out_stride, q_starts, context_lens, block_tables,    \
-                                  max_blocks, n_requests, max_q_len, reach, n_heads, n_kv_heads, page_shift, window, scale, options, stream)
+                                  max_blocks, n_requests, rows, max_q_len, reach, n_heads, n_kv_heads, page_shift, window, scale, options, stream)
     if (dtype == MLLM_BF16 && (!wide_out || ((size_t)out) % 16 == 0) &&
         prefill_stream::takes<bf16_t>(head_size, page_size, max_q_len, scale, q_stride, out_stride, q, out)) {
         // long portions, rows of 64 / 128 / 256 bytes, pages of 32 keys or more: keys and values stream from the pages straight into LDS

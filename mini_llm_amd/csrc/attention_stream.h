@@ -156,18 +156,82 @@ struct Layout {
     static __device__ __forceinline__ int v_turn(int key) { return FP32 || ROW_BYTES == 64 ? 0 : (ROW_BYTES == 128 ? ((key >> 1) & 1) * 4 : (key & 3) * 4); }
 };
 
+// The (request, tile of queries) that place `slot` of a launch stands for: the tiles of all portions in the order of their place in the portion, the
+// last ones (which have the most keys) first, portions that have no such tile left out. False: the launch has more places than tiles. So a launch
+// has as many blocks a head as there can be tiles in its rows, and not one for every tile of the longest portion a padded shape allows, times its
+// requests: 64 prompts of 32 tokens x 25 heads in a step of 2,048 rows took 51,200 blocks of which 1,600 had work, and 60 us; 26 us without the others.
+// Padding requests (a negative context) have no tiles. Every lane holds the tiles of one request (of each 64 of them), and what is below is the same in
+// all lanes. The lengths are asked for at once: a trip to memory, as for one request's.
+template <int QUERIES>
+__device__ __forceinline__ bool tile_of_slot(int slot, int n_requests, const int* q_starts, const int* context_lens, int& request, int& q_first, int& q_len, int& context, int& tile) {
+    const int lane = threadIdx.x % WAVE;
+    for (int group = 0; group < n_requests; group += WAVE) {
+        const int mine = group + lane;
+        const bool real = mine < n_requests;
+        const int first = real ? q_starts[mine] : 0, length = real ? q_starts[mine + 1] - first : 0, stored = real ? context_lens[mine] : -1;
+        const int tiles = stored < 0 ? 0 : max(0, length + QUERIES - 1) / QUERIES;
+        // places(at): the tiles at place `at` of their portion and behind it; the slot falls where places(at) > slot >= places(at + 1)
+        int at = 0, before_it = 0;
+        bool found = false;
+        if (n_requests <= 8) {   // few portions: every lane takes a place (the search below, six dependent sums over a wave, costs a block 0.4 us)
+            int behind_lane = 0;
+            for (int r = 0; r < n_requests; r++) behind_lane += max(0, __builtin_amdgcn_readlane(tiles, r) - lane);
+            const unsigned long long more = __ballot(behind_lane > slot);
+            if (more == 0) return false;
+            if (more != ~0ull) {
+                at = __popcll(more) - 1;
+                before_it = __builtin_amdgcn_readlane(behind_lane, at + 1);
+                found = true;
+            }
+        }
+        if (!found) {   // many portions, which in a step's rows are short ones, or one of more than 64 tiles
+            auto places = [&](int at) { return (int)wave_total((float)max(0, tiles - at)); };   // (exact: far below 2^24)
+            const int all = places(0);
+            if (slot >= all) {
+                slot -= all;
+                continue;
+            }
+            int behind = (int)wave_max_total((float)tiles);
+            while (behind - at > 1) {
+                const int middle = (at + behind) / 2, count = places(middle);
+                if (count > slot) at = middle;
+                else behind = middle, before_it = count;
+            }
+        }
+        unsigned long long has = __ballot(tiles > at);
+        for (int skip = slot - before_it; skip > 0; skip--) has &= has - 1;
+        const int from = __ffsll(has) - 1;
+        request = group + from;
+        q_first = __builtin_amdgcn_readlane(first, from);
+        q_len = __builtin_amdgcn_readlane(length, from);
+        context = __builtin_amdgcn_readlane(stored, from);
+        tile = at;
+        return true;
+    }
+    return false;
+}
+
 // QUERIES: 64 queries a block (two sub-tiles of 32, both held by every wave), or 32 where that would leave compute units
 // without a block: what the kernel waits for is the wave with the most tiles, and a tile of 32 queries takes it half as long.
 // SPLITS: four waves a block, or eight where the portions reach far back: the kernel's time is the time of the wave with
 // the most tiles (it pays every tile's chain in full), which eight waves halve; a block then has a compute unit to itself.
-// KEPT: a window with kept first keys (ScoreOptions). A kernel of its own: the fragments of the next tile sit in registers that nothing may copy
-// until they have landed, so the kernel without kept keys carries nothing for them.
-template <typename T, int HD, int QUERIES, int SPLITS, bool KEPT>
+// FORM: which of the options on scores a launch has, as kernels of their own. The loop is written for the registers it has (the fragments of the
+// next tile sit in registers that nothing may copy until they have landed), and a cap in a branch that a launch never takes cost the
+// 64-query kernel for heads of 64 51 spilled registers: two prompts of 1,024 tokens x 12 heads 36 us, 16 without them.
+enum Form : int {
+    CAUSAL = 0,   // every key up to the query
+    MASKED = 1,   // a window or chunks
+    CAPPED = 2,   // capped scores, with or without a window or chunks
+    KEPT = 3,     // a window with kept first keys, with or without a cap
+};
+
+template <typename T, int HD, int QUERIES, int SPLITS, int FORM>
 __global__ __launch_bounds__(64 * SPLITS, (HD * sizeof(T) <= 128 && SPLITS == 4) ? 2 : 1) void attention_prefill_stream_kernel(
     const T* __restrict__ q, int q_stride, const T* __restrict__ k_pages, const T* __restrict__ v_pages,
     T* __restrict__ out, int out_stride, const int* __restrict__ q_starts, const int* __restrict__ context_lens,
-    const int* __restrict__ block_tables, int max_blocks, int n_heads, int n_kv_heads, int page_shift, int window, float scale, ScoreOptions options) {
+    const int* __restrict__ block_tables, int max_blocks, int n_requests, int n_heads, int n_kv_heads, int page_shift, int given_window, float scale, ScoreOptions options) {
     typedef Layout<T, HD, SPLITS> L;
+    const int window = FORM == CAUSAL ? 0 : given_window, chunk = FORM == CAUSAL ? 0 : options.chunk;
     constexpr bool FP32 = L::FP32;
     constexpr int QSUB = QUERIES / 32;
     static_assert(QUERIES == 32 || QUERIES == 64, "one or two sub-tiles of queries");
@@ -181,13 +245,14 @@ __global__ __launch_bounds__(64 * SPLITS, (HD * sizeof(T) <= 128 && SPLITS == 4)
     const int tid = threadIdx.x, lane = tid % WAVE;
     const int wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
     const int lane32 = lane % 32, half = lane / 32;
-    const int request = blockIdx.x / n_heads, head = blockIdx.x % n_heads;
-    const int q_first = q_starts[request];
-    const int q_len = q_starts[request + 1] - q_first;
-    const int tile_q0 = (gridDim.y - 1 - blockIdx.y) * QUERIES;  // the blocks with the most keys start first
-    if (tile_q0 >= q_len) return;
-    const int context = context_lens[request];
-    if (context < 0) return;  // a padding request of a padded batch: its rows (if it has any) are nobody's, and it has no pages
+    // places one after the other, the heads of a place side by side: the blocks with the most keys start first, whatever their head. Of each eight
+    // heads one belongs to an XCD (which has every eighth block), so that its keys and values are read through one L2; the heads beyond a multiple of
+    // eight are where they fall.
+    const int slot = blockIdx.x / n_heads, at = blockIdx.x % n_heads;
+    const int head = at < (n_heads & ~7) ? (at & ~7) | (blockIdx.x & 7) : at;
+    int request, q_first, q_len, context, query_tile;
+    if (!tile_of_slot<QUERIES>(slot, n_requests, q_starts, context_lens, request, q_first, q_len, context, query_tile)) return;
+    const int tile_q0 = query_tile * QUERIES;
     const int kv_head = head / (n_heads / n_kv_heads);
     const int* table = block_tables + (size_t)request * max_blocks;
     const int page_mask = (1 << page_shift) - 1;
@@ -207,10 +272,10 @@ __global__ __launch_bounds__(64 * SPLITS, (HD * sizeof(T) <= 128 && SPLITS == 4)
     }
 
     const int block_last_position = context + min(tile_q0 + QUERIES, q_len) - 1;
-    const int block_first_key = first_visible_key(context + tile_q0, window, options.chunk);
+    const int block_first_key = first_visible_key(context + tile_q0, window, chunk);
     const int first_base = (block_first_key / KEYS) * KEYS;
     // with kept first keys: the tiles that hold them come first, the tiles between them and the window are passed over
-    const int kept_tiles = KEPT ? min((options.keep + KEYS - 1) / KEYS, first_base / KEYS) : 0;
+    const int kept_tiles = FORM == KEPT ? min((options.keep + KEYS - 1) / KEYS, first_base / KEYS) : 0;
     const int n_tiles = kept_tiles + (block_last_position - first_base) / KEYS + 1;
     const int n_mine = n_tiles > wave ? (n_tiles - wave + SPLITS - 1) / SPLITS : 0;  // tiles wave, wave + SPLITS, ...
 
@@ -220,7 +285,7 @@ __global__ __launch_bounds__(64 * SPLITS, (HD * sizeof(T) <= 128 && SPLITS == 4)
     unsigned char* const wave_lds = lds + wave * L::WAVE_BYTES;
     auto tile_base = [&](int i) {
         const int tile = wave + SPLITS * min(i, n_mine - 1);
-        return KEPT && tile < kept_tiles ? tile * KEYS : first_base + (tile - kept_tiles) * KEYS;
+        return FORM == KEPT && tile < kept_tiles ? tile * KEYS : first_base + (tile - kept_tiles) * KEYS;
     };
     // a lane's place among the rows of a whole tile, in bytes: the same for every tile, so an address is a base all lanes
     // share plus this (worked out anew for every load it was a sixth of the loop's vector instructions)
@@ -324,7 +389,7 @@ __global__ __launch_bounds__(64 * SPLITS, (HD * sizeof(T) <= 128 && SPLITS == 4)
 
     auto tile = [&](int i, f32x16 (&s_acc)[QSUB], f32x16 (&s_next)[QSUB]) {
         const int page_next = table[tile_base(i + 4) >> page_shift];
-        const int k0 = KEPT ? tile_base(i) : first_base + (wave + SPLITS * i) * KEYS;
+        const int k0 = FORM == KEPT ? tile_base(i) : first_base + (wave + SPLITS * i) * KEYS;
         const unsigned char* v_tile = wave_lds + 2 * L::TILE_BYTES + (i % 2) * L::TILE_BYTES;
         const unsigned char* k_next = wave_lds + ((i + 1) % 2) * L::TILE_BYTES;
         bf16x8 p[QSUB][2];  // the probabilities of a sub-tile of queries, as the second product's operand: keys 0-15 and 16-31 of the tile
@@ -337,9 +402,9 @@ __global__ __launch_bounds__(64 * SPLITS, (HD * sizeof(T) <= 128 && SPLITS == 4)
         // ---- mask (only where the tile touches the diagonal, a window or the portion's end), maximum, exponentials ----
         auto softmax = [&](int qs) {
             const int sub_first_position = context + tile_q0 + qs * 32;
-            const bool interior = window == 0 && options.chunk == 0 && tile_q0 + qs * 32 + 31 < q_len && k0 + KEYS - 1 <= sub_first_position;
+            const bool interior = window == 0 && chunk == 0 && tile_q0 + qs * 32 + 31 < q_len && k0 + KEYS - 1 <= sub_first_position;
             float tile_max = -INFINITY;
-            if (options.softcap > 0.0f) {   // a capped score, left divided by the scale as the plain ones are: cap tanh(scale s / cap) / scale
+            if ((FORM == CAPPED || FORM == KEPT) && options.softcap > 0.0f) {   // a capped score, left divided by the scale as the plain ones are: cap tanh(scale s / cap) / scale
                 const float back = options.softcap / scale, into = scale / options.softcap;
 #pragma unroll
                 for (int v = 0; v < 16; v++) {
@@ -352,12 +417,12 @@ __global__ __launch_bounds__(64 * SPLITS, (HD * sizeof(T) <= 128 && SPLITS == 4)
 #pragma unroll
                 for (int v = 0; v < 16; v++) tile_max = fmaxf(tile_max, s_acc[qs][v]);
             } else {
-                const int first_allowed = q_position[qs] < 0 ? 0 : first_visible_key(q_position[qs], window, options.chunk);
+                const int first_allowed = q_position[qs] < 0 ? 0 : first_visible_key(q_position[qs], window, chunk);
                 const int key0 = k0 + 4 * half;
 #pragma unroll
                 for (int v = 0; v < 16; v++) {
                     const int key = key0 + 8 * (v / 4) + (v % 4);
-                    const bool allowed = (key <= q_position[qs]) & ((key >= first_allowed) | (KEPT && key < options.keep));
+                    const bool allowed = (key <= q_position[qs]) & ((key >= first_allowed) | (FORM == KEPT && key < options.keep));
                     s_acc[qs][v] = allowed ? s_acc[qs][v] : -INFINITY;
                     tile_max = fmaxf(tile_max, s_acc[qs][v]);
                 }
@@ -529,58 +594,68 @@ inline bool takes(int head_size, int page_size, int max_q_len, float scale, int 
     return (q_stride * sizeof(T)) % 16 == 0 && (out_stride * sizeof(T)) % (4 * sizeof(T)) == 0 && ((size_t)q) % 16 == 0 && ((size_t)out) % (4 * sizeof(T)) == 0;
 }
 
-template <typename T, int HD, int QUERIES, int SPLITS, bool KEPT>
+// The most tiles of queries that portions of `rows` rows in sum, none longer than max_q_len, can have: what a launch needs a place for.
+inline int most_tiles(int queries, int n_requests, int rows, int max_q_len) {
+    const long by_rows = (long)rows / queries + n_requests, by_length = (long)n_requests * ceil_div(max_q_len, queries);
+    return (int)(by_rows < by_length ? by_rows : by_length);
+}
+
+template <typename T, int HD, int QUERIES, int SPLITS, int FORM>
 void launch_with(const void* q, int q_stride, const void* k_pages, const void* v_pages, void* out, int out_stride, const int* q_starts,
-                    const int* context_lens, const int* block_tables, int max_blocks, int n_requests, int max_q_len, int n_heads, int n_kv_heads,
+                    const int* context_lens, const int* block_tables, int max_blocks, int n_requests, int rows, int max_q_len, int n_heads, int n_kv_heads,
                     int page_shift, int window, float scale, ScoreOptions options, hipStream_t stream) {
     constexpr int LDS_BYTES = Layout<T, HD, SPLITS>::LDS_BYTES;
     static bool raised = false;  // per instantiation: the limit on dynamic LDS is a property of the kernel
     if (!raised && LDS_BYTES > 60 * 1024)  // (if this fails the launch below fails too, and the entry point reports that)
-        raised = hipFuncSetAttribute((const void*)attention_prefill_stream_kernel<T, HD, QUERIES, SPLITS, KEPT>, hipFuncAttributeMaxDynamicSharedMemorySize, LDS_BYTES) == hipSuccess;
-    // x: (request, head), so that with a multiple of eight heads the blocks of one head share an XCD's L2; y: tiles of queries
-    dim3 grid(n_heads * n_requests, ceil_div(max_q_len, QUERIES));
+        raised = hipFuncSetAttribute((const void*)attention_prefill_stream_kernel<T, HD, QUERIES, SPLITS, FORM>, hipFuncAttributeMaxDynamicSharedMemorySize, LDS_BYTES) == hipSuccess;
+    const int grid = n_heads * most_tiles(QUERIES, n_requests, rows, max_q_len);
     mllm_count_kernel(MLLM_K_ATTENTION_PREFILL_STREAM);
-    attention_prefill_stream_kernel<T, HD, QUERIES, SPLITS, KEPT><<<grid, 64 * SPLITS, LDS_BYTES, stream>>>(
+    attention_prefill_stream_kernel<T, HD, QUERIES, SPLITS, FORM><<<grid, 64 * SPLITS, LDS_BYTES, stream>>>(
         (const T*)q, q_stride, (const T*)k_pages, (const T*)v_pages, (T*)out, out_stride, q_starts, context_lens,
-        block_tables, max_blocks, n_heads, n_kv_heads, page_shift, window, scale, options);
+        block_tables, max_blocks, n_requests, n_heads, n_kv_heads, page_shift, window, scale, options);
 }
 
 template <typename T, int HD, int QUERIES, int SPLITS>
 void launch_queries(const void* q, int q_stride, const void* k_pages, const void* v_pages, void* out, int out_stride, const int* q_starts,
-                    const int* context_lens, const int* block_tables, int max_blocks, int n_requests, int max_q_len, int n_heads, int n_kv_heads,
+                    const int* context_lens, const int* block_tables, int max_blocks, int n_requests, int rows, int max_q_len, int n_heads, int n_kv_heads,
                     int page_shift, int window, float scale, ScoreOptions options, hipStream_t stream) {
-#define MLLM_STREAM_WITH(QUERIES, KEPT)                                                                                                        \
-    launch_with<T, HD, QUERIES, SPLITS, KEPT>(q, q_stride, k_pages, v_pages, out, out_stride, q_starts, context_lens, block_tables, max_blocks, \
-                                              n_requests, max_q_len, n_heads, n_kv_heads, page_shift, window, scale, options, stream)
-    constexpr int KEPT_QUERIES = HD * sizeof(T) > 128 ? 32 : QUERIES;   // (rows of 256 bytes with 64 queries leave no register for the second mask)
-    if (options.keep > 0) MLLM_STREAM_WITH(KEPT_QUERIES, true);
-    else MLLM_STREAM_WITH(QUERIES, false);
+#define MLLM_STREAM_WITH(QUERIES, FORM)                                                                                                        \
+    launch_with<T, HD, QUERIES, SPLITS, FORM>(q, q_stride, k_pages, v_pages, out, out_stride, q_starts, context_lens, block_tables, max_blocks, \
+                                              n_requests, rows, max_q_len, n_heads, n_kv_heads, page_shift, window, scale, options, stream)
+    // a cap with 64 queries spills (51 registers for heads of 64, 53 for heads of 128), and so may what the fragments in flight must not be moved by:
+    // two prompts of 1,024 tokens x 12 heads of 64 over a window of 512, capped 28.0 us with 64 queries, 19.0 with 32; with kept keys 27.5 and 18.1
+    constexpr int CAPPED_QUERIES = HD >= 64 ? 32 : QUERIES;
+    if (options.keep > 0) MLLM_STREAM_WITH(CAPPED_QUERIES, KEPT);
+    else if (options.softcap > 0.0f) MLLM_STREAM_WITH(CAPPED_QUERIES, CAPPED);
+    else if (window > 0 || options.chunk > 0) MLLM_STREAM_WITH(QUERIES, MASKED);
+    else MLLM_STREAM_WITH(QUERIES, CAUSAL);
 #undef MLLM_STREAM_WITH
 }
 
 template <typename T, int HD>
 void launch(const void* q, int q_stride, const void* k_pages, const void* v_pages, void* out, int out_stride, const int* q_starts,
-            const int* context_lens, const int* block_tables, int max_blocks, int n_requests, int max_q_len, int max_len, int n_heads,
+            const int* context_lens, const int* block_tables, int max_blocks, int n_requests, int rows, int max_q_len, int max_len, int n_heads,
             int n_kv_heads, int page_shift, int window, float scale, ScoreOptions options, hipStream_t stream) {
 #define MLLM_STREAM_LAUNCH(QUERIES, SPLITS)                                                                                                 \
     launch_queries<T, HD, QUERIES, SPLITS>(q, q_stride, k_pages, v_pages, out, out_stride, q_starts, context_lens, block_tables, max_blocks, \
-                                           n_requests, max_q_len, n_heads, n_kv_heads, page_shift, window, scale, options, stream)
+                                           n_requests, rows, max_q_len, n_heads, n_kv_heads, page_shift, window, scale, options, stream)
     if constexpr (sizeof(T) == 4) {
         // 32-bit: the matrix cores are what a wave waits for (a tile of 32 keys is 96 products of 64 cycles for 32 queries),
         // so blocks of 32 queries, which the compute units take in turn, the ones with the most keys first
         // (blocks of 64 queries: 59.2 against 62.1 us for two prompts of 1,024 tokens x 12 heads of 64, 35.0 against 32.2 us for eight of 256)
         MLLM_STREAM_LAUNCH(32, 4);
     } else {
-        // blocks of 64 queries where they give every compute unit a block (measured: 2 x 1,024 tokens x 12 heads 15.9 against 17.2 us),
+        // blocks of 64 queries where they give every compute unit a block (measured: 2 x 1,024 tokens x 12 heads 15.9 against 17.2 us; 16.8 with the walk
+        // over the portions in front),
         // else of 32 (4 x 128 tokens on 896 cached: 9.7 against 13.0 us; 512 on 7,680: 46.7 against 66.0 us)
-        const bool wide = (long)n_heads * n_requests * ceil_div(max_q_len, 64) >= 256;
+        const bool wide = (long)n_heads * most_tiles(64, n_requests, rows, max_q_len) >= 256;
         // Eight waves a block where the block of the last queries has sixteen tiles of keys or more to walk (max_len: the longest
         // sequence after this step, or what bounds it; a window bounds the keys too) AND every block still finds a compute
         // unit of its own at once (eight waves' tiles leave room for one block a unit): a long context with few queries.
         // Measured, heads of 64: 512 queries on 7,680 cached keys 38.2 against 46.7 us with four waves; but two prompts of 1,024
         // tokens (384 blocks: a second round) 19.1 against 15.9 us, one of 4,096 64.8 against 57 us.
         const int reach = options.chunk > 0 ? min(max_len, options.chunk + 64) : (window > 0 ? min(max_len, window + options.keep + 64) : max_len);
-        const long blocks = (long)n_heads * n_requests * ceil_div(max_q_len, wide ? 64 : 32);
+        const long blocks = (long)n_heads * most_tiles(wide ? 64 : 32, n_requests, rows, max_q_len);
         bool eight = false;
         if constexpr (HD * sizeof(T) <= 128) {  // (eight waves' tiles of rows of 256 bytes do not fit a compute unit's LDS)
             eight = reach >= 16 * KEYS && blocks <= 256;

@@ -501,6 +501,47 @@ def test_decode_attention_with_the_keys_in_runs(K, monkeypatch, dtype, n_heads, 
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("lengths,contexts", [
+    ([2200, 1, 97], [0, 40, 3]),                                            # few portions, one of more than 64 tiles of 32 queries
+    ([33, 64, 65, 1, 128, 129, 31, 300], [0, 5, 0, 70, 64, 0, 1, 0]),       # eight: every lane takes a place
+    ([33, 64, 65, 1, 128, 129, 31, 300, 96], [0, 5, 0, 70, 64, 0, 1, 0, 0]),   # nine: a search
+    ([1 + (37 * i) % 70 for i in range(70)], [(11 * i) % 40 for i in range(70)]),   # more than a wave has lanes
+])
+def test_prompt_attention_finds_every_tile_of_a_padded_shape(K, dtype, lengths, contexts):
+    # The portions of a padded shape: the longest is named as all rows, and padding requests (no rows, a stored length of -1) stand between
+    # the real ones. Every real row comes out, the rows behind them are nobody's.
+    rng = np.random.default_rng(len(lengths))
+    rnd = lambda *s: bf16_round(rng.standard_normal(s)) if dtype == torch.bfloat16 else rng.standard_normal(s).astype(np.float32).astype(np.float64)
+    heads, size, page = 3, 64, 64
+    need = [-(-(c + n) // page) for c, n in zip(contexts, lengths)]
+    kp = torch.full((sum(need), heads, page, size), float("nan"), device=DEV).to(dtype)
+    vp = torch.full_like(kp, float("nan"))
+    order, tables, starts, stored, rows, refs = rng.permutation(sum(need)).tolist(), [], [0], [], [], []
+    for i, (ctx, new, blocks) in enumerate(zip(contexts, lengths, need)):
+        k, v, q = rnd(ctx + new, heads * size), rnd(ctx + new, heads * size), rnd(new, heads * size)
+        pages = [order.pop() for _ in range(blocks)]
+        slots = np.array([pages[p // page] * page + p % page for p in range(ctx + new)], dtype=np.int32)
+        K.cache_write(dev(k, dtype), dev(v, dtype), kp, vp, dev(slots, torch.int32), heads, size)
+        tables.append(pages + [-1] * (max(need) - blocks))
+        starts.append(starts[-1] + new)
+        stored.append(ctx)
+        rows.append(q)
+        refs.append(plain_paged_attention(q, k, v, heads, heads, None))
+        if i % 4 == 2:   # a padding request
+            tables.append([-1] * max(need))
+            starts.append(starts[-1])
+            stored.append(-1)
+    real, total = starts[-1], -(-(starts[-1] + 1) // 64) * 64
+    q = np.concatenate(rows + [np.zeros((total - real, heads * size))])
+    out = torch.zeros((total, heads * size), device=DEV, dtype=dtype)
+    K.paged_attention(dev(q, dtype), kp, vp, dev(np.zeros(total), torch.int32), dev(np.zeros(total), torch.int32), dev(tables, torch.int32), heads, heads, size,
+                      1.0 / math.sqrt(size), max_q_len=total, max_len=4096, q_starts=dev(starts, torch.int32), context_lens=dev(stored, torch.int32), out=out)
+    tol = 2e-5 if dtype == torch.float32 else 2e-2   # as the tests of the same kernel above
+    np.testing.assert_allclose(host(out)[:real], np.concatenate(refs), rtol=tol, atol=tol)
+    assert not host(out)[real:].any()
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize(
     "n_heads,n_kv_heads,head_size,page_size,window",
     [(3, 3, 32, 16, 0), (2, 2, 64, 64, 0), (4, 2, 64, 16, 150), (2, 1, 128, 8, 0), (2, 2, 128, 256, 0), (3, 3, 32, 32, 70),
