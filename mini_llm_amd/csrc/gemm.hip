@@ -1,8 +1,8 @@
 // Matrix products on the matrix cores: out[M,N] = act(A[M,K] . W[N,K]^T + bias[N]) (+ residual).
 //
 // W is [out, in], either row-major (rows contiguous in K: what the tied head's token table
-// already is) or in the packed layout (common.h), which the weights of the layers are kept in. 32-bit inputs use the 32-bit MFMA (no reduced-precision
-// matrix mode); bfloat16 inputs use the bf16 MFMA; sums are 32-bit in both. Replaces the
+// already is) or in the packed layout (common.h), which the weights of the layers are kept in. 32-bit inputs use the 32-bit MFMA or,
+// for many rows, the bf16 MFMA on all 24 bits of them in pieces (gemm_pieces.h); bfloat16 inputs use the bf16 MFMA; sums are 32-bit in all. Replaces the
 // reference's mult_kernel + add_bias + gelu + vector_addition (engine/src/matrixmult.cu:7-34,
 // linear.cu:9-18) and its epilogue order sum -> +bias -> activation -> residual + that
 // (engine/include/matvec_common.h:40-54).
@@ -41,6 +41,7 @@ struct Tile<bf16_t> {
 }  // namespace
 
 #include "gemm_stream.h"
+#include "gemm_pieces.h"
 
 namespace {
 
@@ -564,7 +565,7 @@ __global__ __launch_bounds__(64 * KSPLIT) void gemm_skinny_kernel(
 }
 
 template <typename T, typename OutT, int MT>
-void launch_skinny(const T* a, const T* w, bool packed, const float* bias, const float* residual, OutT* o, int M,
+void launch_skinny(const T* a, const T* w, int packed, const float* bias, const float* residual, OutT* o, int M,
                    int N, int K, int epilogue, hipStream_t stream, CacheScatter scatter = CacheScatter{}, int k_blocks = 1,
                    int x_packed = 0, int out_packed = 0) {
     constexpr int KSTEP = 4 * Tile<T>::VEC;
@@ -609,6 +610,7 @@ template <typename T>
 int tiled_k_blocks(int M, int N, int K) {
     int tiles = ceil_div(M, 128) * ceil_div(N, 64);
     int k_blocks = 1;
+    if (sizeof(T) == 4 && K % pieces::BK == 0 && N % 4 == 0) return pieces::split_blocks(ceil_div(M, 128) * 128, N, K);   // (by whole tiles of 128 rows, as the rest)
     if (sizeof(T) == 4 && tiles > 128) {
         // In 32-bit the matrix cores set the pace, and a block has two waves on each of them: what counts is that every
         // compute unit gets the same number of blocks. 192 tiles (2,048 x 768) whole keep 192 units busy for a block's
@@ -631,7 +633,7 @@ int tiled_k_blocks(int M, int N, int K) {
 }
 
 template <typename T, typename OutT, bool ALIGNED, int BM, int BN, int WAVES_M, int WAVES_N>
-void launch_tile(const T* a, const T* w, bool packed, const float* bias, const float* residual, OutT* o, int M, int N,
+void launch_tile(const T* a, const T* w, int packed, const float* bias, const float* residual, OutT* o, int M, int N,
                  int K, int epilogue, hipStream_t stream, CacheScatter scatter, int k_blocks) {
     dim3 grid(ceil_div(N, BN), ceil_div(M, BM), k_blocks);
     constexpr int PAIR = 2 * Tile<T>::BK;  // the kernel's loop takes two LDS tiles a turn
@@ -642,11 +644,17 @@ void launch_tile(const T* a, const T* w, bool packed, const float* bias, const f
 }
 
 template <typename T, typename OutT, bool ALIGNED>
-void launch_tiled(const T* a, const T* w, bool packed, const float* bias, const float* residual, OutT* o, int M, int N,
+void launch_tiled(const T* a, const T* w, int packed, const float* bias, const float* residual, OutT* o, int M, int N,
                   int K, int epilogue, hipStream_t stream, CacheScatter scatter = CacheScatter{}, int k_blocks = 1) {
     if constexpr (sizeof(T) == 2) {  // bfloat16 with many rows and a packed W: the kernel that streams its operands straight into LDS
-        if (ALIGNED && stream::takes(M, N, K, packed, scatter, sizeof(OutT))) {
+        if (ALIGNED && stream::takes(M, N, K, packed != 0, scatter, sizeof(OutT))) {
             stream::dispatch<OutT>(a, w, bias, residual, o, M, N, K, epilogue, stream, scatter, k_blocks);
+            return;
+        }
+    }
+    if constexpr (sizeof(T) == 4) {
+        if (ALIGNED && pieces::takes(a, bias, residual, o, M, N, K, ceil_div(N, 16), packed, scatter)) {
+            pieces::dispatch(a, w, bias, residual, o, M, N, K, epilogue, stream, scatter, k_blocks);
             return;
         }
     }
@@ -683,7 +691,7 @@ bool takes_few_row_kernel(int M, int N, int K) {
 }
 
 template <typename T, typename OutT>
-void launch_gemm(const void* A, const void* W, bool packed, const float* bias, const float* residual, void* out,
+void launch_gemm(const void* A, const void* W, int packed, const float* bias, const float* residual, void* out,
                  int M, int N, int K, int epilogue, int x_packed, int out_packed, hipStream_t stream) {
     const T* a = (const T*)A;
     const T* w = (const T*)W;
@@ -723,11 +731,11 @@ MLLM_API int mllm_gemm(const void* A, const void* W, int w_packed, const float* 
     MLLM_REQUIRE(residual == nullptr || out_dtype == MLLM_F32, "gemm: a residual sum is 32-bit, the output asked for is not");
     if (M == 0) return 0;
     if (in_dtype == MLLM_F32 && out_dtype == MLLM_F32)
-        launch_gemm<float, float>(A, W, w_packed != 0, bias, residual, out, M, N, K, epilogue, x_packed, out_packed, stream);
+        launch_gemm<float, float>(A, W, w_packed, bias, residual, out, M, N, K, epilogue, x_packed, out_packed, stream);
     else if (in_dtype == MLLM_BF16 && out_dtype == MLLM_BF16)
-        launch_gemm<bf16_t, bf16_t>(A, W, w_packed != 0, bias, residual, out, M, N, K, epilogue, x_packed, out_packed, stream);
+        launch_gemm<bf16_t, bf16_t>(A, W, w_packed, bias, residual, out, M, N, K, epilogue, x_packed, out_packed, stream);
     else if (in_dtype == MLLM_BF16 && out_dtype == MLLM_F32)
-        launch_gemm<bf16_t, float>(A, W, w_packed != 0, bias, residual, out, M, N, K, epilogue, x_packed, out_packed, stream);
+        launch_gemm<bf16_t, float>(A, W, w_packed, bias, residual, out, M, N, K, epilogue, x_packed, out_packed, stream);
     else
         MLLM_REQUIRE(false, "gemm: no kernel for input dtype %d with output dtype %d", in_dtype, out_dtype);
     return mllm_check_launch("gemm");
@@ -810,10 +818,10 @@ MLLM_API int mllm_gemm_split(const void* A, const void* W, int w_packed, float* 
     MLLM_REQUIRE(K % (in_dtype == MLLM_F32 ? 4 : 8) == 0, "gemm_split: K=%d is not a multiple of a 16-byte piece", K);
     if (M == 0) return 0;
 #define MLLM_SPLIT_CASE(T)                                                                                                     \
-    if (M <= 16) launch_skinny<T, float, 1>((const T*)A, (const T*)W, w_packed != 0, nullptr, nullptr, partials, M, N, K, 0, stream, CacheScatter{}, k_blocks, x_packed);      \
-    else if (M <= 32) launch_skinny<T, float, 2>((const T*)A, (const T*)W, w_packed != 0, nullptr, nullptr, partials, M, N, K, 0, stream, CacheScatter{}, k_blocks, x_packed); \
-    else if (M <= 64) launch_skinny<T, float, 4>((const T*)A, (const T*)W, w_packed != 0, nullptr, nullptr, partials, M, N, K, 0, stream, CacheScatter{}, k_blocks, x_packed); \
-    else launch_tiled<T, float, true>((const T*)A, (const T*)W, w_packed != 0, nullptr, nullptr, partials, M, N, K, 0, stream, CacheScatter{}, k_blocks);
+    if (M <= 16) launch_skinny<T, float, 1>((const T*)A, (const T*)W, w_packed, nullptr, nullptr, partials, M, N, K, 0, stream, CacheScatter{}, k_blocks, x_packed);      \
+    else if (M <= 32) launch_skinny<T, float, 2>((const T*)A, (const T*)W, w_packed, nullptr, nullptr, partials, M, N, K, 0, stream, CacheScatter{}, k_blocks, x_packed); \
+    else if (M <= 64) launch_skinny<T, float, 4>((const T*)A, (const T*)W, w_packed, nullptr, nullptr, partials, M, N, K, 0, stream, CacheScatter{}, k_blocks, x_packed); \
+    else launch_tiled<T, float, true>((const T*)A, (const T*)W, w_packed, nullptr, nullptr, partials, M, N, K, 0, stream, CacheScatter{}, k_blocks);
     if (in_dtype == MLLM_F32) { MLLM_SPLIT_CASE(float) } else { MLLM_SPLIT_CASE(bf16_t) }
 #undef MLLM_SPLIT_CASE
     return mllm_check_launch("gemm_split");
@@ -837,10 +845,10 @@ MLLM_API int mllm_gemm_qkv_cache(const void* A, const void* W, int w_packed, con
     MLLM_REQUIRE(!x_packed || mllm_gemm_takes_packed_rows(M, N, K, dtype),
                  "gemm_qkv_cache: rows in the packed layout are for the kernel for few rows, which M=%d N=%d K=%d do not take", M, N, K);
 #define MLLM_QKV_CASE(T)                                                                                              \
-    if (!takes_few_row_kernel<T>(M, N, K)) launch_tiled<T, T, true>((const T*)A, (const T*)W, w_packed != 0, bias, nullptr, (T*)out_q, M, N, K, 0, stream, scatter); \
-    else if (M <= 16) launch_skinny<T, T, 1>((const T*)A, (const T*)W, w_packed != 0, bias, nullptr, (T*)out_q, M, N, K, 0, stream, scatter, 1, x_packed);      \
-    else if (M <= 32) launch_skinny<T, T, 2>((const T*)A, (const T*)W, w_packed != 0, bias, nullptr, (T*)out_q, M, N, K, 0, stream, scatter, 1, x_packed); \
-    else launch_skinny<T, T, 4>((const T*)A, (const T*)W, w_packed != 0, bias, nullptr, (T*)out_q, M, N, K, 0, stream, scatter, 1, x_packed);
+    if (!takes_few_row_kernel<T>(M, N, K)) launch_tiled<T, T, true>((const T*)A, (const T*)W, w_packed, bias, nullptr, (T*)out_q, M, N, K, 0, stream, scatter); \
+    else if (M <= 16) launch_skinny<T, T, 1>((const T*)A, (const T*)W, w_packed, bias, nullptr, (T*)out_q, M, N, K, 0, stream, scatter, 1, x_packed);      \
+    else if (M <= 32) launch_skinny<T, T, 2>((const T*)A, (const T*)W, w_packed, bias, nullptr, (T*)out_q, M, N, K, 0, stream, scatter, 1, x_packed); \
+    else launch_skinny<T, T, 4>((const T*)A, (const T*)W, w_packed, bias, nullptr, (T*)out_q, M, N, K, 0, stream, scatter, 1, x_packed);
     if (dtype == MLLM_F32) { MLLM_QKV_CASE(float) } else { MLLM_QKV_CASE(bf16_t) }
 #undef MLLM_QKV_CASE
     return mllm_check_launch("gemm_qkv_cache");
@@ -879,13 +887,17 @@ int check_experts(const char* what, int entries, int max_tiles, int units, int w
 // hidden [entries, units]: the gate unit of row a_row[i] of x [.., width] with its expert's matrices, W [n_experts * 2 * units, width] packed, an
 // expert's rows 32 gate rows and 32 up rows in turn; units a multiple of 64. tiles / n_tiles / max_tiles: see ExpertTiles.
 MLLM_API int mllm_experts_up(const void* x, const void* W, void* hidden, const int* tiles, const int* n_tiles, const int* a_row, const float* weight, int entries,
-                             int max_tiles, int units, int width, float limit, float alpha, float shift, int weigh_input, int dtype, hipStream_t stream) {
+                             int max_tiles, int experts, int units, int width, float limit, float alpha, float shift, int weigh_input, int w_packed, int dtype,
+                             hipStream_t stream) {
     if (int status = check_experts("experts_up", entries, max_tiles, units, width, dtype)) return status;
     MLLM_REQUIRE(x && W && hidden && tiles && n_tiles && a_row && weight && limit > 0.0f && ((uintptr_t)tiles & 15) == 0, "experts_up: a missing operand");
     if (entries == 0) return 0;
     const stream::ExpertTiles<true> group{(const int4*)tiles, n_tiles, a_row, nullptr, weight, GateUnit{limit, alpha, shift}, weigh_input};
     if (dtype == MLLM_F32) {
-        if (width % 4 == 0) launch_tiled_experts<float, float, true>(x, W, hidden, entries, max_tiles, 2 * units, width, group, stream);
+        const int matrix_tiles = experts * ceil_div(2 * units, 16);
+        if (pieces::takes(x, nullptr, nullptr, hidden, entries + 65, 2 * units, width, matrix_tiles, w_packed, CacheScatter{}))   // (whatever the rows: the kernel for few is another)
+            pieces::launch_grouped((const float*)x, (const float*)W, (float*)hidden, entries, max_tiles, 2 * units, width, matrix_tiles, group, stream);
+        else if (width % 4 == 0) launch_tiled_experts<float, float, true>(x, W, hidden, entries, max_tiles, 2 * units, width, group, stream);
         else launch_tiled_experts<float, float, false>(x, W, hidden, entries, max_tiles, 2 * units, width, group, stream);
     } else if (width % 64 == 0) {
         stream::launch_grouped<bf16_t, EXPERT_TILE, 128, 2, 2, 3>((const bf16_t*)x, (const bf16_t*)W, (bf16_t*)hidden, entries, max_tiles, 2 * units, width, group, stream);
@@ -899,13 +911,16 @@ MLLM_API int mllm_experts_up(const void* x, const void* W, void* hidden, const i
 
 // out row out_row[i] = hidden row i . its expert's down matrix^T, 32-bit; W packed, every expert's [width, units] filled up to whole sixteens of rows.
 MLLM_API int mllm_experts_down(const void* hidden, const void* W, float* out, const int* tiles, const int* n_tiles, const int* out_row, int entries, int max_tiles,
-                               int units, int width, int dtype, hipStream_t stream) {
+                               int experts, int units, int width, int w_packed, int dtype, hipStream_t stream) {
     if (int status = check_experts("experts_down", entries, max_tiles, units, width, dtype)) return status;
     MLLM_REQUIRE(hidden && W && out && tiles && n_tiles && out_row && ((uintptr_t)tiles & 15) == 0, "experts_down: a missing operand");
     if (entries == 0) return 0;
     const stream::ExpertTiles<false> group{(const int4*)tiles, n_tiles, nullptr, out_row, nullptr, GateUnit{1.0f, 1.0f, 0.0f}, 0};
     if (dtype == MLLM_F32) {
-        launch_tiled_experts<float, float, true>(hidden, W, out, entries, max_tiles, width, units, group, stream);
+        const int matrix_tiles = experts * ceil_div(width, 16);
+        if (pieces::takes(hidden, nullptr, nullptr, out, entries + 65, width, units, matrix_tiles, w_packed, CacheScatter{}))
+            pieces::launch_grouped((const float*)hidden, (const float*)W, out, entries, max_tiles, width, units, matrix_tiles, group, stream);
+        else launch_tiled_experts<float, float, true>(hidden, W, out, entries, max_tiles, width, units, group, stream);
     } else if (width % 8 != 0) {
         launch_tiled_experts<bf16_t, float, true>(hidden, W, out, entries, max_tiles, width, units, group, stream);
     } else {

@@ -1,0 +1,350 @@
+// The 32-bit product for many rows on the bfloat16 matrix cores. Included by gemm.hip.
+//
+// A 32-bit number is the sum of three bfloat16 ones, exactly (eight bits each, cut off and not rounded, so that all three have its sign and none
+// overflows), and a product of two such numbers is the sum of nine products of pieces, each exact in 32-bit. The six largest reach down to the 24th bit;
+// the matrix instruction for bfloat16 does in 32 cycles sixteen times the work that the 32-bit one does in 64, so six of them are 2.7 times faster, and
+// there are fewer roundings of a running sum (six for sixteen numbers of K instead of eight). Measured against 64-bit sums over rows of 768 to 3,072
+// normally distributed numbers: 4.3e-7 to 8.7e-7 of the result's norm, 5.0e-7 to 9.9e-7 with the 32-bit instruction.
+//
+// W's pieces are laid out once, when the matrix is packed (common.h: packed_pieces): the chunks of the packed layout for bfloat16, the three of a k-step
+// behind each other. A's rows come as they are, and a wave splits the fragments it has read.
+// A block of four waves owns BM x BN outputs and walks K in tiles of 32: rows of A and chunks of W go from memory straight into LDS
+// (global_load_lds_dwordx4), one tile ahead of the products, in two stages. The stages leave room for two blocks a compute unit: one's splitting,
+// fragment reads and barriers run under the other's products. Fragment reads are inline assembly with waits of their own: through the compiler each
+// would wait for the loads into LDS that are under way.
+#pragma once
+
+namespace pieces {
+
+typedef int i32x4 __attribute__((ext_vector_type(4)));
+
+constexpr int BK = 32;   // numbers of K in a tile
+
+template <int BM, int BN>
+constexpr int stage_bytes() {
+    return BM * BK * 4 + BN / 16 * 3 * 1024;
+}
+
+template <int OFFSET>
+__device__ __forceinline__ void ask(i32x4& to, unsigned address) {
+    asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(to) : "v"(address), "n"(OFFSET));
+}
+__device__ __forceinline__ void landed(i32x4& first) { asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(first)); }
+__device__ __forceinline__ void this_too(i32x4& fragment) { asm volatile("" : "+v"(fragment)); }
+
+// Eight numbers -> three operands of pieces.
+__device__ __forceinline__ void split(const i32x4 (&raw)[2], bf16x8 (&out)[3], float& largest) {
+    uint32_t rest[8];
+#pragma unroll
+    for (int e = 0; e < 8; e++) rest[e] = (uint32_t)raw[e / 4][e % 4];
+#pragma unroll
+    for (int e = 0; e < 8; e += 2) largest = fmaxf(fmaxf(fabsf(__builtin_bit_cast(float, rest[e])), fabsf(__builtin_bit_cast(float, rest[e + 1]))), largest);
+#pragma unroll
+    for (int p = 0; p < 3; p++) {
+        uint32_t pairs[4];
+#pragma unroll
+        for (int e = 0; e < 4; e++) pairs[e] = __builtin_amdgcn_perm(rest[2 * e + 1], rest[2 * e], 0x07060302);   // the upper halves of two
+        out[p] = *reinterpret_cast<bf16x8*>(pairs);
+        if (p < 2) {
+#pragma unroll
+            for (int e = 0; e < 8; e++) rest[e] = __builtin_bit_cast(uint32_t, __builtin_bit_cast(float, rest[e]) - __builtin_bit_cast(float, rest[e] & 0xffff0000u));
+        }
+    }
+}
+
+// The whole product (Group: stream::Whole) or one over rows grouped by expert (stream::ExpertTiles, a one-dimensional grid). W: packed, its pieces behind its
+// `matrix_tiles` row tiles. gridDim.z blocks along K take k_per_block of it each (a multiple of 32) and leave partial products.
+// W is the first operand of the matrix instruction, so that a lane holds four consecutive columns of a row; the results pass through LDS 32 rows at a time
+// and leave in whole rows of a wave's columns. (Stored from where the sums lie, number by number, a block of 128 x 128 took 12 us behind its loop.)
+template <int BM, int BN, int WAVES_M, int WAVES_N, typename Group>
+__global__ __launch_bounds__(64 * WAVES_M * WAVES_N, 2) void gemm_pieces_kernel(const float* __restrict__ A, const float* __restrict__ W, const float* __restrict__ bias,
+                                                                               const float* __restrict__ residual, float* __restrict__ out, int M, int N, int K, int matrix_tiles,
+                                                                               int epilogue, CacheScatter scatter, int k_per_block, Group group) {
+    constexpr int WAVES = WAVES_M * WAVES_N, STAGE = stage_bytes<BM, BN>(), A_BYTES = BM * BK * 4;
+    constexpr int WM = BM / WAVES_M, WN = BN / WAVES_N, TM = WM / 32, TN = WN / 32;
+    constexpr int A_LOADS = BM / 8 / WAVES, W_CHUNKS = BN / 16 * 3, W_LOADS = W_CHUNKS / WAVES;
+    static_assert(TM >= 1 && TN >= 1 && BM / 8 % WAVES == 0 && W_CHUNKS % WAVES == 0, "every wave asks for as much");
+    extern __shared__ __attribute__((aligned(16))) unsigned char piece_lds[];
+    const int lane = threadIdx.x % WAVE, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+    const int wave_m = wave / WAVES_N, wave_n = wave % WAVES_N, half = lane / 32, lane32 = lane % 32;
+    const int row_tiles = ceil_div(N, 16), k_steps = ceil_div(K, BK);
+    int m0 = blockIdx.y * BM, n0 = blockIdx.x * BN, m_end = M, first_tile = 0;
+    if constexpr (Group::GROUPED) {
+        stream::GroupTile tile;
+        if (!stream::group_tile(group, N, BN, tile)) return;  // (the whole block leaves)
+        m0 = tile.m0, m_end = tile.m_end, n0 = tile.n0;
+        first_tile = tile.expert * row_tiles;
+    }
+    const int k_begin = blockIdx.z * k_per_block, k_end = min(K, k_begin + k_per_block);
+    out += (size_t)blockIdx.z * M * N;
+    const unsigned char* w_pieces = reinterpret_cast<const unsigned char*>(W) + packed_pieces_at(matrix_tiles, packed_k_steps<float>(K));
+    auto a_row = [&](int r) {   // of the block's tile; beyond the last: that row again, never stored
+        const int row = min(m0 + r, m_end - 1);
+        if constexpr (Group::GROUPED) return group.a_row ? group.a_row[row] : row;
+        else return row;
+    };
+
+    // what this lane asks for: eight lanes the 128 bytes a row of A has in a tile, its 16-byte pieces turned by the row (so that the fragment reads of
+    // sixteen rows, two of which fill all banks once, meet different ones); a chunk of W as it lies
+    unsigned a_from[A_LOADS], w_from[W_LOADS];
+#pragma unroll
+    for (int l = 0; l < A_LOADS; l++) {
+        const int row = (wave + l * WAVES) * 8 + lane / 8;
+        a_from[l] = (unsigned)a_row(row) * (unsigned)K * 4u + (unsigned)(((lane % 8) ^ (row / 2 % 8)) * 16);
+    }
+#pragma unroll
+    for (int l = 0; l < W_LOADS; l++) {
+        const int chunk = wave + l * WAVES, row_tile = first_tile + min(n0 / 16 + chunk / 3, row_tiles - 1);
+        w_from[l] = ((unsigned)row_tile * (unsigned)k_steps * 3u + (unsigned)(chunk % 3)) * 1024u + lane * 16u;
+    }
+    const unsigned char* a_tile = reinterpret_cast<const unsigned char*>(A + k_begin);
+    const unsigned char* w_tile = w_pieces + (size_t)(k_begin / BK) * 3072;
+    auto issue = [&](int stage) {   // the next tile
+        unsigned char* place = piece_lds + stage * STAGE;
+#pragma unroll
+        for (int l = 0; l < A_LOADS; l++)
+            __builtin_amdgcn_global_load_lds((const void __attribute__((address_space(1)))*)(a_tile + a_from[l]),
+                                             (void __attribute__((address_space(3)))*)(place + (wave + l * WAVES) * 1024), 16, 0, 0);
+#pragma unroll
+        for (int l = 0; l < W_LOADS; l++)
+            __builtin_amdgcn_global_load_lds((const void __attribute__((address_space(1)))*)(w_tile + w_from[l]),
+                                             (void __attribute__((address_space(3)))*)(place + A_BYTES + (wave + l * WAVES) * 1024), 16, 0, 0);
+        a_tile += BK * 4;
+        w_tile += 3072;
+    };
+
+    f32x16 acc[TN][TM];
+#pragma unroll
+    for (int j = 0; j < TN; j++)
+#pragma unroll
+        for (int i = 0; i < TM; i++)
+#pragma unroll
+            for (int v = 0; v < 16; v++) acc[j][i][v] = 0.0f;
+    const unsigned base = (unsigned)(size_t)(const __attribute__((address_space(3))) unsigned char*)piece_lds;
+    unsigned a_at[2][2];   // [step of 16][piece]
+#pragma unroll
+    for (int kk = 0; kk < 2; kk++)
+#pragma unroll
+        for (int q = 0; q < 2; q++) a_at[kk][q] = base + (wave_m * WM + lane32) * 128 + (((kk * 4 + half * 2 + q) ^ (lane32 / 2 % 8)) * 16);
+    const unsigned w_at = base + A_BYTES + (wave_n * TN * 2 + lane32 / 16) * 3072 + half * 256 + (lane % 16) * 16;
+
+    float largest = 0.0f;   // the largest magnitude this lane has met in A
+    const int tiles = (k_end - k_begin + BK - 1) / BK;
+    if (tiles > 0) issue(0);
+    for (int t = 0; t < tiles; t++) {
+        // this wave's loads of the tile have landed; behind the barrier everybody's have, and nobody reads the other stage any more
+        __builtin_amdgcn_s_waitcnt(0);
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_sched_barrier(0);
+        if (t + 1 < tiles) issue((t + 1) & 1);
+        const unsigned stage = (t & 1) * STAGE;
+        i32x4 raw[2][TM][2], w[2][3][TN];
+        auto ask_step = [&](auto step) {
+            constexpr int kk = decltype(step)::value;
+            stream::static_for<TM>([&](auto i) {
+                ask<i * 32 * 128>(raw[kk][i][0], a_at[kk][0] + stage);
+                ask<i * 32 * 128>(raw[kk][i][1], a_at[kk][1] + stage);
+            });
+            stream::static_for<3>([&](auto p) { stream::static_for<TN>([&](auto j) { ask<j * 2 * 3072 + p * 1024 + kk * 512>(w[kk][p][j], w_at + stage); }); });
+        };
+        auto wait_step = [&](int kk) {
+            landed(raw[kk][0][0]);
+#pragma unroll
+            for (int i = 0; i < TM; i++) this_too(raw[kk][i][0]), this_too(raw[kk][i][1]);
+#pragma unroll
+            for (int p = 0; p < 3; p++)
+#pragma unroll
+                for (int j = 0; j < TN; j++) this_too(w[kk][p][j]);
+        };
+        bf16x8 a[2][TM][3];
+        auto multiply = [&](int kk) {
+            constexpr int OF_A[6] = {2, 0, 1, 1, 0, 0}, OF_W[6] = {0, 2, 1, 0, 1, 0};   // the smallest products first
+#pragma unroll
+            for (int c = 0; c < 6; c++)
+#pragma unroll
+                for (int i = 0; i < TM; i++)
+#pragma unroll
+                    for (int j = 0; j < TN; j++)
+                        acc[j][i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*reinterpret_cast<const bf16x8*>(&w[kk][OF_W[c]][j]), a[kk][i][OF_A[c]], acc[j][i], 0, 0, 0);
+        };
+        ask_step(std::integral_constant<int, 0>{});
+        wait_step(0);
+        ask_step(std::integral_constant<int, 1>{});
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int i = 0; i < TM; i++) split(raw[0][i], a[0][i], largest);
+        multiply(0);
+        wait_step(1);
+#pragma unroll
+        for (int i = 0; i < TM; i++) split(raw[1][i], a[1][i], largest);
+        multiply(1);
+    }
+
+    // An infinity has no pieces: a wave that met one (its own rows', or anywhere in W) takes its sums again, number by number.
+    const int infinite = *reinterpret_cast<const int*>(w_pieces + packed_pieces_bytes(matrix_tiles, K));
+    const int row0 = m0 + wave_m * WM, col0 = n0 + wave_n * WN;
+    __syncthreads();   // the slabs below lie where the tiles did (and a flag shared through LDS would leave no room for two blocks of 80 KiB)
+    if (__any(largest == INFINITY) || infinite) {
+        const float* w_rows = W + packed_offset<float>(first_tile, 0, packed_k_steps<float>(K), 0);
+#pragma unroll 1
+        for (int v = 0; v < 16 * TM * TN; v++) {
+            const int j = v / (16 * TM), i = v / 16 % TM, u = v % 16;
+            const int r = wave_m * WM + i * 32 + lane32, col = col0 + j * 32 + 8 * (u / 4) + 4 * half + (u % 4);
+            float sum = 0.0f;
+            if (m0 + r < m_end && col < N) {
+                const float* row = A + (size_t)a_row(r) * K;
+                for (int k = k_begin; k < k_end; k++) sum = __builtin_fmaf(row[k], w_rows[packed_element<float>(col, k, K)], sum);
+            }
+#pragma unroll
+            for (int x = 0; x < 16 * TM * TN; x++) acc[x / (16 * TM)][x / 16 % TM][x % 16] = x == v ? sum : acc[x / (16 * TM)][x / 16 % TM][x % 16];
+        }
+    }
+
+    // 32 rows of the wave's columns at a time through LDS of its own, 16 bytes of padding a row. GATED: 32 gate and 32 up columns become 32 units.
+    constexpr int OUT_COLS = Group::GATED ? WN / 2 : WN, SLAB_ROW = OUT_COLS + 4, LANES_A_ROW = OUT_COLS / 4, ROWS = WAVE / LANES_A_ROW;
+    static_assert(!Group::GATED || TN % 2 == 0, "a wave holds gate and up columns of the same units");
+    static_assert(WAVES * 32 * SLAB_ROW * 4 <= 2 * STAGE, "the slabs fit the stages");
+    float* const slab = reinterpret_cast<float*>(piece_lds) + wave * 32 * SLAB_ROW;
+    const int out_cols = Group::GATED ? N / 2 : N, out_col = (Group::GATED ? col0 / 2 : col0) + (lane % LANES_A_ROW) * 4;
+    // a q/k/v projection: four columns lie in one head (the host sees to it), a lane's columns are the same in every row
+    const int width = scatter.enabled ? scatter.q_width : out_cols;
+    float* pages = nullptr;
+    int kv_head = 0, d = 0;
+    if (!Group::GROUPED && scatter.enabled && out_col >= scatter.q_width && out_col < N) {
+        int c = out_col - scatter.q_width;
+        pages = (float*)(c < scatter.kv_width ? scatter.k_pages : scatter.v_pages);
+        if (c >= scatter.kv_width) c -= scatter.kv_width;
+        kv_head = c / scatter.head_size, d = c % scatter.head_size;
+    }
+    auto leave = [&](auto kind) {
+        constexpr int KIND = decltype(kind)::value;
+#pragma unroll
+        for (int i = 0; i < TM; i++) {
+            float in_weight = 1.0f, out_weight = 1.0f;
+            if constexpr (Group::GATED) {
+                const float weight = group.weight[min(row0 + i * 32 + lane32, m_end - 1)];
+                in_weight = group.weigh_input ? weight : 1.0f, out_weight = group.weigh_input ? 1.0f : weight;
+            }
+#pragma unroll
+            for (int j = 0; j < TN; j += Group::GATED ? 2 : 1)
+#pragma unroll
+                for (int g = 0; g < 4; g++) {
+                    f32x4 value;
+                    if constexpr (Group::GATED) {
+#pragma unroll
+                        for (int e = 0; e < 4; e++)
+                            value[e] = gated(acc[j][i][4 * g + e] * in_weight, acc[j + 1][i][4 * g + e] * in_weight, group.unit) * out_weight;
+                    } else {
+                        const int col = col0 + j * 32 + 8 * g + 4 * half;
+                        f32x4 b = {0.0f, 0.0f, 0.0f, 0.0f};
+                        if (!Group::GROUPED && bias && col < N) b = *reinterpret_cast<const f32x4*>(bias + col);
+#pragma unroll
+                        for (int e = 0; e < 4; e++) value[e] = apply_activation<KIND>(acc[j][i][4 * g + e] + b[e]);
+                    }
+                    *reinterpret_cast<f32x4*>(slab + lane32 * SLAB_ROW + (Group::GATED ? j / 2 : j) * 32 + 8 * g + 4 * half) = value;
+                }
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma unroll
+            for (int r = 0; r < 32 / ROWS; r++) {
+                const int in_slab = r * ROWS + lane / LANES_A_ROW, row = row0 + i * 32 + in_slab;
+                f32x4 value = *reinterpret_cast<const f32x4*>(slab + in_slab * SLAB_ROW + (lane % LANES_A_ROW) * 4);
+                if (row >= m_end || out_col >= out_cols) continue;
+                if (!Group::GROUPED && pages) {
+                    const int slot = scatter.slots[row];
+                    if (slot < 0) continue;
+                    const int page = slot >> scatter.page_shift, offset = slot & ((1 << scatter.page_shift) - 1);
+                    *reinterpret_cast<f32x4*>(pages + ((((size_t)page * scatter.n_kv_heads + kv_head) << scatter.page_shift) + offset) * scatter.head_size + d) = value;
+                    continue;
+                }
+                int to = row;
+                if constexpr (Group::GROUPED && !Group::GATED) to = group.out_row ? group.out_row[row] : row;
+                const size_t at = (size_t)to * width + out_col;
+                if (!Group::GROUPED && residual) value = *reinterpret_cast<const f32x4*>(residual + at) + value;
+                *reinterpret_cast<f32x4*>(out + at) = value;
+            }
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        }
+    };
+    using std::integral_constant;
+    if (Group::GROUPED || epilogue == MLLM_EPI_NONE) leave(integral_constant<int, MLLM_EPI_NONE>{});
+    else if (epilogue == MLLM_EPI_GELU_TANH) leave(integral_constant<int, MLLM_EPI_GELU_TANH>{});
+    else if (epilogue == MLLM_EPI_GELU_ERF) leave(integral_constant<int, MLLM_EPI_GELU_ERF>{});
+    else leave(integral_constant<int, MLLM_EPI_SQUARED_RELU>{});
+}
+
+// Whether a product takes this kernel: a W that was packed with its pieces, more rows than the kernel for few rows takes, whole tiles of K, whole pieces of
+// 16 bytes in every row and pointer, operands whose bytes a 32-bit offset reaches, and in a q/k/v projection four columns never in two heads.
+inline bool takes(const void* a, const void* bias, const void* residual, const void* out, int M, int N, int K, int matrix_tiles, int packed, const CacheScatter& scatter) {
+    if (packed != PACKED_WITH_PIECES || M <= 64 || K % BK != 0 || N % 4 != 0) return false;
+    if (((size_t)a | (size_t)bias | (size_t)residual | (size_t)out) % 16 != 0) return false;
+    if ((long long)M * K * 4 >= (1LL << 32) || packed_pieces_bytes(matrix_tiles, K) >= (1LL << 32)) return false;
+    return !scatter.enabled || (scatter.q_width % 4 == 0 && scatter.kv_width % 4 == 0 && scatter.head_size % 4 == 0 && (((size_t)scatter.k_pages | (size_t)scatter.v_pages) % 16) == 0);
+}
+
+template <int BM, int BN, int WAVES_M, int WAVES_N, typename Group>
+void launch(const float* a, const float* w, const float* bias, const float* residual, float* o, int M, int N, int K, int matrix_tiles, int epilogue, hipStream_t stream,
+            const CacheScatter& scatter, int k_blocks, dim3 grid, const Group& group) {
+    constexpr int LDS_BYTES = 2 * stage_bytes<BM, BN>();
+    static bool raised = false;  // per instantiation: the limit on dynamic LDS is a property of the kernel
+    if (!raised && LDS_BYTES > 60 * 1024)  // (if this fails the launch below fails too, and the entry point reports that)
+        raised = hipFuncSetAttribute((const void*)gemm_pieces_kernel<BM, BN, WAVES_M, WAVES_N, Group>, hipFuncAttributeMaxDynamicSharedMemorySize, LDS_BYTES) == hipSuccess;
+    const int k_per_block = ceil_div(ceil_div(K, k_blocks), BK) * BK;
+    mllm_count_kernel(MLLM_K_GEMM_TILED);
+    gemm_pieces_kernel<BM, BN, WAVES_M, WAVES_N, Group><<<grid, 64 * WAVES_M * WAVES_N, LDS_BYTES, stream>>>(a, w, bias, residual, o, M, N, K, matrix_tiles, epilogue, scatter,
+                                                                                                          k_per_block, group);
+}
+
+template <int BM, int BN, int WAVES_M, int WAVES_N>
+void launch_whole(const float* a, const float* w, const float* bias, const float* residual, float* o, int M, int N, int K, int epilogue, hipStream_t stream, const CacheScatter& scatter,
+                  int k_blocks) {
+    launch<BM, BN, WAVES_M, WAVES_N>(a, w, bias, residual, o, M, N, K, ceil_div(N, 16), epilogue, stream, scatter, k_blocks, dim3(ceil_div(N, BN), ceil_div(M, BM), k_blocks), stream::Whole{});
+}
+
+// The tiles, and what a tile of K costs a block in microseconds: alone on its compute unit, and beside others (a round of 256 blocks). Measured over
+// 130 to 8,192 rows at GPT-2's widths. A compute unit brings most out of 128 x 128; narrow outputs and few rows fill the chip with smaller ones.
+struct Choice {
+    int bm, bn;
+    float alone, shared;
+};
+constexpr Choice CHOICES[3] = {{128, 128, 1.27f, 1.28f}, {128, 64, 0.83f, 0.72f}, {64, 64, 0.50f, 0.41f}};
+
+// Microseconds of a product cut into k_blocks along K with the best of the tiles (`best`): the rounds of blocks, the start and end of a block, and the sums
+// that are written (6 TB/s). Within a tenth of what was measured from 2,048 x 768 x 768 (24.4 us whole, 20.3 in two) to 2,048 x 768 x 3,072 (78 whole,
+// 58 in four, 67 in eight) and 130 x 768 x 768 (14.5 whole, 5.1 in six).
+inline float cost(int M, int N, int K, int k_blocks, int& best) {
+    float best_cost = 0.0f;
+    for (int c = 0; c < 3; c++) {
+        const int rounds = (int)(((long long)ceil_div(M, CHOICES[c].bm) * ceil_div(N, CHOICES[c].bn) * k_blocks + 255) / 256), tiles = ceil_div(ceil_div(K, k_blocks), BK);
+        const float us = tiles * (rounds == 1 ? CHOICES[c].alone : rounds * CHOICES[c].shared) + 3.0f + (float)M * N * k_blocks * (4.0f / 6e6f);
+        if (c == 0 || us < best_cost) best = c, best_cost = us;
+    }
+    return best_cost;
+}
+
+inline void dispatch(const float* a, const float* w, const float* bias, const float* residual, float* o, int M, int N, int K, int epilogue, hipStream_t stream,
+                     const CacheScatter& scatter, int k_blocks) {
+    int best = 0;
+    cost(M, N, K, k_blocks, best);
+    if (best == 0) launch_whole<128, 128, 2, 2>(a, w, bias, residual, o, M, N, K, epilogue, stream, scatter, k_blocks);
+    else if (best == 1) launch_whole<128, 64, 4, 1>(a, w, bias, residual, o, M, N, K, epilogue, stream, scatter, k_blocks);
+    else launch_whole<64, 64, 2, 2>(a, w, bias, residual, o, M, N, K, epilogue, stream, scatter, k_blocks);
+}
+
+// Into how many partial products a product with sums to be taken by whoever reads them is cut: they are read once more there.
+inline int split_blocks(int M, int N, int K) {
+    int best = 1, tile = 0;
+    float best_cost = 0.0f;
+    for (int cuts = 1; cuts <= 8 && (cuts == 1 || K >= 4 * BK * cuts); cuts++) {
+        const float us = cost(M, N, K, cuts, tile) + (float)M * N * cuts * (4.0f / 6e6f);
+        if (cuts == 1 || us < best_cost) best = cuts, best_cost = us;
+    }
+    return best;
+}
+
+// The same over rows grouped by expert: a tile of the lists is 128 entries.
+template <typename Group>
+void launch_grouped(const float* a, const float* w, float* o, int entries, int max_tiles, int N, int K, int matrix_tiles, const Group& group, hipStream_t stream) {
+    launch<128, 128, 2, 2>(a, w, nullptr, nullptr, o, entries, N, K, matrix_tiles, MLLM_EPI_NONE, stream, CacheScatter{}, 1, dim3(ceil_div(max_tiles * ceil_div(N, 128), 8) * 8), group);
+}
+
+}  // namespace pieces

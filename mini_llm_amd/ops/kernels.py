@@ -180,10 +180,11 @@ def add(a, b, out=None):
 class PackedMatrix:
     """A weight matrix [rows (out), cols (in)] in the packed layout of the matrix kernels: chunks
     of 16 rows x 64 bytes, each chunk's 16-byte pieces in the order the lanes of a wave take them
-    as matrix-core operands, zeros beyond the matrix. ``data`` is the flat device tensor."""
+    as matrix-core operands, zeros beyond the matrix. ``data`` is the flat device tensor. ``pieces``: a 32-bit matrix whose
+    bfloat16 pieces (csrc/gemm_pieces.h) lie behind it in the same allocation, for the products of many rows."""
 
-    def __init__(self, data: torch.Tensor, rows: int, cols: int):
-        self.data, self.rows, self.cols = data, rows, cols
+    def __init__(self, data: torch.Tensor, rows: int, cols: int, pieces: bool = False):
+        self.data, self.rows, self.cols, self.pieces = data, rows, cols, pieces
 
     @property
     def shape(self):
@@ -239,16 +240,20 @@ def pack_matrix(src, dtype=None, transpose=False) -> PackedMatrix:
     rows, cols = (src.shape[1], src.shape[0]) if transpose else src.shape
     _require(rows > 0 and cols > 0, "an empty matrix cannot be packed")
     lib = library()
-    data = torch.empty((lib.mllm_packed_elements(rows, cols, _code(dtype)),), dtype=dtype, device=src.device)
+    elements = lib.mllm_packed_elements(rows, cols, _code(dtype))
+    pieces = dtype == torch.float32
+    data = torch.empty((elements + (lib.mllm_pieces_bytes(rows, cols) // 4 if pieces else 0),), dtype=dtype, device=src.device)
     check(lib.mllm_pack_matrix(_ptr(src), _ptr(data), rows, cols, _code(src.dtype), _code(dtype), int(bool(transpose)), _stream()))
-    return PackedMatrix(data, rows, cols)
+    if pieces:
+        check(lib.mllm_pack_pieces(_ptr(data), rows, cols, _stream()))
+    return PackedMatrix(data[:elements], rows, cols, pieces)
 
 
 def _matrix(weight, name, dtype):
     """(pointer, packed flag, rows, cols) of a weight given row-major or packed."""
     if isinstance(weight, PackedMatrix):
         _device_tensor(weight.data, name, dtype, 1)
-        return _ptr(weight.data), 1, weight.rows, weight.cols
+        return _ptr(weight.data), 2 if weight.pieces else 1, weight.rows, weight.cols
     _device_tensor(weight, name, dtype, 2)
     return _ptr(weight), 0, weight.shape[0], weight.shape[1]
 
@@ -1451,9 +1456,10 @@ def grouped_experts(x, picks: Picks, up: PackedMatrix, down: PackedMatrix, n_exp
     weights, n_tiles = lists[4 * max_tiles + 2 * entries : 4 * max_tiles + 3 * entries], lists[4 * max_tiles + 3 * entries :]
     check(lib.mllm_expert_lists(_ptr(picks.experts), _ptr(picks.weights), n, top, int(n_experts), tile, _ptr(rows), _ptr(places), _ptr(weights), _ptr(tiles), _ptr(n_tiles),
                                 _stream()))
-    check(lib.mllm_experts_up(_ptr(x), _ptr(up.data), _ptr(hidden), _ptr(tiles), _ptr(n_tiles), _ptr(rows), _ptr(weights), entries, max_tiles, int(units), width, *unit, code,
-                              _stream()))
-    check(lib.mllm_experts_down(_ptr(hidden), _ptr(down.data), _ptr(out), _ptr(tiles), _ptr(n_tiles), _ptr(places), entries, max_tiles, int(units), width, code, _stream()))
+    check(lib.mllm_experts_up(_ptr(x), _ptr(up.data), _ptr(hidden), _ptr(tiles), _ptr(n_tiles), _ptr(rows), _ptr(weights), entries, max_tiles, int(n_experts), int(units), width, *unit,
+                              2 if up.pieces else 1, code, _stream()))
+    check(lib.mllm_experts_down(_ptr(hidden), _ptr(down.data), _ptr(out), _ptr(tiles), _ptr(n_tiles), _ptr(places), entries, max_tiles, int(n_experts), int(units), width,
+                                2 if down.pieces else 1, code, _stream()))
     return out
 
 

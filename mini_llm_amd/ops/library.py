@@ -26,6 +26,8 @@ _SIGNATURES = {
     "mllm_convert": [P, P, c_int, c_int, c_int, c_int, c_int, P],
     "mllm_pack_matrix": [P, P, c_int, c_int, c_int, c_int, c_int, P],
     "mllm_packed_elements": [c_int, c_int, c_int],
+    "mllm_pieces_bytes": [c_int, c_int],
+    "mllm_pack_pieces": [P, c_int, c_int, P],
     "mllm_probe_read": [P, c_longlong, P, c_int, P],
     "mllm_probe_mfma": [P, c_int, c_int, c_int, P],
     "mllm_cache_write": [P, P, c_int, P, P, P, c_int, c_int, c_int, c_int, c_int, P],
@@ -60,8 +62,8 @@ _SIGNATURES = {
     "mllm_expert_tile_rows": [],
     "mllm_experts_few_rows": [c_int, c_int],
     "mllm_expert_lists": [P, P, c_int, c_int, c_int, c_int, P, P, P, P, P, P],
-    "mllm_experts_up": [P, P, P, P, P, P, P, c_int, c_int, c_int, c_int, c_float, c_float, c_float, c_int, c_int, P],
-    "mllm_experts_down": [P, P, P, P, P, P, c_int, c_int, c_int, c_int, c_int, P],
+    "mllm_experts_up": [P, P, P, P, P, P, P, c_int, c_int, c_int, c_int, c_int, c_float, c_float, c_float, c_int, c_int, c_int, P],
+    "mllm_experts_down": [P, P, P, P, P, P, c_int, c_int, c_int, c_int, c_int, c_int, c_int, P],
     "mllm_experts_few_up": [P, P, P, P, P, c_int, c_int, c_int, c_int, c_int, c_float, c_float, c_float, c_int, c_int, P],
     "mllm_experts_few_down": [P, P, P, P, c_int, c_int, c_int, c_int, c_int, c_int, P],
     "mllm_expert_unit": [P, P, P, c_int, c_int, c_int, c_int, c_int, P, P, c_int, c_int, c_int, P],
@@ -123,7 +125,7 @@ def library() -> ctypes.CDLL:
             fn = getattr(lib, name)
             fn.argtypes = argtypes
             fn.restype = c_int
-        lib.mllm_packed_elements.restype = c_longlong
+        lib.mllm_packed_elements.restype = lib.mllm_pieces_bytes.restype = c_longlong
         lib.mllm_static_scratch_bytes.restype = c_longlong
         lib.mllm_static_scratch_bytes.argtypes = []
         lib.mllm_last_error.restype = ctypes.c_char_p

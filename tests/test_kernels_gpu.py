@@ -1083,6 +1083,47 @@ def test_linear_split_leaves_partial_products(K, m, n, k, k_blocks, dtype, packe
         assert (host(partials) != 0).any(axis=(1, 2)).all()  # every block had its share
 
 
+@pytest.mark.parametrize("m,n,k,scale", [(65, 100, 32, 1.0), (130, 132, 96, 1.0), (200, 64, 3072, 1.0), (700, 776, 320, 1e-18), (2100, 2008, 128, 1e15), (8200, 1028, 64, 1.0)])
+def test_32_bit_products_in_pieces_are_no_less_exact_than_32_bit_ones(K, m, n, k, scale):
+    # the kernel that multiplies in bfloat16 pieces (65 rows or more, a packed W, K in whole tiles of 32) against 64-bit sums, over numbers of many
+    # magnitudes, beside the kernel with the 32-bit matrix instruction (a row-major W takes it)
+    rng = np.random.default_rng(m + n)
+    x = (rng.standard_normal((m, k)) * np.exp(rng.normal(0, 2, (m, k))) * scale).astype(np.float32)
+    w = (rng.standard_normal((n, k)) * np.exp(rng.normal(0, 2, (n, k)))).astype(np.float32)
+    ref = x.astype(np.float64) @ w.astype(np.float64).T
+    size = np.abs(x).astype(np.float64) @ np.abs(w).astype(np.float64).T   # what a rounding of a sum is relative to
+    errors = [np.linalg.norm((host(K.linear(dev(x), weight)) - ref) / size) for weight in (K.pack_matrix(dev(w)), dev(w))]
+    assert errors[0] <= 1.2 * errors[1]
+    # every matrix instruction may leave the running sum a unit in its last place off (2^-23 of at most `size`), and there are six for sixteen numbers of
+    # K; the pieces' products that are left out are below 2^-22 of a product
+    bound = 2**-23 * (6 * k / 16 + 2)
+    assert np.abs((host(K.linear(dev(x), K.pack_matrix(dev(w)))) - ref) / size).max() < bound
+    for blocks in (2, 5):   # (with fewer tiles of K than blocks the last ones have none: zeros)
+        got = host(K.linear_split(dev(x), K.pack_matrix(dev(w)), blocks)).sum(axis=0)
+        assert np.abs((got - ref) / size).max() < bound
+
+
+def test_32_bit_products_in_pieces_with_infinities_and_no_numbers(K):
+    # an infinity has no pieces: what comes out is what sums of 32-bit products give; other rows and columns know nothing of it
+    rng = np.random.default_rng(3)
+    x, w = rng.standard_normal((130, 64)).astype(np.float32), rng.standard_normal((72, 64)).astype(np.float32)
+    w[5], x[0] = bf16_round(w[5]), bf16_round(x[0])   # numbers whose lower pieces are zero
+    x[7, 3], x[70, 10], x[100, 1], x[129, 0] = np.inf, -np.inf, np.nan, np.finfo(np.float32).max
+    got, ref = host(K.linear(dev(x), K.pack_matrix(dev(w)))), x.astype(np.float64) @ w.astype(np.float64).T
+    np.testing.assert_array_equal(np.isnan(got), np.isnan(ref))
+    np.testing.assert_array_equal(got[[7, 70]], ref[[7, 70]])
+    rest = [r for r in range(129) if r not in (7, 70, 100)]
+    np.testing.assert_allclose(got[rest], ref[rest], rtol=2e-5, atol=2e-5)
+    with np.errstate(over="ignore"):
+        np.testing.assert_array_equal(np.isinf(got[129]), np.isinf(ref[129].astype(np.float32)))
+    w[40, 9] = np.inf
+    x[[7, 70, 100, 129]] = 1.0
+    got, ref = host(K.linear(dev(x), K.pack_matrix(dev(w)))), x.astype(np.float64) @ w.astype(np.float64).T
+    np.testing.assert_array_equal(got[:, 40], ref[:, 40])
+    rest = [c for c in range(72) if c != 40]
+    np.testing.assert_allclose(got[:, rest], ref[:, rest], rtol=2e-5, atol=2e-5)
+
+
 def test_split_blocks_follow_the_shape(K):
     # few output columns and a long K are cut; many columns, or a short K, are not
     big = lambda n, k, dtype, rows=1: K.split_blocks(torch.empty((n, k), dtype=dtype, device=DEV), dtype, rows)
