@@ -78,6 +78,7 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N, 2) void gemm_pieces_kernel(
     const int k_begin = blockIdx.z * k_per_block, k_end = min(K, k_begin + k_per_block);
     out += (size_t)blockIdx.z * M * N;
     const unsigned char* w_pieces = reinterpret_cast<const unsigned char*>(W) + packed_pieces_at(matrix_tiles, packed_k_steps<float>(K));
+    const int infinite = *reinterpret_cast<const int*>(w_pieces + packed_pieces_bytes(matrix_tiles, K));   // whether W holds an infinity: asked for early
     auto a_row = [&](int r) {   // of the block's tile; beyond the last: that row again, never stored
         const int row = min(m0 + r, m_end - 1);
         if constexpr (Group::GROUPED) return group.a_row ? group.a_row[row] : row;
@@ -97,8 +98,7 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N, 2) void gemm_pieces_kernel(
         const int chunk = wave + l * WAVES, row_tile = first_tile + min(n0 / 16 + chunk / 3, row_tiles - 1);
         w_from[l] = ((unsigned)row_tile * (unsigned)k_steps * 3u + (unsigned)(chunk % 3)) * 1024u + lane * 16u;
     }
-    const unsigned char* a_tile = reinterpret_cast<const unsigned char*>(A + k_begin);
-    const unsigned char* w_tile = w_pieces + (size_t)(k_begin / BK) * 3072;
+    const unsigned char *a_tile, *w_tile;
     auto issue = [&](int stage) {   // the next tile
         unsigned char* place = piece_lds + stage * STAGE;
 #pragma unroll
@@ -114,12 +114,6 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N, 2) void gemm_pieces_kernel(
     };
 
     f32x16 acc[TN][TM];
-#pragma unroll
-    for (int j = 0; j < TN; j++)
-#pragma unroll
-        for (int i = 0; i < TM; i++)
-#pragma unroll
-            for (int v = 0; v < 16; v++) acc[j][i][v] = 0.0f;
     const unsigned base = (unsigned)(size_t)(const __attribute__((address_space(3))) unsigned char*)piece_lds;
     unsigned a_at[2][2];   // [step of 16][piece]
 #pragma unroll
@@ -130,80 +124,79 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N, 2) void gemm_pieces_kernel(
 
     float largest = 0.0f;   // the largest magnitude this lane has met in A
     const int tiles = (k_end - k_begin + BK - 1) / BK;
-    if (tiles > 0) issue(0);
-    for (int t = 0; t < tiles; t++) {
-        // this wave's loads of the tile have landed; behind the barrier everybody's have, and nobody reads the other stage any more
-        __builtin_amdgcn_s_waitcnt(0);
-        __builtin_amdgcn_s_barrier();
-        __builtin_amdgcn_sched_barrier(0);
-        if (t + 1 < tiles) issue((t + 1) & 1);
-        const unsigned stage = (t & 1) * STAGE;
-        i32x4 raw[2][TM][2], w[2][3][TN];
-        auto ask_step = [&](auto step) {
-            constexpr int kk = decltype(step)::value;
-            stream::static_for<TM>([&](auto i) {
-                ask<i * 32 * 128>(raw[kk][i][0], a_at[kk][0] + stage);
-                ask<i * 32 * 128>(raw[kk][i][1], a_at[kk][1] + stage);
-            });
-            stream::static_for<3>([&](auto p) { stream::static_for<TN>([&](auto j) { ask<j * 2 * 3072 + p * 1024 + kk * 512>(w[kk][p][j], w_at + stage); }); });
-        };
-        auto wait_step = [&](int kk) {
-            landed(raw[kk][0][0]);
+    // the sums of the last `count` of the six products of pieces; nobody reads the stages when it begins
+    auto walk = [&](auto count) {
+        constexpr int FIRST = 6 - decltype(count)::value;
+        a_tile = reinterpret_cast<const unsigned char*>(A + k_begin);
+        w_tile = w_pieces + (size_t)(k_begin / BK) * 3072;
 #pragma unroll
-            for (int i = 0; i < TM; i++) this_too(raw[kk][i][0]), this_too(raw[kk][i][1]);
+        for (int j = 0; j < TN; j++)
 #pragma unroll
-            for (int p = 0; p < 3; p++)
+            for (int i = 0; i < TM; i++)
 #pragma unroll
-                for (int j = 0; j < TN; j++) this_too(w[kk][p][j]);
-        };
-        bf16x8 a[2][TM][3];
-        auto multiply = [&](int kk) {
-            constexpr int OF_A[6] = {2, 0, 1, 1, 0, 0}, OF_W[6] = {0, 2, 1, 0, 1, 0};   // the smallest products first
+                for (int v = 0; v < 16; v++) acc[j][i][v] = 0.0f;
+        if (tiles > 0) issue(0);
+        for (int t = 0; t < tiles; t++) {
+            // this wave's loads of the tile have landed; behind the barrier everybody's have, and nobody reads the other stage any more
+            __builtin_amdgcn_s_waitcnt(0);
+            __builtin_amdgcn_s_barrier();
+            __builtin_amdgcn_sched_barrier(0);
+            if (t + 1 < tiles) issue((t + 1) & 1);
+            const unsigned stage = (t & 1) * STAGE;
+            i32x4 raw[2][TM][2], w[2][3][TN];
+            auto ask_step = [&](auto step) {
+                constexpr int kk = decltype(step)::value;
+                stream::static_for<TM>([&](auto i) {
+                    ask<i * 32 * 128>(raw[kk][i][0], a_at[kk][0] + stage);
+                    ask<i * 32 * 128>(raw[kk][i][1], a_at[kk][1] + stage);
+                });
+                stream::static_for<3>([&](auto p) { stream::static_for<TN>([&](auto j) { ask<j * 2 * 3072 + p * 1024 + kk * 512>(w[kk][p][j], w_at + stage); }); });
+            };
+            auto wait_step = [&](int kk) {
+                landed(raw[kk][0][0]);
 #pragma unroll
-            for (int c = 0; c < 6; c++)
+                for (int i = 0; i < TM; i++) this_too(raw[kk][i][0]), this_too(raw[kk][i][1]);
 #pragma unroll
-                for (int i = 0; i < TM; i++)
+                for (int p = 0; p < 3; p++)
 #pragma unroll
-                    for (int j = 0; j < TN; j++)
-                        acc[j][i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*reinterpret_cast<const bf16x8*>(&w[kk][OF_W[c]][j]), a[kk][i][OF_A[c]], acc[j][i], 0, 0, 0);
-        };
-        ask_step(std::integral_constant<int, 0>{});
-        wait_step(0);
-        ask_step(std::integral_constant<int, 1>{});
-        __builtin_amdgcn_sched_barrier(0);
+                    for (int j = 0; j < TN; j++) this_too(w[kk][p][j]);
+            };
+            bf16x8 a[2][TM][3];
+            auto multiply = [&](int kk) {
+                constexpr int OF_A[6] = {2, 0, 1, 1, 0, 0}, OF_W[6] = {0, 2, 1, 0, 1, 0};   // the smallest products first
 #pragma unroll
-        for (int i = 0; i < TM; i++) split(raw[0][i], a[0][i], largest);
-        multiply(0);
-        wait_step(1);
+                for (int c = FIRST; c < 6; c++)
 #pragma unroll
-        for (int i = 0; i < TM; i++) split(raw[1][i], a[1][i], largest);
-        multiply(1);
-    }
-
-    // An infinity has no pieces: a wave that met one (its own rows', or anywhere in W) takes its sums again, number by number.
-    const int infinite = *reinterpret_cast<const int*>(w_pieces + packed_pieces_bytes(matrix_tiles, K));
-    const int row0 = m0 + wave_m * WM, col0 = n0 + wave_n * WN;
-    __syncthreads();   // the slabs below lie where the tiles did (and a flag shared through LDS would leave no room for two blocks of 80 KiB)
-    if (__any(largest == INFINITY) || infinite) {
-        const float* w_rows = W + packed_offset<float>(first_tile, 0, packed_k_steps<float>(K), 0);
-#pragma unroll 1
-        for (int v = 0; v < 16 * TM * TN; v++) {
-            const int j = v / (16 * TM), i = v / 16 % TM, u = v % 16;
-            const int r = wave_m * WM + i * 32 + lane32, col = col0 + j * 32 + 8 * (u / 4) + 4 * half + (u % 4);
-            float sum = 0.0f;
-            if (m0 + r < m_end && col < N) {
-                const float* row = A + (size_t)a_row(r) * K;
-                for (int k = k_begin; k < k_end; k++) sum = __builtin_fmaf(row[k], w_rows[packed_element<float>(col, k, K)], sum);
-            }
+                    for (int i = 0; i < TM; i++)
 #pragma unroll
-            for (int x = 0; x < 16 * TM * TN; x++) acc[x / (16 * TM)][x / 16 % TM][x % 16] = x == v ? sum : acc[x / (16 * TM)][x / 16 % TM][x % 16];
+                        for (int j = 0; j < TN; j++)
+                            acc[j][i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*reinterpret_cast<const bf16x8*>(&w[kk][OF_W[c]][j]), a[kk][i][OF_A[c]], acc[j][i], 0, 0, 0);
+            };
+            ask_step(std::integral_constant<int, 0>{});
+            wait_step(0);
+            ask_step(std::integral_constant<int, 1>{});
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int i = 0; i < TM; i++) split(raw[0][i], a[0][i], largest);
+            multiply(0);
+            wait_step(1);
+#pragma unroll
+            for (int i = 0; i < TM; i++) split(raw[1][i], a[1][i], largest);
+            multiply(1);
         }
-    }
+    };
+    walk(std::integral_constant<int, 6>{});
+
+    const int row0 = m0 + wave_m * WM, col0 = n0 + wave_n * WN;
+    __syncthreads();   // the slabs below lie where the tiles did
+    int* const met = reinterpret_cast<int*>(piece_lds + 2 * STAGE) - WAVES;   // behind the slabs: whether each wave has met an infinity (`again` below)
+    if (lane == 0) met[wave] = 0;
+    if (__any(largest == INFINITY) && lane == 0) met[wave] = 1;
 
     // 32 rows of the wave's columns at a time through LDS of its own, 16 bytes of padding a row. GATED: 32 gate and 32 up columns become 32 units.
     constexpr int OUT_COLS = Group::GATED ? WN / 2 : WN, SLAB_ROW = OUT_COLS + 4, LANES_A_ROW = OUT_COLS / 4, ROWS = WAVE / LANES_A_ROW;
     static_assert(!Group::GATED || TN % 2 == 0, "a wave holds gate and up columns of the same units");
-    static_assert(WAVES * 32 * SLAB_ROW * 4 <= 2 * STAGE, "the slabs fit the stages");
+    static_assert(WAVES * 32 * SLAB_ROW * 4 + WAVES * 4 <= 2 * STAGE, "the slabs fit the stages");
     float* const slab = reinterpret_cast<float*>(piece_lds) + wave * 32 * SLAB_ROW;
     const int out_cols = Group::GATED ? N / 2 : N, out_col = (Group::GATED ? col0 / 2 : col0) + (lane % LANES_A_ROW) * 4;
     // a q/k/v projection: four columns lie in one head (the host sees to it), a lane's columns are the same in every row
@@ -270,6 +263,56 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N, 2) void gemm_pieces_kernel(
     else if (epilogue == MLLM_EPI_GELU_TANH) leave(integral_constant<int, MLLM_EPI_GELU_TANH>{});
     else if (epilogue == MLLM_EPI_GELU_ERF) leave(integral_constant<int, MLLM_EPI_GELU_ERF>{});
     else leave(integral_constant<int, MLLM_EPI_SQUARED_RELU>{});
+
+    // An infinity has no pieces (its middle would be no number, and a lower piece of zero times it is none either), but the sums it belongs to are settled
+    // by the products of the high pieces alone: infinite or no number. A block that met one, in its rows or anywhere in W, takes those products once more
+    // and writes the sums that are not finite again. (Rows that nobody reads may hold anything, so this has to be cheap too.)
+    __syncthreads();
+    bool again = infinite != 0;
+#pragma unroll
+    for (int w = 0; w < WAVES; w++) again |= met[w] != 0;
+    if (!again) return;
+    __syncthreads();   // (everybody has read what the tiles will lie over)
+    walk(std::integral_constant<int, 1>{});
+#pragma unroll
+    for (int i = 0; i < TM; i++) {
+        const int row = row0 + i * 32 + lane32;
+        if (row >= m_end) continue;
+#pragma unroll
+        for (int j = 0; j < TN; j += Group::GATED ? 2 : 1)
+#pragma unroll
+            for (int v = 0; v < 16; v++) {
+                const int col = col0 + j * 32 + 8 * (v / 4) + 4 * half + v % 4;
+                if (col >= N) continue;
+                float value = acc[j][i][v];
+                if constexpr (Group::GATED) {
+                    const float up = acc[j + 1][i][v], weight = group.weight[row];
+                    if (fabsf(value) < INFINITY && fabsf(up) < INFINITY) continue;
+                    const float in_weight = group.weigh_input ? weight : 1.0f, out_weight = group.weigh_input ? 1.0f : weight;
+                    out[(size_t)row * (N / 2) + col0 / 2 + j / 2 * 32 + 8 * (v / 4) + 4 * half + v % 4] = gated(value * in_weight, up * in_weight, group.unit) * out_weight;
+                } else if constexpr (Group::GROUPED) {
+                    if (!(fabsf(value) < INFINITY)) out[(size_t)(group.out_row ? group.out_row[row] : row) * N + col] = value;
+                } else {
+                    if (fabsf(value) < INFINITY) continue;
+                    if (bias) value += bias[col];
+                    if (epilogue == MLLM_EPI_GELU_TANH) value = gelu_tanh(value);
+                    else if (epilogue == MLLM_EPI_GELU_ERF) value = gelu_erf(value);
+                    else if (epilogue == MLLM_EPI_SQUARED_RELU) value = squared_relu(value);
+                    if (!scatter.enabled || col < scatter.q_width) {
+                        const size_t at = (size_t)row * (scatter.enabled ? scatter.q_width : N) + col;
+                        out[at] = residual && residual != out ? residual[at] + value : value;   // (in place the residual is gone, and changes nothing that is not finite)
+                        continue;
+                    }
+                    const int slot = scatter.slots[row];
+                    if (slot < 0) continue;
+                    int c = col - scatter.q_width;
+                    float* to = (float*)(c < scatter.kv_width ? scatter.k_pages : scatter.v_pages);
+                    if (c >= scatter.kv_width) c -= scatter.kv_width;
+                    const int page = slot >> scatter.page_shift, offset = slot & ((1 << scatter.page_shift) - 1);
+                    to[((((size_t)page * scatter.n_kv_heads + c / scatter.head_size) << scatter.page_shift) + offset) * scatter.head_size + c % scatter.head_size] = value;
+                }
+            }
+    }
 }
 
 // Whether a product takes this kernel: a W that was packed with its pieces, more rows than the kernel for few rows takes, whole tiles of K, whole pieces of
