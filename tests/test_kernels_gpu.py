@@ -1124,6 +1124,24 @@ def test_32_bit_products_in_pieces_with_infinities_and_no_numbers(K):
     np.testing.assert_allclose(got[:, rest], ref[:, rest], rtol=2e-5, atol=2e-5)
 
 
+@pytest.mark.parametrize("m", [17, 32, 33, 64])
+@pytest.mark.parametrize("n,k,k_blocks", [(4616, 320, 1), (4632, 1400, 1), (8184, 256, 1), (1592, 2048, 5), (2304, 1288, 2), (4618, 256, 1)])
+def test_products_of_few_rows_with_two_tiles_of_columns_a_block(K, m, n, k, k_blocks):
+    # bfloat16, more than 288 tiles of 16 columns (parts of K counted): an odd tile at the end, columns that fill no tile, K that ends inside a round,
+    # in one and in two rounds of loads; and (the last) columns that are no whole pieces of four
+    rng = np.random.default_rng(n + m)
+    x, w, b = bf16_round(rng.standard_normal((m, k))), bf16_round(rng.standard_normal((n, k)) / math.sqrt(k)), rng.standard_normal(n).astype(np.float32)
+    weight, ref = K.pack_matrix(dev(w, torch.bfloat16)), x @ w.T
+    for rows in (dev(x, torch.bfloat16), packed_rows_of(K, x, torch.bfloat16)):
+        got = host(K.linear_split(rows, weight, k_blocks)).sum(axis=0)
+        np.testing.assert_allclose(got, ref, rtol=2e-5, atol=2e-5)
+        if k_blocks == 1:
+            out = K.linear(rows, weight, dev(b), activation="gelu_new", packed_out=True)
+            np.testing.assert_allclose(unpacked(out), P.gelu_new(ref + b), rtol=1e-2, atol=1e-2)
+            residual = rng.standard_normal((m, n)).astype(np.float32)
+            np.testing.assert_allclose(host(K.linear(rows, weight, dev(b), residual=dev(residual))), ref + b + residual, rtol=2e-5, atol=2e-5)
+
+
 def test_split_blocks_follow_the_shape(K):
     # few output columns and a long K are cut; many columns, or a short K, are not
     big = lambda n, k, dtype, rows=1: K.split_blocks(torch.empty((n, k), dtype=dtype, device=DEV), dtype, rows)
