@@ -800,11 +800,12 @@ __global__ __launch_bounds__(256) void pending_sum_kernel(PendingSum in, float* 
 // GROUPS > 1 (a row of many partial rows, few of them in a launch: the rows a decode step's last layer leaves for the
 // final norm): the block's threads in so many groups of `group_lanes`, each of which adds up every GROUPS-th partial row,
 // all asked for at once; their shares meet in LDS, in a fixed order.
-template <typename OutT, int GROUPS>
-__global__ __launch_bounds__(GROUPS == 1 ? 256 : 1024) void pending_layernorm_kernel(
+// THREADS: as many as a row has pieces of four columns, up to 1,024, so that a thread's pieces are one trip to memory and not two behind each other.
+template <typename OutT, int GROUPS, int THREADS>
+__global__ __launch_bounds__(THREADS) void pending_layernorm_kernel(
     PendingSum in, const int* __restrict__ row_index, const float* __restrict__ gamma, const float* __restrict__ beta,
     OutT* __restrict__ out, float* __restrict__ summed, int width, float eps, int packed_out, int group_lanes) {
-    constexpr int THREADS = GROUPS == 1 ? 256 : 1024, WAVES = THREADS / WAVE;
+    constexpr int WAVES = THREADS / WAVE;
     extern __shared__ f32x4 row_pieces[];  // width / 4, and behind them GROUPS x width / 4 for the groups' shares
     __shared__ float red[2][WAVES];
     const int tid = threadIdx.x, n_pieces = width / 4;
@@ -1014,11 +1015,14 @@ MLLM_API int mllm_pending_layernorm(const float* base, const float* partials, co
     // groups of threads take every fourth partial row each. Where the rows are many the compute units are busy as it is.
     const int group_lanes = (width / 4 + WAVE - 1) / WAVE * WAVE;
     const bool grouped = n_partials >= 16 && n_rows <= 64 && 4 * group_lanes <= 1024;
-#define MLLM_PENDING_NORM(OutT)                                                                                              \
-    if (grouped)                                                                                                             \
-        pending_layernorm_kernel<OutT, 4><<<n_rows, 1024, (size_t)width * 4 * 5, stream>>>(in, row_index, gamma, beta, (OutT*)out, summed, width, eps, packed_out, group_lanes); \
-    else                                                                                                                     \
-        pending_layernorm_kernel<OutT, 1><<<n_rows, 256, (size_t)width * 4, stream>>>(in, row_index, gamma, beta, (OutT*)out, summed, width, eps, packed_out, group_lanes);
+    // (rows of 1,600 with 256 threads took 144 of them through two trips to memory: 64 rows in a decode step 5.9 us, with 512 threads 5.0)
+#define MLLM_PENDING_NORM_WITH(OutT, GROUPS, THREADS) \
+    pending_layernorm_kernel<OutT, GROUPS, THREADS><<<n_rows, THREADS, (size_t)width * 4 * (GROUPS == 1 ? 1 : 1 + GROUPS), stream>>>(in, row_index, gamma, beta, (OutT*)out, summed, width, eps, packed_out, group_lanes)
+#define MLLM_PENDING_NORM(OutT)                                            \
+    if (grouped) MLLM_PENDING_NORM_WITH(OutT, 4, 1024);                    \
+    else if (width <= 1024) MLLM_PENDING_NORM_WITH(OutT, 1, 256);          \
+    else if (width <= 2048) MLLM_PENDING_NORM_WITH(OutT, 1, 512);          \
+    else MLLM_PENDING_NORM_WITH(OutT, 1, 1024);
     if (out_dtype == MLLM_F32) {
         MLLM_PENDING_NORM(float)
     } else if (out_dtype == MLLM_BF16) {
@@ -1027,5 +1031,6 @@ MLLM_API int mllm_pending_layernorm(const float* base, const float* partials, co
         MLLM_REQUIRE(false, "pending_layernorm: unknown output dtype %d", out_dtype);
     }
 #undef MLLM_PENDING_NORM
+#undef MLLM_PENDING_NORM_WITH
     return mllm_check_launch("pending_layernorm");
 }
