@@ -221,7 +221,73 @@ __global__ __launch_bounds__(64 * HEADS_FEW_WAVES) void heads_few_kernel(const X
     store_from_float(out, (size_t)row * out_row_stride + (size_t)head * out_head_stride + n, out_code, value);
 }
 
-constexpr int LATENT_ROWS = 4;   // rows of the batch a block takes, a wave each
+// The same for 32-bit rows and matrices with K a multiple of 16, on the 32-bit matrix instructions, a wave a tile [16 columns, 16 rows]. A
+// lane reads four numbers of its W row and of its x row at once and the four products take one of them each, so the numbers of a piece
+// meet in pairs whatever K index the instruction means by them. BY_K: the four waves of a block take a quarter of one tile's K each and
+// their sums meet in LDS, else they take four neighbouring tiles of columns. What bounds few rows is the trip to memory: with twelve heads
+// the kernel above has twelve blocks, which walk K one 16-byte piece behind the other. Twelve heads, [256, 64] / [64, 256] matrices, that
+// kernel -> this one: 6 rows 9.0 -> 2.8 / 11.8 -> 3.1 us, 260 rows 10.7 -> 7.2 / 14.2 -> 6.1, 2,048 rows 30.9 -> 30.3 / 48.5 -> 25.5.
+// HEADS_BY_K_TILES: where the tiles alone give the 256 compute units two blocks each, cutting K as well no longer pays: 384 tiles by K / by
+// columns 4.2 / 5.9 us (K = 256) and 3.6 / 3.4 (K = 64), 768 tiles of K = 64 4.3 / 3.5.
+constexpr int HEADS_BY_K_TILES = 512;
+
+template <bool BY_K>
+__global__ __launch_bounds__(64 * HEADS_FEW_WAVES) void heads_tile_f32_kernel(const float* __restrict__ x, int x_row_stride, int x_head_stride, const float* __restrict__ w,
+                                                                              const void* __restrict__ gate, int gate_code, int gate_row_stride, int gate_per_head,
+                                                                              void* __restrict__ out, int out_code, int out_row_stride, int out_head_stride, int n_rows,
+                                                                              int N, int K) {
+    const int lane = threadIdx.x % WAVE, wave = threadIdx.x / WAVE, row16 = lane % 16, quad = lane / 16;
+    const int head = blockIdx.y, n0 = (BY_K ? blockIdx.z : blockIdx.z * HEADS_FEW_WAVES + wave) * 16, row0 = blockIdx.x * 16, row = row0 + row16;
+    const float* w_row = w + ((size_t)head * N + min(n0 + row16, N - 1)) * K + 4 * quad;
+    const float* x_row = x + (size_t)min(row, n_rows - 1) * x_row_stride + (size_t)head * x_head_stride + 4 * quad;
+    auto finish = [&](int n, float value) {
+        if (row >= n_rows || n >= N) return;
+        if (gate) {
+            const float g = load_as_float(gate, (size_t)row * gate_row_stride + (gate_per_head ? (size_t)head : (size_t)head * N + n), gate_code);
+            value *= 1.0f / (1.0f + expf(-g));
+        }
+        store_from_float(out, (size_t)row * out_row_stride + (size_t)head * out_head_stride + n, out_code, value);
+    };
+    f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+    const int steps = K / 16;
+    constexpr int AHEAD = 4, STRIDE = BY_K ? HEADS_FEW_WAVES : 1;
+    for (int step0 = BY_K ? wave : 0; step0 < steps; step0 += STRIDE * AHEAD) {
+        f32x4 a[AHEAD], b[AHEAD];
+#pragma unroll
+        for (int u = 0; u < AHEAD; u++) {
+            const int k = min(step0 + u * STRIDE, steps - 1) * 16;   // beyond the end: the last step again, not used
+            a[u] = *reinterpret_cast<const f32x4*>(w_row + k);
+            b[u] = *reinterpret_cast<const f32x4*>(x_row + k);
+        }
+#pragma unroll
+        for (int u = 0; u < AHEAD; u++)
+            if (step0 + u * STRIDE < steps)
+#pragma unroll
+                for (int e = 0; e < 4; e++) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[u][e], b[u][e], acc, 0, 0, 0);
+    }
+    // acc[r] of a lane: column 4 * (lane / 16) + r, row lane % 16
+    if constexpr (BY_K) {
+        __shared__ float sums[HEADS_FEW_WAVES][4][WAVE];
+#pragma unroll
+        for (int r = 0; r < 4; r++) sums[wave][r][lane] = acc[r];
+        __syncthreads();
+        float value = 0.0f;
+#pragma unroll
+        for (int w4 = 0; w4 < HEADS_FEW_WAVES; w4++) value += sums[w4][wave][lane];
+        finish(n0 + 4 * quad + wave, value);
+    } else {
+#pragma unroll
+        for (int r = 0; r < 4; r++) finish(n0 + 4 * quad + r, acc[r]);
+    }
+}
+
+constexpr int LATENT_ROWS = 4;   // rows of the batch a block takes, a wave each (or waves that share a row)
+
+// Up to this many (row, group of heads) pairs the block's waves share a row. Rows of 288 floats, 12 heads (two groups), a wave a row /
+// shared, 32-bit and bfloat16: 6 rows of 200 keys 37.6 / 18.8 us and 38.3 / 16.9, 64 of 640 38.6 / 37.3 and 39.6 / 29.1, a prompt of 260
+// 60.5 / 38.2 and 56 / 38, of 640 195 / 135 and 192 / 120. At 2,048 pairs a prompt of 1,024 still gains (400 / 300), rows of few keys lose (32
+// portions of 32 rows 25.6 / 28.2), and the launch does not know which it has.
+constexpr int LATENT_SHARED_PAIRS = 1536;
 
 template <typename T>
 __device__ __forceinline__ float piece_element(const Vec16& piece, int e) {
@@ -247,14 +313,22 @@ __device__ __forceinline__ float lane_value(float v, int lane) {
 // each head is read out of the lane that holds it. So a cached element costs one load and HG multiply-adds. Keys in
 // tiles of 64 with online softmax statistics per head. n_runs = 1: out [rows, n_heads, R] holds the finished sums, sink
 // included. More runs: every run leaves its unnormalised sums, maximum and weight in parts [rows, n_heads, runs, R + 2].
-template <typename T, int HG, int RV>
+//
+// SHARED, for launches of few rows: the four waves of a block take one row. Of the scores of a tile each adds up a quarter of the row's
+// pieces (the four sums meet in LDS), of the weighted sum each takes every fourth eight keys, and the first wave adds the others' up. What
+// bounds few rows is the chain of trips to memory of a tile of 64 keys, 26 of them in rows of 288 floats; it becomes a quarter as long. The
+// wave a row stays for many rows: there it is the work that counts, and summing up in LDS adds to it where a row has few keys.
+template <typename T, int HG, int RV, bool SHARED>
 __global__ __launch_bounds__(64 * LATENT_ROWS) void latent_attention_kernel(
     const float* __restrict__ q, const T* __restrict__ pages, const float* __restrict__ sinks, float* __restrict__ out, float* __restrict__ parts,
     const int* __restrict__ token_request, const int* __restrict__ positions, const int* __restrict__ block_tables, int max_blocks,
     int n_rows, int n_heads, int R, int D, int page_size, float scale, int run_length) {
     const int lane = threadIdx.x % WAVE;
-    const int token = blockIdx.x * LATENT_ROWS + __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
-    if (token >= n_rows) return;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+    const int token = SHARED ? blockIdx.x : blockIdx.x * LATENT_ROWS + wave;
+    if (token >= n_rows) return;   // SHARED: never, the grid is exact
+    constexpr int SCORE_FLOATS = LATENT_ROWS * HG * WAVE, SUM_FLOATS = (LATENT_ROWS - 1) * HG * RV * WAVE;
+    __shared__ float shared_sums[SHARED ? (SCORE_FLOATS > SUM_FLOATS ? SCORE_FLOATS : SUM_FLOATS) : 1];
     const int run = blockIdx.y, n_runs = gridDim.y, head0 = blockIdx.z * HG;
     const int request = token_request[token];
 
@@ -285,8 +359,10 @@ __global__ __launch_bounds__(64 * LATENT_ROWS) void latent_attention_kernel(
 #pragma unroll
             for (int h = 0; h < HG; h++) s[h] = 0.0f;
             // four pieces of the lane's row are asked for at a time, so that their ways from memory overlap
-            int d0 = 0;
-            for (; d0 + 4 * VEC <= D; d0 += 4 * VEC) {
+            const int share = SHARED ? ceil_div(D / VEC, LATENT_ROWS) * VEC : D;
+            const int d_end = SHARED ? min(D, (wave + 1) * share) : D;
+            int d0 = SHARED ? wave * share : 0;
+            for (; d0 + 4 * VEC <= d_end; d0 += 4 * VEC) {
                 Vec16 pieces[4];
 #pragma unroll
                 for (int u = 0; u < 4; u++) pieces[u] = *reinterpret_cast<const Vec16*>(row + d0 + u * VEC);
@@ -299,7 +375,7 @@ __global__ __launch_bounds__(64 * LATENT_ROWS) void latent_attention_kernel(
                         for (int h = 0; h < HG; h++) s[h] = __builtin_fmaf(q_head[h][d0 + u * VEC + e], k, s[h]);
                     }
             }
-            for (; d0 < D; d0 += VEC) {
+            for (; d0 < d_end; d0 += VEC) {
                 const Vec16 piece = *reinterpret_cast<const Vec16*>(row + d0);
 #pragma unroll
                 for (int e = 0; e < VEC; e++) {
@@ -307,6 +383,18 @@ __global__ __launch_bounds__(64 * LATENT_ROWS) void latent_attention_kernel(
 #pragma unroll
                     for (int h = 0; h < HG; h++) s[h] = __builtin_fmaf(q_head[h][d0 + e], k, s[h]);
                 }
+            }
+            if constexpr (SHARED) {   // every wave of the block walks the same tiles
+#pragma unroll
+                for (int h = 0; h < HG; h++) shared_sums[(wave * HG + h) * WAVE + lane] = s[h];
+                __syncthreads();
+#pragma unroll
+                for (int h = 0; h < HG; h++) {
+                    s[h] = 0.0f;
+#pragma unroll
+                    for (int other = 0; other < LATENT_ROWS; other++) s[h] += shared_sums[(other * HG + h) * WAVE + lane];
+                }
+                __syncthreads();
             }
             float p[HG];
 #pragma unroll
@@ -324,7 +412,7 @@ __global__ __launch_bounds__(64 * LATENT_ROWS) void latent_attention_kernel(
             // for at a time; lanes beyond the tile's keys hold a weight of zero and the place of a key that exists
             const int in_tile = min(WAVE, last_key - tile0 + 1);
             constexpr int KEYS = 8;
-            for (int j0 = 0; j0 < in_tile; j0 += KEYS) {
+            for (int j0 = SHARED ? wave * KEYS : 0; j0 < in_tile; j0 += SHARED ? LATENT_ROWS * KEYS : KEYS) {
                 float v[KEYS][RV];
 #pragma unroll
                 for (int u = 0; u < KEYS; u++) {
@@ -353,6 +441,21 @@ __global__ __launch_bounds__(64 * LATENT_ROWS) void latent_attention_kernel(
                     }
             }
         }
+    }
+    if constexpr (SHARED) {   // maxima and weights are the same in every wave
+        if (wave > 0)
+#pragma unroll
+            for (int h = 0; h < HG; h++)
+#pragma unroll
+                for (int r = 0; r < RV; r++) shared_sums[(((wave - 1) * HG + h) * RV + r) * WAVE + lane] = o[h][r];
+        __syncthreads();
+        if (wave > 0) return;
+#pragma unroll
+        for (int other = 0; other < LATENT_ROWS - 1; other++)
+#pragma unroll
+            for (int h = 0; h < HG; h++)
+#pragma unroll
+                for (int r = 0; r < RV; r++) o[h][r] += shared_sums[((other * HG + h) * RV + r) * WAVE + lane];
     }
 #pragma unroll
     for (int h = 0; h < HG; h++) {
@@ -695,10 +798,14 @@ struct LatentArgs {
 
 template <typename T, int HG, int RV>
 void launch_latent(const LatentArgs& a) {
-    dim3 grid(ceil_div(a.n_rows, LATENT_ROWS), a.n_runs, ceil_div(a.n_heads, HG));
-    latent_attention_kernel<T, HG, RV><<<grid, 64 * LATENT_ROWS, 0, a.stream>>>(a.q, (const T*)a.pages, a.sinks, a.out, a.parts, a.token_request, a.positions,
-                                                                                a.block_tables, a.max_blocks, a.n_rows, a.n_heads, a.R, a.D, a.page_size,
-                                                                                a.scale, a.run_length);
+    const int groups = ceil_div(a.n_heads, HG);
+    auto go = [&](auto kernel, int blocks) {
+        kernel<<<dim3(blocks, a.n_runs, groups), 64 * LATENT_ROWS, 0, a.stream>>>(a.q, (const T*)a.pages, a.sinks, a.out, a.parts, a.token_request, a.positions,
+                                                                                  a.block_tables, a.max_blocks, a.n_rows, a.n_heads, a.R, a.D, a.page_size,
+                                                                                  a.scale, a.run_length);
+    };
+    if ((long long)a.n_rows * groups <= LATENT_SHARED_PAIRS) go(latent_attention_kernel<T, HG, RV, true>, a.n_rows);
+    else go(latent_attention_kernel<T, HG, RV, false>, ceil_div(a.n_rows, LATENT_ROWS));
 }
 
 template <typename T, int HG>
@@ -755,6 +862,18 @@ MLLM_API int mllm_heads_linear(const void* x, int x_dtype, int x_row_stride, int
         else
             heads_linear_mfma_kernel<bf16_t><<<tiles, 256, 0, stream>>>((const bf16_t*)x, x_row_stride, x_head_stride, (const bf16_t*)w, gate, gate_dtype,
                                                                         gate_row_stride, gate_per_head, out, out_dtype, out_row_stride, out_head_stride, n_rows, N, K);
+        return mllm_check_launch("heads_linear");
+    }
+    if (w_dtype == MLLM_F32 && x_dtype == MLLM_F32 && K % 16 == 0 && x_row_stride % 4 == 0 && x_head_stride % 4 == 0 && (size_t)x % 16 == 0 && (size_t)w % 16 == 0 &&
+        n_heads <= 65535 && ceil_div(N, 16) <= 65535) {
+        auto go = [&](auto kernel, int columns) {
+            kernel<<<dim3(ceil_div(n_rows, 16), n_heads, columns), 64 * HEADS_FEW_WAVES, 0, stream>>>((const float*)x, x_row_stride, x_head_stride, (const float*)w, gate,
+                                                                                                      gate_dtype, gate_row_stride, gate_per_head, out, out_dtype,
+                                                                                                      out_row_stride, out_head_stride, n_rows, N, K);
+        };
+        const long long tiles = (long long)ceil_div(n_rows, 16) * n_heads * ceil_div(N, 16);
+        if (tiles <= HEADS_BY_K_TILES) go(heads_tile_f32_kernel<true>, ceil_div(N, 16));
+        else go(heads_tile_f32_kernel<false>, ceil_div(N, 16 * HEADS_FEW_WAVES));
         return mllm_check_launch("heads_linear");
     }
     dim3 grid(ceil_div(n_rows, HEADS_ROWS), n_heads);

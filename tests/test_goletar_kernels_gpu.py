@@ -357,3 +357,44 @@ def test_norm_with_one_gain():
     x, stream = rng.normal(0, 0.05, (9, 70)), rng.normal(0, 1, (9, 70))
     np.testing.assert_allclose(part.forward(gpu(x), torch.float32).cpu().numpy(), plain.rms_norm(x, 0.37, 1e-3), atol=1e-6, rtol=1e-5)
     np.testing.assert_allclose(part.forward_added(gpu(stream), gpu(x)).cpu().numpy(), stream + plain.rms_norm(x, 0.37, 1e-3), atol=1e-6, rtol=1e-5)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("rows", [1536, 1537])   # up to 1,536 (row, group of heads) pairs the waves of a block share a row
+@pytest.mark.parametrize("rank,rot", [(21, 8), (300, 16)])
+def test_latent_attention_at_the_most_rows_that_waves_share(dtype, rows, rank, rot):
+    # bounds as for few rows above: sums of at most 97 keys in 32 bits on either side of the line
+    k = kernels()
+    rng = np.random.default_rng(rows + rank)
+    page_size, length, per, scale = 16, 97, 64, 0.3
+    n_requests, row_size = -(-rows // per), k.latent_row_size(rank + rot)
+    blocks = -(-length // page_size)
+    pages = torch.tensor(rng.normal(0, 1, (n_requests * blocks, 1, page_size, row_size)), dtype=torch.float32).to(dtype)
+    pages[..., rank + rot :] = 0
+    tables = rng.permutation(n_requests * blocks).reshape(n_requests, blocks).astype(np.int32)
+    owner, positions = np.arange(rows, dtype=np.int32) // per, (np.arange(rows, dtype=np.int32) % per) + length - per
+    q = torch.tensor(rng.normal(0, 1, (rows, 1, row_size)), dtype=torch.float32)
+    got = k.latent_attention(q.cuda(), pages.cuda(), None, torch.tensor(owner).cuda(), torch.tensor(positions).cuda(), torch.tensor(tables).cuda(), rank, scale,
+                             max_len=length).cpu().double()
+    cached = pages[torch.tensor(tables).long().view(-1)].double().view(n_requests, blocks * page_size, row_size)
+    for r in range(n_requests):
+        mine = owner == r
+        keys = cached[r, :length]
+        scores = (q[mine, 0].double() @ keys.T) * scale
+        scores[torch.arange(length)[None, :] > torch.tensor(positions[mine])[:, None]] = -float("inf")
+        np.testing.assert_allclose(got[mine, 0].numpy(), (scores.softmax(1) @ keys[:, :rank]).numpy(), atol=2e-5, rtol=2e-4)
+
+
+@pytest.mark.parametrize("rows,heads,n,k_size", [(816, 2, 65, 48), (819, 2, 80, 48), (1030, 3, 130, 80), (1, 3, 1, 16), (15, 2, 17, 272)])
+def test_heads_linear_in_32_bit_tiles(rows, heads, n, k_size):
+    # around the number of tiles (512) beyond which a block takes columns instead of pieces of K; sums of at most 272 products of
+    # numbers around 1 are off by less than k 2^-24 |sum of magnitudes| ~ 272 * 6e-8 * 272 = 4.4e-3 at the very worst, and by its square root's like in fact
+    k = kernels()
+    rng = np.random.default_rng(rows)
+    x, w, gate = rng.normal(0, 1, (rows, heads, k_size + 4)), rng.normal(0, 1, (heads, n, k_size)), rng.normal(0, 2, (rows, heads * n))
+    x, w, gate = (torch.tensor(t, dtype=torch.float32) for t in (x, w, gate))
+    out = torch.full((rows, heads, n + 1), 5.0).cuda()
+    k.heads_linear(x.cuda().view(rows, -1), w.cuda(), out, n_heads=heads, k=k_size, x_head_stride=k_size + 4, gate=gate.cuda())
+    want = torch.einsum("rhk,hnk->rhn", x[:, :, :k_size].double(), w.double()) * torch.sigmoid(gate.double()).view(rows, heads, n)
+    np.testing.assert_allclose(out.cpu()[:, :, :n].double().numpy(), want.numpy(), atol=1e-4, rtol=1e-4)
+    assert (out[:, :, n:] == 5).all()
