@@ -53,18 +53,16 @@ __global__ __launch_bounds__(256) void pack_kernel(const S* __restrict__ src, D*
 }
 
 // The pieces of the packed 32-bit matrix in front of them (gemm_pieces.h): a wave 16 rows x 32 columns.
-__global__ __launch_bounds__(256) void pack_pieces_kernel(const float* __restrict__ packed, unsigned char* __restrict__ pieces, int* __restrict__ infinite, int row_tiles, int cols) {
+__global__ __launch_bounds__(256) void pack_pieces_kernel(const float* __restrict__ packed, unsigned char* __restrict__ pieces, int row_tiles, int cols) {
     const int k_steps = ceil_div(cols, 32);
     const size_t step = (size_t)blockIdx.x * (blockDim.x / WAVE) + threadIdx.x / WAVE;
     if (step >= (size_t)row_tiles * k_steps) return;
     const int lane = threadIdx.x % WAVE, row_tile = (int)(step / k_steps), k_step = (int)(step % k_steps);
     bf16x8 out[3];
-    bool met = false;
 #pragma unroll
     for (int e = 0; e < 8; e++) {
         const int col = k_step * 32 + (lane / 16) * 8 + e;   // the bfloat16 chunk's place: row lane % 16, columns 8 (lane / 16) ..
         float rest = col < cols ? packed[packed_element<float>(row_tile * 16 + lane % 16, col, cols)] : 0.0f;
-        met |= fabsf(rest) == INFINITY;
 #pragma unroll
         for (int p = 0; p < 3; p++) {
             const uint32_t bits = __builtin_bit_cast(uint32_t, rest) & 0xffff0000u;
@@ -73,12 +71,9 @@ __global__ __launch_bounds__(256) void pack_pieces_kernel(const float* __restric
             rest -= __builtin_bit_cast(float, bits);
         }
     }
-    if (met) *infinite = 1;   // (whoever writes writes the same)
 #pragma unroll
     for (int p = 0; p < 3; p++) *reinterpret_cast<bf16x8*>(pieces + (step * 3 + p) * 1024 + lane * 16) = out[p];
 }
-
-__global__ void no_infinite_kernel(int* infinite) { *infinite = 0; }
 
 template <typename S, typename D>
 void launch_pack(const void* src, void* dst, int rows, int cols, int transpose, hipStream_t stream) {
@@ -129,19 +124,16 @@ MLLM_API int mllm_pack_matrix(const void* src, void* dst, int rows, int cols, in
     return mllm_check_launch("pack_matrix");
 }
 
-// Bytes the pieces of a packed 32-bit matrix take behind it (the number that tells of infinities included).
-MLLM_API long long mllm_pieces_bytes(int rows, int cols) { return packed_pieces_bytes(ceil_div(rows, 16), cols) + 16; }
+// Bytes the pieces of a packed 32-bit matrix take behind it.
+MLLM_API long long mllm_pieces_bytes(int rows, int cols) { return packed_pieces_bytes(ceil_div(rows, 16), cols); }
 
 // Lays the pieces of a packed 32-bit matrix [rows, cols] behind it, at packed + mllm_packed_elements.
 MLLM_API int mllm_pack_pieces(float* packed, int rows, int cols, hipStream_t stream) {
     MLLM_REQUIRE(rows > 0 && cols > 0 && packed != nullptr, "pack_pieces: bad size %d x %d", rows, cols);
     const int row_tiles = ceil_div(rows, 16);
     unsigned char* pieces = reinterpret_cast<unsigned char*>(packed) + packed_pieces_at(row_tiles, packed_k_steps<float>(cols));
-    int* infinite = reinterpret_cast<int*>(pieces + packed_pieces_bytes(row_tiles, cols));
     const size_t steps = (size_t)row_tiles * ceil_div(cols, 32);
     mllm_count_kernel(MLLM_K_PACK);
-    no_infinite_kernel<<<1, 1, 0, stream>>>(infinite);
-    mllm_count_kernel(MLLM_K_PACK);
-    pack_pieces_kernel<<<(unsigned)((steps + 3) / 4), 256, 0, stream>>>(packed, pieces, infinite, row_tiles, cols);
+    pack_pieces_kernel<<<(unsigned)((steps + 3) / 4), 256, 0, stream>>>(packed, pieces, row_tiles, cols);
     return mllm_check_launch("pack_pieces");
 }

@@ -33,12 +33,10 @@ __device__ __forceinline__ void landed(i32x4& first) { asm volatile("s_waitcnt l
 __device__ __forceinline__ void this_too(i32x4& fragment) { asm volatile("" : "+v"(fragment)); }
 
 // Eight numbers -> three operands of pieces.
-__device__ __forceinline__ void split(const i32x4 (&raw)[2], bf16x8 (&out)[3], float& largest) {
+__device__ __forceinline__ void split(const i32x4 (&raw)[2], bf16x8 (&out)[3]) {
     uint32_t rest[8];
 #pragma unroll
     for (int e = 0; e < 8; e++) rest[e] = (uint32_t)raw[e / 4][e % 4];
-#pragma unroll
-    for (int e = 0; e < 8; e += 2) largest = fmaxf(fmaxf(fabsf(__builtin_bit_cast(float, rest[e])), fabsf(__builtin_bit_cast(float, rest[e + 1]))), largest);
 #pragma unroll
     for (int p = 0; p < 3; p++) {
         uint32_t pairs[4];
@@ -78,7 +76,6 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N, 2) void gemm_pieces_kernel(
     const int k_begin = blockIdx.z * k_per_block, k_end = min(K, k_begin + k_per_block);
     out += (size_t)blockIdx.z * M * N;
     const unsigned char* w_pieces = reinterpret_cast<const unsigned char*>(W) + packed_pieces_at(matrix_tiles, packed_k_steps<float>(K));
-    const int infinite = *reinterpret_cast<const int*>(w_pieces + packed_pieces_bytes(matrix_tiles, K));   // whether W holds an infinity: asked for early
     auto a_row = [&](int r) {   // of the block's tile; beyond the last: that row again, never stored
         const int row = min(m0 + r, m_end - 1);
         if constexpr (Group::GROUPED) return group.a_row ? group.a_row[row] : row;
@@ -98,7 +95,7 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N, 2) void gemm_pieces_kernel(
         const int chunk = wave + l * WAVES, row_tile = first_tile + min(n0 / 16 + chunk / 3, row_tiles - 1);
         w_from[l] = ((unsigned)row_tile * (unsigned)k_steps * 3u + (unsigned)(chunk % 3)) * 1024u + lane * 16u;
     }
-    const unsigned char *a_tile, *w_tile;
+    const unsigned char *a_tile = reinterpret_cast<const unsigned char*>(A + k_begin), *w_tile = w_pieces + (size_t)(k_begin / BK) * 3072;
     auto issue = [&](int stage) {   // the next tile
         unsigned char* place = piece_lds + stage * STAGE;
 #pragma unroll
@@ -122,93 +119,137 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N, 2) void gemm_pieces_kernel(
         for (int q = 0; q < 2; q++) a_at[kk][q] = base + (wave_m * WM + lane32) * 128 + (((kk * 4 + half * 2 + q) ^ (lane32 / 2 % 8)) * 16);
     const unsigned w_at = base + A_BYTES + (wave_n * TN * 2 + lane32 / 16) * 3072 + half * 256 + (lane % 16) * 16;
 
-    float largest = 0.0f;   // the largest magnitude this lane has met in A
     const int tiles = (k_end - k_begin + BK - 1) / BK;
-    // the sums of the last `count` of the six products of pieces; nobody reads the stages when it begins
-    auto walk = [&](auto count) {
-        constexpr int FIRST = 6 - decltype(count)::value;
-        a_tile = reinterpret_cast<const unsigned char*>(A + k_begin);
-        w_tile = w_pieces + (size_t)(k_begin / BK) * 3072;
 #pragma unroll
-        for (int j = 0; j < TN; j++)
+    for (int j = 0; j < TN; j++)
 #pragma unroll
-            for (int i = 0; i < TM; i++)
+        for (int i = 0; i < TM; i++)
 #pragma unroll
-                for (int v = 0; v < 16; v++) acc[j][i][v] = 0.0f;
-        if (tiles > 0) issue(0);
-        for (int t = 0; t < tiles; t++) {
-            // this wave's loads of the tile have landed; behind the barrier everybody's have, and nobody reads the other stage any more
-            __builtin_amdgcn_s_waitcnt(0);
-            __builtin_amdgcn_s_barrier();
-            __builtin_amdgcn_sched_barrier(0);
-            if (t + 1 < tiles) issue((t + 1) & 1);
-            const unsigned stage = (t & 1) * STAGE;
-            i32x4 raw[2][TM][2], w[2][3][TN];
-            auto ask_step = [&](auto step) {
-                constexpr int kk = decltype(step)::value;
-                stream::static_for<TM>([&](auto i) {
-                    ask<i * 32 * 128>(raw[kk][i][0], a_at[kk][0] + stage);
-                    ask<i * 32 * 128>(raw[kk][i][1], a_at[kk][1] + stage);
-                });
-                stream::static_for<3>([&](auto p) { stream::static_for<TN>([&](auto j) { ask<j * 2 * 3072 + p * 1024 + kk * 512>(w[kk][p][j], w_at + stage); }); });
-            };
-            auto wait_step = [&](int kk) {
-                landed(raw[kk][0][0]);
+            for (int v = 0; v < 16; v++) acc[j][i][v] = 0.0f;
+    if (tiles > 0) issue(0);
+    for (int t = 0; t < tiles; t++) {
+        // this wave's loads of the tile have landed; behind the barrier everybody's have, and nobody reads the other stage any more
+        __builtin_amdgcn_s_waitcnt(0);
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_sched_barrier(0);
+        if (t + 1 < tiles) issue((t + 1) & 1);
+        const unsigned stage = (t & 1) * STAGE;
+        i32x4 raw[2][TM][2], w[2][3][TN];
+        auto ask_step = [&](auto step) {
+            constexpr int kk = decltype(step)::value;
+            stream::static_for<TM>([&](auto i) {
+                ask<i * 32 * 128>(raw[kk][i][0], a_at[kk][0] + stage);
+                ask<i * 32 * 128>(raw[kk][i][1], a_at[kk][1] + stage);
+            });
+            stream::static_for<3>([&](auto p) { stream::static_for<TN>([&](auto j) { ask<j * 2 * 3072 + p * 1024 + kk * 512>(w[kk][p][j], w_at + stage); }); });
+        };
+        auto wait_step = [&](int kk) {
+            landed(raw[kk][0][0]);
 #pragma unroll
-                for (int i = 0; i < TM; i++) this_too(raw[kk][i][0]), this_too(raw[kk][i][1]);
+            for (int i = 0; i < TM; i++) this_too(raw[kk][i][0]), this_too(raw[kk][i][1]);
 #pragma unroll
-                for (int p = 0; p < 3; p++)
+            for (int p = 0; p < 3; p++)
 #pragma unroll
-                    for (int j = 0; j < TN; j++) this_too(w[kk][p][j]);
-            };
-            bf16x8 a[2][TM][3];
-            auto multiply = [&](int kk) {
-                constexpr int OF_A[6] = {2, 0, 1, 1, 0, 0}, OF_W[6] = {0, 2, 1, 0, 1, 0};   // the smallest products first
+                for (int j = 0; j < TN; j++) this_too(w[kk][p][j]);
+        };
+        bf16x8 a[2][TM][3];
+        auto multiply = [&](int kk) {
+            constexpr int OF_A[6] = {2, 0, 1, 1, 0, 0}, OF_W[6] = {0, 2, 1, 0, 1, 0};   // the smallest products first
 #pragma unroll
-                for (int c = FIRST; c < 6; c++)
+            for (int c = 0; c < 6; c++)
 #pragma unroll
-                    for (int i = 0; i < TM; i++)
+                for (int i = 0; i < TM; i++)
 #pragma unroll
-                        for (int j = 0; j < TN; j++)
-                            acc[j][i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*reinterpret_cast<const bf16x8*>(&w[kk][OF_W[c]][j]), a[kk][i][OF_A[c]], acc[j][i], 0, 0, 0);
-            };
-            ask_step(std::integral_constant<int, 0>{});
-            wait_step(0);
-            ask_step(std::integral_constant<int, 1>{});
-            __builtin_amdgcn_sched_barrier(0);
+                    for (int j = 0; j < TN; j++)
+                        acc[j][i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*reinterpret_cast<const bf16x8*>(&w[kk][OF_W[c]][j]), a[kk][i][OF_A[c]], acc[j][i], 0, 0, 0);
+        };
+        ask_step(std::integral_constant<int, 0>{});
+        wait_step(0);
+        ask_step(std::integral_constant<int, 1>{});
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int i = 0; i < TM; i++) split(raw[0][i], a[0][i], largest);
-            multiply(0);
-            wait_step(1);
+        for (int i = 0; i < TM; i++) split(raw[0][i], a[0][i]);
+        multiply(0);
+        wait_step(1);
 #pragma unroll
-            for (int i = 0; i < TM; i++) split(raw[1][i], a[1][i], largest);
-            multiply(1);
-        }
-    };
-    walk(std::integral_constant<int, 6>{});
+        for (int i = 0; i < TM; i++) split(raw[1][i], a[1][i]);
+        multiply(1);
+    }
 
     const int row0 = m0 + wave_m * WM, col0 = n0 + wave_n * WN;
     __syncthreads();   // the slabs below lie where the tiles did
-    int* const met = reinterpret_cast<int*>(piece_lds + 2 * STAGE) - WAVES;   // behind the slabs: whether each wave has met an infinity (`again` below)
-    if (lane == 0) met[wave] = 0;
-    if (__any(largest == INFINITY) && lane == 0) met[wave] = 1;
+
+    // An infinity has no pieces (its middle is no number), so every sum it belongs to comes out as no number, whatever it should be. The rows of this wave
+    // with a sum that is not finite (bit r: row r of the WM) are left out of what is stored below and taken again in 32-bit at the end.
+    // What a row holds that is no number itself makes all its sums none, as it should: such a row stays as it is. (Rows that nobody reads may hold anything,
+    // and those with an infinity become that behind the next norm.)
+    static_assert(TM <= 2, "a bit a row");
+    unsigned long long bad = 0;
+#pragma unroll
+    for (int i = 0; i < TM; i++) {
+        float any = 0.0f;
+#pragma unroll
+        for (int j = 0; j < TN; j++)
+#pragma unroll
+            for (int v = 0; v < 16; v++) any = __builtin_fmaf(acc[j][i][v], 0.0f, any);   // no number where one of them is not finite
+        const unsigned long long lanes = __ballot(any != any);
+        bad |= (unsigned long long)((unsigned)lanes | (unsigned)(lanes >> 32)) << (32 * i);
+    }
+    const int row16 = lane % 16, quad = lane / 16, rows_here = m_end - row0;
+    if (rows_here < WM) bad = rows_here > 0 ? bad & ((1ull << rows_here) - 1) : 0;   // (beyond the last row: that row again)
+    if (bad != 0) {
+#pragma unroll 1
+        for (int g = 0; g < WM / 16; g++) {
+            if ((bad >> (16 * g) & 0xffff) == 0) continue;
+            const float* x = A + (size_t)a_row(wave_m * WM + g * 16 + row16) * K + 4 * quad;
+            bool none = false;
+            for (int k = k_begin; k < k_end; k += 16) {
+                const f32x4 piece = *reinterpret_cast<const f32x4*>(x + k);
+#pragma unroll
+                for (int e = 0; e < 4; e++) none |= piece[e] != piece[e];
+            }
+            const unsigned long long lanes = __ballot(none);
+            bad &= ~(((lanes | lanes >> 16 | lanes >> 32 | lanes >> 48) & 0xffff) << (16 * g));
+        }
+    }
 
     // 32 rows of the wave's columns at a time through LDS of its own, 16 bytes of padding a row. GATED: 32 gate and 32 up columns become 32 units.
     constexpr int OUT_COLS = Group::GATED ? WN / 2 : WN, SLAB_ROW = OUT_COLS + 4, LANES_A_ROW = OUT_COLS / 4, ROWS = WAVE / LANES_A_ROW;
     static_assert(!Group::GATED || TN % 2 == 0, "a wave holds gate and up columns of the same units");
-    static_assert(WAVES * 32 * SLAB_ROW * 4 + WAVES * 4 <= 2 * STAGE, "the slabs fit the stages");
+    static_assert(WAVES * 32 * SLAB_ROW * 4 <= 2 * STAGE, "the slabs fit the stages");
     float* const slab = reinterpret_cast<float*>(piece_lds) + wave * 32 * SLAB_ROW;
     const int out_cols = Group::GATED ? N / 2 : N, out_col = (Group::GATED ? col0 / 2 : col0) + (lane % LANES_A_ROW) * 4;
-    // a q/k/v projection: four columns lie in one head (the host sees to it), a lane's columns are the same in every row
     const int width = scatter.enabled ? scatter.q_width : out_cols;
-    float* pages = nullptr;
-    int kv_head = 0, d = 0;
-    if (!Group::GROUPED && scatter.enabled && out_col >= scatter.q_width && out_col < N) {
-        int c = out_col - scatter.q_width;
-        pages = (float*)(c < scatter.kv_width ? scatter.k_pages : scatter.v_pages);
-        if (c >= scatter.kv_width) c -= scatter.kv_width;
-        kv_head = c / scatter.head_size, d = c % scatter.head_size;
-    }
+    // where four columns of a q/k/v projection go: they lie in one head (the host sees to it)
+    struct Place {
+        float* pages;   // null: the output
+        int kv_head, d;
+    };
+    auto place_of = [&](int col) {
+        Place place = {nullptr, 0, 0};
+        if (!Group::GROUPED && scatter.enabled && col >= scatter.q_width && col < N) {
+            int c = col - scatter.q_width;
+            place.pages = (float*)(c < scatter.kv_width ? scatter.k_pages : scatter.v_pages);
+            if (c >= scatter.kv_width) c -= scatter.kv_width;
+            place.kv_head = c / scatter.head_size, place.d = c % scatter.head_size;
+        }
+        return place;
+    };
+    auto put = [&](int row, int col, const Place& place, f32x4 value) {
+        if (!Group::GROUPED && place.pages) {
+            const int slot = scatter.slots[row];
+            if (slot < 0) return;
+            const int page = slot >> scatter.page_shift, offset = slot & ((1 << scatter.page_shift) - 1);
+            *reinterpret_cast<f32x4*>(place.pages + ((((size_t)page * scatter.n_kv_heads + place.kv_head) << scatter.page_shift) + offset) * scatter.head_size + place.d) = value;
+            return;
+        }
+        int to = row;
+        if constexpr (Group::GROUPED && !Group::GATED) to = group.out_row ? group.out_row[row] : row;
+        const size_t at = (size_t)to * width + col;
+        if (!Group::GROUPED && residual) value = *reinterpret_cast<const f32x4*>(residual + at) + value;
+        *reinterpret_cast<f32x4*>(out + at) = value;
+    };
+    const Place place = place_of(out_col);   // a lane's columns are the same in every row
     auto leave = [&](auto kind) {
         constexpr int KIND = decltype(kind)::value;
 #pragma unroll
@@ -241,19 +282,8 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N, 2) void gemm_pieces_kernel(
             for (int r = 0; r < 32 / ROWS; r++) {
                 const int in_slab = r * ROWS + lane / LANES_A_ROW, row = row0 + i * 32 + in_slab;
                 f32x4 value = *reinterpret_cast<const f32x4*>(slab + in_slab * SLAB_ROW + (lane % LANES_A_ROW) * 4);
-                if (row >= m_end || out_col >= out_cols) continue;
-                if (!Group::GROUPED && pages) {
-                    const int slot = scatter.slots[row];
-                    if (slot < 0) continue;
-                    const int page = slot >> scatter.page_shift, offset = slot & ((1 << scatter.page_shift) - 1);
-                    *reinterpret_cast<f32x4*>(pages + ((((size_t)page * scatter.n_kv_heads + kv_head) << scatter.page_shift) + offset) * scatter.head_size + d) = value;
-                    continue;
-                }
-                int to = row;
-                if constexpr (Group::GROUPED && !Group::GATED) to = group.out_row ? group.out_row[row] : row;
-                const size_t at = (size_t)to * width + out_col;
-                if (!Group::GROUPED && residual) value = *reinterpret_cast<const f32x4*>(residual + at) + value;
-                *reinterpret_cast<f32x4*>(out + at) = value;
+                if (row >= m_end || out_col >= out_cols || (bad >> (i * 32 + in_slab) & 1)) continue;
+                put(row, out_col, place, value);
             }
             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         }
@@ -264,54 +294,58 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N, 2) void gemm_pieces_kernel(
     else if (epilogue == MLLM_EPI_GELU_ERF) leave(integral_constant<int, MLLM_EPI_GELU_ERF>{});
     else leave(integral_constant<int, MLLM_EPI_SQUARED_RELU>{});
 
-    // An infinity has no pieces (its middle would be no number, and a lower piece of zero times it is none either), but the sums it belongs to are settled
-    // by the products of the high pieces alone: infinite or no number. A block that met one, in its rows or anywhere in W, takes those products once more
-    // and writes the sums that are not finite again. (Rows that nobody reads may hold anything, so this has to be cheap too.)
-    __syncthreads();
-    bool again = infinite != 0;
+    // the rows left out, in groups of sixteen that hold one, with the 32-bit instruction and operands straight from memory
+    constexpr int TILES = WN / 16;
+#pragma unroll 1
+    for (int g = 0; g < WM / 16; g++) {
+        const unsigned rows = (unsigned)(bad >> (16 * g)) & 0xffff;
+        if (rows == 0) continue;
+        const float* x = A + (size_t)a_row(wave_m * WM + g * 16 + row16) * K + 4 * quad;
+        f32x4 sum[TILES];
 #pragma unroll
-    for (int w = 0; w < WAVES; w++) again |= met[w] != 0;
-    if (!again) return;
-    __syncthreads();   // (everybody has read what the tiles will lie over)
-    walk(std::integral_constant<int, 1>{});
+        for (int t = 0; t < TILES; t++) sum[t] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll 1
+        for (int k = k_begin; k < k_end; k += 16) {
+            const f32x4 b = *reinterpret_cast<const f32x4*>(x + k);
+            f32x4 a[TILES];
 #pragma unroll
-    for (int i = 0; i < TM; i++) {
-        const int row = row0 + i * 32 + lane32;
-        if (row >= m_end) continue;
+            for (int t = 0; t < TILES; t++)
+                a[t] = *reinterpret_cast<const f32x4*>(W + packed_offset<float>(first_tile + min(col0 / 16 + t, row_tiles - 1), k / 16, packed_k_steps<float>(K), lane));
 #pragma unroll
-        for (int j = 0; j < TN; j += Group::GATED ? 2 : 1)
+            for (int t = 0; t < TILES; t++)
 #pragma unroll
-            for (int v = 0; v < 16; v++) {
-                const int col = col0 + j * 32 + 8 * (v / 4) + 4 * half + v % 4;
-                if (col >= N) continue;
-                float value = acc[j][i][v];
-                if constexpr (Group::GATED) {
-                    const float up = acc[j + 1][i][v], weight = group.weight[row];
-                    if (fabsf(value) < INFINITY && fabsf(up) < INFINITY) continue;
-                    const float in_weight = group.weigh_input ? weight : 1.0f, out_weight = group.weigh_input ? 1.0f : weight;
-                    out[(size_t)row * (N / 2) + col0 / 2 + j / 2 * 32 + 8 * (v / 4) + 4 * half + v % 4] = gated(value * in_weight, up * in_weight, group.unit) * out_weight;
-                } else if constexpr (Group::GROUPED) {
-                    if (!(fabsf(value) < INFINITY)) out[(size_t)(group.out_row ? group.out_row[row] : row) * N + col] = value;
-                } else {
-                    if (fabsf(value) < INFINITY) continue;
-                    if (bias) value += bias[col];
-                    if (epilogue == MLLM_EPI_GELU_TANH) value = gelu_tanh(value);
-                    else if (epilogue == MLLM_EPI_GELU_ERF) value = gelu_erf(value);
-                    else if (epilogue == MLLM_EPI_SQUARED_RELU) value = squared_relu(value);
-                    if (!scatter.enabled || col < scatter.q_width) {
-                        const size_t at = (size_t)row * (scatter.enabled ? scatter.q_width : N) + col;
-                        out[at] = residual && residual != out ? residual[at] + value : value;   // (in place the residual is gone, and changes nothing that is not finite)
-                        continue;
-                    }
-                    const int slot = scatter.slots[row];
-                    if (slot < 0) continue;
-                    int c = col - scatter.q_width;
-                    float* to = (float*)(c < scatter.kv_width ? scatter.k_pages : scatter.v_pages);
-                    if (c >= scatter.kv_width) c -= scatter.kv_width;
-                    const int page = slot >> scatter.page_shift, offset = slot & ((1 << scatter.page_shift) - 1);
-                    to[((((size_t)page * scatter.n_kv_heads + c / scatter.head_size) << scatter.page_shift) + offset) * scatter.head_size + c % scatter.head_size] = value;
-                }
+                for (int e = 0; e < 4; e++) sum[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[t][e], b[e], sum[t], 0, 0, 0);
+        }
+        // sum[t][e] of a lane: row lane % 16, column 16 t + 4 (lane / 16) + e of the wave's
+        const int row = row0 + g * 16 + row16;
+        if (row >= m_end || !(rows >> row16 & 1)) continue;
+        if constexpr (Group::GATED) {
+            const float weight = group.weight[row], in_weight = group.weigh_input ? weight : 1.0f, out_weight = group.weigh_input ? 1.0f : weight;
+#pragma unroll
+            for (int t = 0; t < TILES / 2; t++) {   // 32 gate columns, two tiles of them, and the 32 up columns behind them
+                const int col = col0 / 2 + t * 16 + 4 * quad, gate = t / 2 * 4 + t % 2;
+                if (col >= out_cols) continue;
+                f32x4 value;
+#pragma unroll
+                for (int e = 0; e < 4; e++) value[e] = gated(sum[gate][e] * in_weight, sum[gate + 2][e] * in_weight, group.unit) * out_weight;
+                put(row, col, Place{nullptr, 0, 0}, value);
             }
+        } else {
+#pragma unroll
+            for (int t = 0; t < TILES; t++) {
+                const int col = col0 + t * 16 + 4 * quad;
+                if (col >= out_cols) continue;
+                f32x4 value = sum[t];
+                if (!Group::GROUPED && bias) value += *reinterpret_cast<const f32x4*>(bias + col);
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    if (!Group::GROUPED && epilogue == MLLM_EPI_GELU_TANH) value[e] = gelu_tanh(value[e]);
+                    else if (!Group::GROUPED && epilogue == MLLM_EPI_GELU_ERF) value[e] = gelu_erf(value[e]);
+                    else if (!Group::GROUPED && epilogue == MLLM_EPI_SQUARED_RELU) value[e] = squared_relu(value[e]);
+                }
+                put(row, col, place_of(col), value);
+            }
+        }
     }
 }
 

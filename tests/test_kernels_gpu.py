@@ -1124,6 +1124,65 @@ def test_32_bit_products_in_pieces_with_infinities_and_no_numbers(K):
     np.testing.assert_allclose(got[:, rest], ref[:, rest], rtol=2e-5, atol=2e-5)
 
 
+def test_32_bit_products_in_pieces_settle_infinities_in_every_output(K):
+    # bias and activation, a residual added in place, q/k/v columns into pages, a product cut along K: against the 32-bit instruction (a row-major W takes
+    # it). Bounds: sums of 96 numbers around 1.
+    rng = np.random.default_rng(11)
+    heads, size, page = 2, 16, 32
+    m, n, k = 150, 3 * heads * size, 96
+    x, w, b = rng.standard_normal((m, k)).astype(np.float32), rng.standard_normal((n, k)).astype(np.float32), rng.standard_normal(n).astype(np.float32)
+    x[7, 3], x[70, 40], x[100, 1], x[149, 0], x[149, 50], x[33, 0] = np.inf, -np.inf, np.nan, np.inf, -np.inf, np.finfo(np.float32).max
+    w[41, 9], w[n - 1, 60] = np.inf, np.nan
+    packed, plain = K.pack_matrix(dev(w)), dev(w)
+    same = lambda got, want: np.testing.assert_allclose(host(got), host(want), rtol=2e-5, atol=2e-5)   # (infinities and what is no number in the same places)
+    for activation in (None, "gelu_new", "gelu", "squared_relu"):
+        same(K.linear(dev(x), packed, dev(b), activation), K.linear(dev(x), plain, dev(b), activation))
+    residual = rng.standard_normal((m, n)).astype(np.float32)
+    residual[7, ::2], residual[70, ::3], residual[50, 41], residual[51, 41], residual[8] = -np.inf, np.inf, np.nan, -np.inf, np.inf
+    there, here = dev(residual), dev(residual)
+    want = K.linear(dev(x), plain, dev(b), residual=dev(residual))
+    same(K.linear(dev(x), packed, dev(b), residual=there), want)
+    same(K.linear(dev(x), packed, dev(b), residual=here, out=here), want)
+    slots = rng.permutation(5 * page)[:m].astype(np.int32)
+    slots[12] = -1
+    taken = []
+    for weight in (packed, plain):
+        k_pages = torch.zeros((5, heads, page, size), device=DEV)
+        v_pages = torch.zeros_like(k_pages)
+        taken.append((K.linear_qkv_cache(dev(x), weight, dev(b), k_pages, v_pages, dev(slots, torch.int32), heads, heads, size), k_pages, v_pages))
+    for got, want in zip(*taken):
+        same(got, want)
+    whole = host(K.linear(dev(x), plain))
+    with np.errstate(invalid="ignore"):
+        for blocks in (2, 3):
+            parts = host(K.linear_split(dev(x), packed, blocks))
+            np.testing.assert_allclose(parts.sum(axis=0), whole, rtol=2e-5, atol=2e-5)
+
+
+@pytest.mark.parametrize("limit", [7.0, None])
+def test_grouped_experts_in_pieces_with_an_infinity_beside_a_finite_sum(K, limit):
+    # a gate or up sum that is infinite is clamped, and its partner counts in full: bounds of the routed experts' tests in 32-bit
+    rng = np.random.default_rng(12)
+    rows, experts, units, width, top = 260, 3, 64, 96, 2
+    x = rng.standard_normal((rows, width)).astype(np.float32)
+    gate, up = (rng.standard_normal((experts, units, width)).astype(np.float32) * 0.2 for _ in range(2))
+    down = rng.standard_normal((experts, width, units)).astype(np.float32)
+    up[0, 5, 17], gate[1, 9, 30], x[20, 4], x[21, 5] = np.inf, np.inf, np.inf, np.nan
+    picked = np.stack([np.arange(rows) % experts, (np.arange(rows) + 1) % experts], axis=1).astype(np.int32)
+    weights = rng.uniform(0.5, 1.5, (rows, top)).astype(np.float32)
+    laid = np.stack([gate.reshape(experts, units // 32, 32, width), up.reshape(experts, units // 32, 32, width)], axis=2).reshape(-1, width)
+    out = host(K.grouped_experts(dev(x), K.Picks(dev(picked, torch.int32), dev(weights)), K.pack_matrix(dev(laid)), K.pack_matrix(dev(down.reshape(-1, units))), experts, units,
+                                 limit=limit, alpha=1.702, shift=1.0))
+    bound = np.inf if limit is None else limit
+    with np.errstate(invalid="ignore", over="ignore"):
+        for place in range(top):
+            for r in range(rows):
+                e = picked[r, place]
+                g, u = np.fmin(gate[e].astype(np.float64) @ x[r], bound), np.fmin(np.fmax(up[e].astype(np.float64) @ x[r], -bound), bound)
+                want = down[e].astype(np.float64) @ (g / (1 + np.exp(-1.702 * g)) * (u + 1) * weights[r, place])
+                np.testing.assert_allclose(out[place, r], want, rtol=2e-4, atol=2e-4)
+
+
 @pytest.mark.parametrize("m", [17, 32, 33, 64])
 @pytest.mark.parametrize("n,k,k_blocks", [(4616, 320, 1), (4632, 1400, 1), (8184, 256, 1), (1592, 2048, 5), (2304, 1288, 2), (4618, 256, 1)])
 def test_products_of_few_rows_with_two_tiles_of_columns_a_block(K, m, n, k, k_blocks):
