@@ -58,7 +58,7 @@ __host__ __device__ __forceinline__ size_t packed_element(int row, int col, int 
 }
 
 // How a matrix is given to a product (w_packed): row-major, packed, or packed with its pieces behind it (32-bit only; gemm_pieces.h). The pieces: for
-// every 16 rows x 32 columns three chunks of 1 KiB in the packed layout for bfloat16 (high, middle and low eight bits), row tiles outermost, behind the
+// every 16 rows x 32 columns three chunks of 1 KiB in the packed layout for bfloat16 (the number rounded, what that leaves rounded, and the rest), row tiles outermost, behind the
 // last chunk of the packed matrix.
 enum MllmPacked : int { ROW_MAJOR = 0, PACKED = 1, PACKED_WITH_PIECES = 2 };
 __host__ __device__ __forceinline__ long long packed_pieces_at(int row_tiles, int k_steps) { return (long long)row_tiles * k_steps * 1024; }

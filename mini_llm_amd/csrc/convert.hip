@@ -65,10 +65,13 @@ __global__ __launch_bounds__(256) void pack_pieces_kernel(const float* __restric
         float rest = col < cols ? packed[packed_element<float>(row_tile * 16 + lane % 16, col, cols)] : 0.0f;
 #pragma unroll
         for (int p = 0; p < 3; p++) {
-            const uint32_t bits = __builtin_bit_cast(uint32_t, rest) & 0xffff0000u;
-            const uint16_t upper = (uint16_t)(bits >> 16);
-            out[p][e] = __builtin_bit_cast(bf16_t, upper);
-            rest -= __builtin_bit_cast(float, bits);
+            bf16_t piece = from_float<bf16_t>(rest);
+            if (fabsf(to_float(piece)) == INFINITY && fabsf(rest) < INFINITY) {   // rounded beyond the largest: cut off instead
+                const uint16_t upper = (uint16_t)(__builtin_bit_cast(uint32_t, rest) >> 16);
+                piece = __builtin_bit_cast(bf16_t, upper);
+            }
+            out[p][e] = piece;
+            rest -= to_float(piece);
         }
     }
 #pragma unroll

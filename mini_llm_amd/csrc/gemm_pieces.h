@@ -1,10 +1,11 @@
 // The 32-bit product for many rows on the bfloat16 matrix cores. Included by gemm.hip.
 //
-// A 32-bit number is the sum of three bfloat16 ones, exactly (eight bits each, cut off and not rounded, so that all three have its sign and none
-// overflows), and a product of two such numbers is the sum of nine products of pieces, each exact in 32-bit. The six largest reach down to the 24th bit;
-// the matrix instruction for bfloat16 does in 32 cycles sixteen times the work that the 32-bit one does in 64, so six of them are 2.7 times faster, and
+// A 32-bit number is the sum of three bfloat16 ones, each what the one before leaves, rounded to the nearest, and a product of two such numbers is the sum of
+// nine products of pieces, each exact in 32-bit. The three left out are at most 2^-24 of the product and lie on either side of it. (Pieces cut off instead
+// of rounded leave out up to 2^-21, always on the product's own side: over 3,072 positive numbers the sums came out 6.5e-6 too small, 7e-8 with rounding.)
+// The matrix instruction for bfloat16 does in 32 cycles eight times the work that the 32-bit one does in 64, so six of them are 2.7 times faster, and
 // there are fewer roundings of a running sum (six for sixteen numbers of K instead of eight). Measured against 64-bit sums over rows of 768 to 3,072
-// normally distributed numbers: 4.3e-7 to 8.7e-7 of the result's norm, 5.0e-7 to 9.9e-7 with the 32-bit instruction.
+// normally distributed numbers: 4.2e-7 to 8.6e-7 of the result's norm, 5.0e-7 to 9.9e-7 with the 32-bit instruction.
 //
 // W's pieces are laid out once, when the matrix is packed (common.h: packed_pieces): the chunks of the packed layout for bfloat16, the three of a k-step
 // behind each other. A's rows come as they are, and a wave splits the fragments it has read.
@@ -32,21 +33,28 @@ __device__ __forceinline__ void ask(i32x4& to, unsigned address) {
 __device__ __forceinline__ void landed(i32x4& first) { asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(first)); }
 __device__ __forceinline__ void this_too(i32x4& fragment) { asm volatile("" : "+v"(fragment)); }
 
-// Eight numbers -> three operands of pieces.
+// Eight numbers -> three operands of pieces. (A number that the first rounding makes infinite leaves sums that are not finite, as an infinity does.)
 __device__ __forceinline__ void split(const i32x4 (&raw)[2], bf16x8 (&out)[3]) {
-    uint32_t rest[8];
+    typedef float f32x2 __attribute__((ext_vector_type(2)));
+    typedef bf16_t bf16x2 __attribute__((ext_vector_type(2)));
+    float rest[8];
 #pragma unroll
-    for (int e = 0; e < 8; e++) rest[e] = (uint32_t)raw[e / 4][e % 4];
+    for (int e = 0; e < 8; e++) {
+        const int bits = raw[e / 4][e % 4];
+        rest[e] = __builtin_bit_cast(float, bits);
+    }
 #pragma unroll
     for (int p = 0; p < 3; p++) {
         uint32_t pairs[4];
 #pragma unroll
-        for (int e = 0; e < 4; e++) pairs[e] = __builtin_amdgcn_perm(rest[2 * e + 1], rest[2 * e], 0x07060302);   // the upper halves of two
-        out[p] = *reinterpret_cast<bf16x8*>(pairs);
-        if (p < 2) {
-#pragma unroll
-            for (int e = 0; e < 8; e++) rest[e] = __builtin_bit_cast(uint32_t, __builtin_bit_cast(float, rest[e]) - __builtin_bit_cast(float, rest[e] & 0xffff0000u));
+        for (int e = 0; e < 4; e++) {
+            pairs[e] = __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2{rest[2 * e], rest[2 * e + 1]}), bf16x2));
+            if (p < 2) {
+                rest[2 * e] -= __builtin_bit_cast(float, pairs[e] << 16);
+                rest[2 * e + 1] -= __builtin_bit_cast(float, pairs[e] & 0xffff0000u);
+            }
         }
+        out[p] = *reinterpret_cast<bf16x8*>(pairs);
     }
 }
 

@@ -1095,7 +1095,7 @@ def test_32_bit_products_in_pieces_are_no_less_exact_than_32_bit_ones(K, m, n, k
     errors = [np.linalg.norm((host(K.linear(dev(x), weight)) - ref) / size) for weight in (K.pack_matrix(dev(w)), dev(w))]
     assert errors[0] <= 1.2 * errors[1]
     # every matrix instruction may leave the running sum a unit in its last place off (2^-23 of at most `size`), and there are six for sixteen numbers of
-    # K; the pieces' products that are left out are below 2^-22 of a product
+    # K; the pieces' products that are left out are at most 2^-24 of a product
     bound = 2**-23 * (6 * k / 16 + 2)
     assert np.abs((host(K.linear(dev(x), K.pack_matrix(dev(w)))) - ref) / size).max() < bound
     for blocks in (2, 5):   # (with fewer tiles of K than blocks the last ones have none: zeros)
@@ -1122,6 +1122,26 @@ def test_32_bit_products_in_pieces_with_infinities_and_no_numbers(K):
     np.testing.assert_array_equal(got[:, 40], ref[:, 40])
     rest = [c for c in range(72) if c != 40]
     np.testing.assert_allclose(got[:, rest], ref[:, rest], rtol=2e-5, atol=2e-5)
+
+
+def test_32_bit_products_in_pieces_lean_to_no_side(K):
+    # numbers of one sign: what the pieces leave out must not always lie on the same side
+    rng = np.random.default_rng(21)
+    x, w = np.abs(rng.standard_normal((300, 3072))).astype(np.float32), np.abs(rng.standard_normal((260, 3072))).astype(np.float32)
+    ref = x.astype(np.float64) @ w.astype(np.float64).T
+    pieces, plain = (host(K.linear(dev(x), weight)) / ref - 1 for weight in (K.pack_matrix(dev(w)), dev(w)))
+    assert np.linalg.norm(pieces) <= np.linalg.norm(plain) and abs(pieces.mean()) < 2**-22
+    # one product a sum, of numbers whose lower sixteen bits are all set and others: the left out (at most 2^-24 of the product) and two roundings of the sum
+    # that a matrix instruction may leave a unit in the last place off
+    a = ((rng.integers(100, 150, (96, 1)) << 23) | rng.integers(0, 2**23, (96, 1))).astype(np.uint32)
+    a[:40] = (a[:40] & 0xffff0000) | 0xffff
+    a = a.view(np.float32)
+    x = np.zeros((96, 64), dtype=np.float32)
+    x[:, 5:6] = a
+    w = np.zeros((96, 64), dtype=np.float32)
+    w[:, 5:6] = a
+    ref = x.astype(np.float64) @ w.astype(np.float64).T
+    assert np.abs(host(K.linear(dev(x), K.pack_matrix(dev(w)))) / ref - 1).max() < 2**-24 + 2 * 2**-24
 
 
 def test_32_bit_products_in_pieces_settle_infinities_in_every_output(K):
