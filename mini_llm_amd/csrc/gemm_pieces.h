@@ -3,9 +3,12 @@
 // A 32-bit number is the sum of three bfloat16 ones, each what the one before leaves, rounded to the nearest, and a product of two such numbers is the sum of
 // nine products of pieces, each exact in 32-bit. The three left out are at most 2^-24 of the product and lie on either side of it. (Pieces cut off instead
 // of rounded leave out up to 2^-21, always on the product's own side: over 3,072 positive numbers the sums came out 6.5e-6 too small, 7e-8 with rounding.)
-// The matrix instruction for bfloat16 does in 32 cycles eight times the work that the 32-bit one does in 64, so six of them are 2.7 times faster, and
-// there are fewer roundings of a running sum (six for sixteen numbers of K instead of eight). Measured against 64-bit sums over rows of 768 to 3,072
-// normally distributed numbers: 4.2e-7 to 8.6e-7 of the result's norm, 5.0e-7 to 9.9e-7 with the 32-bit instruction.
+// The matrix instruction for bfloat16 does in 32 cycles eight times the work that the 32-bit one does in 64, so six of them are 2.7 times faster. The five
+// smaller products have a running sum of their own, added to the large one at the end: in one sum they are lost to its rounding once it is long, and it is
+// rounded six times for sixteen numbers of K instead of once (the 32-bit instruction: eight times). Measured against 64-bit sums over rows of 768 and 3,072
+// normally distributed numbers: 1.6e-7 and 3.4e-7 of the result's norm, in one sum 4.2e-7 and 8.6e-7, with the 32-bit instruction 5.0e-7 and 9.9e-7; over
+// rows of which half are zero, as behind a clamp, 1.2e-7 and 2.7e-7, 4.0e-7 and 8.2e-7, 3.5e-7 and 7.1e-7. It is the 64 registers that the 128 x 128 tile
+// has left (188 -> 252, none spilled), and no time: 2,048 x 3,072 x 768 60.6 us, 61.6 in one sum.
 //
 // W's pieces are laid out once, when the matrix is packed (common.h: packed_pieces): the chunks of the packed layout for bfloat16, the three of a k-step
 // behind each other. A's rows come as they are, and a wave splits the fragments it has read.
@@ -118,7 +121,7 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N, 2) void gemm_pieces_kernel(
         w_tile += 3072;
     };
 
-    f32x16 acc[TN][TM];
+    f32x16 acc[TN][TM], low[TN][TM];   // the sums of the high pieces' products, and of the five others
     const unsigned base = (unsigned)(size_t)(const __attribute__((address_space(3))) unsigned char*)piece_lds;
     unsigned a_at[2][2];   // [step of 16][piece]
 #pragma unroll
@@ -133,7 +136,7 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N, 2) void gemm_pieces_kernel(
 #pragma unroll
         for (int i = 0; i < TM; i++)
 #pragma unroll
-            for (int v = 0; v < 16; v++) acc[j][i][v] = 0.0f;
+            for (int v = 0; v < 16; v++) acc[j][i][v] = low[j][i][v] = 0.0f;
     if (tiles > 0) issue(0);
     for (int t = 0; t < tiles; t++) {
         // this wave's loads of the tile have landed; behind the barrier everybody's have, and nobody reads the other stage any more
@@ -168,8 +171,10 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N, 2) void gemm_pieces_kernel(
 #pragma unroll
                 for (int i = 0; i < TM; i++)
 #pragma unroll
-                    for (int j = 0; j < TN; j++)
-                        acc[j][i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*reinterpret_cast<const bf16x8*>(&w[kk][OF_W[c]][j]), a[kk][i][OF_A[c]], acc[j][i], 0, 0, 0);
+                    for (int j = 0; j < TN; j++) {
+                        f32x16& to = c < 5 ? low[j][i] : acc[j][i];
+                        to = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*reinterpret_cast<const bf16x8*>(&w[kk][OF_W[c]][j]), a[kk][i][OF_A[c]], to, 0, 0, 0);
+                    }
         };
         ask_step(std::integral_constant<int, 0>{});
         wait_step(0);
@@ -184,6 +189,10 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N, 2) void gemm_pieces_kernel(
         multiply(1);
     }
 
+#pragma unroll
+    for (int j = 0; j < TN; j++)
+#pragma unroll
+        for (int i = 0; i < TM; i++) acc[j][i] += low[j][i];
     const int row0 = m0 + wave_m * WM, col0 = n0 + wave_n * WN;
     __syncthreads();   // the slabs below lie where the tiles did
 

@@ -1144,6 +1144,24 @@ def test_32_bit_products_in_pieces_lean_to_no_side(K):
     assert np.abs(host(K.linear(dev(x), K.pack_matrix(dev(w)))) / ref - 1).max() < 2**-24 + 2 * 2**-24
 
 
+@pytest.mark.parametrize("m,n,k", [(130, 768, 768), (520, 260, 3072), (2048, 200, 320)])   # tiles of each size
+@pytest.mark.parametrize("kind", ["normal", "relu", "one sign"])
+def test_32_bit_products_in_pieces_are_nearer_than_32_bit_ones(K, m, n, k, kind):
+    # the small products have a running sum of their own, so the large one is rounded once for sixteen numbers of K, where the 32-bit instruction rounds
+    # eight times: errors against 64 bits below its own, whatever the signs
+    rng = np.random.default_rng(m + k)
+    x, w = rng.standard_normal((m, k)).astype(np.float32), rng.standard_normal((n, k)).astype(np.float32)
+    if kind != "normal":
+        x = np.maximum(x, 0) if kind == "relu" else np.abs(x)
+    if kind == "one sign":
+        w = np.abs(w)
+    ref = x.astype(np.float64) @ w.astype(np.float64).T
+    pieces, plain = (np.linalg.norm(host(K.linear(dev(x), weight)) - ref) for weight in (K.pack_matrix(dev(w)), dev(w)))
+    assert pieces <= 0.6 * plain
+    parts = np.linalg.norm(host(K.linear_split(dev(x), K.pack_matrix(dev(w)), 2)).sum(axis=0) - ref)
+    assert parts <= 0.6 * plain
+
+
 def test_32_bit_products_in_pieces_settle_infinities_in_every_output(K):
     # bias and activation, a residual added in place, q/k/v columns into pages, a product cut along K: against the 32-bit instruction (a row-major W takes
     # it). Bounds: sums of 96 numbers around 1.
