@@ -233,10 +233,10 @@ def _capture(runner, batch, choice=None, lanes=None):
         from dataclasses import replace
 
         warm["choice"] = replace(choice, token_slots=torch.empty_like(choice.token_slots), host_ring=None, cursor=None, advance=False)
-    side = torch.cuda.Stream(device=runner.device)
-    side.wait_stream(torch.cuda.current_stream())
     cache = getattr(runner, "cache", None)
     kept_state = cache.snapshot_state() if cache is not None else None   # a mixer that keeps state moves it on in place: the warm-up must not count
+    side = torch.cuda.Stream(device=runner.device)
+    side.wait_stream(torch.cuda.current_stream())   # behind the copy of the state: the warm-up changes what is being copied
     with torch.cuda.stream(side):
         runner.forward(batch, **warm)
     torch.cuda.current_stream().wait_stream(side)

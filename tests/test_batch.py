@@ -157,3 +157,54 @@ def test_hot_shapes_beyond_the_kept_graphs_are_not_captured_at_every_turn():
         for entries in shapes[:-1]:
             runner._portion_graph_for(entries)
     assert runner.portion_graphs_made == step_module.PORTION_GRAPHS_KEPT and runner.portion_graphs_dropped == 0
+
+
+def test_the_warm_up_of_a_capture_waits_for_the_copy_of_the_state(monkeypatch):
+    # Streams as sets of what is sure to have ended before whatever is queued next. The warm-up moves the state on in place, so it may begin only behind the
+    # copy, and the copy may be put back only behind the warm-up.
+    import contextlib
+
+    import torch
+
+    from mini_llm_amd.engine import step
+
+    class Stream:
+        def __init__(self, **_):
+            self.behind = set()
+
+        def wait_stream(self, other):
+            self.behind |= other.behind
+
+    main, current, before = Stream(), [], {}
+    current.append(main)
+
+    def queued(name):
+        before[name] = set(current[-1].behind)
+        current[-1].behind.add(name)
+
+    @contextlib.contextmanager
+    def on(stream):
+        current.append(stream)
+        yield
+        current.pop()
+
+    class Cache:
+        def snapshot_state(self):
+            queued("copy")
+            return {"layer": None}
+
+        def restore_state(self, _):
+            queued("put back")
+
+    class Runner:
+        device, cache = "cuda:0", Cache()
+
+        def forward(self, batch, **_):
+            queued("captured" if "warm-up" in before else "warm-up")
+
+    for name, fake in (("Stream", Stream), ("current_stream", lambda *_: current[-1]), ("stream", on), ("synchronize", lambda *_: None),
+                       ("CUDAGraph", object), ("graph", lambda _: on(Stream()))):
+        monkeypatch.setattr(torch.cuda, name, fake)
+    step._capture(Runner(), None)
+    assert "copy" in before["warm-up"]
+    assert "warm-up" in before["put back"]
