@@ -59,10 +59,17 @@ __host__ __device__ __forceinline__ size_t packed_element(int row, int col, int 
 
 // How a matrix is given to a product (w_packed): row-major, packed, or packed with its pieces behind it (32-bit only; gemm_pieces.h). The pieces: for
 // every 16 rows x 32 columns three chunks of 1 KiB in the packed layout for bfloat16 (the number rounded, what that leaves rounded, and the rest), row tiles outermost, behind the
-// last chunk of the packed matrix.
+// last chunk of the packed matrix; behind them what is known of every 16 rows (TileRows).
 enum MllmPacked : int { ROW_MAJOR = 0, PACKED = 1, PACKED_WITH_PIECES = 2 };
 __host__ __device__ __forceinline__ long long packed_pieces_at(int row_tiles, int k_steps) { return (long long)row_tiles * k_steps * 1024; }
 __host__ __device__ __forceinline__ long long packed_pieces_bytes(int row_tiles, int cols) { return (long long)row_tiles * ((cols + 31) / 32) * 3072; }
+
+// Whether numbers with these bits set among them are all below 2^-95, and some are not zero.
+__host__ __device__ __forceinline__ bool tiny(uint32_t bits) { return (bits & 0x70000000u) == 0 && (bits & 0x0fffffffu) != 0; }
+struct TileRows {
+    int tiny;      // bit r: row r is tiny throughout
+    int largest;   // the bits of the largest magnitude
+};
 
 void mllm_set_error(const char* format, ...);
 int mllm_check_launch(const char* what);

@@ -78,6 +78,23 @@ __global__ __launch_bounds__(256) void pack_pieces_kernel(const float* __restric
     for (int p = 0; p < 3; p++) *reinterpret_cast<bf16x8*>(pieces + (step * 3 + p) * 1024 + lane * 16) = out[p];
 }
 
+// What the product in pieces asks of every sixteen rows of the packed 32-bit matrix: a wave each.
+__global__ __launch_bounds__(64) void tile_rows_kernel(const float* __restrict__ packed, TileRows* __restrict__ out, int cols) {
+    const int lane = threadIdx.x, k_steps = packed_k_steps<float>(cols);
+    uint32_t bits = 0, largest = 0;   // of row lane % 16
+    for (int step = 0; step < k_steps; step++) {
+        const Vec16 piece = *reinterpret_cast<const Vec16*>(packed + packed_offset<float>(blockIdx.x, step, k_steps, lane));
+#pragma unroll
+        for (int e = 0; e < 4; e++) bits |= piece.w[e], largest = max(largest, piece.w[e] & 0x7fffffffu);
+    }
+    bits |= (uint32_t)__shfl_xor((int)bits, 16, WAVE);
+    bits |= (uint32_t)__shfl_xor((int)bits, 32, WAVE);
+#pragma unroll
+    for (int offset = 32; offset > 0; offset >>= 1) largest = max(largest, (uint32_t)__shfl_xor((int)largest, offset, WAVE));
+    const unsigned long long lanes = __ballot(tiny(bits));
+    if (lane == 0) out[blockIdx.x] = TileRows{(int)(lanes & 0xffff), (int)largest};
+}
+
 template <typename S, typename D>
 void launch_pack(const void* src, void* dst, int rows, int cols, int transpose, hipStream_t stream) {
     const size_t chunks = (size_t)ceil_div(rows, 16) * ceil_div(cols, 4 * (16 / (int)sizeof(D)));
@@ -127,8 +144,8 @@ MLLM_API int mllm_pack_matrix(const void* src, void* dst, int rows, int cols, in
     return mllm_check_launch("pack_matrix");
 }
 
-// Bytes the pieces of a packed 32-bit matrix take behind it.
-MLLM_API long long mllm_pieces_bytes(int rows, int cols) { return packed_pieces_bytes(ceil_div(rows, 16), cols); }
+// Bytes the pieces of a packed 32-bit matrix take behind it, with what is known of its rows.
+MLLM_API long long mllm_pieces_bytes(int rows, int cols) { return packed_pieces_bytes(ceil_div(rows, 16), cols) + (long long)sizeof(TileRows) * ceil_div(rows, 16); }
 
 // Lays the pieces of a packed 32-bit matrix [rows, cols] behind it, at packed + mllm_packed_elements.
 MLLM_API int mllm_pack_pieces(float* packed, int rows, int cols, hipStream_t stream) {
@@ -138,5 +155,7 @@ MLLM_API int mllm_pack_pieces(float* packed, int rows, int cols, hipStream_t str
     const size_t steps = (size_t)row_tiles * ceil_div(cols, 32);
     mllm_count_kernel(MLLM_K_PACK);
     pack_pieces_kernel<<<(unsigned)((steps + 3) / 4), 256, 0, stream>>>(packed, pieces, row_tiles, cols);
+    mllm_count_kernel(MLLM_K_PACK);
+    tile_rows_kernel<<<row_tiles, 64, 0, stream>>>(packed, reinterpret_cast<TileRows*>(pieces + packed_pieces_bytes(row_tiles, cols)), cols);
     return mllm_check_launch("pack_pieces");
 }

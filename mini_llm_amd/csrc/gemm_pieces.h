@@ -8,7 +8,7 @@
 // rounded six times for sixteen numbers of K instead of once (the 32-bit instruction: eight times). Measured against 64-bit sums over rows of 768 and 3,072
 // normally distributed numbers: 1.6e-7 and 3.4e-7 of the result's norm, in one sum 4.2e-7 and 8.6e-7, with the 32-bit instruction 5.0e-7 and 9.9e-7; over
 // rows of which half are zero, as behind a clamp, 1.2e-7 and 2.7e-7, 4.0e-7 and 8.2e-7, 3.5e-7 and 7.1e-7. It is the 64 registers that the 128 x 128 tile
-// has left (188 -> 252, none spilled), and no time: 2,048 x 3,072 x 768 60.6 us, 61.6 in one sum.
+// has left (188 -> 252, none spilled), and no time: 2,048 x 3,072 x 768 60.6 us, 63.2 in one sum.
 //
 // W's pieces are laid out once, when the matrix is packed (common.h: packed_pieces): the chunks of the packed layout for bfloat16, the three of a k-step
 // behind each other. A's rows come as they are, and a wave splits the fragments it has read.
@@ -130,6 +130,13 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N, 2) void gemm_pieces_kernel(
         for (int q = 0; q < 2; q++) a_at[kk][q] = base + (wave_m * WM + lane32) * 128 + (((kk * 4 + half * 2 + q) ^ (lane32 / 2 % 8)) * 16);
     const unsigned w_at = base + A_BYTES + (wave_n * TN * 2 + lane32 / 16) * 3072 + half * 256 + (lane % 16) * 16;
 
+    // of the wave's columns: whether one has a row of W that is tiny throughout, and the largest magnitude in W
+    int w_tiny = 0, w_largest = 0;
+#pragma unroll
+    for (int t = 0; t < WN / 16; t++) {
+        const TileRows rows = reinterpret_cast<const TileRows*>(w_pieces + packed_pieces_bytes(matrix_tiles, K))[first_tile + min((n0 + wave_n * WN) / 16 + t, row_tiles - 1)];
+        w_tiny |= rows.tiny, w_largest = max(w_largest, rows.largest);
+    }
     const int tiles = (k_end - k_begin + BK - 1) / BK;
 #pragma unroll
     for (int j = 0; j < TN; j++)
@@ -196,37 +203,52 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N, 2) void gemm_pieces_kernel(
     const int row0 = m0 + wave_m * WM, col0 = n0 + wave_n * WN;
     __syncthreads();   // the slabs below lie where the tiles did
 
-    // An infinity has no pieces (its middle is no number), so every sum it belongs to comes out as no number, whatever it should be. The rows of this wave
-    // with a sum that is not finite (bit r: row r of the WM) are left out of what is stored below and taken again in 32-bit at the end.
-    // What a row holds that is no number itself makes all its sums none, as it should: such a row stays as it is. (Rows that nobody reads may hold anything,
-    // and those with an infinity become that behind the next norm.)
+    // An infinity has no pieces (its middle is no number), so every sum it belongs to comes out as no number, whatever it should be. And below 2^-110 the
+    // last piece of a number falls under the smallest bfloat16 number: what is lost, up to 2^-134, counts where a row has nothing larger. The rows of this
+    // wave with a sum that is not finite, and those that are tiny throughout (bit r: row r of the WM), are left out of what is stored below and taken again
+    // in 32-bit at the end. What a row holds that is no number itself makes all its sums none, as it should: such a row stays as it is. (Rows that nobody
+    // reads may hold anything, and those with an infinity become that behind the next norm.)
+    // Whether a row is tiny is not asked while it is split (four instructions for eight numbers: 1.5 % of a pass of ragged prompts) but read again where its
+    // sums are no larger than a tiny row's could be.
     static_assert(TM <= 2, "a bit a row");
-    unsigned long long bad = 0;
+    const float faint_sum = ldexpf(__builtin_bit_cast(float, w_largest), -94) * (float)(k_end - k_begin);   // (twice as much, for the roundings)
+    unsigned long long bad = 0, faint = 0;
 #pragma unroll
     for (int i = 0; i < TM; i++) {
-        float any = 0.0f;
+        float largest = 0.0f;   // no number if one of them is none (the instruction keeps that: one for two sums)
 #pragma unroll
         for (int j = 0; j < TN; j++)
 #pragma unroll
-            for (int v = 0; v < 16; v++) any = __builtin_fmaf(acc[j][i][v], 0.0f, any);   // no number where one of them is not finite
-        const unsigned long long lanes = __ballot(any != any);
+            for (int v = 0; v < 16; v++) largest = __builtin_elementwise_maximum(largest, fabsf(acc[j][i][v]));
+        const unsigned long long lanes = __ballot(!(largest < INFINITY));
         bad |= (unsigned long long)((unsigned)lanes | (unsigned)(lanes >> 32)) << (32 * i);
+        largest = fmaxf(largest, __shfl_xor(largest, 32, WAVE));
+        faint |= (unsigned long long)(unsigned)__ballot(largest > 0.0f && largest <= faint_sum) << (32 * i);
     }
     const int row16 = lane % 16, quad = lane / 16, rows_here = m_end - row0;
-    if (rows_here < WM) bad = rows_here > 0 ? bad & ((1ull << rows_here) - 1) : 0;   // (beyond the last row: that row again)
-    if (bad != 0) {
+    const unsigned long long real = rows_here >= WM ? ~0ull >> (64 - WM) : rows_here > 0 ? (1ull << rows_here) - 1 : 0;   // (beyond the last row: that row again)
+    if (w_tiny != 0) bad = ~0ull;
+    bad &= real, faint &= real;
+    if ((bad | faint) != 0) {
 #pragma unroll 1
         for (int g = 0; g < WM / 16; g++) {
-            if ((bad >> (16 * g) & 0xffff) == 0) continue;
+            if (((bad | faint) >> (16 * g) & 0xffff) == 0) continue;
             const float* x = A + (size_t)a_row(wave_m * WM + g * 16 + row16) * K + 4 * quad;
             bool none = false;
+            uint32_t bits = 0;
             for (int k = k_begin; k < k_end; k += 16) {
-                const f32x4 piece = *reinterpret_cast<const f32x4*>(x + k);
+                const Vec16 piece = *reinterpret_cast<const Vec16*>(x + k);
 #pragma unroll
-                for (int e = 0; e < 4; e++) none |= piece[e] != piece[e];
+                for (int e = 0; e < 4; e++) {
+                    none |= (piece.w[e] & 0x7fffffffu) > 0x7f800000u;
+                    bits |= piece.w[e];
+                }
             }
-            const unsigned long long lanes = __ballot(none);
+            bits |= (uint32_t)__shfl_xor((int)bits, 16, WAVE);
+            bits |= (uint32_t)__shfl_xor((int)bits, 32, WAVE);
+            const unsigned long long lanes = __ballot(none), tiny_rows = __ballot(tiny(bits)) & 0xffff;
             bad &= ~(((lanes | lanes >> 16 | lanes >> 32 | lanes >> 48) & 0xffff) << (16 * g));
+            bad |= faint & tiny_rows << (16 * g);
         }
     }
 
@@ -299,7 +321,7 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N, 2) void gemm_pieces_kernel(
             for (int r = 0; r < 32 / ROWS; r++) {
                 const int in_slab = r * ROWS + lane / LANES_A_ROW, row = row0 + i * 32 + in_slab;
                 f32x4 value = *reinterpret_cast<const f32x4*>(slab + in_slab * SLAB_ROW + (lane % LANES_A_ROW) * 4);
-                if (row >= m_end || out_col >= out_cols || (bad >> (i * 32 + in_slab) & 1)) continue;
+                if (row >= m_end || out_col >= out_cols || ((unsigned)(bad >> (i * 32)) >> in_slab & 1)) continue;
                 put(row, out_col, place, value);
             }
             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");

@@ -1162,6 +1162,26 @@ def test_32_bit_products_in_pieces_are_nearer_than_32_bit_ones(K, m, n, k, kind)
     assert parts <= 0.6 * plain
 
 
+@pytest.mark.parametrize("exponent", [-90, -100, -112, -120, -126])
+@pytest.mark.parametrize("where", ["x", "rows of x", "w", "a row of w"])
+def test_32_bit_products_in_pieces_of_tiny_numbers(K, exponent, where):
+    # a piece of a number below 2^-110 would fall under the smallest bfloat16 number: the bound of the first test above, and what any 32-bit sum may lose
+    # below its smallest number
+    rng = np.random.default_rng(31)
+    m, n, k = 200, 140, 96
+    x, w = rng.standard_normal((m, k)).astype(np.float32), rng.standard_normal((n, k)).astype(np.float32)
+    if where.endswith("x"):
+        x[:: 1 if where == "x" else 7] *= np.float32(2.0**exponent)
+    else:
+        w[slice(None) if where == "w" else slice(77, 78)] *= np.float32(2.0**exponent)
+    ref = x.astype(np.float64) @ w.astype(np.float64).T
+    size = np.abs(x).astype(np.float64) @ np.abs(w).astype(np.float64).T
+    bound = 2**-23 * (6 * k / 16 + 2) * size + k * 2.0**-149
+    packed = K.pack_matrix(dev(w))
+    for got in (host(K.linear(dev(x), packed)), host(K.linear_split(dev(x), packed, 2)).sum(axis=0)):
+        assert (np.abs(got - ref) <= bound).all()
+
+
 def test_32_bit_products_in_pieces_settle_infinities_in_every_output(K):
     # bias and activation, a residual added in place, q/k/v columns into pages, a product cut along K: against the 32-bit instruction (a row-major W takes
     # it). Bounds: sums of 96 numbers around 1.
