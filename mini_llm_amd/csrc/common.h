@@ -57,10 +57,11 @@ __host__ __device__ __forceinline__ size_t packed_element(int row, int col, int 
     return packed_offset<T>(row / 16, col / KC, packed_k_steps<T>(cols), (in_chunk / VEC) * 16 + row % 16) + in_chunk % VEC;
 }
 
-// How a matrix is given to a product (w_packed): row-major, packed, or packed with its pieces behind it (32-bit only; gemm_pieces.h). The pieces: for
+// How a matrix is given to a product (w_packed): row-major (0), packed (any other number), or packed with its pieces behind it (32-bit only;
+// gemm_pieces.h): a number that nobody passes who only says that it is packed. The pieces: for
 // every 16 rows x 32 columns three chunks of 1 KiB in the packed layout for bfloat16 (the number rounded, what that leaves rounded, and the rest), row tiles outermost, behind the
 // last chunk of the packed matrix; behind them what is known of every 16 rows (TileRows).
-enum MllmPacked : int { ROW_MAJOR = 0, PACKED = 1, PACKED_WITH_PIECES = 2 };
+enum MllmPacked : int { ROW_MAJOR = 0, PACKED = 1, PACKED_WITH_PIECES = 0x70696563 };
 __host__ __device__ __forceinline__ long long packed_pieces_at(int row_tiles, int k_steps) { return (long long)row_tiles * k_steps * 1024; }
 __host__ __device__ __forceinline__ long long packed_pieces_bytes(int row_tiles, int cols) { return (long long)row_tiles * ((cols + 31) / 32) * 3072; }
 

@@ -12,7 +12,8 @@
 // out[M, N] (float) = residual + bias + A[M, K] . W[N, K]^T, the product cut along K into k_blocks
 // partial products that a second kernel adds up in a fixed order (the same numbers as
 // mllm_gemm_split followed by mllm_pending_sum). A and W are float or bfloat16 (in_dtype), W
-// row-major or packed (w_packed); bias [N] and residual [M, N] are float and may be null.
+// row-major (w_packed 0) or packed (any other number; MllmPacked in common.h for one that has its pieces
+// behind it); bias [N] and residual [M, N] are float and may be null.
 //
 // The partial products lie in an array of MLLM_STATIC_SCRATCH_BYTES (4 MiB) that every GPU the
 // library runs on holds from the first use until the process ends: k_blocks * M * N floats must

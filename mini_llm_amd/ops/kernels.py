@@ -177,6 +177,9 @@ def add(a, b, out=None):
     return out
 
 
+PACKED_WITH_PIECES = 0x70696563   # MllmPacked in csrc/common.h
+
+
 class PackedMatrix:
     """A weight matrix [rows (out), cols (in)] in the packed layout of the matrix kernels: chunks
     of 16 rows x 64 bytes, each chunk's 16-byte pieces in the order the lanes of a wave take them
@@ -185,6 +188,11 @@ class PackedMatrix:
 
     def __init__(self, data: torch.Tensor, rows: int, cols: int, pieces: bool = False):
         self.data, self.rows, self.cols, self.pieces = data, rows, cols, pieces
+
+    @property
+    def code(self):
+        """How the matrix is named to a product."""
+        return PACKED_WITH_PIECES if self.pieces else 1
 
     @property
     def shape(self):
@@ -253,7 +261,7 @@ def _matrix(weight, name, dtype):
     """(pointer, packed flag, rows, cols) of a weight given row-major or packed."""
     if isinstance(weight, PackedMatrix):
         _device_tensor(weight.data, name, dtype, 1)
-        return _ptr(weight.data), 2 if weight.pieces else 1, weight.rows, weight.cols
+        return _ptr(weight.data), weight.code, weight.rows, weight.cols
     _device_tensor(weight, name, dtype, 2)
     return _ptr(weight), 0, weight.shape[0], weight.shape[1]
 
@@ -1457,9 +1465,9 @@ def grouped_experts(x, picks: Picks, up: PackedMatrix, down: PackedMatrix, n_exp
     check(lib.mllm_expert_lists(_ptr(picks.experts), _ptr(picks.weights), n, top, int(n_experts), tile, _ptr(rows), _ptr(places), _ptr(weights), _ptr(tiles), _ptr(n_tiles),
                                 _stream()))
     check(lib.mllm_experts_up(_ptr(x), _ptr(up.data), _ptr(hidden), _ptr(tiles), _ptr(n_tiles), _ptr(rows), _ptr(weights), entries, max_tiles, int(n_experts), int(units), width, *unit,
-                              2 if up.pieces else 1, code, _stream()))
+                              up.code, code, _stream()))
     check(lib.mllm_experts_down(_ptr(hidden), _ptr(down.data), _ptr(out), _ptr(tiles), _ptr(n_tiles), _ptr(places), entries, max_tiles, int(n_experts), int(units), width,
-                                2 if down.pieces else 1, code, _stream()))
+                                down.code, code, _stream()))
     return out
 
 

@@ -1162,6 +1162,23 @@ def test_32_bit_products_in_pieces_are_nearer_than_32_bit_ones(K, m, n, k, kind)
     assert parts <= 0.6 * plain
 
 
+@pytest.mark.parametrize("packed", [1, 2, -1, 7])
+def test_a_matrix_that_is_only_said_to_be_packed_is_read_no_further(K, packed):
+    # any number but 0 and the one for pieces: what lies behind the matrix (here: no numbers) is not looked at
+    from mini_llm_amd.ops.library import library
+
+    rng, lib, (m, n, k) = np.random.default_rng(5), library(), (130, 64, 96)
+    x, w = rng.standard_normal((m, k)).astype(np.float32), rng.standard_normal((n, k)).astype(np.float32)
+    elements = lib.mllm_packed_elements(n, k, K.F32)
+    memory, out, parts = torch.full((4 * elements,), float("nan"), device=DEV), torch.zeros((m, n), device=DEV), torch.zeros((2, m, n), device=DEV)
+    x, w, ref = dev(x), dev(w), x.astype(np.float64) @ w.astype(np.float64).T
+    assert lib.mllm_pack_matrix(w.data_ptr(), memory.data_ptr(), n, k, K.F32, K.F32, 0, None) == 0
+    assert lib.mllm_gemm(x.data_ptr(), memory.data_ptr(), packed, None, None, out.data_ptr(), m, n, k, K.F32, K.F32, 0, 0, 0, None) == 0
+    assert lib.mllm_gemm_split(x.data_ptr(), memory.data_ptr(), packed, parts.data_ptr(), m, n, k, K.F32, 2, 0, None) == 0
+    np.testing.assert_allclose(host(out), ref, rtol=2e-5, atol=2e-5)
+    np.testing.assert_allclose(host(parts).sum(axis=0), ref, rtol=2e-5, atol=2e-5)
+
+
 @pytest.mark.parametrize("exponent", [-90, -100, -112, -120, -126])
 @pytest.mark.parametrize("where", ["x", "rows of x", "w", "a row of w"])
 def test_32_bit_products_in_pieces_of_tiny_numbers(K, exponent, where):
