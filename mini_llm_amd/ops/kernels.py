@@ -180,14 +180,25 @@ def add(a, b, out=None):
 PACKED_WITH_PIECES = 0x70696563   # MllmPacked in csrc/common.h
 
 
+def _version(tensor):
+    """torch's count of changes in place (it keeps none for tensors made in inference mode)."""
+    return None if tensor.is_inference() else tensor._version
+
+
 class PackedMatrix:
     """A weight matrix [rows (out), cols (in)] in the packed layout of the matrix kernels: chunks
     of 16 rows x 64 bytes, each chunk's 16-byte pieces in the order the lanes of a wave take them
     as matrix-core operands, zeros beyond the matrix. ``data`` is the flat device tensor. ``pieces``: a 32-bit matrix whose
-    bfloat16 pieces (csrc/gemm_pieces.h) lie behind it in the same allocation, for the products of many rows."""
+    bfloat16 pieces (csrc/gemm_pieces.h) lie behind it in the same allocation, for the products of many rows; they count while ``data``
+    is the tensor they were made from and torch has not changed it since (a step captured before keeps reading them)."""
 
     def __init__(self, data: torch.Tensor, rows: int, cols: int, pieces: bool = False):
-        self.data, self.rows, self.cols, self.pieces = data, rows, cols, pieces
+        self.data, self.rows, self.cols = data, rows, cols
+        self._pieces_of = (data, _version(data)) if pieces else None
+
+    @property
+    def pieces(self):
+        return self._pieces_of is not None and self._pieces_of[0] is self.data and self._pieces_of[1] == _version(self.data)
 
     @property
     def code(self):

@@ -1162,6 +1162,20 @@ def test_32_bit_products_in_pieces_are_nearer_than_32_bit_ones(K, m, n, k, kind)
     assert parts <= 0.6 * plain
 
 
+def test_a_packed_matrix_changed_in_place_is_multiplied_as_it_stands(K):
+    rng, (m, n, k) = np.random.default_rng(6), (130, 64, 96)
+    x, w, v = (dev(rng.standard_normal(shape)) for shape in ((m, k), (n, k), (n, k)))
+    weight = K.pack_matrix(w)
+    weight.data.mul_(2)
+    np.testing.assert_allclose(host(K.linear(x, weight)), 2 * host(x) @ host(w).T, rtol=2e-5, atol=2e-5)
+    weight = K.pack_matrix(w)
+    weight.data.copy_(K.pack_matrix(v).data)
+    np.testing.assert_allclose(host(K.linear(x, weight)), host(x) @ host(v).T, rtol=2e-5, atol=2e-5)
+    with torch.inference_mode():
+        weight = K.pack_matrix(w)
+        np.testing.assert_allclose(host(K.linear(x, weight)), host(x) @ host(w).T, rtol=2e-5, atol=2e-5)
+
+
 @pytest.mark.parametrize("packed", [1, 2, -1, 7])
 def test_a_matrix_that_is_only_said_to_be_packed_is_read_no_further(K, packed):
     # any number but 0 and the one for pieces: what lies behind the matrix (here: no numbers) is not looked at
