@@ -144,12 +144,17 @@ MLLM_API int mllm_pack_matrix(const void* src, void* dst, int rows, int cols, in
     return mllm_check_launch("pack_matrix");
 }
 
-// Bytes the pieces of a packed 32-bit matrix take behind it, with what is known of its rows.
-MLLM_API long long mllm_pieces_bytes(int rows, int cols) { return packed_pieces_bytes(ceil_div(rows, 16), cols) + (long long)sizeof(TileRows) * ceil_div(rows, 16); }
+// Bytes the pieces of a packed 32-bit matrix take behind it, with what is known of its rows; 0: no product would take them (pieces::takes_sizes).
+MLLM_API long long mllm_pieces_bytes(int rows, int cols) {
+    const int row_tiles = ceil_div(rows, 16);
+    const long long bytes = packed_pieces_bytes(row_tiles, cols);
+    return cols % 32 != 0 || rows % 4 != 0 || bytes >= (1LL << 32) ? 0 : bytes + (long long)sizeof(TileRows) * row_tiles;
+}
 
 // Lays the pieces of a packed 32-bit matrix [rows, cols] behind it, at packed + mllm_packed_elements.
 MLLM_API int mllm_pack_pieces(float* packed, int rows, int cols, hipStream_t stream) {
     MLLM_REQUIRE(rows > 0 && cols > 0 && packed != nullptr, "pack_pieces: bad size %d x %d", rows, cols);
+    MLLM_REQUIRE(mllm_pieces_bytes(rows, cols) > 0, "pack_pieces: no product takes pieces of a %d x %d matrix", rows, cols);
     const int row_tiles = ceil_div(rows, 16);
     unsigned char* pieces = reinterpret_cast<unsigned char*>(packed) + packed_pieces_at(row_tiles, packed_k_steps<float>(cols));
     const size_t steps = (size_t)row_tiles * ceil_div(cols, 32);

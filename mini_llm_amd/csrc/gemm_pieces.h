@@ -388,12 +388,16 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N, 2) void gemm_pieces_kernel(
     }
 }
 
-// Whether a product takes this kernel: a W that was packed with its pieces, more rows than the kernel for few rows takes, whole tiles of K, whole pieces of
-// 16 bytes in every row and pointer, operands whose bytes a 32-bit offset reaches, and in a q/k/v projection four columns never in two heads.
+// Whether a product takes this kernel: a W that was packed with its pieces (which it is not unless the sizes of W asked for here hold), more rows than the
+// kernel for few rows takes, whole tiles of K, whole pieces of 16 bytes in every row and pointer, operands whose bytes a 32-bit offset reaches, and in a
+// q/k/v projection four columns never in two heads.
+inline bool takes_sizes(int M, int N, int K, int matrix_tiles, int packed) {
+    return packed == PACKED_WITH_PIECES && M > 64 && K % BK == 0 && N % 4 == 0 && (long long)M * K * 4 < (1LL << 32) && packed_pieces_bytes(matrix_tiles, K) < (1LL << 32);
+}
+
 inline bool takes(const void* a, const void* bias, const void* residual, const void* out, int M, int N, int K, int matrix_tiles, int packed, const CacheScatter& scatter) {
-    if (packed != PACKED_WITH_PIECES || M <= 64 || K % BK != 0 || N % 4 != 0) return false;
+    if (!takes_sizes(M, N, K, matrix_tiles, packed)) return false;
     if (((size_t)a | (size_t)bias | (size_t)residual | (size_t)out) % 16 != 0) return false;
-    if ((long long)M * K * 4 >= (1LL << 32) || packed_pieces_bytes(matrix_tiles, K) >= (1LL << 32)) return false;
     return !scatter.enabled || (scatter.q_width % 4 == 0 && scatter.kv_width % 4 == 0 && scatter.head_size % 4 == 0 && (((size_t)scatter.k_pages | (size_t)scatter.v_pages) % 16) == 0);
 }
 

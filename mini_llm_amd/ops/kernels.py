@@ -260,12 +260,12 @@ def pack_matrix(src, dtype=None, transpose=False) -> PackedMatrix:
     _require(rows > 0 and cols > 0, "an empty matrix cannot be packed")
     lib = library()
     elements = lib.mllm_packed_elements(rows, cols, _code(dtype))
-    pieces = dtype == torch.float32
-    data = torch.empty((elements + (lib.mllm_pieces_bytes(rows, cols) // 4 if pieces else 0),), dtype=dtype, device=src.device)
+    pieces = lib.mllm_pieces_bytes(rows, cols) if dtype == torch.float32 else 0
+    data = torch.empty((elements + pieces // 4,), dtype=dtype, device=src.device)
     check(lib.mllm_pack_matrix(_ptr(src), _ptr(data), rows, cols, _code(src.dtype), _code(dtype), int(bool(transpose)), _stream()))
     if pieces:
         check(lib.mllm_pack_pieces(_ptr(data), rows, cols, _stream()))
-    return PackedMatrix(data[:elements], rows, cols, pieces)
+    return PackedMatrix(data[:elements], rows, cols, pieces > 0)
 
 
 def _matrix(weight, name, dtype):

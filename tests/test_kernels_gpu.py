@@ -1176,6 +1176,17 @@ def test_a_packed_matrix_changed_in_place_is_multiplied_as_it_stands(K):
         np.testing.assert_allclose(host(K.linear(x, weight)), host(x) @ host(w).T, rtol=2e-5, atol=2e-5)
 
 
+@pytest.mark.parametrize("n,k,pieces", [(64, 96, True), (20, 32, True), (50, 96, False), (4099, 64, False), (64, 100, False), (64, 48, False)])
+def test_pieces_are_laid_out_where_a_product_takes_them(K, n, k, pieces):
+    rng = np.random.default_rng(n)
+    x, w = rng.standard_normal((130, k)).astype(np.float32), rng.standard_normal((n, k)).astype(np.float32)
+    weight = K.pack_matrix(dev(w))
+    assert weight.pieces == pieces
+    held = weight.data.untyped_storage().nbytes() - 4 * weight.data.numel()
+    assert (held > 0) == pieces
+    np.testing.assert_allclose(host(K.linear(dev(x), weight)), x.astype(np.float64) @ w.astype(np.float64).T, rtol=2e-5, atol=2e-5)
+
+
 @pytest.mark.parametrize("packed", [1, 2, -1, 7])
 def test_a_matrix_that_is_only_said_to_be_packed_is_read_no_further(K, packed):
     # any number but 0 and the one for pieces: what lies behind the matrix (here: no numbers) is not looked at
