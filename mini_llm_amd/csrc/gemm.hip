@@ -465,6 +465,7 @@ __global__ __launch_bounds__(64 * KSPLIT) void gemm_skinny_kernel(
     // the epilogue it would be one more trip to memory at the end of a kernel that is a few long.
     constexpr int ITEMS = (NT * MT * 4 * WAVE + WAVE * KSPLIT - 1) / (WAVE * KSPLIT);  // outputs a thread finishes
     constexpr bool EARLY = MT < 4;  // with four row tiles the registers are better left to the loads of x
+    const bool early = EARLY && !(NT * MT >= 4 && whole_pieces);  // (four columns at a time ask for their own)
     float early_bias[ITEMS], early_residual[ITEMS];
     int early_slot[ITEMS];
 #pragma unroll
@@ -473,7 +474,7 @@ __global__ __launch_bounds__(64 * KSPLIT) void gemm_skinny_kernel(
         int l = index % WAVE, ir = index / WAVE;
         int token = (ir / 4 % MT) * 16 + l % 16;
         int col = n0 + (ir / 4 / MT) * 16 + 4 * (l / 16) + ir % 4;
-        bool wanted = EARLY && index < NT * MT * 4 * WAVE && token < M && col < N;
+        bool wanted = early && index < NT * MT * 4 * WAVE && token < M && col < N;
         early_bias[j] = bias && wanted ? bias[col] : 0.0f;
         early_residual[j] = residual && wanted && !scatter.enabled ? residual[(size_t)token * N + col] : 0.0f;
         early_slot[j] = scatter.enabled && wanted && col >= scatter.q_width ? scatter.slots[token] : -1;
