@@ -385,6 +385,47 @@ def test_latent_attention_at_the_most_rows_that_waves_share(dtype, rows, rank, r
         np.testing.assert_allclose(got[mine, 0].numpy(), (scores.softmax(1) @ keys[:, :rank]).numpy(), atol=2e-5, rtol=2e-4)
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("heads,rows,rank,rot", [(12, 801, 40, 8), (3, 1603, 150, 20), (17, 514, 300, 16)])
+def test_latent_attention_of_more_rows_than_waves_share(dtype, heads, rows, rank, rot):
+    # a wave a row: groups of heads, sinks, rows of no request among the others, one run of keys and several (which some rows end before). Bounds as above:
+    # sums of at most 200 keys in 32 bits.
+    k = kernels()
+    lib = k.library()
+    assert rows * -(-heads // lib.mllm_latent_attention_head_group(heads)) > 1536
+    rng = np.random.default_rng(rows)
+    page_size, length, n_requests, scale = 16, 200, 5, 0.3
+    row_size, blocks = k.latent_row_size(rank + rot), -(-length // page_size)
+    pages = torch.tensor(rng.normal(0, 1, (n_requests * blocks, 1, page_size, row_size)), dtype=torch.float32).to(dtype)
+    pages[..., rank + rot :] = 0
+    tables = rng.permutation(n_requests * blocks).reshape(n_requests, blocks).astype(np.int32)
+    owner, positions = rng.integers(-1, n_requests, rows).astype(np.int32), rng.integers(0, length, rows).astype(np.int32)
+    positions[:4] = 0, 63, 64, length - 1
+    q, sinks = torch.tensor(rng.normal(0, 1, (rows, heads, row_size)), dtype=torch.float32), torch.tensor(rng.normal(0, 2, heads), dtype=torch.float32)
+    cached = pages[torch.tensor(tables).long().view(-1)].double().view(n_requests, blocks * page_size, row_size)[:, :length]
+    want = {}
+    for sink in (True, False):
+        want[sink] = np.zeros((rows, heads, rank))
+        for r in range(n_requests):
+            mine = np.flatnonzero(owner == r)
+            scores = torch.einsum("thd,kd->thk", q[mine].double(), cached[r]) * scale
+            scores.masked_fill_(torch.arange(length)[None, None, :] > torch.tensor(positions[mine])[:, None, None], -float("inf"))
+            if sink:
+                scores = torch.cat([scores, sinks.double()[None, :, None].expand(len(mine), heads, 1)], dim=2)
+            want[sink][mine] = (scores.softmax(2)[:, :, :length] @ cached[r, :, :rank]).numpy()
+    q, pages, owner_gpu, positions_gpu, tables_gpu, sinks = q.cuda(), pages.cuda(), ints(owner), ints(positions), ints(tables), sinks.cuda()
+    for sink in (True, False):
+        got = k.latent_attention(q, pages, sinks if sink else None, owner_gpu, positions_gpu, tables_gpu, rank, scale, max_len=length)
+        np.testing.assert_allclose(got.cpu().numpy(), want[sink], atol=2e-5, rtol=2e-4)
+        for n_runs, run_length in ((2, 128), (3, 64)):
+            out, parts = torch.full((rows, heads, rank), 7.0).cuda(), torch.empty((rows, heads, n_runs, rank + 2)).cuda()
+            status = lib.mllm_latent_attention(q.data_ptr(), pages.data_ptr(), sinks.data_ptr() if sink else None, out.data_ptr(), parts.data_ptr(), owner_gpu.data_ptr(),
+                                               positions_gpu.data_ptr(), tables_gpu.data_ptr(), blocks, rows, heads, rank, row_size, page_size, scale, n_runs, run_length,
+                                               0 if dtype == torch.float32 else 1, None)
+            assert status == 0
+            np.testing.assert_allclose(out.cpu().numpy(), want[sink], atol=2e-5, rtol=2e-4)
+
+
 @pytest.mark.parametrize("rows,heads,n,k_size", [(816, 2, 65, 48), (819, 2, 80, 48), (1030, 3, 130, 80), (1, 3, 1, 16), (15, 2, 17, 272)])
 def test_heads_linear_in_32_bit_tiles(rows, heads, n, k_size):
     # around the number of tiles (512) beyond which a block takes columns instead of pieces of K; sums of at most 272 products of

@@ -238,12 +238,14 @@ def test_few_rows_over_a_large_matrix(K, rows):
         np.testing.assert_allclose(host(vp[slot // page_size, :, slot % page_size]).reshape(-1), ref[r, 2 * width : 3 * width], rtol=2e-2, atol=2e-2)
 
 
-def test_linear_f32_is_true_32_bit(K):
+@pytest.mark.parametrize("packed", [False, True])
+@pytest.mark.parametrize("m", [8, 130])   # the kernel for few rows; many rows: the 32-bit instruction, and with a packed W the product in pieces
+def test_linear_f32_is_true_32_bit(K, m, packed):
     # values that a reduced-precision matrix mode (tf32/bf16 inputs) would round away
-    m, n, k = 8, 64, 64
+    n, k = 64, 64
     x = np.full((m, k), 1.0 + 2.0**-12, dtype=np.float32)  # 12 fraction bits: tf32 keeps 10, bf16 7
     w = np.ones((n, k), dtype=np.float32)
-    out = host(K.linear(dev(x), dev(w)))
+    out = host(K.linear(dev(x), as_weight(K, w, torch.float32, packed)))
     assert (out == k * (1.0 + 2.0**-12)).all()  # exact in float32; a reduced mode gives 64.0
 
 
