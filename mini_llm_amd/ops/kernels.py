@@ -282,7 +282,8 @@ def linear(x, weight, bias=None, activation=None, residual=None, out_dtype=None,
     PackedMatrix; sums are float32. x may be PackedRows, and with ``packed_out`` the result is,
     where ``takes_packed_rows`` says so.
 
-    x and weight share their element type (float32: true 32-bit MFMA; bfloat16: bf16 MFMA);
+    x and weight share their element type (float32: 32-bit MFMA, or with a
+    packed weight and more than 64 rows bf16 MFMA over three pieces of every number, csrc/gemm_pieces.h; bfloat16: bf16 MFMA);
     bias and residual are float32; a residual makes the output float32."""
     x_ptr, x_packed, m, k, x_dtype, device = _rows(x, "x")
     w_ptr, w_packed, n, w_cols = _matrix(weight, "weight", x_dtype)

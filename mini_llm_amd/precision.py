@@ -1,6 +1,7 @@
 """The two precisions a model runs in.
 
-``float32``: every tensor and every product in true 32-bit. ``bfloat16``: matrices, tables,
+``float32``: every tensor in 32-bit, and products of all bits of their operands with 32-bit sums
+(csrc/gemm_pieces.h: on the bfloat16 matrix instructions where rows are many, in pieces). ``bfloat16``: matrices, tables,
 the activations between kernels and the cache pages in bfloat16; sums, norms, softmax, the
 residual stream and the logits in 32-bit, and vectors (biases, norm gains) kept in 32-bit."""
 
