@@ -9,6 +9,7 @@
 #include "common.h"
 #include "no_alloc.h"
 
+#include <algorithm>
 #include <mutex>
 
 namespace {
@@ -705,14 +706,16 @@ int skinny_k_blocks(int N, int K) {
 // 256 rows a block may go down to four LDS tiles: the partial products are small then, and a
 // 128 x 768 x 768 product takes 6.1 us in two cuts against 7.9 us whole (bfloat16; in 32-bit 8.6 us
 // in four cuts against 12.6 us in two).
+//
+// most: the most partial products there is room for, asked by the rule for products in pieces alone, which cuts finer than the rules below.
 template <typename T>
-int tiled_k_blocks(int M, int N, int K) {
+int tiled_k_blocks(int M, int N, int K, int most) {
     int tiles = ceil_div(M, 128) * ceil_div(N, 64);
     int k_blocks = 1;
     // By whole tiles of 128 rows, as the rest. A W without pieces takes the 32-bit instruction with this count too, and loses nothing by it, the reading of the
     // partial products included: with the rule below / with this one 700 x 1,024 x 4,096 75.1 us in four / 62.6 in five, 300 x 1,600 x 1,600 29.8 in four /
     // 28.2 in six, 577 x 768 x 3,072 34.5 in four / 34.0 in eight, 2,048 x 768 x 768 30.4 in four / 32.7 in two (12.6 MB less to read).
-    if (sizeof(T) == 4 && K % pieces::BK == 0 && N % 4 == 0) return pieces::split_blocks(ceil_div(M, 128) * 128, N, K);
+    if (sizeof(T) == 4 && K % pieces::BK == 0 && N % 4 == 0) return pieces::split_blocks(ceil_div(M, 128) * 128, N, K, most);
     if (sizeof(T) == 4 && tiles > 128) {
         // In 32-bit the matrix cores set the pace, and a block has two waves on each of them: what counts is that every
         // compute unit gets the same number of blocks. 192 tiles (2,048 x 768) whole keep 192 units busy for a block's
@@ -899,14 +902,24 @@ MLLM_API int mllm_gemm_best(const void* A, const void* W, int w_packed, const fl
     return mllm_check_launch("gemm_best");
 }
 
-// How many partial products mllm_gemm_split should be asked for at these sizes (1: the product is
-// better left whole).
-MLLM_API int mllm_gemm_split_blocks(int M, int N, int K, int in_dtype) {
+constexpr size_t STATIC_SCRATCH_FLOATS = (size_t)1 << 20;  // 4 MiB: what mllm_linear_split_static has room for
+
+static int split_blocks_of_at_most(int M, int N, int K, int in_dtype, int most) {
     if (M <= 0 || N <= 0 || K <= 0) return 1;
-    if (in_dtype == MLLM_F32) return K % 4 ? 1 : (M <= 64 ? skinny_k_blocks<float>(N, K) : tiled_k_blocks<float>(M, N, K));
-    if (in_dtype == MLLM_BF16) return K % 8 ? 1 : (M <= 64 ? skinny_k_blocks<bf16_t>(N, K) : tiled_k_blocks<bf16_t>(M, N, K));
+    if (in_dtype == MLLM_F32) return K % 4 ? 1 : (M <= 64 ? skinny_k_blocks<float>(N, K) : tiled_k_blocks<float>(M, N, K, most));
+    if (in_dtype == MLLM_BF16) return K % 8 ? 1 : (M <= 64 ? skinny_k_blocks<bf16_t>(N, K) : tiled_k_blocks<bf16_t>(M, N, K, most));
     return 1;
 }
+
+// How many partial products mllm_gemm_split should be asked for at these sizes (1: the product is better left whole), for a caller who may take the
+// answer to mllm_linear_split_static: no more than fit its array, where one fits.
+MLLM_API int mllm_gemm_split_blocks(int M, int N, int K, int in_dtype) {
+    const long long one = (long long)M * N;
+    return split_blocks_of_at_most(M, N, K, in_dtype, one > 0 && one <= (long long)STATIC_SCRATCH_FLOATS ? (int)std::min<long long>(8, STATIC_SCRATCH_FLOATS / one) : 8);
+}
+
+// The same for a caller who brings the memory: the fastest count, however much its partial products take.
+MLLM_API int mllm_gemm_split_blocks_anywhere(int M, int N, int K, int in_dtype) { return split_blocks_of_at_most(M, N, K, in_dtype, 8); }
 
 // A . W^T as k_blocks partial products over consecutive parts of K: partials [k_blocks, M, N] in
 // 32-bit, whose sum (in any fixed order) is the product. For a long K with few output columns;
@@ -1043,7 +1056,6 @@ MLLM_API int mllm_experts_down(const void* hidden, const void* W, float* out, co
 // ------------------------------------------------------------------------------------------------
 namespace {
 
-constexpr size_t STATIC_SCRATCH_FLOATS = (size_t)1 << 20;  // 4 MiB
 // Each GPU holds its own copy of this array at its own address. In host code the name is only a
 // handle for hipGetSymbolAddress: kernels get the address that call returns, never the name.
 static __device__ __align__(256) float scratch[STATIC_SCRATCH_FLOATS];

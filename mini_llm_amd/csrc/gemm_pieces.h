@@ -450,11 +450,11 @@ inline void dispatch(const float* a, const float* w, const float* bias, const fl
     else launch_whole<64, 64, 2, 2>(a, w, bias, residual, o, M, N, K, epilogue, stream, scatter, k_blocks);
 }
 
-// Into how many partial products a product with sums to be taken by whoever reads them is cut: they are read once more there.
-inline int split_blocks(int M, int N, int K) {
+// Into how many partial products a product with sums to be taken by whoever reads them is cut, `most` at most: they are read once more there.
+inline int split_blocks(int M, int N, int K, int most) {
     int best = 1, tile = 0;
     float best_cost = 0.0f;
-    for (int cuts = 1; cuts <= 8 && (cuts == 1 || K >= 4 * BK * cuts); cuts++) {
+    for (int cuts = 1; cuts <= most && (cuts == 1 || K >= 4 * BK * cuts); cuts++) {
         const float us = cost(M, N, K, cuts, tile) + (float)M * N * cuts * (4.0f / 6e6f);
         if (cuts == 1 || us < best_cost) best = cuts, best_cost = us;
     }

@@ -322,7 +322,7 @@ def split_blocks(weight, dtype, rows: int = 1) -> int:
     columns meet a long K. The same for all row counts up to 64, and for all that need the same
     number of 128-row tiles."""
     _, _, n, k = _matrix(weight, "weight", dtype)
-    return int(library().mllm_gemm_split_blocks(int(rows), n, k, _code(dtype)))
+    return int(library().mllm_gemm_split_blocks_anywhere(int(rows), n, k, _code(dtype)))
 
 
 def linear_split(x, weight, k_blocks: int, out=None):

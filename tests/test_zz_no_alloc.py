@@ -88,6 +88,20 @@ def test_two_calls_in_a_row_the_second_smaller(lib, dtype, code):
     np.testing.assert_allclose(out.cpu().numpy(), x.double().cpu().numpy() @ w.double().cpu().numpy().T, rtol=2e-5, atol=2e-4)
 
 
+@pytest.mark.parametrize("m,n,k", [(65, 3088, 8192), (577, 768, 768), (700, 736, 768), (1024, 1024, 1024), (65, 16128, 768), (1024, 1020, 4096)])
+def test_the_count_the_library_names_fits(lib, m, n, k):
+    # in 32-bit, where the product in pieces is cut finest: whatever can be held in one product or more is cut no finer than there is room for
+    assert m * n <= 1 << 20
+    blocks = lib.mllm_gemm_split_blocks(m, n, k, F32)
+    assert 1 <= blocks and blocks * m * n <= 1 << 20
+    x, w, bias, residual = operands(m + n, m, n, k, torch.float32)
+    out = torch.empty((m, n), dtype=torch.float32, device="cuda")
+    assert lib.mllm_linear_split_static(x.data_ptr(), w.data_ptr(), 0, bias.data_ptr(), residual.data_ptr(), out.data_ptr(), m, n, k, F32, blocks, None) == 0, lib.mllm_last_error()
+    ref = x.double().cpu() @ w.double().cpu().T + bias.double().cpu() + residual.double().cpu()
+    np.testing.assert_allclose(out.cpu().numpy(), ref.numpy(), rtol=2e-5, atol=2e-4 * (k / 256) ** 0.5)   # (K roundings at random of a sum of about 0.1 sqrt(K), 2^-23 of it each: 7e-5 at K = 8,192)
+    assert lib.mllm_gemm_split_blocks_anywhere(m, n, k, F32) >= blocks
+
+
 def test_what_does_not_fit_is_refused(lib):
     x, w, bias, residual = operands(1, 4, 64, 64, torch.float32)
     out = torch.zeros((4, 64), dtype=torch.float32, device="cuda")
