@@ -180,11 +180,6 @@ def add(a, b, out=None):
 PACKED_WITH_PIECES = 0x70696563   # MllmPacked in csrc/common.h
 
 
-def _version(tensor):
-    """torch's count of changes in place (it keeps none for tensors made in inference mode)."""
-    return None if tensor.is_inference() else tensor._version
-
-
 class PackedMatrix:
     """A weight matrix [rows (out), cols (in)] in the packed layout of the matrix kernels: chunks
     of 16 rows x 64 bytes, each chunk's 16-byte pieces in the order the lanes of a wave take them
@@ -194,11 +189,11 @@ class PackedMatrix:
 
     def __init__(self, data: torch.Tensor, rows: int, cols: int, pieces: bool = False):
         self.data, self.rows, self.cols = data, rows, cols
-        self._pieces_of = (data, _version(data)) if pieces else None
+        self._pieces_of = (data, data._version) if pieces else None
 
     @property
     def pieces(self):
-        return self._pieces_of is not None and self._pieces_of[0] is self.data and self._pieces_of[1] == _version(self.data)
+        return self._pieces_of is not None and self._pieces_of[0] is self.data and self._pieces_of[1] == self.data._version
 
     @property
     def code(self):
@@ -261,11 +256,13 @@ def pack_matrix(src, dtype=None, transpose=False) -> PackedMatrix:
     lib = library()
     elements = lib.mllm_packed_elements(rows, cols, _code(dtype))
     pieces = lib.mllm_pieces_bytes(rows, cols) if dtype == torch.float32 else 0
-    data = torch.empty((elements + pieces // 4,), dtype=dtype, device=src.device)
+    with torch.inference_mode(False):   # (torch counts no changes of tensors made in inference mode)
+        data = torch.empty((elements + pieces // 4,), dtype=dtype, device=src.device)
+        matrix = data[:elements]
     check(lib.mllm_pack_matrix(_ptr(src), _ptr(data), rows, cols, _code(src.dtype), _code(dtype), int(bool(transpose)), _stream()))
     if pieces:
         check(lib.mllm_pack_pieces(_ptr(data), rows, cols, _stream()))
-    return PackedMatrix(data[:elements], rows, cols, pieces > 0)
+    return PackedMatrix(matrix, rows, cols, pieces > 0)
 
 
 def _matrix(weight, name, dtype):

@@ -1175,7 +1175,10 @@ def test_a_packed_matrix_changed_in_place_is_multiplied_as_it_stands(K):
     np.testing.assert_allclose(host(K.linear(x, weight)), host(x) @ host(v).T, rtol=2e-5, atol=2e-5)
     with torch.inference_mode():
         weight = K.pack_matrix(w)
+        assert weight.pieces
         np.testing.assert_allclose(host(K.linear(x, weight)), host(x) @ host(w).T, rtol=2e-5, atol=2e-5)
+        weight.data.mul_(2)
+        np.testing.assert_allclose(host(K.linear(x, weight)), 2 * host(x) @ host(w).T, rtol=2e-5, atol=2e-5)
 
 
 @pytest.mark.parametrize("n,k,pieces", [(64, 96, True), (20, 32, True), (50, 96, False), (4099, 64, False), (64, 100, False), (64, 48, False)])
