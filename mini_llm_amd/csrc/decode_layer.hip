@@ -910,8 +910,11 @@ MLLM_API int mllm_decode_layer_supported(int width, int head_size, int page_size
 // width (0: never). A property of the kernels, measured on MI355X: every (token, head) block pulls
 // its own copy of the partial rows and of its head's matrices through one compute unit, which grows
 // with the width, while what the fusion saves (five kernel boundaries a layer) does not. Up to 768
-// columns the fused kernels win up to 16 rows (by 2 % at 1 row, 11 % at 8, 12 % at 16, and lose by
-// 4 % at 32); at 1,024 columns they lose at every row count (1.10 against 0.96 ms a step at 1 row).
+// columns the fused kernels win up to 16 rows (a decode step of GPT-2 small, fused / one by one: 0.380 to
+// 0.385 / 0.388 ms at 1 row, 0.373 / 0.392 at 2, 0.386 / 0.406 at 4, 0.401 / 0.440 at 8, 0.420 / 0.465 at 16; at
+// 32 they lose by 4 %); at 1,024 columns they lose at every row count (1.10 against 0.96 ms a step at 1 row).
+// The row counts 32 and the wider layers were measured before the products of few rows last became faster,
+// which can only have widened what is lost there.
 MLLM_API int mllm_decode_layer_rows(int width) {
     if (!mllm_decode_layer_supported(width, 0, 0, 0)) return 0;
     return width <= 768 ? 16 : 0;

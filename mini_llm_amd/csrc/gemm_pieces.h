@@ -8,7 +8,7 @@
 // rounded six times for sixteen numbers of K instead of once (the 32-bit instruction: eight times). Measured against 64-bit sums over rows of 768 and 3,072
 // normally distributed numbers: 1.6e-7 and 3.4e-7 of the result's norm, in one sum 4.2e-7 and 8.6e-7, with the 32-bit instruction 5.0e-7 and 9.9e-7; over
 // rows of which half are zero, as behind a clamp, 1.2e-7 and 2.7e-7, 4.0e-7 and 8.2e-7, 3.5e-7 and 7.1e-7. It is the 64 registers that the 128 x 128 tile
-// has left (188 -> 252, none spilled), and no time: 2,048 x 3,072 x 768 60.6 us, 63.2 in one sum.
+// has left (188 -> 252, none spilled), and little time: 2,048 x 3,072 x 768 60.6 us, 63.2 in one sum, on another machine 64.4 and 63.3.
 //
 // W's pieces are laid out once, when the matrix is packed (common.h: packed_pieces): the chunks of the packed layout for bfloat16, the three of a k-step
 // behind each other. A's rows come as they are, and a wave splits the fragments it has read.
@@ -429,8 +429,10 @@ struct Choice {
 constexpr Choice CHOICES[3] = {{128, 128, 1.27f, 1.28f}, {128, 64, 0.83f, 0.72f}, {64, 64, 0.50f, 0.41f}};
 
 // Microseconds of a product cut into k_blocks along K with the best of the tiles (`best`): the rounds of blocks, the start and end of a block, and the sums
-// that are written (6 TB/s). Within a tenth of what was measured from 2,048 x 768 x 768 (24.4 us whole, 20.3 in two) to 2,048 x 768 x 3,072 (78 whole,
-// 58 in four, 67 in eight) and 130 x 768 x 768 (14.5 whole, 5.1 in six).
+// that are written (6 TB/s). Within a sixth of what was measured from 2,048 x 768 x 768 (21.4 us whole, 19.8 in two) to 2,048 x 768 x 3,072 (72 whole,
+// 62 in four, 63 in eight) and 130 x 768 x 768 (15.0 whole, 5.2 in six). With each tile in turn, 128 x 128 / 128 x 64 / 64 x 64: 2,048 x 2,304 x 768 58.8 /
+// 57.0 / 53.8 us, 8,192 x 3,072 x 768 213 / 237 / 253, 130 x 768 x 768 35.6 / 21.4 / 14.9; the rule's is the best of the three or within 3 % of it, but for
+// 1,500 x 2,304 x 768 (39.5 / 34.9 / 41.4, it takes the first).
 inline float cost(int M, int N, int K, int k_blocks, int& best) {
     float best_cost = 0.0f;
     for (int c = 0; c < 3; c++) {
