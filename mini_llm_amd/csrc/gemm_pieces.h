@@ -1,6 +1,6 @@
 // The 32-bit product for many rows on the bfloat16 matrix cores. Included by gemm.hip.
 //
-// A 32-bit number is the sum of three bfloat16 ones, each what the one before leaves, rounded to the nearest, and a product of two such numbers is the sum of
+// A 32-bit number (of 2^-110 or more; smaller ones and infinities: at the kernel's end) is the sum of three bfloat16 ones, each what the one before leaves, rounded to the nearest, and a product of two such numbers is the sum of
 // nine products of pieces, each exact in 32-bit (the method: Henry, Tang and Heinecke, "Leveraging the bfloat16 Artificial Intelligence Datatype For
 // Higher-Precision Computations", 2019). The three left out are at most 2^-24 of the product and lie on either side of it. (Pieces cut off instead
 // of rounded leave out up to 2^-21, always on the product's own side: over 3,072 positive numbers the sums came out 6.5e-6 too small, 7e-8 with rounding.)
