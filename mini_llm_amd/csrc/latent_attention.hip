@@ -761,15 +761,254 @@ __global__ __launch_bounds__(64 * LATENT_WAVES, 2) void latent_attention_mfma_ke
     }
 }
 
+// The same for 32-bit caches of those row sizes, on the 32-bit matrix instruction (32 x 32 x 2): for many rows what bounds the wave a row above is its
+// multiply-adds, each of which reads a weight or a query's element of its own; here 32 (token, head) pairs of a request share every operand.
+// A block takes 32 pairs and its eight waves the tiles of 32 keys in turn, each with sums and softmax statistics of its own that meet in LDS at the end, so
+// that the longest rows are not a chain of one wave; a block fills a compute unit, so that the blocks, longest first, go to whichever unit is free (blocks of
+// four waves, two a unit: the second of a unit's blocks is placed before it is known which unit will be late, and a prompt of 1,024 took 118 us where it takes 87). The queries lie in LDS; keys come from memory as operands, a lane four numbers of its key's row at
+// once, which the four products take one of each: the numbers meet in pairs whatever K index the instruction means by them. The scores S^T = C Q^T come out
+// with a pair a lane and keys 8 g + 4 half + e in the registers, which is what the weighted sum O^T = C_latent^T P^T takes as its other operand if its step
+// (g, e) means key 8 g + e in one half of the lanes and 8 g + 4 + e in the other: weights never leave their registers. A key's latent is read four elements a
+// lane, an element for each of four output tiles (tile e of four: elements 128 j + 4 i + e).
+// Keys are asked for a chunk ahead of the products, behind scheduling borders: moved up further they would not fit 256 registers, which two waves a SIMD leave
+// each (one covers the other's softmax).
+// Rows of 288 floats, 12 heads, a wave a row (or shared) -> here: six prompts of 19 to 640 304 -> 119 us, one of 1,024 401 -> 87 (79 TFLOP/s of the instruction's 157).
+constexpr int LATENT_F32_KEYS = 32, LATENT_F32_WAVES = 8;
+
+template <int DK>
+__global__ __launch_bounds__(64 * LATENT_F32_WAVES) void latent_attention_f32_mfma_kernel(
+    const float* __restrict__ q, const float* __restrict__ pages, const float* __restrict__ sinks, float* __restrict__ out, float* __restrict__ parts,
+    const int* __restrict__ token_request, int n_rows,
+    const int* __restrict__ q_starts, const int* __restrict__ context_lens, const int* __restrict__ block_tables, int max_blocks,
+    int n_heads, int R, int page_size, float scale, int run_length) {
+    constexpr int D = 16 * DK, GROUPS = D / 8, CHUNK = GROUPS % 6 == 0 ? 6 : 4, CHUNKS = GROUPS / CHUNK;   // a group: a piece of four numbers in either half
+    constexpr int FOURS = D > 128 ? 2 : 1;                                                              // times four output tiles of 32 latent elements (R <= 256)
+    constexpr int Q_ROW = D + 4, SLOT_ROW = WAVE * 4 + 4;                                               // floats; padded by a piece
+    constexpr int MERGE_FLOATS = LATENT_F32_WAVES * 8 * SLOT_ROW, LDS_FLOATS = 32 * Q_ROW > MERGE_FLOATS ? 32 * Q_ROW : MERGE_FLOATS;
+    static_assert(GROUPS % CHUNK == 0, "whole chunks");
+    __shared__ __attribute__((aligned(16))) float lds[LDS_FLOATS];   // the queries, then the waves' sums
+    __shared__ float wave_top[LATENT_F32_WAVES][32], wave_weight[LATENT_F32_WAVES][32];
+    __shared__ int wave_endless[LATENT_F32_WAVES];
+    const int lane = threadIdx.x % WAVE, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE), lane32 = lane % 32, half = lane / 32;
+    const int request = blockIdx.y, run = blockIdx.z, n_runs = gridDim.z;
+    if (n_runs == 1 && request == 0) {   // rows of no request are zero, as above
+        for (int row0 = (blockIdx.x * LATENT_F32_WAVES + wave) * WAVE; row0 < n_rows; row0 += gridDim.x * LATENT_F32_WAVES * WAVE) {
+            unsigned long long nobodys = __ballot(row0 + lane < n_rows && token_request[min(row0 + lane, n_rows - 1)] < 0);
+            for (; nobodys; nobodys &= nobodys - 1) {
+                float* row = out + (size_t)(row0 + __builtin_ctzll(nobodys)) * n_heads * R;
+                for (int i = lane; i < n_heads * R; i += WAVE) row[i] = 0.0f;
+            }
+        }
+    }
+    const int context = context_lens[request];
+    if (context < 0) return;   // a padding request
+    const int q_first = q_starts[request], q_len = q_starts[request + 1] - q_first;
+    const int pair0 = (gridDim.x - 1 - blockIdx.x) * 32, n_pairs = q_len * n_heads;   // (a portion's last pairs, which have the most keys, go first)
+    if (pair0 >= n_pairs) return;
+    const int position = context + min((pair0 + lane32) / n_heads, q_len - 1);   // of this lane's pair
+    const int* table = block_tables + (size_t)request * max_blocks;
+    const int first_position = context + pair0 / n_heads, last_position = context + min(q_len - 1, (pair0 + 31) / n_heads);
+    const int first_key = run * run_length, last_key = run == n_runs - 1 ? last_position : min(last_position, first_key + run_length - 1);
+
+    auto slot_of = [&](int kt) {   // this lane's key of a tile (the same in both halves), from a clamped place
+        const int key = max(min(kt + lane32, last_key), 0);
+        return table[key / page_size] * page_size + key % page_size;
+    };
+    f32x4 key_piece[2][CHUNK];
+    auto ask_keys = [&](int slot, int chunk, int to) {
+        const float* row = pages + (size_t)slot * D + 4 * half + 8 * CHUNK * chunk;
+#pragma unroll
+        for (int c = 0; c < CHUNK; c++) key_piece[to][c] = *reinterpret_cast<const f32x4*>(row + 8 * c);
+    };
+    constexpr int STRIDE = LATENT_F32_WAVES * LATENT_F32_KEYS;
+    const int first_tile = first_key + LATENT_F32_KEYS * wave;
+    int slot = 0, next_slot = 0;
+    if (first_tile <= last_key) {   // (uniform over the wave, as the loop below is)
+        slot = slot_of(first_tile);
+        next_slot = slot_of(first_tile + STRIDE);
+        ask_keys(slot, 0, 0);
+    }
+    for (int i = threadIdx.x; i < 32 * (D / 4); i += 64 * LATENT_F32_WAVES) {   // pairs lie in (token, head) order, as q's rows do
+        const int p = i / (D / 4), piece = i % (D / 4);
+        *reinterpret_cast<f32x4*>(lds + p * Q_ROW + 4 * piece) = *reinterpret_cast<const f32x4*>(q + ((size_t)q_first * n_heads + min(pair0 + p, n_pairs - 1)) * D + 4 * piece);
+    }
+    __syncthreads();
+    const float* q_row = lds + lane32 * Q_ROW + 4 * half;
+
+    f32x16 o[FOURS][4];
+#pragma unroll
+    for (int j = 0; j < FOURS; j++)
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+#pragma unroll
+            for (int v = 0; v < 16; v++) o[j][e][v] = 0.0f;
+    float top = -INFINITY, weight = 0.0f;   // the pair's maximum over this wave's keys, and its weights' sum over those of this half
+    unsigned endless = 0;                   // whether one of the elements set to zero below was none
+
+    for (int kt = first_tile; kt <= last_key; kt += STRIDE) {
+        f32x16 s;
+#pragma unroll
+        for (int v = 0; v < 16; v++) s[v] = 0.0f;
+        // the latents of two steps: this half's key of step v = 4 g + e is 8 g + 4 half + e
+        f32x4 latent[2][2][FOURS];
+        auto ask_latents = [&](int pair_of_steps, int to) {
+#pragma unroll
+            for (int u = 0; u < 2; u++) {
+                const int v = 2 * pair_of_steps + u, low = 8 * (v / 4) + v % 4;
+                const int at = half ? __builtin_amdgcn_readlane(slot, low + 4) : __builtin_amdgcn_readlane(slot, low);
+                const float* row = pages + (size_t)at * D;
+#pragma unroll
+                for (int j = 0; j < FOURS; j++) latent[to][u][j] = *reinterpret_cast<const f32x4*>(row + min(128 * j + 4 * lane32, D - 4));   // beyond R: never stored
+            }
+        };
+#pragma unroll
+        for (int chunk = 0; chunk < CHUNKS; chunk++) {
+            if (chunk + 1 < CHUNKS) ask_keys(slot, chunk + 1, (chunk + 1) & 1);
+            else ask_latents(0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int c = 0; c < CHUNK; c++) {
+                const f32x4 query = *reinterpret_cast<const f32x4*>(q_row + 8 * (CHUNK * chunk + c));
+#pragma unroll
+                for (int e = 0; e < 4; e++) s = __builtin_amdgcn_mfma_f32_32x32x2f32(key_piece[chunk & 1][c][e], query[e], s, 0, 0, 0);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        float tile_top = -INFINITY;
+#pragma unroll
+        for (int v = 0; v < 16; v++) {
+            const int at = kt + 8 * (v / 4) + 4 * half + (v % 4);
+            s[v] = at <= position && at <= last_key ? s[v] * scale : -INFINITY;
+            tile_top = fmaxf(tile_top, s[v]);
+        }
+        const float new_top = fmaxf(top, fmaxf(tile_top, __shfl_xor(tile_top, 32, WAVE)));
+        const float safe_top = new_top == -INFINITY ? 0.0f : new_top;   // a pair none of whose keys has come yet
+        if (__any(new_top != top)) {
+            const float rescale = expf(top - safe_top);
+            weight *= rescale;
+#pragma unroll
+            for (int j = 0; j < FOURS; j++)
+#pragma unroll
+                for (int e = 0; e < 4; e++)
+#pragma unroll
+                    for (int v = 0; v < 16; v++) o[j][e][v] *= rescale;
+        }
+        top = new_top;
+#pragma unroll
+        for (int v = 0; v < 16; v++) {
+            s[v] = expf(s[v] - safe_top);
+            weight += s[v];
+        }
+        // A key that some of the pairs do not see meets their weight of zero, and an infinity in it would leave them no number: in a tile that reaches
+        // beyond the block's first position those elements are taken as zero and made up for below.
+        const bool ragged = kt + LATENT_F32_KEYS - 1 > first_position;   // uniform over the wave
+#pragma unroll
+        for (int two = 0; two < 8; two++) {
+            if (two + 1 < 8) ask_latents(two + 1, (two + 1) & 1);
+            else ask_keys(next_slot, 0, 0);   // the next tile's (behind the last tile: the last key's row, not used)
+            __builtin_amdgcn_sched_barrier(0);
+            if (ragged) {
+#pragma unroll
+                for (int u = 0; u < 2; u++)
+#pragma unroll
+                    for (int j = 0; j < FOURS; j++)
+#pragma unroll
+                        for (int e = 0; e < 4; e++) {
+                            const float value = latent[two & 1][u][j][e];
+                            const bool finite = fabsf(value) < INFINITY;
+                            endless |= finite ? 0u : 1u;
+                            latent[two & 1][u][j][e] = finite ? value : 0.0f;
+                        }
+            }
+#pragma unroll
+            for (int u = 0; u < 2; u++)
+#pragma unroll
+                for (int j = 0; j < FOURS; j++)
+#pragma unroll
+                    for (int e = 0; e < 4; e++) o[j][e] = __builtin_amdgcn_mfma_f32_32x32x2f32(latent[two & 1][u][j][e], s[2 * two + u], o[j][e], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        slot = next_slot;
+        next_slot = slot_of(kt + 2 * STRIDE);
+    }
+    weight += __shfl_xor(weight, 32, WAVE);
+    if (half == 0) wave_top[wave][lane32] = top, wave_weight[wave][lane32] = weight;
+    const bool wave_has = __any(endless != 0);
+    if (lane == 0) wave_endless[wave] = wave_has;
+    __syncthreads();   // (and nobody reads the queries any more)
+    int some_endless = 0;
+    float all_top = -INFINITY;
+#pragma unroll
+    for (int w = 0; w < LATENT_F32_WAVES; w++) {
+        all_top = fmaxf(all_top, wave_top[w][lane32]);
+        some_endless |= wave_endless[w];
+    }
+    const float share = top == -INFINITY ? 0.0f : expf(top - all_top);
+    // The waves' sums, eight registers of four tiles at a time: a thread takes four neighbouring latent elements of a pair, sixteen threads a run of 64 (row
+    // 2 v0 + i of the tiles is register v0 + 4 (i / 8) + i % 4 of half i / 4 % 2).
+    const int i = threadIdx.x % 16, p = threadIdx.x / 16;
+    const bool stores = pair0 + p < n_pairs;
+    const size_t item = (size_t)q_first * n_heads + min(pair0 + p, n_pairs - 1);
+    float* const to = n_runs == 1 ? out + item * R : parts + (item * n_runs + run) * (R + 2);
+    float pair_top = -INFINITY, total = 0.0f, factor = 1.0f;
+#pragma unroll
+    for (int w = 0; w < LATENT_F32_WAVES; w++) pair_top = fmaxf(pair_top, wave_top[w][p]);
+#pragma unroll
+    for (int w = 0; w < LATENT_F32_WAVES; w++) total += wave_top[w][p] == -INFINITY ? 0.0f : wave_weight[w][p] * expf(wave_top[w][p] - pair_top);
+    if (n_runs == 1) {   // the finished sums: the sink joins the denominator once, measured from the larger of the two
+        factor = 1.0f / total;
+        if (sinks) {
+            const float sink = sinks[(pair0 + p) % n_heads], highest = fmaxf(pair_top, sink), shrink = expf(pair_top - highest);
+            factor = shrink / (total * shrink + expf(sink - highest));
+        }
+    } else if (i == 0 && stores) {
+        to[R] = pair_top;   // -inf and 0 for a run without keys
+        to[R + 1] = total;
+    }
+#pragma unroll
+    for (int round = 0; round < 2 * FOURS; round++) {
+        const int j = round / 2, v0 = 8 * (round % 2), d = 128 * j + 4 * (2 * v0 + i);
+#pragma unroll
+        for (int v = 0; v < 8; v++)
+            *reinterpret_cast<f32x4*>(lds + (wave * 8 + v) * SLOT_ROW + 4 * lane) = f32x4{o[j][0][v0 + v], o[j][1][v0 + v], o[j][2][v0 + v], o[j][3][v0 + v]} * share;
+        __syncthreads();
+        f32x4 sum = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int w = 0; w < LATENT_F32_WAVES; w++)
+            sum += *reinterpret_cast<const f32x4*>(lds + (w * 8 + 4 * (i / 8) + i % 4) * SLOT_ROW + 4 * (p + 32 * (i / 4 % 2)));
+        if (some_endless && stores && d < R) {   // what of them the pair does see (one of an earlier tile counted twice stays what it is)
+            const int sees = min(last_key, context + (pair0 + p) / n_heads);
+            for (int key = max(first_key, first_position - LATENT_F32_KEYS); key <= sees; key++) {
+                const f32x4 value = *reinterpret_cast<const f32x4*>(pages + ((size_t)table[key / page_size] * page_size + key % page_size) * D + d);
+#pragma unroll
+                for (int e = 0; e < 4; e++) sum[e] += fabsf(value[e]) < INFINITY ? 0.0f : value[e];
+            }
+        }
+        sum *= factor;
+        if (stores && n_runs == 1 && R % 4 == 0) {
+            if (d < R) *reinterpret_cast<f32x4*>(to + d) = sum;
+        } else if (stores) {
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+                if (d + e < R) to[d + e] = sum[e];
+        }
+        if (round + 1 < 2 * FOURS) __syncthreads();
+    }
+}
+
 struct LatentMfmaArgs {
-    const float* q; const bf16_t* pages; const float* sinks; float* out; float* parts; const int* token_request; int n_rows;
+    const float* q; const void* pages; const float* sinks; float* out; float* parts; const int* token_request; int n_rows;
     const int* q_starts; const int* context_lens; const int* block_tables; int max_blocks, n_heads, R, page_size; float scale; int run_length; dim3 grid; hipStream_t stream;
 };
 
 template <int DK>
-void launch_latent_mfma(const LatentMfmaArgs& a) {
-    latent_attention_mfma_kernel<DK><<<a.grid, 64 * LATENT_WAVES, 0, a.stream>>>(a.q, a.pages, a.sinks, a.out, a.parts, a.token_request, a.n_rows, a.q_starts, a.context_lens, a.block_tables,
-                                                                                 a.max_blocks, a.n_heads, a.R, a.page_size, a.scale, a.run_length);
+void launch_latent_mfma(const LatentMfmaArgs& a, int dtype) {
+    auto go = [&](auto kernel, auto pages, int waves) {
+        kernel<<<a.grid, 64 * waves, 0, a.stream>>>(a.q, pages, a.sinks, a.out, a.parts, a.token_request, a.n_rows, a.q_starts, a.context_lens, a.block_tables,
+                                                           a.max_blocks, a.n_heads, a.R, a.page_size, a.scale, a.run_length);
+    };
+    if (dtype == MLLM_F32) go(latent_attention_f32_mfma_kernel<DK>, (const float*)a.pages, LATENT_F32_WAVES);
+    else go(latent_attention_mfma_kernel<DK>, (const bf16_t*)a.pages, LATENT_WAVES);
 }
 
 template <typename KernelT>
@@ -929,7 +1168,7 @@ MLLM_API int mllm_latent_mfma_row_size(int needed) {
 }
 
 MLLM_API int mllm_latent_attention_mfma_supported(int R, int D, int dtype) {
-    return dtype == MLLM_BF16 && R > 0 && R <= D && R <= 256 && mllm_latent_mfma_row_size(D) == D;
+    return (dtype == MLLM_BF16 || dtype == MLLM_F32) && R > 0 && R <= D && R <= 256 && mllm_latent_mfma_row_size(D) == D;
 }
 
 // q_starts [requests + 1] and context_lens [requests] (negative: a padding request): each request's rows are consecutive, its
@@ -937,24 +1176,24 @@ MLLM_API int mllm_latent_attention_mfma_supported(int R, int D, int dtype) {
 MLLM_API int mllm_latent_attention_mfma(const float* q, const void* pages, const float* sinks, float* out, float* parts, const int* token_request,
                                         const int* q_starts, const int* context_lens, const int* block_tables, int max_blocks, int n_rows,
                                         int n_requests, int max_pairs, int n_heads, int R, int D, int page_size, float scale, int n_runs,
-                                        int run_length, hipStream_t stream) {
+                                        int run_length, int dtype, hipStream_t stream) {
     MLLM_REQUIRE(n_rows >= 0 && n_requests >= 0 && n_heads > 0 && max_blocks > 0 && page_size > 0 && max_pairs > 0, "latent_attention_mfma: bad sizes");
-    MLLM_REQUIRE(mllm_latent_attention_mfma_supported(R, D, MLLM_BF16), "latent_attention_mfma: no kernel for rows of %d elements with a latent of %d", D, R);
+    MLLM_REQUIRE(mllm_latent_attention_mfma_supported(R, D, dtype), "latent_attention_mfma: no kernel for rows of %d elements with a latent of %d", D, R);
     MLLM_REQUIRE(n_runs >= 1 && n_runs <= MERGE_MAX_RUNS && n_requests <= 65535 && run_length >= 1 && (n_runs == 1 || run_length % 64 == 0), "latent_attention_mfma: bad runs");
     MLLM_REQUIRE(n_runs == 1 || parts != nullptr, "latent_attention_mfma: runs need room for their sums");
     MLLM_REQUIRE(token_request != nullptr || n_rows == 0, "latent_attention_mfma: no token_request");
     if (n_rows == 0 || n_requests == 0) return 0;
     if (n_runs == 1) run_length = 1 << 30;
-    LatentMfmaArgs a{q, (const bf16_t*)pages, sinks, out, parts, token_request, n_rows, q_starts, context_lens, block_tables, max_blocks, n_heads, R, page_size, scale, run_length,
+    LatentMfmaArgs a{q, pages, sinks, out, parts, token_request, n_rows, q_starts, context_lens, block_tables, max_blocks, n_heads, R, page_size, scale, run_length,
                      dim3(ceil_div(max_pairs, 32), n_requests, n_runs), stream};
     mllm_count_kernel(MLLM_K_LATENT_ATTENTION);
     switch (D / 16) {
-        case 2: launch_latent_mfma<2>(a); break;
-        case 4: launch_latent_mfma<4>(a); break;
-        case 6: launch_latent_mfma<6>(a); break;
-        case 8: launch_latent_mfma<8>(a); break;
-        case 12: launch_latent_mfma<12>(a); break;
-        case 18: launch_latent_mfma<18>(a); break;
+        case 2: launch_latent_mfma<2>(a, dtype); break;
+        case 4: launch_latent_mfma<4>(a, dtype); break;
+        case 6: launch_latent_mfma<6>(a, dtype); break;
+        case 8: launch_latent_mfma<8>(a, dtype); break;
+        case 12: launch_latent_mfma<12>(a, dtype); break;
+        case 18: launch_latent_mfma<18>(a, dtype); break;
     }
     int status = mllm_check_launch("latent_attention_mfma");
     if (status || n_runs == 1) return status;

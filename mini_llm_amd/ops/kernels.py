@@ -1055,6 +1055,13 @@ def heads_linear(x, weight, out, *, n_heads, k, x_head_stride, n_out=None, gate=
 LATENT_RUN_MIN = 64        # cached rows a run of a token's keys should at least hold: a tile of the kernel
 LATENT_TARGET_BLOCKS = 256   # blocks (four waves that share the keys of 32 pairs) the matrix-core kernel's launch should have before keys are left whole
 LATENT_BLOCK_RUN_MIN = 128   # and the cached rows its runs are multiples of there: what a block takes at a time
+# A 32-bit cache runs through the matrix-core kernel from so many (token, head) pairs on, if a sequence may be longer than so many keys. The kernel of a wave (or
+# block) a row / it, us, rows of 288 floats, 12 heads: a prompt of 128 19.0 / 19.5, of 260 39.0 / 37.0, of 640 136 / 57, of 1,024 401 / 87, six prompts of 19 to
+# 640 304 / 119; 6 heads over rows of 192: 260 (1,560 pairs) 24.7 / 30.1, 508 (3,048) 45 / 48, 640 62 / 41; 64 single tokens over 600 keys 37.5 / 32.7, 256 of
+# them 124 / 60. Short sequences leave seven of a block's eight waves without a tile: 100 prompts of 20 35 / 75, 256 single tokens over 60 keys 14.9 / 19.7, 64
+# portions of 8 over 60 37 / 20.
+LATENT_F32_PAIRS = 3072
+LATENT_F32_KEYS = 64
 LATENT_TARGET_WAVES = 2048   # waves a launch should have before a token's keys are left whole (eight to a compute unit)
 
 
@@ -1076,8 +1083,8 @@ def latent_attention(q_full, pages, sinks, token_request, positions, block_table
     q_full: float32 [rows, n_heads, row_size]; pages [num_pages, 1, page_size, row_size]. Returns float32 [rows, n_heads,
     rank]. Few rows with many keys are cut into runs of keys (``max_len``: the longest sequence of the batch).
     With ``q_starts`` ([requests + 1]: each request's rows are consecutive), ``context_lens`` ([requests]: the position of a
-    request's first row; negative: a padding request) and ``max_q_len``, a bfloat16 cache of a row size the matrix-core kernel
-    takes runs through that kernel (32 (token, head) pairs of a request to a block)."""
+    request's first row; negative: a padding request) and ``max_q_len``, a cache of a row size the matrix-core kernels
+    take runs through them (32 (token, head) pairs of a request to a block; a 32-bit cache where LATENT_F32_PAIRS and LATENT_F32_KEYS say so)."""
     _device_tensor(q_full, "q_full", torch.float32, 3)
     _device_tensor(pages, "pages", dim=4)
     n, n_heads, row_size = q_full.shape
@@ -1097,6 +1104,7 @@ def latent_attention(q_full, pages, sinks, token_request, positions, block_table
     reach = block_tables.shape[1] * page_size
     longest = reach if max_len is None else max(1, min(int(max_len), reach))
     if (q_starts is not None and context_lens is not None and max_q_len is not None
+            and (pages.dtype != torch.float32 or (n * n_heads >= LATENT_F32_PAIRS and longest > LATENT_F32_KEYS))
             and lib.mllm_latent_attention_mfma_supported(int(rank), row_size, _code(pages.dtype))):
         _device_tensor(q_starts, "q_starts", torch.int32, 1)
         _device_tensor(context_lens, "context_lens", torch.int32, 1)
@@ -1110,7 +1118,7 @@ def latent_attention(q_full, pages, sinks, token_request, positions, block_table
         _require(n_requests >= 1, "rows of no request")
         check(lib.mllm_latent_attention_mfma(_ptr(q_full), _ptr(pages), _ptr(sinks), _ptr(out), _ptr(parts), _ptr(token_request), _ptr(q_starts),
                                              _ptr(context_lens), _ptr(block_tables), block_tables.shape[1], n, n_requests, max_pairs, n_heads,
-                                             int(rank), row_size, page_size, float(scale), n_runs, run_length, _stream()))
+                                             int(rank), row_size, page_size, float(scale), n_runs, run_length, _code(pages.dtype), _stream()))
         return out
     # a wave takes a row's keys for a group of heads: few rows with many keys are cut into runs, a wave each
     waves = n * -(-n_heads // int(library().mllm_latent_attention_head_group(n_heads)))

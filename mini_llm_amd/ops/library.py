@@ -85,7 +85,7 @@ _SIGNATURES = {
     "mllm_latent_attention_head_group": [c_int],
     "mllm_latent_mfma_row_size": [c_int],
     "mllm_latent_attention_mfma_supported": [c_int, c_int, c_int],
-    "mllm_latent_attention_mfma": [P, P, P, P, P, P, P, P, P, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_float, c_int, c_int, P],
+    "mllm_latent_attention_mfma": [P, P, P, P, P, P, P, P, P, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_float, c_int, c_int, c_int, P],
     "mllm_latent_attention": [P, P, P, P, P, P, P, P, c_int, c_int, c_int, c_int, c_int, c_int, c_float, c_int, c_int, c_int, P],
     "mllm_projection_rows": [P, c_int, P, c_int, P, c_int, P, c_int, P, P, P, c_float, P, c_int, P, P, P, P, P, c_int, c_int, c_int, c_int, c_int, c_int, c_int,
                              c_int, c_int, P],
