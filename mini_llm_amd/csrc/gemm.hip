@@ -731,6 +731,21 @@ int tiled_k_blocks(int M, int N, int K, int most) {
         }
         return best;
     }
+    if (sizeof(T) == 2 && K % 64 == 0 && N % 8 == 0) {
+        // By the costs of the streaming kernel's tiles and what the partial products cost: each is written and read, whoever adds them up reads the stream and
+        // writes it again (at 5.5 TB/s), and has one more load under way. With the layer norm behind it, whole / as this rule cuts it, us: 80 x 768 x 3,072 18.3 /
+        // 10.3 (in eight), 528 x 1,024 x 4,096 23.4 / 17 (three), 1,024 x 768 x 3,072 20.8 / 18.7 (two), 1,500 x 1,600 x 6,400 49.0 / 45.2 (two); left whole:
+        // 2,048 x 768 x 3,072 23.1 (24.5 in two), 528 x 1,024 x 1,024 12.5 (12.9 in two), 2,048 x 1,600 x 6,400 55.2 (57.6 in two).
+        const int rows = ceil_div(M, 128) * 128;
+        const float output_us = (float)rows * (float)N * 4.0f / 5.5e6f;
+        int best = 1;
+        float best_us = 0.0f;
+        for (int cuts = 1; cuts <= std::min(8, most) && (cuts == 1 || K >= 4 * 64 * cuts); cuts++) {
+            const float us = stream::product_us(stream::tile_costs()[stream::best_tile(rows, N, K, cuts)], rows, N, K, cuts) + (cuts == 1 ? 0.0f : output_us * (3.0f + 1.3f * (float)cuts) + 0.15f * (float)cuts);
+            if (cuts == 1 || us < best_us) best = cuts, best_us = us;
+        }
+        return best;
+    }
     if (tiles > 128) return 1;
     const int least_tiles = M <= 256 ? 4 : 8;
     while (k_blocks < 8 && tiles * k_blocks * 2 <= 384 && K >= least_tiles * Tile<T>::BK * k_blocks * 2) k_blocks *= 2;

@@ -20,7 +20,7 @@
 //  * With loads into LDS under way the compiler can only wait for all LDS operations at once before
 //    the first use of any value read from LDS. The fragment reads are therefore inline assembly the
 //    compiler does not see through, with the wave's own counted waits.
-//  * The blocks of one XCD take the tiles of one rectangle of the output: the eight L2 caches then
+//  * The blocks of one XCD take neighbouring tiles of the output, about a rectangle: the eight L2 caches then
 //    each fetch a part of A and W once (taking tiles in turn, every XCD reads nearly all of both:
 //    21.4 -> 18.3 us for 2,048 x 768 x 3,072).
 //  * W is the first operand of the matrix instruction: a lane then holds four consecutive columns
@@ -82,18 +82,28 @@ __device__ __forceinline__ void fragments_landed(i32x4& first) {
 __device__ __forceinline__ void and_this_one(i32x4& fragment) { asm volatile("" : "+v"(fragment)); }
 __device__ __forceinline__ void still_written(const i32x4& fragment) { asm volatile("" : : "v"(fragment)); }
 
-// Eight rectangles of 'wide' x 'high' tiles, 'across' of them side by side along N, cover the tiles of the output.
+// Where blocks find their tiles. The tiles of the output lie in strips of `strip` rows of tiles, a strip column by column; each part of K has them all, the parts
+// behind each other; and an XCD takes the next `per_xcd` of that list, which is about a rectangle of the output.
 struct XcdTiles {
-    int across, wide, high;
+    int tiles_m, tiles_n, strip, per_xcd, count;
 };
-// the split of the eight rectangles (1 x 8, 2 x 4, 4 x 2 or 8 x 1) whose rectangle needs the fewest rows of A and W together
-inline XcdTiles place_tiles(int tiles_m, int tiles_n, int bm, int bn) {
-    XcdTiles best{1, tiles_n, ceil_div(tiles_m, 8)};
+// The strip is as high as makes the rows of A and W that the XCDs read the fewest. Equal shares come first: one block more than 32 on one XCD is a second round
+// of its compute units (rectangles of equal sides that cover the tiles give some XCDs full ones and others a remainder: 528 x 1,024 x 4,096 in three parts along K,
+// 240 blocks, were 36 on six of them: 23.6 us).
+inline XcdTiles place_tiles(int tiles_m, int tiles_n, int bm, int bn, int k_blocks) {
+    const int tiles = tiles_m * tiles_n, count = tiles * k_blocks, per_xcd = ceil_div(count, 8);
+    XcdTiles best{tiles_m, tiles_n, 1, per_xcd, count};
     long best_rows = -1;
-    for (int across = 1; across <= 8; across *= 2) {
-        const int wide = ceil_div(tiles_n, across), high = ceil_div(tiles_m, 8 / across);
-        const long rows = (long)wide * bn + (long)high * bm;
-        if (best_rows < 0 || rows < best_rows) best = XcdTiles{across, wide, high}, best_rows = rows;
+    for (int strip = 1; strip <= tiles_m && strip <= 16; strip++) {
+        const int in_strip = strip * tiles_n;
+        long rows = 0;
+        for (int xcd = 0; xcd < 8; xcd++) {
+            const int from = xcd * per_xcd % tiles, to = from + (per_xcd < tiles ? per_xcd : tiles) - 1;   // (of the parts along K the first it takes)
+            const int strips = to / in_strip - from / in_strip + 1, first = from % in_strip / strip, last = to % in_strip / strip;
+            const int columns = strips == 1 ? last - first + 1 : strips == 2 && last < first ? tiles_n - first + last + 1 : tiles_n;
+            rows += (long)strips * strip * bm + (long)columns * bn;
+        }
+        if (best_rows < 0 || rows < best_rows) best.strip = strip, best_rows = rows;
     }
     return best;
 }
@@ -179,8 +189,8 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N * WAVES_K) void gemm_stream_
     const int tid = threadIdx.x, lane = tid % WAVE;
     const int wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
     const int wave_k = wave / (WAVES_M * WAVES_N), wave_m = wave / WAVES_N % WAVES_M, wave_n = wave % WAVES_N;
-    // Blocks go round the eight XCDs in turn, each with an L2 of its own: the blocks of one XCD take the tiles of one
-    // rectangle of the output, so that the rows of A and of W an XCD reads are few and each is fetched into its L2 once.
+    // Blocks go round the eight XCDs in turn, each with an L2 of its own: the blocks of one XCD take neighbouring tiles of the
+    // output, so that the rows of A and of W an XCD reads are few and each is fetched into its L2 once.
     const int xcd = blockIdx.x % 8, in_xcd = blockIdx.x / 8;
     int block_k = 0, m0, n0, m_end = M, w_first_tile = 0;
     if constexpr (GROUPED) {
@@ -191,11 +201,13 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N * WAVES_K) void gemm_stream_
         n0 = tile.n0;
         w_first_tile = tile.expert * ((N + 15) / 16);
     } else {
-        block_k = in_xcd / (places.wide * places.high);
-        const int in_rectangle = in_xcd % (places.wide * places.high);
-        m0 = ((xcd / places.across) * places.high + in_rectangle / places.wide) * BM;
-        n0 = ((xcd % places.across) * places.wide + in_rectangle % places.wide) * BN;
-        if (m0 >= M || n0 >= N) return;  // (the rectangles cover more than the matrix; the whole block leaves)
+        const int item = xcd * places.per_xcd + in_xcd, tiles = places.tiles_m * places.tiles_n;
+        if (item >= places.count) return;  // (eight equal shares may be a few more; the whole block leaves)
+        block_k = item / tiles;
+        const int tile = item % tiles, strip = tile / (places.strip * places.tiles_n), in_strip = tile % (places.strip * places.tiles_n);
+        const int high = min(places.strip, places.tiles_m - strip * places.strip);
+        m0 = (strip * places.strip + in_strip % high) * BM;
+        n0 = in_strip / high * BN;
     }
     const int n_out = GATED ? N / 2 : N;
     const int k_begin = block_k * k_per_block, k_end = min(K, k_begin + k_per_block);
@@ -557,9 +569,9 @@ void launch(const bf16_t* a, const bf16_t* w, const float* bias, const float* re
                                      hipFuncAttributeMaxDynamicSharedMemorySize, LDS_BYTES) == hipSuccess;
     }
     const int k_per_block = k_blocks == 1 ? K : ceil_div(ceil_div(K, k_blocks), 64) * 64;
-    const XcdTiles places = place_tiles(ceil_div(M, BM), ceil_div(N, BN), BM, BN);
+    const XcdTiles places = place_tiles(ceil_div(M, BM), ceil_div(N, BN), BM, BN, k_blocks);
     mllm_count_kernel(MLLM_K_GEMM_STREAM);
-    gemm_stream_kernel<OutT, BM, BN, WAVES_M, WAVES_N, WAVES_K, STAGES, Whole><<<8 * places.wide * places.high * k_blocks, 64 * NW, LDS_BYTES, stream>>>(
+    gemm_stream_kernel<OutT, BM, BN, WAVES_M, WAVES_N, WAVES_K, STAGES, Whole><<<8 * places.per_xcd, 64 * NW, LDS_BYTES, stream>>>(
         a, w, bias, residual, o, M, N, K, epilogue, scatter, k_per_block, places, Whole{});
 }
 
@@ -576,7 +588,7 @@ void launch_grouped(const bf16_t* a, const bf16_t* w, OutT* o, int entries, int 
     const int blocks = ceil_div(max_tiles * ceil_div(N, BN), 8) * 8;
     mllm_count_kernel(MLLM_K_GEMM_STREAM);
     gemm_stream_kernel<OutT, BM, BN, WAVES_M, WAVES_N, 1, STAGES, Group><<<blocks, 64 * NW, LDS_BYTES, stream>>>(
-        a, w, nullptr, nullptr, o, entries, N, K, MLLM_EPI_NONE, CacheScatter{}, K, XcdTiles{1, 1, 1}, group);
+        a, w, nullptr, nullptr, o, entries, N, K, MLLM_EPI_NONE, CacheScatter{}, K, XcdTiles{1, 1, 1, 1, 1}, group);
 }
 
 // Whether the product takes this kernel: bfloat16 with a packed W, whole tiles of K, whole 16-byte pieces of output
@@ -591,47 +603,76 @@ inline bool takes(int M, int N, int K, bool packed, const CacheScatter& scatter,
     return true;
 }
 
-// The tile is chosen by what the busiest compute unit has to do: every block keeps a compute unit to itself (its
-// stages fill most of the LDS), so the blocks run in rounds of 256, and a round costs what a tile of K costs the block
-// (measured at GPT-2's three widths, 512 to 4,096 rows: 0.57 us at 128 x 192, 0.45 at 128 x 128, 0.70 at 256 x 128,
-// 0.30 at 128 x 64). Wide tiles win where they still fill a round; narrow outputs take 128 x 64, with two waves
-// sharing each 64 x 64 tile along K and a fourth stage where K is long.
+// The tile is chosen by what the busiest compute unit has to do: every block keeps a compute unit to itself (its stages fill most of the LDS), so the
+// blocks run in rounds of 256, and a round costs what a block costs before and behind its loop and what a tile of K costs it. Measured at GPT-2's three
+// widths, 300 to 4,096 rows, K of 768 to 6,400 (start_us without the 3 us that any kernel takes in a chain of them). Wide tiles win where they still fill a
+// round; 192 rows where that makes one round of what would be a few blocks more than one, or fewer and fuller blocks.
+// Stages: four of 128 x 128 and 128 x 64. With three the loads of a tile have two tiles' products to land, which at these sizes is too little, and a fifth is
+// slower again: us with three / four / five stages, 2,048 rows: 128 x 128 at 1,600 x 6,400 49.5 / 47.1 / 49.9, at 1,600 x 1,600 18.3 / 17.5 / 18.6; 528 rows at
+// 4,096 x 1,024 11.2 / 10.4 / 11.4; 128 x 64 at 768 x 768 8.8 / 8.4. The larger tiles stay at three: with a fourth, all 160 KB of a unit's LDS, a layer's up
+// product (128 x 192, 2,048 x 3,072 x 768) took 18.1 us inside a prompt step where it takes 17.1.
+// 192 x 128 at 2,304 x 768, inside a prompt step: 14.6 where 128 x 192 takes 15.0; at 1,500 rows of 3,072 x 768 12.2 and 13.1.
+struct TileCost {
+    int bm, bn;
+    float start_us, tile_us;
+};
+constexpr int TILES = 5;
+inline const TileCost* tile_costs() {
+    static const TileCost costs[TILES] = {{128, 192, 5.1f, 0.46f}, {192, 128, 4.6f, 0.46f}, {256, 128, 4.2f, 0.62f}, {128, 128, 3.7f, 0.42f}, {128, 64, 2.2f, 0.28f}};
+    return costs;
+}
+// us of the product with that tile in k_blocks parts along K
+inline float product_us(const TileCost& tile, int M, int N, int K, int k_blocks) {
+    const long blocks = (long)ceil_div(M, tile.bm) * ceil_div(N, tile.bn) * k_blocks;
+    return (float)((blocks + 255) / 256) * (tile.start_us + (float)ceil_div(ceil_div(K, k_blocks), 64) * tile.tile_us);
+}
+inline int best_tile(int M, int N, int K, int k_blocks) {
+    int best = 0;
+    for (int c = 1; c < TILES; c++)
+        if (product_us(tile_costs()[c], M, N, K, k_blocks) < product_us(tile_costs()[best], M, N, K, k_blocks)) best = c;   // (equal costs: the wider tile, which reads less)
+    return best;
+}
+
 template <typename OutT>
 void dispatch(const bf16_t* a, const bf16_t* w, const float* bias, const float* residual, OutT* o, int M, int N, int K, int epilogue,
              hipStream_t stream, CacheScatter scatter, int k_blocks) {
 #define MLLM_STREAM(BM, BN, WM_, WN_, WK_, ST) launch<OutT, BM, BN, WM_, WN_, WK_, ST>(a, w, bias, residual, o, M, N, K, epilogue, stream, scatter, k_blocks)
-    struct Choice {
-        int bm, bn;
-        float tile_us;
-    };
-    static const Choice choices[4] = {{128, 192, 0.57f}, {256, 128, 0.70f}, {128, 128, 0.45f}, {128, 64, 0.30f}};
-    int best = 0;
-    float best_cost = 0.0f;
-    for (int c = 0; c < 4; c++) {
-        const long blocks = (long)ceil_div(M, choices[c].bm) * ceil_div(N, choices[c].bn) * k_blocks;
-        const float cost = (float)((blocks + 255) / 256) * choices[c].tile_us;
-        if (c == 0 || cost < best_cost) best = c, best_cost = cost;  // (equal costs: the wider tile, which reads less)
-    }
     // 256 x 256 (four waves of 128 x 128; the LDS holds two stages of it) brings a compute unit 40k outputs a microsecond
     // and tile of K where the others bring 30k, but only in full rounds of at least 150 blocks: from 2,048 x 6,400 on.
-    // Measured against the choice among the others (whose costs above are those of smaller products: at these sizes
-    // they take 1.45 times as long), on one machine in one run: 2,048 x 6,400 x 1,600 52 against 59 us (as a layer's up
+    // Measured against the best of the others, on one machine in one run: 2,048 x 6,400 x 1,600 52 against 59 us (as a layer's up
     // product with its GELU 52.5 against 56.2), 8,192 x 4,096 x 1,024 74 against 85, 8,192 x 6,400 x 1,600 186 against 194;
     // but 2,048 x 4,096 x 1,024 (128 blocks) 30.7 against 23.2. (Machines of this kind differ by a tenth between them:
-    // another one took 45.2 and 52.4 us for the first of these.)
+    // another one took 45.2 and 52.4 us for the first of these.) In such rounds a tile of K costs it 1.6 us and the others 1.45 times these:
     // (Only with bfloat16 out, which is what the products of that size write: with 32-bit out and a residual asked for
     // before the loop, a lane's 256 sums and 256 residual values do not fit its registers.)
     if constexpr (sizeof(OutT) == 2) {
+        static const float in_full_rounds[4][3] = {{128, 192, 0.57f}, {256, 128, 0.70f}, {128, 128, 0.45f}, {128, 64, 0.30f}};
         const long large = (long)ceil_div(M, 256) * ceil_div(N, 256), rounds = (large + 255) / 256;
-        if (k_blocks == 1 && large >= 150 && large * 10 >= rounds * 256 * 7 && (float)rounds * 1.6f < best_cost * 1.45f) {
-            MLLM_STREAM(256, 256, 2, 2, 1, 2);
-            return;
+        if (k_blocks == 1 && large >= 150 && large * 10 >= rounds * 256 * 7) {
+            float others = 1e30f;
+            for (const auto& tile : in_full_rounds) {
+                const long blocks = (long)ceil_div(M, (int)tile[0]) * ceil_div(N, (int)tile[1]);
+                others = fminf(others, (float)((blocks + 255) / 256) * tile[2]);
+            }
+            if ((float)rounds * 1.6f < others * 1.45f) {
+                MLLM_STREAM(256, 256, 2, 2, 1, 2);
+                return;
+            }
         }
     }
+    const int best = best_tile(M, N, K, k_blocks), k_part = ceil_div(K, k_blocks);
+    const bool one_round = (long)ceil_div(M, 128) * ceil_div(N, 64) * k_blocks <= 256;
     if (best == 0) MLLM_STREAM(128, 192, 2, 2, 1, 3);
-    else if (best == 1) MLLM_STREAM(256, 128, 4, 2, 1, 3);
-    else if (best == 2) MLLM_STREAM(128, 128, 2, 2, 1, 3);
-    else if (K / k_blocks >= 1536) MLLM_STREAM(128, 64, 2, 1, 2, 4);
+    else if (best == 1) MLLM_STREAM(192, 128, 2, 2, 1, 3);
+    else if (best == 2) MLLM_STREAM(256, 128, 4, 2, 1, 3);
+    // eight waves of 64 x 32, two a SIMD, cover each other's way out of the loop where four of 64 x 64 read less in it: 528 x 4,096 x 1,024 10.1 and 10.5 us, 1,500 x
+    // 3,072 x 768 17.3 and 18.1; GPT-2 XL's output and down products, 2,048 rows, inside a prompt step 41.4 and 42.3 on average
+    else if (best == 3) MLLM_STREAM(128, 128, 2, 4, 1, 4);
+    // narrow outputs in one round of blocks: four stages (a layer's down product, 2,048 x 768 x 3,072, 22.8 us in a prompt step, 23.4 with two waves sharing each
+    // 64 x 64 tile along K, 26.0 with three stages); in more rounds two waves share a tile along K where K is long, and else three stages leave room for two blocks
+    // a compute unit
+    else if (one_round) MLLM_STREAM(128, 64, 2, 2, 1, 4);
+    else if (k_part >= 1536) MLLM_STREAM(128, 64, 2, 1, 2, 4);
     else MLLM_STREAM(128, 64, 2, 2, 1, 3);
 #undef MLLM_STREAM
 }
