@@ -768,24 +768,42 @@ __device__ __forceinline__ f32x4 pending_piece(const PendingSum& in, int row_ind
     return value;
 }
 
-// The share of group `group` of `n_groups` in those four columns: the partial rows group, group + n_groups, ..., and with
-// group 0 the base row and the bias.
-__device__ __forceinline__ f32x4 pending_piece_share(const PendingSum& in, int row_index, int width, int piece, int group, int n_groups) {
-    f32x4 value = {0.0f, 0.0f, 0.0f, 0.0f};
-    if (group == 0) {
-        value = load4(in.base + (size_t)row_index * width + 4 * piece);
-        if (in.bias) value += load4(in.bias + 4 * piece);
+// The same as loads alone, all of them under way before the first is waited for (a bias added under a condition made the partial rows wait for it): up to
+// eight partial rows; take() adds up, the further ones eight at a time.
+struct PendingLoads {
+    f32x4 base, bias, part[8];
+    __device__ __forceinline__ void ask(const PendingSum& in, int row_index, int width, int piece, int first, int step) {
+        base = load4(in.base + (size_t)row_index * width + 4 * piece);
+        bias = load4(in.bias ? in.bias + 4 * piece : in.base + (size_t)row_index * width + 4 * piece);   // a vector that is there stands in for one that is not
+        ask_parts(in, row_index, width, piece, first, step);
     }
-    for (int s0 = group; s0 < in.n_partials; s0 += 8 * n_groups) {
-        f32x4 part[8];
+    __device__ __forceinline__ void ask_parts(const PendingSum& in, int row_index, int width, int piece, int first, int step) {
+        const float* rows = in.n_partials > 0 ? in.partials : in.base;
+        auto ask_part = [&](int u) {
+            const size_t matrix = in.n_partials > 0 ? (size_t)min(first + u * step, in.n_partials - 1) * in.rows : 0;
+            part[u] = load4(rows + (matrix + row_index) * width + 4 * piece);
+        };
 #pragma unroll
-        for (int u = 0; u < 8; u++)
-            part[u] = load4(in.partials + ((size_t)min(s0 + u * n_groups, in.n_partials - 1) * in.rows + row_index) * width + 4 * piece);
+        for (int u = 0; u < 4; u++) ask_part(u);
+        if (in.n_partials > 4 * step) {   // (the same for the whole launch)
 #pragma unroll
-        for (int u = 0; u < 8; u++) value += part[u] * (s0 + u * n_groups < in.n_partials ? 1.0f : 0.0f);
+            for (int u = 4; u < 8; u++) ask_part(u);
+        } else {
+#pragma unroll
+            for (int u = 4; u < 8; u++) part[u] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        }
     }
-    return value;
-}
+    __device__ __forceinline__ f32x4 take(const PendingSum& in, int row_index, int width, int piece, int first, int step) {
+        f32x4 value = {0.0f, 0.0f, 0.0f, 0.0f};
+        if (first == 0) value = in.bias ? base + bias : base;
+        for (int s0 = first; s0 < in.n_partials; s0 += 8 * step) {
+            if (s0 > first) ask_parts(in, row_index, width, piece, s0, step);
+#pragma unroll
+            for (int u = 0; u < 8; u++) value += part[u] * (s0 + u * step < in.n_partials ? 1.0f : 0.0f);
+        }
+        return value;
+    }
+};
 
 // out = base + bias + the partial rows: the pending stream as plain rows, for whatever does not
 // take it pending. grid (pieces of 256 x 4 columns, rows).
@@ -795,37 +813,73 @@ __global__ __launch_bounds__(256) void pending_sum_kernel(PendingSum in, float* 
     *reinterpret_cast<f32x4*>(out + (size_t)row_index * width + 4 * piece) = pending_piece(in, row_index, width, piece);
 }
 
-// Row LayerNorm of pending rows (the sums are taken on the way in): a block a row, the row kept in LDS; row_index, if
-// given, names the pending row of each output row. Centred, in 32-bit, like the norm of plain rows (elementwise.hip).
-// GROUPS > 1 (a row of many partial rows, few of them in a launch: the rows a decode step's last layer leaves for the
-// final norm): the block's threads in so many groups of `group_lanes`, each of which adds up every GROUPS-th partial row,
-// all asked for at once; their shares meet in LDS, in a fixed order.
-// THREADS: as many as a row has pieces of four columns, up to 1,024, so that a thread's pieces are one trip to memory and not two behind each other.
+// Row LayerNorm of pending rows (the sums are taken on the way in): a block a row; row_index, if given, names the pending row of each output row. Centred, in
+// 32-bit, like the norm of plain rows (elementwise.hip). THREADS: as many as a row has pieces of four columns, rounded up, so that a thread owns one piece and
+// everything it needs of it (the row, its bias, up to eight partial rows, gain and offset) is one trip to memory: a kernel of few rows is little else. With the
+// partial rows asked for behind the bias and gain and offset behind the statistics, three trips, 64 rows of 1,024 with four partial rows took PENDING_FIGURES
+// GROUPS > 1 (a row of many partial rows, few of them in a launch: the rows a decode step's last layer leaves for the final norm): the block's threads in so many
+// groups of `group_lanes`, each of which adds up every GROUPS-th partial row, all asked for at once; their shares meet in LDS, in a fixed order.
 template <typename OutT, int GROUPS, int THREADS>
 __global__ __launch_bounds__(THREADS) void pending_layernorm_kernel(
     PendingSum in, const int* __restrict__ row_index, const float* __restrict__ gamma, const float* __restrict__ beta,
     OutT* __restrict__ out, float* __restrict__ summed, int width, float eps, int packed_out, int group_lanes) {
     constexpr int WAVES = THREADS / WAVE;
-    extern __shared__ f32x4 row_pieces[];  // width / 4, and behind them GROUPS x width / 4 for the groups' shares
+    extern __shared__ f32x4 group_shares[];  // GROUPS > 1: GROUPS x width / 4
     __shared__ float red[2][WAVES];
     const int tid = threadIdx.x, n_pieces = width / 4;
     const int source = row_index ? row_index[blockIdx.x] : blockIdx.x;
+    const bool owns = tid < n_pieces;
+    const int own_piece = min(tid, n_pieces - 1);
+    PendingLoads loads;
+    const int group = GROUPS > 1 ? tid / group_lanes : 0, piece = GROUPS > 1 ? min(tid % group_lanes, n_pieces - 1) : own_piece;
+    loads.ask(in, source, width, piece, group, GROUPS);
+    const f32x4 gain = load4(gamma + 4 * own_piece), offset = load4(beta + 4 * own_piece);
+    keep_order();
+    f32x4 value = loads.take(in, source, width, piece, group, GROUPS);
     if constexpr (GROUPS > 1) {
-        const int group = tid / group_lanes, piece = tid % group_lanes;
-        if (group < GROUPS && piece < n_pieces)
-            row_pieces[(1 + group) * n_pieces + piece] = pending_piece_share(in, source, width, piece, group, GROUPS);
+        if (group < GROUPS && tid % group_lanes < n_pieces) group_shares[group * n_pieces + piece] = value;
         __syncthreads();
+        value = group_shares[own_piece];
+#pragma unroll
+        for (int g = 1; g < GROUPS; g++) value += group_shares[g * n_pieces + own_piece];
     }
+    if (summed && owns) *reinterpret_cast<f32x4*>(summed + (size_t)blockIdx.x * width + 4 * tid) = value;  // the row with its sums taken
+    const float sum = wave_total(owns ? (value[0] + value[1]) + (value[2] + value[3]) : 0.0f);
+    if (tid % WAVE == 0) red[0][tid / WAVE] = sum;
+    __syncthreads();
+    const float n = (float)width;
+    float total = 0.0f;
+#pragma unroll
+    for (int w = 0; w < WAVES; w += 4) total += (red[0][w] + red[0][w + 1]) + (red[0][w + 2] + red[0][w + 3]);
+    const f32x4 centred = value - total / n;
+    const float squares = wave_total(owns ? (centred[0] * centred[0] + centred[1] * centred[1]) + (centred[2] * centred[2] + centred[3] * centred[3]) : 0.0f);
+    if (tid % WAVE == 0) red[1][tid / WAVE] = squares;
+    __syncthreads();
+    total = 0.0f;
+#pragma unroll
+    for (int w = 0; w < WAVES; w += 4) total += (red[1][w] + red[1][w + 1]) + (red[1][w + 2] + red[1][w + 3]);
+    const float inverse_stddev = 1.0f / sqrtf(total / n + eps);
+    if (!owns) return;
+    const f32x4 y = centred * inverse_stddev * gain + offset;
+    // four consecutive columns lie together in the packed layout too (inside one 16-byte piece)
+    OutT* at = out + (packed_out ? packed_element<OutT>(blockIdx.x, 4 * tid, width) : (size_t)blockIdx.x * width + 4 * tid);
+    if constexpr (sizeof(OutT) == 2) store_bf16x4(at, y);
+    else *reinterpret_cast<f32x4*>(at) = y;
+}
+
+// The same for rows of more than 4,096, of which a thread takes several pieces and the row lies in LDS meanwhile.
+template <typename OutT, int THREADS>
+__global__ __launch_bounds__(THREADS) void pending_layernorm_long_kernel(
+    PendingSum in, const int* __restrict__ row_index, const float* __restrict__ gamma, const float* __restrict__ beta,
+    OutT* __restrict__ out, float* __restrict__ summed, int width, float eps, int packed_out) {
+    constexpr int WAVES = THREADS / WAVE;
+    extern __shared__ f32x4 row_pieces[];  // width / 4
+    __shared__ float red[2][WAVES];
+    const int tid = threadIdx.x, n_pieces = width / 4;
+    const int source = row_index ? row_index[blockIdx.x] : blockIdx.x;
     float sum = 0.0f;
     for (int piece = tid; piece < n_pieces; piece += THREADS) {
-        f32x4 value;
-        if constexpr (GROUPS > 1) {
-            value = row_pieces[n_pieces + piece];
-#pragma unroll
-            for (int g = 1; g < GROUPS; g++) value += row_pieces[(1 + g) * n_pieces + piece];
-        } else {
-            value = pending_piece(in, source, width, piece);
-        }
+        const f32x4 value = pending_piece(in, source, width, piece);
         row_pieces[piece] = value;
         if (summed) *reinterpret_cast<f32x4*>(summed + (size_t)blockIdx.x * width + 4 * piece) = value;  // the row with its sums taken
         sum += (value[0] + value[1]) + (value[2] + value[3]);
@@ -1018,14 +1072,14 @@ MLLM_API int mllm_pending_layernorm(const float* base, const float* partials, co
     // groups of threads take every fourth partial row each. Where the rows are many the compute units are busy as it is.
     const int group_lanes = (width / 4 + WAVE - 1) / WAVE * WAVE;
     const bool grouped = n_partials >= 16 && n_rows <= 64 && 4 * group_lanes <= 1024;
-    // (rows of 1,600 with 256 threads took 144 of them through two trips to memory: 64 rows in a decode step 5.9 us, with 512 threads 5.0)
 #define MLLM_PENDING_NORM_WITH(OutT, GROUPS, THREADS) \
-    pending_layernorm_kernel<OutT, GROUPS, THREADS><<<n_rows, THREADS, (size_t)width * 4 * (GROUPS == 1 ? 1 : 1 + GROUPS), stream>>>(in, row_index, gamma, beta, (OutT*)out, summed, width, eps, packed_out, group_lanes)
+    pending_layernorm_kernel<OutT, GROUPS, THREADS><<<n_rows, THREADS, (size_t)width * 4 * (GROUPS == 1 ? 0 : GROUPS), stream>>>(in, row_index, gamma, beta, (OutT*)out, summed, width, eps, packed_out, group_lanes)
 #define MLLM_PENDING_NORM(OutT)                                            \
     if (grouped) MLLM_PENDING_NORM_WITH(OutT, 4, 1024);                    \
     else if (width <= 1024) MLLM_PENDING_NORM_WITH(OutT, 1, 256);          \
     else if (width <= 2048) MLLM_PENDING_NORM_WITH(OutT, 1, 512);          \
-    else MLLM_PENDING_NORM_WITH(OutT, 1, 1024);
+    else if (width <= 4096) MLLM_PENDING_NORM_WITH(OutT, 1, 1024);         \
+    else pending_layernorm_long_kernel<OutT, 1024><<<n_rows, 1024, (size_t)width * 4, stream>>>(in, row_index, gamma, beta, (OutT*)out, summed, width, eps, packed_out);
     if (out_dtype == MLLM_F32) {
         MLLM_PENDING_NORM(float)
     } else if (out_dtype == MLLM_BF16) {
