@@ -127,6 +127,89 @@ __global__ __launch_bounds__(256) void rms_norm_kernel(const float* __restrict__
     }
 }
 
+// The same, a block a row, a thread four neighbouring columns (width a multiple of 4, up to 4 * THREADS; operands on their own size's borders): all a thread
+// needs is a handful of 16-byte loads in one trip to memory. A wave a row asks for its columns one number at a time, five arrays of up to sixteen loads a
+// lane before it can add anything up. A wave a row / a block a row, us, in 32-bit with a residual and a second norm: rows of 768, 8 of them 4.1 / 2.7 (two partial
+// products 4.2 / 3.0, five 5.1 / 3.1), 256 4.4 / 2.9, 2,048 6.3 / 5.9; rows of 1,600, 8 of them 6.2 / 2.9, 2,048 14.2 / 10.1; without either, rows of 768, 8 of
+// them 3.8 / 2.4, 2,048 4.8 / 4.1. Where many rows are narrow most of a block has nothing to do (4,096 rows of 60 2.9 / 4.8), and many thousand rows with many partial
+// products are bound by their bytes either way (32,768 rows of 768 with five 141 / 147): a wave a row there.
+template <int THREADS>
+__global__ __launch_bounds__(THREADS) void rms_norm_row_kernel(const float* __restrict__ x, const void* __restrict__ y, int y_code, float alpha,
+                                                               const int* __restrict__ row_index, const float* __restrict__ weight, int one_plus,
+                                                               float eps, float* __restrict__ stream, void* __restrict__ rows, int rows_code, int width,
+                                                               int n_partials, long long partial_stride, const float* __restrict__ residual,
+                                                               const float* __restrict__ next_weight) {
+    constexpr int WAVES = THREADS / WAVE, AHEAD = 8;
+    __shared__ float shares[2][WAVES];
+    const int row = blockIdx.x, source = row_index ? row_index[row] : row, column = 4 * threadIdx.x;
+    const bool owns = column < width;
+    const int at = min(column, width - 4);
+    const size_t in_at = (size_t)source * width + at, out_at = (size_t)row * width + at;
+    const float plus = one_plus ? 1.0f : 0.0f;
+    // (an array that is there stands in for one that is not)
+    const f32x4 own = *reinterpret_cast<const f32x4*>(x + in_at), gain = *reinterpret_cast<const f32x4*>(weight + at);
+    const f32x4 base = *reinterpret_cast<const f32x4*>(residual ? residual + out_at : x + in_at);
+    const f32x4 next_gain = *reinterpret_cast<const f32x4*>((next_weight ? next_weight : weight) + at);
+    f32x4 part[AHEAD];
+    const float* parts = reinterpret_cast<const float*>(y);
+    auto ask = [&](int p0, int u) { part[u] = *reinterpret_cast<const f32x4*>(parts + min(p0 + u, n_partials - 1) * partial_stride + in_at); };
+    bf16x4 narrow = {};
+    if (y && y_code == MLLM_F32) {
+        ask(0, 0);
+        if (n_partials > 1) {   // (the same for the whole launch, as the next)
+#pragma unroll
+            for (int u = 1; u < 4; u++) ask(0, u);
+        }
+        if (n_partials > 4) {
+#pragma unroll
+            for (int u = 4; u < AHEAD; u++) ask(0, u);
+        }
+    } else if (y) {
+        narrow = *reinterpret_cast<const bf16x4*>(reinterpret_cast<const bf16_t*>(y) + in_at);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    f32x4 added = {0.0f, 0.0f, 0.0f, 0.0f};
+    if (y && y_code == MLLM_F32) {
+        added = part[0];
+        for (int p0 = 0; p0 < n_partials; p0 += AHEAD) {
+            if (p0 > 0)
+#pragma unroll
+                for (int u = 0; u < AHEAD; u++) ask(p0, u);
+#pragma unroll
+            for (int u = 0; u < AHEAD; u++)
+                if (p0 + u > 0 && p0 + u < n_partials) added += part[u];
+        }
+    } else if (y) {
+#pragma unroll
+        for (int e = 0; e < 4; e++) added[e] = static_cast<float>(narrow[e]);
+    }
+    auto mean_square = [&](f32x4 v, int which) {   // over the row; two barriers a row at most, each with shares of its own
+        const float mine = wave_total(owns ? (v[0] * v[0] + v[1] * v[1]) + (v[2] * v[2] + v[3] * v[3]) : 0.0f);
+        if (threadIdx.x % WAVE == 0) shares[which][threadIdx.x / WAVE] = mine;
+        __syncthreads();
+        float total = 0.0f;
+#pragma unroll
+        for (int w = 0; w < WAVES; w++) total += shares[which][w];
+        return total / (float)width;
+    };
+    const f32x4 h = own * alpha + added;
+    f32x4 value = h * (1.0f / sqrtf(mean_square(h, 0) + eps)) * (gain + plus);
+    if (residual) value = base + value;
+    f32x4 result = value;
+    if (next_weight) result = value * (1.0f / sqrtf(mean_square(value, 1) + eps)) * (next_gain + plus);   // (the same for the whole launch)
+    if (!owns) return;
+    if (stream) *reinterpret_cast<f32x4*>(stream + out_at) = value;
+    if (!rows) return;
+    if (rows_code == MLLM_F32) {
+        *reinterpret_cast<f32x4*>(reinterpret_cast<float*>(rows) + out_at) = result;
+    } else {
+        bf16x4 rounded;
+#pragma unroll
+        for (int e = 0; e < 4; e++) rounded[e] = static_cast<bf16_t>(result[e]);
+        *reinterpret_cast<bf16x4*>(reinterpret_cast<bf16_t*>(rows) + out_at) = rounded;
+    }
+}
+
 // The heads of a fused q/k/v product, a wave per (row, head): query heads are RMS-normed over their `dim` elements with one
 // gain vector, multiplied by the row's temperature 1 + coef * ln(floor((p + 1) / every) + 1) and stored as q [rows,
 // n_heads * head_size]; key heads are normed with their gain vector and stored in the key pages; value heads go to the
@@ -354,6 +437,15 @@ MLLM_API int mllm_rms_norm(const float* x, const void* y, int y_dtype, float alp
     if (n_rows == 0) return 0;
     const int waves = 4, blocks = ceil_div(n_rows, waves);
     mllm_count_kernel(MLLM_K_RMS_NORM);
+    const size_t wide = (size_t)x | (size_t)weight | (size_t)residual | (size_t)next_weight | (size_t)stream_out | (y_dtype == MLLM_F32 ? (size_t)y : 0) |
+                        (rows_dtype == MLLM_F32 ? (size_t)rows_out : 0) | (size_t)(partial_stride * (n_partials > 1 ? 4 : 0));
+    if ((width >= 512 || n_rows <= 256) && n_rows <= 16384 && width % 4 == 0 && width <= 2048 && wide % 16 == 0 && (((size_t)y | (size_t)rows_out) & 7) == 0) {
+#define LAUNCH(THREADS) rms_norm_row_kernel<THREADS><<<n_rows, THREADS, 0, stream>>>(x, y, y_dtype, alpha, row_index, weight, one_plus, eps, stream_out, rows_out, rows_dtype, width, n_partials, partial_stride, residual, next_weight)
+        if (width <= 1024) LAUNCH(256);
+        else LAUNCH(512);
+#undef LAUNCH
+        return mllm_check_launch("rms_norm");
+    }
 #define LAUNCH(REGS) rms_norm_kernel<REGS><<<blocks, 64 * waves, 0, stream>>>(x, y, y_dtype, alpha, row_index, weight, one_plus, eps, stream_out, rows_out, rows_dtype, n_rows, width, n_partials, partial_stride, residual, next_weight)
     if (width <= 256) LAUNCH(4);
     else if (width <= 512) LAUNCH(8);

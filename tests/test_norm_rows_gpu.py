@@ -1,0 +1,34 @@
+"""RMS norm with a block a row: widths at the edges of its threads, partial products beyond those asked for at once, every option."""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("rows,width", [(1, 4), (3, 60), (257, 512), (5, 1024), (300, 1028), (2, 2048), (9, 2052), (7, 770)])
+@pytest.mark.parametrize("partials", [0, 1, 2, 4, 5, 9])
+@pytest.mark.parametrize("out_dtype", [torch.float32, torch.bfloat16])
+def test_norm_of_a_row_by_a_block(rows, width, partials, out_dtype):
+    from mini_llm_amd.ops import kernels as K
+
+    generator = torch.Generator(device="cuda").manual_seed(rows * width + partials)
+    draw = lambda *shape: torch.randn(*shape, generator=generator, device="cuda")
+    x, weight, residual, following = draw(rows, width), draw(width), draw(rows, width), draw(width)
+    addend = draw(partials, rows, width) if partials else None
+    if partials == 1:
+        addend = addend[0].to(out_dtype)
+    eps, alpha = 1e-5, 0.7
+    h = x.double() * alpha + (0 if addend is None else addend.double().reshape(-1, rows, width).sum(0))
+    norm = lambda v, g: v / (v.pow(2).mean(1, keepdim=True) + eps).sqrt() * (1.0 + g.double())
+    want = residual.double() + norm(h, weight)
+    # 32-bit sums of up to 11 addends and of 2,052 squares, a square root and a division: some 2^-23 times twenty of numbers around 10
+    close = lambda got, ref: (got.double() - ref).abs().max() <= 2e-5 + (ref.abs().max() * 2.0 ** -8 if got.dtype == torch.bfloat16 else 0)
+    assert close(K.rms_norm(x, weight, eps, addend=addend, alpha=alpha, one_plus=True, residual=residual), want)
+    stream, normed = K.rms_norm(x, weight, eps, addend=addend, alpha=alpha, one_plus=True, residual=residual, with_stream=True, out_dtype=out_dtype)
+    assert close(stream, want) and close(normed, want)
+    if width <= 2048:
+        stream, twice = K.rms_norm(x, weight, eps, addend=addend, alpha=alpha, one_plus=True, residual=residual, with_stream=True, out_dtype=out_dtype, next_weight=following)
+        assert close(stream, want) and close(twice, norm(want, following))
+    index = torch.randint(rows, (rows + 2,), generator=generator, device="cuda").int()
+    assert close(K.rms_norm(x, weight, eps, one_plus=True, row_index=index, out_dtype=out_dtype), norm(x.double(), weight)[index.long()])
