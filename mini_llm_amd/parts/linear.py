@@ -60,20 +60,28 @@ class BranchProduct:
     or, where few rows meet few output columns and a long K (the library says: ``kernels.split_blocks``), cut along K into
     partial products [n, rows, out] that the norm adds up on its way in. With a residual the sum is taken inside the product, and
     so is a bias's.
-    Up to FEW_ROWS rows the product stays whole: measured on MI355X at width 768, a decode step of 64 rows gains 5 % from the
-    cut (0.990 -> 0.939 ms), one of 8 rows or of a single row loses 3 % (the norm's extra trips to memory cost more than the
-    product saves)."""
+    Up to FEW_ROWS rows only a long K is cut (``cut_few_rows``): a short one loses more to the norm's further loads than the product saves. With the norm
+    behind it, whole / cut, us: 8 rows in 32-bit 768 x 768 7.3 / 6.8, 1,600 x 1,024 8.0 / 8.1, 768 x 2,048 10.0 / 8.1, 1,600 x 2,048 10.7 / 9.2; in bfloat16
+    768 x 768 5.5 / 5.9, 768 x 2,048 7.1 / 6.5, 1,600 x 2,048 7.3 / 7.5, 1,600 x 3,072 8.1 / 7.7; a single row 0.2 to 0.5 less of a gain."""
 
     FEW_ROWS = 16
 
     def __init__(self):
         self._split_blocks = {}
 
+    @staticmethod
+    def cut_few_rows(weight, dtype) -> bool:
+        import torch
+
+        n, k = (weight.rows, weight.cols) if isinstance(weight, kernels.PackedMatrix) else weight.shape
+        return k >= 1536 if dtype == torch.float32 else k >= (2048 if n <= 1024 else 3072)
+
     def blocks(self, x, weight) -> int:
-        """Into how many partial products the product of these rows is cut (1: it stays whole)."""
+        """Into how many partial products the product of these rows is cut (1: it stays whole, as all of up to FEW_ROWS rows do)."""
+        return 1 if x.shape[0] <= self.FEW_ROWS else self._blocks(x, weight)
+
+    def _blocks(self, x, weight) -> int:
         rows = x.shape[0]
-        if rows <= self.FEW_ROWS:
-            return 1
         bucket = 0 if rows <= 64 else -(-rows // 128)   # the answer is the same inside a bucket
         k_blocks = self._split_blocks.get((bucket, x.dtype))
         if k_blocks is None:
@@ -83,8 +91,8 @@ class BranchProduct:
     def __call__(self, x, weight, residual=None, bias=None):
         import torch
 
-        if residual is None and bias is None:
-            k_blocks = self.blocks(x, weight)
+        if residual is None and bias is None and (x.shape[0] > self.FEW_ROWS or self.cut_few_rows(weight, x.dtype)):
+            k_blocks = self._blocks(x, weight)
             if k_blocks > 1:
                 return kernels.linear_split(x, weight, k_blocks)
         return kernels.linear(x, weight, bias, residual=residual, out_dtype=torch.float32)
