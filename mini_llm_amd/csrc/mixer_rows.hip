@@ -25,8 +25,13 @@ __device__ __forceinline__ float sigmoid_f(float z) { return 1.0f / (1.0f + expf
 // [rows, n_heads * head_size]; keys to the key pages; values [n_kv_heads * vdim], blended with another layer's values of
 // the same row where v_other is given (v <- (1 - mix) v + mix v_other, mix read from the device), to the value pages. The
 // pages' heads hold head_size >= dim, vdim elements, zeros beyond a head's own. A negative slot stores nothing.
+// A thread takes pairs of the queries and, behind them, of the keys; its first one stays in registers from the norm's sums to the rotation, whose angle (64-bit)
+// and sine and cosine are worked out while the row's other numbers are on their way. Few rows get as many threads as a row has pairs: the kernel is then one
+// trip to memory and one pair. Eight rows of twelve heads of 64 and three key heads, in 32-bit, inside a decode step: 8.0 -> 5.3 us.
+constexpr int PROJECTION_WIDE_ROWS = 256;   // up to as many rows as there are compute units
+
 template <typename T>
-__global__ __launch_bounds__(256) void projection_rows_kernel(const float* __restrict__ q, int q_stride, const float* __restrict__ k, int k_stride,
+__global__ __launch_bounds__(1024) void projection_rows_kernel(const float* __restrict__ q, int q_stride, const float* __restrict__ k, int k_stride,
                                                               const float* __restrict__ v, int v_stride, const float* __restrict__ v_other,
                                                               int v_other_stride, const float* __restrict__ mix, const float* __restrict__ q_gain,
                                                               const float* __restrict__ k_gain, float eps, const double* __restrict__ frequencies,
@@ -42,11 +47,44 @@ __global__ __launch_bounds__(256) void projection_rows_kernel(const float* __res
     const int position_of_row = positions[row];
     const int slot = write_cache ? slots[row] : -1;
     const float blend = v_other ? mix[0] : 0.0f;
+    const int half_head = head_size / 2, q_items = n_heads * half_head, items = q_items + n_kv_heads * half_head;   // (heads in pages are multiples of 16 wide)
+    const double position = (double)position_of_row;
+    // a pair of neighbouring elements of a head: d its first element's place in the head (even); elements beyond the head's own are zero
+    struct Pair {
+        int head, d;
+        bool is_q;
+        float first, second, sine, cosine;
+    };
+    auto load_pair = [&](int i) {
+        Pair pair;
+        pair.is_q = i < q_items;
+        const int within = pair.is_q ? i : i - q_items;
+        pair.head = within / half_head, pair.d = 2 * (within % half_head);
+        const float* in = (pair.is_q ? q_row : k_row) + pair.head * dim + pair.d;
+        pair.first = pair.d < dim ? in[0] : 0.0f;
+        pair.second = pair.d + 1 < dim ? in[1] : 0.0f;
+        return pair;
+    };
+    auto find_angle = [&](Pair& pair) {
+        if (pair.d >= rot_dims) return;
+        // the angle in 64-bit (a 32-bit product of a position in the thousands is good to 1e-4 only), brought into -pi .. pi,
+        // where its sine and cosine are taken in 32-bit
+        const double angle = position * frequencies[pair.d >> 1];
+        const double turns = rint(angle * 0.15915494309189535);
+        sincosf((float)(angle - turns * 6.283185307179586), &pair.sine, &pair.cosine);
+    };
     float q_squares = 0.0f, k_squares = 0.0f;
-    if (q_gain)
-        for (int i = threadIdx.x; i < q_width; i += blockDim.x) q_squares += q_row[i] * q_row[i];
-    if (k_gain)
-        for (int i = threadIdx.x; i < k_width; i += blockDim.x) k_squares += k_row[i] * k_row[i];
+    Pair first_pair = {};
+    if ((int)threadIdx.x < items) {
+        first_pair = load_pair(threadIdx.x);
+        find_angle(first_pair);
+    }
+    for (int i = threadIdx.x; i < items; i += blockDim.x) {
+        const Pair pair = i == (int)threadIdx.x ? first_pair : load_pair(i);
+        const float squares = pair.first * pair.first + pair.second * pair.second;
+        if (pair.is_q) q_squares += squares;
+        else k_squares += squares;
+    }
     q_squares = wave_sum(q_squares);
     k_squares = wave_sum(k_squares);
     if (threadIdx.x % WAVE == 0) {
@@ -61,48 +99,39 @@ __global__ __launch_bounds__(256) void projection_rows_kernel(const float* __res
     }
     const float q_factor = q_gain ? 1.0f / sqrtf(q_squares / (float)q_width + eps) : 1.0f;
     const float k_factor = k_gain ? 1.0f / sqrtf(k_squares / (float)k_width + eps) : 1.0f;
-    const double position = (double)position_of_row;
-    // a pair of neighbouring elements of a normed head, rotated where it lies among the first rot_dims: d its first element's place
-    // in the head (even), `at` the head's first element in the row; elements beyond the head's own are zero
-    auto turned_pair = [&](const float* in, const float* gain, float factor, int at, int d, float& first, float& second) {
-        first = d < dim ? in[at + d] * factor * (gain ? gain[at + d] : 1.0f) : 0.0f;
-        second = d + 1 < dim ? in[at + d + 1] * factor * (gain ? gain[at + d + 1] : 1.0f) : 0.0f;
-        if (d < rot_dims) {
-            // the angle in 64-bit (a 32-bit product of a position in the thousands is good to 1e-4 only), brought into -pi .. pi,
-            // where its sine and cosine are taken in 32-bit
-            const double angle = position * frequencies[d >> 1];
-            const double turns = rint(angle * 0.15915494309189535);
-            float s, c;
-            sincosf((float)(angle - turns * 6.283185307179586), &s, &c);
-            const float u = first, w = second;
-            first = u * c - w * s;
-            second = w * c + u * s;
-        }
-    };
-    const int half_head = head_size / 2;   // (heads in pages are multiples of 16 wide)
-    for (int i = threadIdx.x; i < n_heads * half_head; i += blockDim.x) {
-        const int head = i / half_head, d = 2 * (i % half_head);
-        float first, second;
-        turned_pair(q_row, q_gain, q_factor, head * dim, d, first, second);
-        T* to = q_out + (size_t)row * n_heads * head_size + (size_t)head * head_size + d;
-        to[0] = from_float<T>(first);
-        to[1] = from_float<T>(second);
-    }
-    if (slot < 0) return;   // no cache write, or a padding row
     const int page = slot / page_size, offset = slot % page_size;
-    for (int i = threadIdx.x; i < n_kv_heads * half_head; i += blockDim.x) {
-        const int head = i / half_head, d = 2 * (i % half_head);
-        const size_t at = (((size_t)page * n_kv_heads + head) * page_size + offset) * head_size + d;
-        float first, second;
-        turned_pair(k_row, k_gain, k_factor, head * dim, d, first, second);
+    for (int i = threadIdx.x; i < items; i += blockDim.x) {
+        Pair pair = first_pair;
+        if (i != (int)threadIdx.x) {
+            pair = load_pair(i);
+            find_angle(pair);
+        }
+        if (!pair.is_q && slot < 0) break;   // no cache write, or a padding row; the queries lie in front
+        const float* gain = pair.is_q ? q_gain : k_gain;
+        const float factor = pair.is_q ? q_factor : k_factor;
+        const int at_gain = pair.head * dim + pair.d;
+        float first = pair.d < dim ? pair.first * factor * (gain ? gain[at_gain] : 1.0f) : 0.0f;
+        float second = pair.d + 1 < dim ? pair.second * factor * (gain ? gain[at_gain + 1] : 1.0f) : 0.0f;
+        if (pair.d < rot_dims) {
+            const float u = first, w = second;
+            first = u * pair.cosine - w * pair.sine;
+            second = w * pair.cosine + u * pair.sine;
+        }
+        if (pair.is_q) {
+            T* to = q_out + (size_t)row * n_heads * head_size + (size_t)pair.head * head_size + pair.d;
+            to[0] = from_float<T>(first);
+            to[1] = from_float<T>(second);
+            continue;
+        }
+        const size_t at = (((size_t)page * n_kv_heads + pair.head) * page_size + offset) * head_size + pair.d;
         k_pages[at] = from_float<T>(first);
         k_pages[at + 1] = from_float<T>(second);
 #pragma unroll
         for (int e = 0; e < 2; e++) {
             float value = 0.0f;
-            if (d + e < vdim) {
-                value = v[(size_t)row * v_stride + head * vdim + d + e];
-                if (v_other) value = (1.0f - blend) * value + blend * v_other[(size_t)row * v_other_stride + head * vdim + d + e];
+            if (pair.d + e < vdim) {
+                value = v[(size_t)row * v_stride + pair.head * vdim + pair.d + e];
+                if (v_other) value = (1.0f - blend) * value + blend * v_other[(size_t)row * v_other_stride + pair.head * vdim + pair.d + e];
             }
             v_pages[at + e] = from_float<T>(value);
         }
@@ -281,8 +310,9 @@ MLLM_API int mllm_projection_rows(const float* q, int q_stride, const float* k, 
     mllm_count_kernel(MLLM_K_PROJECTION_ROWS);
 #define PROJECTION_ARGS(T) q, q_stride, k, k_stride, v, v_stride, v_other, v_other_stride, mix, q_gain, k_gain, eps, frequencies, rot_dims, positions, slots, \
                            (T*)q_out, (T*)k_pages, (T*)v_pages, n_heads, n_kv_heads, dim, vdim, head_size, page_size, write_cache
-    if (dtype == MLLM_F32) projection_rows_kernel<float><<<n_rows, 256, 0, stream>>>(PROJECTION_ARGS(float));
-    else if (dtype == MLLM_BF16) projection_rows_kernel<bf16_t><<<n_rows, 256, 0, stream>>>(PROJECTION_ARGS(bf16_t));
+    const int pairs = (n_heads + n_kv_heads) * (head_size / 2), threads = n_rows > PROJECTION_WIDE_ROWS || pairs <= 256 ? 256 : (pairs <= 512 ? 512 : 1024);
+    if (dtype == MLLM_F32) projection_rows_kernel<float><<<n_rows, threads, 0, stream>>>(PROJECTION_ARGS(float));
+    else if (dtype == MLLM_BF16) projection_rows_kernel<bf16_t><<<n_rows, threads, 0, stream>>>(PROJECTION_ARGS(bf16_t));
     else MLLM_REQUIRE(false, "projection_rows: unknown dtype %d", dtype);
 #undef PROJECTION_ARGS
     return mllm_check_launch("projection_rows");
