@@ -418,7 +418,11 @@ def _compute_units(device) -> int:
 DECODE_MAX_Q_LEN = 8        # portions up to this many tokens take the split-key kernel
 DECODE_TARGET_WAVES = 4096  # the most waves a launch should have: 16 to each of 256 compute units are resident at once (measured: a
                             # second round of blocks costs more than longer shares of the keys per wave)
-DECODE_MIN_SPLIT = 64       # keys a wave should at least have
+# What a wave should at least have: 64 keys, and two rounds of its sweep over the cache (16 KiB of keys). Four / eight / sixteen waves a block, us, bfloat16, heads
+# of 64, 12 of them: 8 rows of 200 keys 6.0 / 5.8 / 7.1, of 900 11.6 / 9.2 / 10.1, of 1,500 15.3 / 12.3 / 13.2, of 4,000 39.2 / 30.7 / 30.1; 16 rows of 545 10.7 / 9.7 /
+# 10.5; in 32-bit, 8 rows of 545 13.0 / 11.8 / 11.9, of 900 16.7 (eight) / 15.6 (sixteen).
+DECODE_MIN_SPLIT = 64
+DECODE_MIN_SPLIT_BYTES = 16384
 DECODE_MAX_SPLITS = 16      # waves per block
 DECODE_MAX_PARTS = 64       # runs a token's keys are cut into at most, a block each, where (token, head) pairs are few
 # What such a run should at least hold. Measured on MI355X with heads of 64: up to some 32 pairs (a single token) runs
@@ -521,7 +525,7 @@ def paged_attention(q, k_pages, v_pages, token_request, positions, block_tables,
             and lib.mllm_attention_decode_supported(head_size, page_size, _code(q.dtype))):
         # decoding and short portions: a block per (token, head) whose waves share the keys; as many
         # waves per block as keep the launch within what is resident at once, never more than one
-        # per 64 keys of reach
+        # per DECODE_MIN_SPLIT keys of reach
         reach = block_tables.shape[1] * page_size if max_len is None else max(1, min(max_len, block_tables.shape[1] * page_size))
         if window or chunk:
             reach = min(reach, int(window or chunk) + keep_first)
@@ -532,8 +536,8 @@ def paged_attention(q, k_pages, v_pages, token_request, positions, block_tables,
         while n_parts < DECODE_MAX_PARTS and 2 * n * n_heads * n_parts <= units and 2 * n_parts * min_part <= reach:
             n_parts *= 2
         part_reach = -(-reach // n_parts)
-        n_splits = 1
-        while n_splits < DECODE_MAX_SPLITS and 2 * n * n_heads * n_parts * n_splits <= DECODE_TARGET_WAVES and n_splits * DECODE_MIN_SPLIT < part_reach:
+        n_splits, min_split = 1, max(DECODE_MIN_SPLIT, DECODE_MIN_SPLIT_BYTES // (head_size * q.element_size()))
+        while n_splits < DECODE_MAX_SPLITS and 2 * n * n_heads * n_parts * n_splits <= DECODE_TARGET_WAVES and n_splits * min_split < part_reach:
             n_splits *= 2
         result = out
         if packed_out:
