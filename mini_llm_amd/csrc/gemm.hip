@@ -699,8 +699,8 @@ int skinny_k_blocks(int N, int K) {
     return best;
 }
 
-// The same for more rows (the tiled kernel, 128 x 64 tiles): only a product whose tiles leave half
-// the compute units idle is cut, while the tiles of the cut product are no more than one and a
+// The same for more rows: in 32-bit and in bfloat16 with K in whole tiles by the costs below; else (the tiled kernel, 128 x 64
+// tiles) only a product whose tiles leave half the compute units idle is cut, while the tiles of the cut product are no more than one and a
 // half to a compute unit and every block keeps eight LDS tiles of K (measured: a product that
 // nearly fills the chip gains less from the cut than adding the partial products up costs). Up to
 // 256 rows a block may go down to four LDS tiles: the partial products are small then, and a
