@@ -32,3 +32,22 @@ def test_norm_of_a_row_by_a_block(rows, width, partials, out_dtype):
         assert close(stream, want) and close(twice, norm(want, following))
     index = torch.randint(rows, (rows + 2,), generator=generator, device="cuda").int()
     assert close(K.rms_norm(x, weight, eps, one_plus=True, row_index=index, out_dtype=out_dtype), norm(x.double(), weight)[index.long()])
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("rows,n,k,cut", [(1, 768, 1535, (False, False)), (8, 768, 1536, (True, False)), (16, 1024, 2048, (True, True)), (3, 1040, 2048, (True, False)), (5, 1040, 3072, (True, True))])
+def test_branch_products_of_few_rows_are_cut_from_a_long_k_on(dtype, rows, n, k, cut):
+    from mini_llm_amd.ops import kernels as K
+    from mini_llm_amd.parts.linear import BranchProduct
+
+    generator = torch.Generator(device="cuda").manual_seed(rows + k)
+    k = k // 8 * 8   # (whole 16-byte pieces)
+    x, w = torch.randn(rows, k, generator=generator, device="cuda").to(dtype), (torch.randn(n, k, generator=generator, device="cuda") / k ** 0.5).to(dtype)
+    weight, residual = torch.randn(n, generator=generator, device="cuda"), torch.randn(rows, n, generator=generator, device="cuda")
+    branch = BranchProduct()(x, K.pack_matrix(w))
+    assert (branch.dim() == 3) == cut[dtype == torch.bfloat16]
+    h = x.double() @ w.double().T
+    want = residual.double() + h / (h.pow(2).mean(1, keepdim=True) + 1e-5).sqrt() * weight.double()
+    first, rest = (branch[0], branch[1:]) if branch.dim() == 3 else (branch, None)
+    # sums of k products of numbers around 1 / sqrt(k), each rounding 2^-24 of a partial sum of at most some 5, sixteen terms at a time
+    assert (K.rms_norm(first, weight, 1e-5, addend=rest, residual=residual).double() - want).abs().max() <= 5 * 4 * 2.0 ** -24 * (k / 16) ** 0.5 * 4
