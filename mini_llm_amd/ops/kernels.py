@@ -418,12 +418,16 @@ def _compute_units(device) -> int:
 DECODE_MAX_Q_LEN = 8        # portions up to this many tokens take the split-key kernel
 DECODE_TARGET_WAVES = 4096  # the most waves a launch should have: 16 to each of 256 compute units are resident at once (measured: a
                             # second round of blocks costs more than longer shares of the keys per wave)
-# What a wave should at least have: 64 keys, and two rounds of its sweep over the cache (16 KiB of keys). Four / eight / sixteen waves a block, us, bfloat16, heads
-# of 64, 12 of them: 8 rows of 200 keys 6.0 / 5.8 / 7.1, of 900 11.6 / 9.2 / 10.1, of 1,500 15.3 / 12.3 / 13.2, of 4,000 39.2 / 30.7 / 30.1; 16 rows of 545 10.7 / 9.7 /
-# 10.5; in 32-bit, 8 rows of 545 13.0 / 11.8 / 11.9, of 900 16.7 (eight) / 15.6 (sixteen).
+# What a wave should at least have, and what a run of a token's keys (all its keys, where they are not cut) should hold of a head before its block gets sixteen
+# waves instead of eight: sixteen cost 1.2 us more to start and merge. Runs of exactly these keys, bfloat16, heads of 64, 12 of them, us with 1 / 2 / 4 / 8 / 16 waves:
+# 8 rows of 64 keys 4.1 / 4.3 / 4.9 / 4.9 / 6.2, of 128 5.3 / 4.6 / 5.1 / 5.1 / 6.3, of 200 8.6 / 6.6 / 6.0 / 6.0 / 7.1, of 300 10.2 / 8.1 / 7.4 / 6.8 / 7.9, of 500
+# 14.3 / 9.9 / 8.1 / 7.2 / 8.4, of 900 23.1 / 15.6 / 11.4 / 9.1 / 10.1, of 1,500 41.5 / 26.1 / 18.3 / 14.3 / 15.2, of 3,000 78.5 / 49.8 / 32.3 / 25.1 / 24.8; one
+# row of 128 5.1 / 4.4 / 4.8 / 4.9 / 6.0, of 500 11.9 / 8.1 / 6.6 / 5.9 / 7.0; in 32-bit 8 rows of 900 44.8 / 27.4 / 23.7 / 19.6 / 18.0. (A captured step's run is
+# as long as the cache may become, and its waves the same however few keys there are yet.)
 DECODE_MIN_SPLIT = 64
-DECODE_MIN_SPLIT_BYTES = 16384
+DECODE_WIDE_BYTES = 192 * 1024
 DECODE_MAX_SPLITS = 16      # waves per block
+DECODE_COMMON_SPLITS = 8    # and of a run that holds less than DECODE_WIDE_BYTES
 DECODE_MAX_PARTS = 64       # runs a token's keys are cut into at most, a block each, where (token, head) pairs are few
 # What such a run should at least hold. Measured on MI355X with heads of 64: up to some 32 pairs (a single token) runs
 # of 512 keys pay (12 pairs, 3,000 keys: 15.3 -> 12.4 us in bfloat16, 23.2 -> 15.1 in 32-bit; 32 pairs with heads of
@@ -452,6 +456,15 @@ def _arrivals(k_pages, rows: int, n_heads: int):
             _outgrown_counters.append(counters)
         counters = _arrival_counters[key] = torch.zeros(max(rows * n_heads, 1024), dtype=torch.int32, device=k_pages.device)
     return counters
+
+
+def decode_waves(blocks: int, keys: int, key_bytes: int) -> int:
+    """Waves a block of the decode attention for so many blocks, each with up to ``keys`` keys of ``key_bytes`` bytes."""
+    most = DECODE_MAX_SPLITS if keys * key_bytes >= DECODE_WIDE_BYTES else DECODE_COMMON_SPLITS
+    waves = 1
+    while waves < most and 2 * blocks * waves <= DECODE_TARGET_WAVES and waves * DECODE_MIN_SPLIT < keys:
+        waves *= 2
+    return waves
 
 
 def paged_attention(q, k_pages, v_pages, token_request, positions, block_tables, n_heads, n_kv_heads, head_size, scale, window=0, max_q_len=None, max_len=None, q_starts=None, context_lens=None, out=None,
@@ -536,9 +549,7 @@ def paged_attention(q, k_pages, v_pages, token_request, positions, block_tables,
         while n_parts < DECODE_MAX_PARTS and 2 * n * n_heads * n_parts <= units and 2 * n_parts * min_part <= reach:
             n_parts *= 2
         part_reach = -(-reach // n_parts)
-        n_splits, min_split = 1, max(DECODE_MIN_SPLIT, DECODE_MIN_SPLIT_BYTES // (head_size * q.element_size()))
-        while n_splits < DECODE_MAX_SPLITS and 2 * n * n_heads * n_parts * n_splits <= DECODE_TARGET_WAVES and n_splits * min_split < part_reach:
-            n_splits *= 2
+        n_splits = decode_waves(n * n_heads * n_parts, part_reach, head_size * q.element_size())
         result = out
         if packed_out:
             result = empty_packed_rows(n, width, q.dtype, q.device)
