@@ -3,6 +3,8 @@
 // leaves. Everything is computed in 32-bit; the rows these kernels read (the sums of a fused product) are 32-bit too.
 #include "common.h"
 
+#include <algorithm>
+
 namespace {
 
 __device__ __forceinline__ float block_sum(float v, float* scratch) {
@@ -25,13 +27,17 @@ __device__ __forceinline__ float sigmoid_f(float z) { return 1.0f / (1.0f + expf
 // [rows, n_heads * head_size]; keys to the key pages; values [n_kv_heads * vdim], blended with another layer's values of
 // the same row where v_other is given (v <- (1 - mix) v + mix v_other, mix read from the device), to the value pages. The
 // pages' heads hold head_size >= dim, vdim elements, zeros beyond a head's own. A negative slot stores nothing.
-// A thread takes pairs of the queries and, behind them, of the keys; its first one stays in registers from the norm's sums to the rotation, whose angle (64-bit)
-// and sine and cosine are worked out while the row's other numbers are on their way. Few rows get as many threads as a row has pairs: the kernel is then one
-// trip to memory and one pair. Eight rows of twelve heads of 64 and three key heads, in 32-bit, inside a decode step: 8.0 -> 5.3 us.
-constexpr int PROJECTION_WIDE_ROWS = 256;   // up to as many rows as there are compute units
+// FEW rows: a thread takes pairs of the queries and, behind them, of the keys; its first one stays in registers from the norm's sums to the rotation, whose angle
+// (64-bit) and sine and cosine are worked out while the row's other numbers are on their way. With as many threads as a row has pairs the kernel is one trip to
+// memory and one pair: eight rows of twelve heads of 64 and three key heads, in 32-bit, alone in a loop 5.4 -> 4.2 us. Rows enough to fill the compute units take
+// what asks for the least instead: single numbers for the sums, the queries' pairs and the keys' in loops of their own, 256 threads. In 32-bit, us, 256 threads that
+// hold a first pair / so: 2,048 rows of those heads 11.7 / 10.6, 512 rows of 32 heads of 128 and 8 key heads 17.2 / 12.7, without norms 15.1 / 9.1. Rows of up to
+// 256 pairs, which leave a thread none to load again, hold theirs to four times as many rows: 512 rows of six heads of 64 and two key heads 4.5, in loops 5.2; from
+// 2,048 rows on either is as good (8.1 and 8.3), and without keys to store the loops are the better (7.2 and 6.7).
+constexpr int PROJECTION_FEW_ROWS = 256;   // as many as there are compute units
 
-template <typename T>
-__global__ __launch_bounds__(1024) void projection_rows_kernel(const float* __restrict__ q, int q_stride, const float* __restrict__ k, int k_stride,
+template <typename T, bool FEW>
+__global__ __launch_bounds__(FEW ? 1024 : 256) void projection_rows_kernel(const float* __restrict__ q, int q_stride, const float* __restrict__ k, int k_stride,
                                                               const float* __restrict__ v, int v_stride, const float* __restrict__ v_other,
                                                               int v_other_stride, const float* __restrict__ mix, const float* __restrict__ q_gain,
                                                               const float* __restrict__ k_gain, float eps, const double* __restrict__ frequencies,
@@ -47,24 +53,25 @@ __global__ __launch_bounds__(1024) void projection_rows_kernel(const float* __re
     const int position_of_row = positions[row];
     const int slot = write_cache ? slots[row] : -1;
     const float blend = v_other ? mix[0] : 0.0f;
-    const int half_head = head_size / 2, q_items = n_heads * half_head, items = q_items + n_kv_heads * half_head;   // (heads in pages are multiples of 16 wide)
+    const int half_head = head_size / 2, q_items = n_heads * half_head, k_items = n_kv_heads * half_head;   // (heads in pages are multiples of 16 wide)
+    const int items = q_items + (write_cache ? k_items : 0);
     const double position = (double)position_of_row;
     // a pair of neighbouring elements of a head: d its first element's place in the head (even); elements beyond the head's own are zero
     struct Pair {
         int head, d;
-        bool is_q;
-        float first, second, sine, cosine;
+        float first, second, first_gain, second_gain, sine, cosine;
     };
-    auto load_pair = [&](int i) {
+    auto load_pair = [&](const float* in, const float* gain, int i) {
         Pair pair;
-        pair.is_q = i < q_items;
-        const int within = pair.is_q ? i : i - q_items;
-        pair.head = within / half_head, pair.d = 2 * (within % half_head);
-        const float* in = (pair.is_q ? q_row : k_row) + pair.head * dim + pair.d;
-        pair.first = pair.d < dim ? in[0] : 0.0f;
-        pair.second = pair.d + 1 < dim ? in[1] : 0.0f;
+        pair.head = i / half_head, pair.d = 2 * (i % half_head);
+        const int at = pair.head * dim + pair.d;
+        pair.first = pair.d < dim ? in[at] : 0.0f;
+        pair.second = pair.d + 1 < dim ? in[at + 1] : 0.0f;
+        pair.first_gain = gain && pair.d < dim ? gain[at] : 1.0f;
+        pair.second_gain = gain && pair.d + 1 < dim ? gain[at + 1] : 1.0f;
         return pair;
     };
+    auto load_item = [&](int i) { return i < q_items ? load_pair(q_row, q_gain, i) : load_pair(k_row, k_gain, i - q_items); };
     auto find_angle = [&](Pair& pair) {
         if (pair.d >= rot_dims) return;
         // the angle in 64-bit (a 32-bit product of a position in the thousands is good to 1e-4 only), brought into -pi .. pi,
@@ -73,59 +80,63 @@ __global__ __launch_bounds__(1024) void projection_rows_kernel(const float* __re
         const double turns = rint(angle * 0.15915494309189535);
         sincosf((float)(angle - turns * 6.283185307179586), &pair.sine, &pair.cosine);
     };
-    float q_squares = 0.0f, k_squares = 0.0f;
+    float q_factor = 1.0f, k_factor = 1.0f;
     Pair first_pair = {};
-    if ((int)threadIdx.x < items) {
-        first_pair = load_pair(threadIdx.x);
-        find_angle(first_pair);
+    if constexpr (FEW) {
+        if ((int)threadIdx.x < items) {
+            first_pair = load_item(threadIdx.x);
+            find_angle(first_pair);
+        }
     }
-    for (int i = threadIdx.x; i < items; i += blockDim.x) {
-        const Pair pair = i == (int)threadIdx.x ? first_pair : load_pair(i);
-        const float squares = pair.first * pair.first + pair.second * pair.second;
-        if (pair.is_q) q_squares += squares;
-        else k_squares += squares;
+    if (q_gain || k_gain) {   // (the same for the whole launch)
+        float q_squares = 0.0f, k_squares = 0.0f;
+        if constexpr (FEW) {
+            for (int i = threadIdx.x; i < items; i += blockDim.x) {
+                const Pair pair = i == (int)threadIdx.x ? first_pair : load_item(i);
+                (i < q_items ? q_squares : k_squares) += pair.first * pair.first + pair.second * pair.second;
+            }
+        } else {
+            if (q_gain)
+                for (int i = threadIdx.x; i < q_width; i += blockDim.x) q_squares += q_row[i] * q_row[i];
+            if (k_gain && write_cache)
+                for (int i = threadIdx.x; i < k_width; i += blockDim.x) k_squares += k_row[i] * k_row[i];
+        }
+        q_squares = wave_sum(q_squares);
+        k_squares = wave_sum(k_squares);
+        if (threadIdx.x % WAVE == 0) {
+            scratch[0][threadIdx.x / WAVE] = q_squares;
+            scratch[1][threadIdx.x / WAVE] = k_squares;
+        }
+        __syncthreads();
+        q_squares = k_squares = 0.0f;
+        for (int w = 0; w < (int)blockDim.x / WAVE; w++) {
+            q_squares += scratch[0][w];
+            k_squares += scratch[1][w];
+        }
+        if (q_gain) q_factor = 1.0f / sqrtf(q_squares / (float)q_width + eps);
+        if (k_gain) k_factor = 1.0f / sqrtf(k_squares / (float)k_width + eps);
     }
-    q_squares = wave_sum(q_squares);
-    k_squares = wave_sum(k_squares);
-    if (threadIdx.x % WAVE == 0) {
-        scratch[0][threadIdx.x / WAVE] = q_squares;
-        scratch[1][threadIdx.x / WAVE] = k_squares;
-    }
-    __syncthreads();
-    q_squares = k_squares = 0.0f;
-    for (int w = 0; w < (int)blockDim.x / WAVE; w++) {
-        q_squares += scratch[0][w];
-        k_squares += scratch[1][w];
-    }
-    const float q_factor = q_gain ? 1.0f / sqrtf(q_squares / (float)q_width + eps) : 1.0f;
-    const float k_factor = k_gain ? 1.0f / sqrtf(k_squares / (float)k_width + eps) : 1.0f;
     const int page = slot / page_size, offset = slot % page_size;
-    for (int i = threadIdx.x; i < items; i += blockDim.x) {
-        Pair pair = first_pair;
-        if (i != (int)threadIdx.x) {
-            pair = load_pair(i);
-            find_angle(pair);
-        }
-        if (!pair.is_q && slot < 0) break;   // no cache write, or a padding row; the queries lie in front
-        const float* gain = pair.is_q ? q_gain : k_gain;
-        const float factor = pair.is_q ? q_factor : k_factor;
-        const int at_gain = pair.head * dim + pair.d;
-        float first = pair.d < dim ? pair.first * factor * (gain ? gain[at_gain] : 1.0f) : 0.0f;
-        float second = pair.d + 1 < dim ? pair.second * factor * (gain ? gain[at_gain + 1] : 1.0f) : 0.0f;
+    auto turn = [&](Pair& pair, float factor) {   // normed and rotated; what lies beyond the head is zero whatever the factor
+        pair.first = pair.d < dim ? pair.first * factor * pair.first_gain : 0.0f;
+        pair.second = pair.d + 1 < dim ? pair.second * factor * pair.second_gain : 0.0f;
         if (pair.d < rot_dims) {
-            const float u = first, w = second;
-            first = u * pair.cosine - w * pair.sine;
-            second = w * pair.cosine + u * pair.sine;
+            const float u = pair.first, w = pair.second;
+            pair.first = u * pair.cosine - w * pair.sine;
+            pair.second = w * pair.cosine + u * pair.sine;
         }
-        if (pair.is_q) {
-            T* to = q_out + (size_t)row * n_heads * head_size + (size_t)pair.head * head_size + pair.d;
-            to[0] = from_float<T>(first);
-            to[1] = from_float<T>(second);
-            continue;
-        }
+    };
+    auto leave_query = [&](Pair& pair) {
+        turn(pair, q_factor);
+        T* to = q_out + (size_t)row * n_heads * head_size + (size_t)pair.head * head_size + pair.d;
+        to[0] = from_float<T>(pair.first);
+        to[1] = from_float<T>(pair.second);
+    };
+    auto leave_key = [&](Pair& pair) {   // and the value's elements of the same places
+        turn(pair, k_factor);
         const size_t at = (((size_t)page * n_kv_heads + pair.head) * page_size + offset) * head_size + pair.d;
-        k_pages[at] = from_float<T>(first);
-        k_pages[at + 1] = from_float<T>(second);
+        k_pages[at] = from_float<T>(pair.first);
+        k_pages[at + 1] = from_float<T>(pair.second);
 #pragma unroll
         for (int e = 0; e < 2; e++) {
             float value = 0.0f;
@@ -134,6 +145,30 @@ __global__ __launch_bounds__(1024) void projection_rows_kernel(const float* __re
                 if (v_other) value = (1.0f - blend) * value + blend * v_other[(size_t)row * v_other_stride + pair.head * vdim + pair.d + e];
             }
             v_pages[at + e] = from_float<T>(value);
+        }
+    };
+    if constexpr (FEW) {
+        for (int i = threadIdx.x; i < items; i += blockDim.x) {
+            Pair pair = first_pair;
+            if (i != (int)threadIdx.x) {
+                pair = load_item(i);
+                find_angle(pair);
+            }
+            if (i < q_items) leave_query(pair);
+            else if (slot < 0) break;   // a padding row
+            else leave_key(pair);
+        }
+    } else {
+        for (int i = threadIdx.x; i < q_items; i += blockDim.x) {
+            Pair pair = load_pair(q_row, q_gain, i);
+            find_angle(pair);
+            leave_query(pair);
+        }
+        if (slot < 0) return;   // no cache write, or a padding row
+        for (int i = threadIdx.x; i < k_items; i += blockDim.x) {
+            Pair pair = load_pair(k_row, k_gain, i);
+            find_angle(pair);
+            leave_key(pair);
         }
     }
 }
@@ -310,10 +345,16 @@ MLLM_API int mllm_projection_rows(const float* q, int q_stride, const float* k, 
     mllm_count_kernel(MLLM_K_PROJECTION_ROWS);
 #define PROJECTION_ARGS(T) q, q_stride, k, k_stride, v, v_stride, v_other, v_other_stride, mix, q_gain, k_gain, eps, frequencies, rot_dims, positions, slots, \
                            (T*)q_out, (T*)k_pages, (T*)v_pages, n_heads, n_kv_heads, dim, vdim, head_size, page_size, write_cache
-    const int pairs = (n_heads + n_kv_heads) * (head_size / 2), threads = n_rows > PROJECTION_WIDE_ROWS || pairs <= 256 ? 256 : (pairs <= 512 ? 512 : 1024);
-    if (dtype == MLLM_F32) projection_rows_kernel<float><<<n_rows, threads, 0, stream>>>(PROJECTION_ARGS(float));
-    else if (dtype == MLLM_BF16) projection_rows_kernel<bf16_t><<<n_rows, threads, 0, stream>>>(PROJECTION_ARGS(bf16_t));
+    const int pairs = (n_heads + (write_cache ? n_kv_heads : 0)) * (head_size / 2);
+    const bool few = n_rows <= (pairs <= 256 ? 4 * PROJECTION_FEW_ROWS : PROJECTION_FEW_ROWS);
+    const int threads = few ? std::min(1024, ceil_div(pairs, WAVE) * WAVE) : 256;
+#define LAUNCH(T)                                                                                         \
+    if (few) projection_rows_kernel<T, true><<<n_rows, threads, 0, stream>>>(PROJECTION_ARGS(T));         \
+    else projection_rows_kernel<T, false><<<n_rows, threads, 0, stream>>>(PROJECTION_ARGS(T));
+    if (dtype == MLLM_F32) { LAUNCH(float) }
+    else if (dtype == MLLM_BF16) { LAUNCH(bf16_t) }
     else MLLM_REQUIRE(false, "projection_rows: unknown dtype %d", dtype);
+#undef LAUNCH
 #undef PROJECTION_ARGS
     return mllm_check_launch("projection_rows");
 }

@@ -118,6 +118,45 @@ def test_projection_rows_norms_the_whole_projection_not_each_head():
     assert got[1, 0] < 0.02 < 1.0 < got[0, 0] and (got[:, 8:] == 0).all()
 
 
+# rows that hold a pair a thread (512 and 1,024 threads, with and without pairs that are loaded again) and rows taken in loops, on both sides of each border
+@pytest.mark.parametrize("rows,heads,kv_heads,dim,head_size", [(9, 12, 3, 64, 64), (3, 24, 8, 60, 64), (5, 32, 8, 64, 64), (256, 12, 3, 62, 64), (257, 12, 3, 64, 64), (260, 32, 8, 60, 64),
+                                                               (1024, 6, 2, 64, 64), (1025, 6, 2, 64, 64), (300, 3, 1, 5, 16), (7, 1, 1, 3, 16)])
+@pytest.mark.parametrize("norms", [(True, True), (True, False), (False, False)])
+@pytest.mark.parametrize("write_cache", [True, False])
+def test_projection_rows_at_the_borders_of_their_threads(rows, heads, kv_heads, dim, head_size, norms, write_cache):
+    k = kernels()
+    rng = np.random.default_rng(rows + heads + dim)
+    page_size, eps, rot_dims = 16, 1e-5, dim // 4 * 2
+    n_pages = -(-rows // page_size) + 1
+    f = rng.normal(0, 2, (rows, (heads + 2 * kv_heads) * dim)).astype(np.float32).astype(np.float64)
+    q, key, v = np.split(f, [heads * dim, (heads + kv_heads) * dim], axis=1)
+    gains = [rng.normal(1, 0.2, width).astype(np.float32).astype(np.float64) if there else None for there, width in zip(norms, (heads * dim, kv_heads * dim))]
+    positions = rng.integers(0, 2000, rows)
+    slots = rng.permutation(n_pages * page_size)[:rows]
+    slots[rows // 2] = -1
+    rot = {"dims": rot_dims, "base": 300.0}
+    frequencies = torch.tensor(plain.rotary_frequencies(rot), dtype=torch.float64).cuda() if rot_dims else None
+    pages = [torch.full((n_pages, kv_heads, page_size, head_size), 7.0).cuda() for _ in range(2)]
+    g = gpu(f)
+    got = k.projection_rows(g[:, : q.shape[1]], g[:, q.shape[1] : q.shape[1] + key.shape[1]], g[:, q.shape[1] + key.shape[1] :],
+                            *(None if gain is None else gpu(gain) for gain in gains), eps, frequencies, rot_dims, ints(positions), ints(slots), *pages, heads, kv_heads,
+                            dim, dim, write_cache=write_cache).cpu().numpy().reshape(rows, heads, head_size)
+    def turned(x, gain, n):
+        unit = x if gain is None else plain.rms_unit(x, eps) * gain
+        return plain.rotate_pairs(unit.reshape(rows, n, dim), positions, rot) if rot_dims else unit.reshape(rows, n, dim)
+    np.testing.assert_allclose(got[:, :, :dim], turned(q, gains[0], heads), **tol(torch.float32))
+    assert (got[:, :, dim:] == 0).all()
+    kp, vp = (p.cpu().numpy() for p in pages)
+    stored = slots >= 0 if write_cache else np.zeros(rows, dtype=bool)
+    at = slots[stored]
+    for have, want in ((kp, turned(key, gains[1], kv_heads)), (vp, v.reshape(rows, kv_heads, dim))):
+        np.testing.assert_allclose(have[at // page_size, :, at % page_size, :dim], want[stored], **tol(torch.float32))
+        assert (have[at // page_size, :, at % page_size, dim:] == 0).all()
+        untouched = np.ones((n_pages, page_size), dtype=bool)
+        untouched[at // page_size, at % page_size] = False
+        assert (have.transpose(0, 2, 1, 3)[untouched] == 7).all()
+
+
 def batch_of(portions, slots):
     """q_starts, token_request and state_slots of a step whose requests bring ``portions`` rows each."""
     starts = np.concatenate([[0], np.cumsum(portions)])
