@@ -815,7 +815,9 @@ __global__ __launch_bounds__(256) void pending_sum_kernel(PendingSum in, float* 
 // 32-bit, like the norm of plain rows (elementwise.hip). THREADS: as many as a row has pieces of four columns, rounded up, so that a thread owns one piece and
 // everything it needs of it (the row, its bias, up to eight partial rows, gain and offset) is one trip to memory: a kernel of few rows is little else. With the
 // partial rows asked for behind the bias and gain and offset behind the statistics, three trips: 64 rows of 1,024 with four
-// partial rows, alone in a loop, 3.3 -> 2.9 us, 512 rows 4.0 -> 3.5; 32 tokens of 64 sequences of the medium shape 46.3 -> 44.9 ms.
+// partial rows, alone in a loop, 3.3 -> 2.9 us, 512 rows 4.0 -> 3.5; 32 tokens of 64 sequences of the medium shape 46.3 -> 44.9 ms. Narrow rows have
+// blocks to their measure: waves without a piece, which ask for the row's last, made 8,192 rows of 64 with nine partial rows 20.8 us for 7.9, eight rows with sixteen in
+// groups of threads 4.0 for 3.1 (and a branch around their loads costs all rows 0.1 us).
 // GROUPS > 1 (a row of many partial rows, few of them in a launch: the rows a decode step's last layer leaves for the final norm): the block's threads in so many
 // groups of `group_lanes`, each of which adds up every GROUPS-th partial row, all asked for at once; their shares meet in LDS, in a fixed order.
 template <typename OutT, int GROUPS, int THREADS>
@@ -828,9 +830,19 @@ __global__ __launch_bounds__(THREADS) void pending_layernorm_kernel(
     const int tid = threadIdx.x, n_pieces = width / 4;
     const int source = row_index ? row_index[blockIdx.x] : blockIdx.x;
     const bool owns = tid < n_pieces;
+    auto waves_total = [](const float* of) {
+        float total = of[0];
+        if constexpr (WAVES == 2) total += of[1];
+        if constexpr (WAVES >= 4) {
+            total = (of[0] + of[1]) + (of[2] + of[3]);
+#pragma unroll
+            for (int w = 4; w < WAVES; w += 4) total += (of[w] + of[w + 1]) + (of[w + 2] + of[w + 3]);
+        }
+        return total;
+    };
     const int own_piece = min(tid, n_pieces - 1);
-    PendingLoads loads;
     const int group = GROUPS > 1 ? tid / group_lanes : 0, piece = GROUPS > 1 ? min(tid % group_lanes, n_pieces - 1) : own_piece;
+    PendingLoads loads;
     loads.ask(in, source, width, piece, group, GROUPS);
     const f32x4 gain = load4(gamma + 4 * own_piece), offset = load4(beta + 4 * own_piece);
     keep_order();
@@ -847,16 +859,12 @@ __global__ __launch_bounds__(THREADS) void pending_layernorm_kernel(
     if (tid % WAVE == 0) red[0][tid / WAVE] = sum;
     __syncthreads();
     const float n = (float)width;
-    float total = 0.0f;
-#pragma unroll
-    for (int w = 0; w < WAVES; w += 4) total += (red[0][w] + red[0][w + 1]) + (red[0][w + 2] + red[0][w + 3]);
+    float total = waves_total(red[0]);
     const f32x4 centred = value - total / n;
     const float squares = wave_total(owns ? (centred[0] * centred[0] + centred[1] * centred[1]) + (centred[2] * centred[2] + centred[3] * centred[3]) : 0.0f);
     if (tid % WAVE == 0) red[1][tid / WAVE] = squares;
     __syncthreads();
-    total = 0.0f;
-#pragma unroll
-    for (int w = 0; w < WAVES; w += 4) total += (red[1][w] + red[1][w + 1]) + (red[1][w + 2] + red[1][w + 3]);
+    total = waves_total(red[1]);
     const float inverse_stddev = 1.0f / sqrtf(total / n + eps);
     if (!owns) return;
     const f32x4 y = centred * inverse_stddev * gain + offset;
@@ -1074,7 +1082,11 @@ MLLM_API int mllm_pending_layernorm(const float* base, const float* partials, co
 #define MLLM_PENDING_NORM_WITH(OutT, GROUPS, THREADS) \
     pending_layernorm_kernel<OutT, GROUPS, THREADS><<<n_rows, THREADS, (size_t)width * 4 * (GROUPS == 1 ? 0 : GROUPS), stream>>>(in, row_index, gamma, beta, (OutT*)out, summed, width, eps, packed_out, group_lanes)
 #define MLLM_PENDING_NORM(OutT)                                            \
-    if (grouped) MLLM_PENDING_NORM_WITH(OutT, 4, 1024);                    \
+    if (grouped && width <= 256) MLLM_PENDING_NORM_WITH(OutT, 4, 256);     \
+    else if (grouped && width <= 512) MLLM_PENDING_NORM_WITH(OutT, 4, 512); \
+    else if (grouped) MLLM_PENDING_NORM_WITH(OutT, 4, 1024);               \
+    else if (width <= 256) MLLM_PENDING_NORM_WITH(OutT, 1, 64);            \
+    else if (width <= 512) MLLM_PENDING_NORM_WITH(OutT, 1, 128);           \
     else if (width <= 1024) MLLM_PENDING_NORM_WITH(OutT, 1, 256);          \
     else if (width <= 2048) MLLM_PENDING_NORM_WITH(OutT, 1, 512);          \
     else if (width <= 4096) MLLM_PENDING_NORM_WITH(OutT, 1, 1024);         \

@@ -1,4 +1,4 @@
-"""RMS norm with a block a row: widths at the edges of its threads, partial products beyond those asked for at once, every option."""
+"""Norms with a block a row: widths at the edges of their threads, partial products beyond those asked for at once, every option."""
 
 import pytest
 import torch
@@ -51,3 +51,25 @@ def test_branch_products_of_few_rows_are_cut_from_a_long_k_on(dtype, rows, n, k,
     first, rest = (branch[0], branch[1:]) if branch.dim() == 3 else (branch, None)
     # sums of k products of numbers around 1 / sqrt(k), each rounding 2^-24 of a partial sum of at most some 5, sixteen terms at a time
     assert (K.rms_norm(first, weight, 1e-5, addend=rest, residual=residual).double() - want).abs().max() <= 5 * 4 * 2.0 ** -24 * (k / 16) ** 0.5 * 4
+
+
+# waves without a column, rows of 4,096 (a piece of four columns a thread of the largest block) and of more (several), groups of threads that share a row's sums
+@pytest.mark.parametrize("rows,width,partials", [(3, 4, 1), (2, 4, 16), (300, 60, 9), (64, 64, 17), (9, 260, 20), (2, 1024, 16), (65, 1024, 16), (300, 1028, 8), (3, 2052, 5), (3, 4096, 9), (3, 4100, 9),
+                                                 (2, 8200, 17), (5, 4100, 0)])
+@pytest.mark.parametrize("with_bias", [False, True])
+@pytest.mark.parametrize("out_dtype", [torch.float32, torch.bfloat16])
+def test_layer_norm_of_pending_rows_at_the_borders_of_its_threads(rows, width, partials, with_bias, out_dtype):
+    from mini_llm_amd.ops import kernels as K
+
+    generator = torch.Generator(device="cuda").manual_seed(rows * width + partials)
+    draw = lambda *shape: torch.randn(*shape, generator=generator, device="cuda")
+    base, parts, bias, gain, offset = draw(rows, width), draw(partials, rows, width), draw(width), draw(width), draw(width)
+    pending = K.PendingRows(base, parts if partials else None, bias if with_bias else None)
+    total = base.double() + parts.double().sum(0) + (bias.double() if with_bias else 0)
+    want = torch.nn.functional.layer_norm(total, (width,), gain.double(), offset.double(), 1e-5)
+    # 32-bit sums of up to 19 addends and of 8,200 numbers, a square root and a division: some 2^-23 times twenty of numbers around 10
+    close = lambda got, ref: (got.double() - ref).abs().max() <= 2e-5 + (ref.abs().max() * 2.0 ** -8 if got.dtype == torch.bfloat16 else 0)
+    normed, summed = K.layernorm(pending, gain, offset, 1e-5, out_dtype=out_dtype, with_sums=True)
+    assert close(normed, want) and close(summed, total)
+    index = torch.randint(rows, (rows + 2,), generator=generator, device="cuda").int()
+    assert close(K.layernorm(pending, gain, offset, 1e-5, out_dtype=out_dtype, row_index=index), want[index.long()])
