@@ -131,8 +131,11 @@ __global__ __launch_bounds__(256) void rms_norm_kernel(const float* __restrict__
 // needs is a handful of 16-byte loads in one trip to memory. A wave a row asks for its columns one number at a time, five arrays of up to sixteen loads a
 // lane before it can add anything up. A wave a row / a block a row, us, in 32-bit with a residual and a second norm: rows of 768, 8 of them 4.1 / 2.7 (two partial
 // products 4.2 / 3.0, five 5.1 / 3.1), 256 4.4 / 2.9, 2,048 6.3 / 5.9; rows of 1,600, 8 of them 6.2 / 2.9, 2,048 14.2 / 10.1; without either, rows of 768, 8 of
-// them 3.8 / 2.4, 2,048 4.8 / 4.1. Where many rows are narrow most of a block has nothing to do (4,096 rows of 60 2.9 / 4.8), and many thousand rows with many partial
-// products are bound by their bytes either way (32,768 rows of 768 with five 141 / 147): a wave a row there.
+// them 3.8 / 2.4, 2,048 4.8 / 4.1. What stays with a wave a row (block_a_row below): rows of up to 256, of which a wave asks for four numbers a lane and most of a block
+// has nothing to do (8 rows of 64 with five partial products 2.9 / 3.2, 64 of 256 with an addend 3.0 / 3.1); of up to 512, its eight numbers a lane, from some 512 rows on
+// (512 of 512 with four 4.1 / 3.7, 768 with nine 4.6 / 5.1, 2,048 with one 4.6 / 5.7; behind 512 it asks for sixteen: 2,048 of 576 with four 0.87 of its time); and
+// thousands of rows with many partial products, which are bound by their bytes (32,768 rows of 768 with five 141 / 147; of 1,024, whose blocks are as large as 768's
+// and hold a third more, 2,048 with sixteen 24.4 / 27.0, 8,192 with eight 54.4 / 56.7; of 1,600, 8,192 with eight 124 / 103 the other way).
 template <int THREADS>
 __global__ __launch_bounds__(THREADS) void rms_norm_row_kernel(const float* __restrict__ x, const void* __restrict__ y, int y_code, float alpha,
                                                                const int* __restrict__ row_index, const float* __restrict__ weight, int one_plus,
@@ -423,6 +426,13 @@ __global__ __launch_bounds__(256) void silu_mul_kernel(const T* __restrict__ bot
 
 }  // namespace
 
+// Whether so many rows take the kernel with a block a row, if their operands lie on their borders: the lines and what was measured are named there.
+MLLM_API int mllm_rms_norm_block_a_row(int n_rows, int width, int n_partials) {
+    if (width % 4 != 0 || width > 2048 || n_rows > 16384) return 0;
+    if (width <= 512) return width > 256 && n_rows <= 512;
+    return width <= 768 || width > 1024 || n_partials < 8 || (long long)n_rows * n_partials < 32768;
+}
+
 MLLM_API int mllm_rms_norm(const float* x, const void* y, int y_dtype, float alpha, const int* row_index, const float* weight, int one_plus,
                            float eps, float* stream_out, void* rows_out, int rows_dtype, int n_rows, int width, int n_partials,
                            long long partial_stride, const float* residual, const float* next_weight, hipStream_t stream) {
@@ -439,7 +449,7 @@ MLLM_API int mllm_rms_norm(const float* x, const void* y, int y_dtype, float alp
     mllm_count_kernel(MLLM_K_RMS_NORM);
     const size_t wide = (size_t)x | (size_t)weight | (size_t)residual | (size_t)next_weight | (size_t)stream_out | (y_dtype == MLLM_F32 ? (size_t)y : 0) |
                         (rows_dtype == MLLM_F32 ? (size_t)rows_out : 0) | (size_t)(partial_stride * (n_partials > 1 ? 4 : 0));
-    if ((width >= 512 || n_rows <= 256) && n_rows <= 16384 && width % 4 == 0 && width <= 2048 && wide % 16 == 0 && (((size_t)y | (size_t)rows_out) & 7) == 0) {
+    if (mllm_rms_norm_block_a_row(n_rows, width, n_partials) && wide % 16 == 0 && (((size_t)y | (size_t)rows_out) & 7) == 0) {
 #define LAUNCH(THREADS) rms_norm_row_kernel<THREADS><<<n_rows, THREADS, 0, stream>>>(x, y, y_dtype, alpha, row_index, weight, one_plus, eps, stream_out, rows_out, rows_dtype, width, n_partials, partial_stride, residual, next_weight)
         if (width <= 1024) LAUNCH(256);
         else LAUNCH(512);
