@@ -87,18 +87,21 @@ __device__ __forceinline__ void still_written(const i32x4& fragment) { asm volat
 struct XcdTiles {
     int tiles_m, tiles_n, strip, per_xcd, count;
 };
-// The strip is as high as makes the rows of A and W that the XCDs read the fewest. Equal shares come first: one block more than 32 on one XCD is a second round
-// of its compute units (rectangles of equal sides that cover the tiles give some XCDs full ones and others a remainder: 528 x 1,024 x 4,096 in three parts along K,
-// 240 blocks, were 36 on six of them: 23.6 us).
+// The strip is as high as makes the rows of A and W that the XCDs read in one round, a block on each of their 32 compute units, the fewest (over a share of many rounds
+// it would be as high as the tiles are, and a round columns of 16 tiles that read sixteen times the rows of A for two of W: with 32-bit out 16,384 x 4,800 x 1,600
+// 343 us, in strips of four 335, 8,192 x 4,096 x 1,024 114 and 108). Equal shares come first: one block more than 32 on one XCD is a second round of its compute units
+// (rectangles of equal sides that cover the tiles give some XCDs full ones and others a remainder: 528 x 1,024 x 4,096 in three parts along K, 240 blocks, were 36 on
+// six of them: 23.6 us).
 inline XcdTiles place_tiles(int tiles_m, int tiles_n, int bm, int bn, int k_blocks) {
     const int tiles = tiles_m * tiles_n, count = tiles * k_blocks, per_xcd = ceil_div(count, 8);
+    const int at_once = per_xcd < 32 ? per_xcd : 32;
     XcdTiles best{tiles_m, tiles_n, 1, per_xcd, count};
     long best_rows = -1;
     for (int strip = 1; strip <= tiles_m && strip <= 16; strip++) {
         const int in_strip = strip * tiles_n;
         long rows = 0;
         for (int xcd = 0; xcd < 8; xcd++) {
-            const int from = xcd * per_xcd % tiles, to = from + (per_xcd < tiles ? per_xcd : tiles) - 1;   // (of the parts along K the first it takes)
+            const int from = xcd * per_xcd % tiles, to = from + (at_once < tiles ? at_once : tiles) - 1;   // (of the parts along K the first it takes)
             const int strips = to / in_strip - from / in_strip + 1, first = from % in_strip / strip, last = to % in_strip / strip;
             const int columns = strips == 1 ? last - first + 1 : strips == 2 && last < first ? tiles_n - first + last + 1 : tiles_n;
             rows += (long)strips * strip * bm + (long)columns * bn;
