@@ -837,6 +837,14 @@ MLLM_API int mllm_gemm_takes_packed_rows(int M, int N, int K, int in_dtype) {
     return 0;
 }
 
+// The tile of outputs with which a bfloat16 product of M rows and a packed W runs, in k_blocks parts along K: 10,000 times its rows and 10 times its columns, and of
+// 128 x 64 which of its kernels (0; 1: two waves share a tile along K; 2: two blocks a compute unit). 0: another kernel than the streaming one.
+MLLM_API int mllm_gemm_stream_tile(int M, int N, int K, int k_blocks, int out_dtype) {
+    if (M <= 0 || N <= 0 || K <= 0 || k_blocks < 1 || !stream::takes(M, N, K, true, CacheScatter{}, out_dtype == MLLM_F32 ? 4 : 2)) return 0;
+    static const int tiles[] = {1281920, 1921280, 2561280, 1281280, 1280640, 1280641, 1280642, 2562560};
+    return tiles[stream::choose(M, N, K, k_blocks, out_dtype == MLLM_BF16)];
+}
+
 // x_packed: A is in the packed layout of an [M, K] matrix; out_packed: out is written in the packed
 // layout of an [M, N] matrix (no residual then). Both only where mllm_gemm_takes_packed_rows says so.
 MLLM_API int mllm_gemm(const void* A, const void* W, int w_packed, const float* bias, const float* residual,

@@ -10,9 +10,10 @@
 //    of a row touched every line twice: 18.3 -> 18.0 us at 2,048 x 768 x 3,072); a row's eight pieces lie in LDS rotated by the row
 //    (piece ^ (row / 2) % 8), so that the sixteen lanes of a fragment read fall on sixteen different
 //    groups of banks.
-//  * A block has a compute unit to itself and a wave a SIMD: whatever a wave waits for, its matrix
-//    core waits for too. So a wave owns 64 x 64 outputs or more (at 64 x 32 the fragment reads, not
-//    the products, set the pace); fragments are asked for two steps of K before their products; a
+//  * A block has a compute unit to itself, and most tiles a wave a SIMD: whatever a wave waits for, its matrix
+//    core waits for too. So a wave owns 64 x 64 outputs or more (at 64 x 32 the fragment reads, not the products,
+//    set the pace of the loop: so in 128 x 64, which has no more for four waves, and in 128 x 128, which pays it for two
+//    waves a SIMD, one computing while the other is on its way out); fragments are asked for two steps of K before their products; a
 //    tile's loads from memory go out a few at a time between the products of earlier tiles (a compute
 //    unit takes a load of 1 KiB every 16 cycles or so: a wave that issues a whole tile's loads at
 //    once stands still meanwhile); and the order of all this is pinned (sched_barrier), because left
@@ -626,8 +627,10 @@ inline const TileCost* tile_costs() {
 }
 // us of the product with that tile in k_blocks parts along K
 inline float product_us(const TileCost& tile, int M, int N, int K, int k_blocks) {
-    const long blocks = (long)ceil_div(M, tile.bm) * ceil_div(N, tile.bn) * k_blocks;
-    return (float)((blocks + 255) / 256) * (tile.start_us + (float)ceil_div(ceil_div(K, k_blocks), 64) * tile.tile_us);
+    const long rounds = ((long)ceil_div(M, tile.bm) * ceil_div(N, tile.bn) * k_blocks + 255) / 256;
+    // in many rounds what a tile reads weighs more: 16,384 x 1,600 x 6,400 takes 256 x 128 358 us and 192 x 128 379
+    const float tile_us = tile.bm == 256 && rounds >= 4 ? 0.95f * tile.tile_us : tile.tile_us;
+    return (float)rounds * (tile.start_us + (float)ceil_div(ceil_div(K, k_blocks), 64) * tile_us);
 }
 inline int best_tile(int M, int N, int K, int k_blocks) {
     int best = 0;
@@ -636,10 +639,10 @@ inline int best_tile(int M, int N, int K, int k_blocks) {
     return best;
 }
 
-template <typename OutT>
-void dispatch(const bf16_t* a, const bf16_t* w, const float* bias, const float* residual, OutT* o, int M, int N, int K, int epilogue,
-             hipStream_t stream, CacheScatter scatter, int k_blocks) {
-#define MLLM_STREAM(BM, BN, WM_, WN_, WK_, ST) launch<OutT, BM, BN, WM_, WN_, WK_, ST>(a, w, bias, residual, o, M, N, K, epilogue, stream, scatter, k_blocks)
+// The kernels of the products, by their tiles.
+enum Shape { S128x192, S192x128, S256x128, S128x128, S128x64, S128x64_SHARED, S128x64_ROUNDS, S256x256 };
+
+inline Shape choose(int M, int N, int K, int k_blocks, bool bf16_out) {
     // 256 x 256 (four waves of 128 x 128; the LDS holds two stages of it) brings a compute unit 40k outputs a microsecond
     // and tile of K where the others bring 30k, but only in full rounds of at least 150 blocks: from 2,048 x 6,400 on.
     // Measured against the best of the others, on one machine in one run: 2,048 x 6,400 x 1,600 52 against 59 us (as a layer's up
@@ -648,35 +651,50 @@ void dispatch(const bf16_t* a, const bf16_t* w, const float* bias, const float* 
     // another one took 45.2 and 52.4 us for the first of these.) In such rounds a tile of K costs it 1.6 us and the others 1.45 times these:
     // (Only with bfloat16 out, which is what the products of that size write: with 32-bit out and a residual asked for
     // before the loop, a lane's 256 sums and 256 residual values do not fit its registers.)
-    if constexpr (sizeof(OutT) == 2) {
+    if (bf16_out && k_blocks == 1) {
         static const float in_full_rounds[4][3] = {{128, 192, 0.57f}, {256, 128, 0.70f}, {128, 128, 0.45f}, {128, 64, 0.30f}};
         const long large = (long)ceil_div(M, 256) * ceil_div(N, 256), rounds = (large + 255) / 256;
-        if (k_blocks == 1 && large >= 150 && large * 10 >= rounds * 256 * 7) {
+        if (large >= 150 && large * 10 >= rounds * 256 * 7) {
             float others = 1e30f;
             for (const auto& tile : in_full_rounds) {
                 const long blocks = (long)ceil_div(M, (int)tile[0]) * ceil_div(N, (int)tile[1]);
                 others = fminf(others, (float)((blocks + 255) / 256) * tile[2]);
             }
-            if ((float)rounds * 1.6f < others * 1.45f) {
-                MLLM_STREAM(256, 256, 2, 2, 1, 2);
-                return;
-            }
+            if ((float)rounds * 1.6f < others * 1.45f) return S256x256;
         }
     }
-    const int best = best_tile(M, N, K, k_blocks), k_part = ceil_div(K, k_blocks);
-    const bool one_round = (long)ceil_div(M, 128) * ceil_div(N, 64) * k_blocks <= 256;
-    if (best == 0) MLLM_STREAM(128, 192, 2, 2, 1, 3);
-    else if (best == 1) MLLM_STREAM(192, 128, 2, 2, 1, 3);
-    else if (best == 2) MLLM_STREAM(256, 128, 4, 2, 1, 3);
-    // eight waves of 64 x 32, two a SIMD, cover each other's way out of the loop where four of 64 x 64 read less in it: 528 x 4,096 x 1,024 10.1 and 10.5 us, 1,500 x
-    // 3,072 x 768 17.3 and 18.1; GPT-2 XL's output and down products, 2,048 rows, inside a prompt step 41.4 and 42.3 on average
-    else if (best == 3) MLLM_STREAM(128, 128, 2, 4, 1, 4);
-    // narrow outputs in one round of blocks: four stages (a layer's down product, 2,048 x 768 x 3,072, 22.8 us in a prompt step, 23.4 with two waves sharing each
-    // 64 x 64 tile along K, 26.0 with three stages); in more rounds two waves share a tile along K where K is long, and else three stages leave room for two blocks
-    // a compute unit
-    else if (one_round) MLLM_STREAM(128, 64, 2, 2, 1, 4);
-    else if (k_part >= 1536) MLLM_STREAM(128, 64, 2, 1, 2, 4);
-    else MLLM_STREAM(128, 64, 2, 2, 1, 3);
+    static const Shape by_cost[TILES] = {S128x192, S192x128, S256x128, S128x128, S128x64};
+    const Shape best = by_cost[best_tile(M, N, K, k_blocks)];
+    if (best != S128x64) return best;
+    // Narrow outputs in one round of blocks: four stages (a layer's down product, 2,048 x 768 x 3,072, 22.8 us in a prompt step, 26.0 with three). Two waves that share
+    // each 64 x 64 tile along K have half the reads of A's rows under way at a time: the better for a long K whose rows lie whole multiples of 8 KiB apart, where the
+    // rows of a load meet in the same channels of memory (K of 4,096, us, four stages / shared: 65 rows of 1,024 20.0 / 19.0, 300 20.6 / 20.0, 1,500 22.4 / 22.0; K of
+    // 8,192 0.95 of its time; of 3,072, 3,584, 5,632 and 6,400 from 128 rows on 1.01 to 1.02), or of little more than half a tile of rows (65 rows, K of 3,072 to 6,400:
+    // 0.97 to 0.92); short ones lose by it (K of 768 1.08, of 1,600 1.02, of 2,560 1.03).
+    // In more rounds, which take outputs of up to 64 columns and many thousand rows, three stages leave room for two blocks a compute unit (65,536 x 64 x 768 20.3 us,
+    // with four stages 23.7; x 2,048 44.6, 46.2, shared 47.6).
+    if ((long)ceil_div(M, 128) * ceil_div(N, 64) * k_blocks > 256) return S128x64_ROUNDS;
+    return ceil_div(K, k_blocks) >= 3072 && (K % 4096 == 0 || M <= 96) ? S128x64_SHARED : S128x64;
+}
+
+template <typename OutT>
+void dispatch(const bf16_t* a, const bf16_t* w, const float* bias, const float* residual, OutT* o, int M, int N, int K, int epilogue,
+              hipStream_t stream, CacheScatter scatter, int k_blocks) {
+#define MLLM_STREAM(BM, BN, WM_, WN_, WK_, ST) launch<OutT, BM, BN, WM_, WN_, WK_, ST>(a, w, bias, residual, o, M, N, K, epilogue, stream, scatter, k_blocks)
+    switch (choose(M, N, K, k_blocks, sizeof(OutT) == 2)) {
+        case S128x192: MLLM_STREAM(128, 192, 2, 2, 1, 3); break;
+        case S192x128: MLLM_STREAM(192, 128, 2, 2, 1, 3); break;
+        case S256x128: MLLM_STREAM(256, 128, 4, 2, 1, 3); break;
+        // eight waves of 64 x 32, two a SIMD, cover each other's way out of the loop where four of 64 x 64 read less in it: 528 x 4,096 x 1,024 10.1 and 10.5 us, 1,500 x
+        // 3,072 x 768 17.3 and 18.1; GPT-2 XL's output and down products, 2,048 rows, inside a prompt step 41.4 and 42.3 on average
+        case S128x128: MLLM_STREAM(128, 128, 2, 4, 1, 4); break;
+        case S128x64: MLLM_STREAM(128, 64, 2, 2, 1, 4); break;
+        case S128x64_SHARED: MLLM_STREAM(128, 64, 2, 1, 2, 4); break;
+        case S128x64_ROUNDS: MLLM_STREAM(128, 64, 2, 2, 1, 3); break;
+        case S256x256:
+            if constexpr (sizeof(OutT) == 2) MLLM_STREAM(256, 256, 2, 2, 1, 2);
+            break;
+    }
 #undef MLLM_STREAM
 }
 

@@ -21,6 +21,7 @@ _SIGNATURES = {
     "mllm_gemm": [P, P, c_int, P, P, P, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, P],
     "mllm_gemm_takes_packed_rows": [c_int, c_int, c_int, c_int],
     "mllm_gemm_split": [P, P, c_int, P, c_int, c_int, c_int, c_int, c_int, c_int, P],
+    "mllm_gemm_stream_tile": [c_int, c_int, c_int, c_int, c_int],
     "mllm_gemm_split_blocks": [c_int, c_int, c_int, c_int],
     "mllm_gemm_split_blocks_anywhere": [c_int, c_int, c_int, c_int],
     "mllm_gemm_qkv_cache": [P, P, c_int, P, P, P, P, P, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, P],

@@ -27,3 +27,27 @@ def test_rms_norm_with_a_block_or_a_wave_a_row(rows, width, partials, block):
     from mini_llm_amd.ops.library import library
 
     assert library().mllm_rms_norm_block_a_row(rows, width, partials) == block
+
+
+def test_every_tile_of_the_streaming_product_has_a_shape_in_its_test():
+    from mini_llm_amd.ops.library import library
+    from test_stream_tiles_gpu import SHAPES
+
+    tile = library().mllm_gemm_stream_tile
+    for m, n, k, tile_f32, tile_bf16, tile_cut in SHAPES:
+        assert (tile(m, n, k, 1, 0), tile(m, n, k, 1, 1), tile(m, n, k, 3, 0)) == (tile_f32, tile_bf16, tile_cut)
+    assert {shape[3] for shape in SHAPES} == {1281920, 1921280, 2561280, 1281280, 1280640, 1280641, 1280642}
+    assert {shape[4] for shape in SHAPES} == {1281920, 1921280, 2561280, 1281280, 1280640, 1280641, 1280642, 2562560}
+    assert tile(64, 768, 768, 1, 0) == tile(65, 770, 768, 1, 0) == tile(65, 768, 736, 1, 0) == 0   # other kernels'
+
+
+@pytest.mark.parametrize("m,n,k,out,tile", [
+    # a long K in one round of narrow tiles: shared where measured faster (see the kernel's rule)
+    (65, 1024, 4096, 0, 1280641), (1500, 1024, 4096, 0, 1280641), (300, 2048, 8192, 1, 1280641), (65, 1600, 6400, 1, 1280641), (128, 1600, 6400, 0, 1280640),
+    (2048, 768, 3072, 0, 1280640), (300, 768, 2048, 0, 1280640), (65, 768, 2048, 0, 1280640),
+    # many rounds
+    (16384, 1600, 6400, 0, 2561280), (65536, 64, 768, 0, 1280642)])
+def test_tiles_of_the_streaming_product_by_measurement(m, n, k, out, tile):
+    from mini_llm_amd.ops.library import library
+
+    assert library().mllm_gemm_stream_tile(m, n, k, 1, out) == tile
