@@ -707,9 +707,10 @@ int skinny_k_blocks(int N, int K) {
 // 128 x 768 x 768 product takes 6.1 us in two cuts against 7.9 us whole (bfloat16; in 32-bit 8.6 us
 // in four cuts against 12.6 us in two).
 //
-// most: the most partial products there is room for, asked by the rule for products in pieces alone, which cuts finer than the rules below.
+// most: the most partial products there is room for (asked by the two rules of costs, which cut finer than the ones below them). packed: W's layout, which in bfloat16
+// decides between two kernels of different costs.
 template <typename T>
-int tiled_k_blocks(int M, int N, int K, int most) {
+int tiled_k_blocks(int M, int N, int K, int most, bool packed) {
     int tiles = ceil_div(M, 128) * ceil_div(N, 64);
     int k_blocks = 1;
     // By whole tiles of 128 rows, as the rest. A W without pieces takes the 32-bit instruction with this count too, and loses nothing by it, the reading of the
@@ -732,16 +733,33 @@ int tiled_k_blocks(int M, int N, int K, int most) {
         return best;
     }
     if (sizeof(T) == 2 && K % 64 == 0 && N % 8 == 0) {
-        // By the costs of the streaming kernel's tiles and what the partial products cost: each is written and read, whoever adds them up reads the stream and
-        // writes it again (at 5.5 TB/s), and has one more load under way. With the layer norm behind it, whole / as this rule cuts it, us: 80 x 768 x 3,072 18.3 /
-        // 10.3 (in eight), 528 x 1,024 x 4,096 23.4 / 17 (three), 1,024 x 768 x 3,072 20.8 / 18.7 (two), 1,500 x 1,600 x 6,400 49.0 / 45.2 (two); left whole:
-        // 2,048 x 768 x 3,072 23.1 (24.5 in two), 528 x 1,024 x 1,024 12.5 (12.9 in two), 2,048 x 1,600 x 6,400 55.2 (57.6 in two).
+        // By what the product and the partial products cost. Each partial product is written and read (at 5.5 TB/s; behind 12 MB of them a third time: they no longer lie in
+        // the caches), whoever adds them up has one more load under way; what is read and written besides them the whole product has too. With the layer norm
+        // behind it, whole / as this rule cuts it, us: 100 x 768 x 3,072 18.9 / 10.3 (in eight), 400 x 1,600 x 1,600 16.9 / 15.2 (two), 528 x 1,024 x 4,096 23.6 /
+        // 17.5 (three), 528 x 1,280 x 5,120 30.7 / 22.1 (two; 25.0 in five), 1,000 x 768 x 3,072 20.1 / 17.9 (two), 1,500 x 1,600 x 6,400 55.5 / 49.1 (two); left
+        // whole: 2,048 x 768 x 3,072 23.1 (24.5 in two). Over 224 sizes of 65 to 3,000 rows 0.8 % behind the best count of each.
         const int rows = ceil_div(M, 128) * 128;
+        const bool streams = stream::takes(rows, N, K, packed, CacheScatter{}, 4);
         const float output_us = (float)rows * (float)N * 4.0f / 5.5e6f;
         int best = 1;
         float best_us = 0.0f;
         for (int cuts = 1; cuts <= std::min(8, most) && (cuts == 1 || K >= 4 * 64 * cuts); cuts++) {
-            const float us = stream::product_us(stream::tile_costs()[stream::best_tile(rows, N, K, cuts)], rows, N, K, cuts) + (cuts == 1 ? 0.0f : output_us * (3.0f + 1.3f * (float)cuts) + 0.15f * (float)cuts);
+            float us;
+            if (streams) {
+                us = stream::product_us(stream::tile_costs()[stream::best_tile(rows, N, K, cuts)], rows, N, K, cuts);
+                if (cuts > 1) us += output_us * (0.5f + 1.8f * (float)cuts) + 0.15f * (float)cuts + std::max(0.0f, output_us * (float)cuts - 12.0f / 5.5f);
+            } else {
+                // The tiled kernel (a row-major W, or rows of 4 GiB and more), whose tiles find room beside each other on a compute unit, so that a remainder of a round
+                // costs half of one: as above, 257 x 1,280 x 1,280 15.3 / 12.8 (two), 400 x 1,600 x 1,600 18.8 / 16.6 (two), 1,500 x 768 x 3,072 28.4 / 26.4
+                // (three), 2,048 x 2,048 x 5,632 102.4 / 89.2 (two), 1,000 x 1,600 x 6,400 53.9 / 55.2 (two; 59.1 in three, as the streaming
+                // kernel's costs would have it); over the same sizes 0.8 % behind the best.
+                const int blocks = ceil_div(M, 128) * ceil_div(N, 64) * cuts, large = ceil_div(M, 256) * ceil_div(N, 128);
+                const float k_tiles = (float)ceil_div(ceil_div(K, cuts), 64), rounds = (float)blocks / 256.0f;
+                if (cuts == 1 && rows >= 256 && large >= 128) us = (float)ceil_div(large, 256) * k_tiles * 1.0f;
+                else if (blocks <= 128) us = k_tiles * 0.34f;
+                else us = std::max(1.0f, 0.5f * ((float)ceil_div(blocks, 256) + rounds)) * k_tiles * 0.42f;
+                if (cuts > 1) us += output_us * (0.5f + 1.4f * (float)cuts) + 0.15f * (float)cuts;
+            }
             if (cuts == 1 || us < best_us) best = cuts, best_us = us;
         }
         return best;
@@ -927,10 +945,10 @@ MLLM_API int mllm_gemm_best(const void* A, const void* W, int w_packed, const fl
 
 constexpr size_t STATIC_SCRATCH_FLOATS = (size_t)1 << 20;  // 4 MiB: what mllm_linear_split_static has room for
 
-static int split_blocks_of_at_most(int M, int N, int K, int in_dtype, int most) {
+static int split_blocks_of_at_most(int M, int N, int K, int in_dtype, int most, bool packed) {
     if (M <= 0 || N <= 0 || K <= 0) return 1;
-    if (in_dtype == MLLM_F32) return K % 4 ? 1 : (M <= 64 ? skinny_k_blocks<float>(N, K) : tiled_k_blocks<float>(M, N, K, most));
-    if (in_dtype == MLLM_BF16) return K % 8 ? 1 : (M <= 64 ? skinny_k_blocks<bf16_t>(N, K) : tiled_k_blocks<bf16_t>(M, N, K, most));
+    if (in_dtype == MLLM_F32) return K % 4 ? 1 : (M <= 64 ? skinny_k_blocks<float>(N, K) : tiled_k_blocks<float>(M, N, K, most, packed));
+    if (in_dtype == MLLM_BF16) return K % 8 ? 1 : (M <= 64 ? skinny_k_blocks<bf16_t>(N, K) : tiled_k_blocks<bf16_t>(M, N, K, most, packed));
     return 1;
 }
 
@@ -938,11 +956,12 @@ static int split_blocks_of_at_most(int M, int N, int K, int in_dtype, int most) 
 // answer to mllm_linear_split_static: no more than fit its array, where one fits.
 MLLM_API int mllm_gemm_split_blocks(int M, int N, int K, int in_dtype) {
     const long long one = (long long)M * N;
-    return split_blocks_of_at_most(M, N, K, in_dtype, one > 0 && one <= (long long)STATIC_SCRATCH_FLOATS ? (int)std::min<long long>(8, STATIC_SCRATCH_FLOATS / one) : 8);
+    return split_blocks_of_at_most(M, N, K, in_dtype, one > 0 && one <= (long long)STATIC_SCRATCH_FLOATS ? (int)std::min<long long>(8, STATIC_SCRATCH_FLOATS / one) : 8, true);
 }
 
-// The same for a caller who brings the memory: the fastest count, however much its partial products take.
-MLLM_API int mllm_gemm_split_blocks_anywhere(int M, int N, int K, int in_dtype) { return split_blocks_of_at_most(M, N, K, in_dtype, 8); }
+// The same for a caller who brings the memory: the fastest count, however much its partial products take. (Both for a packed W, a row-major one below.)
+MLLM_API int mllm_gemm_split_blocks_anywhere(int M, int N, int K, int in_dtype) { return split_blocks_of_at_most(M, N, K, in_dtype, 8, true); }
+MLLM_API int mllm_gemm_split_blocks_row_major(int M, int N, int K, int in_dtype) { return split_blocks_of_at_most(M, N, K, in_dtype, 8, false); }
 
 // A . W^T as k_blocks partial products over consecutive parts of K: partials [k_blocks, M, N] in
 // 32-bit, whose sum (in any fixed order) is the product. For a long K with few output columns;

@@ -318,8 +318,9 @@ def split_blocks(weight, dtype, rows: int = 1) -> int:
     rows with this weight (1: better left whole): more than one where few rows and few output
     columns meet a long K. The same for all row counts up to 64, and for all that need the same
     number of 128-row tiles."""
-    _, _, n, k = _matrix(weight, "weight", dtype)
-    return int(library().mllm_gemm_split_blocks_anywhere(int(rows), n, k, _code(dtype)))
+    _, packed, n, k = _matrix(weight, "weight", dtype)
+    lib = library()
+    return int((lib.mllm_gemm_split_blocks_anywhere if packed else lib.mllm_gemm_split_blocks_row_major)(int(rows), n, k, _code(dtype)))
 
 
 def linear_split(x, weight, k_blocks: int, out=None):

@@ -24,6 +24,7 @@ _SIGNATURES = {
     "mllm_gemm_stream_tile": [c_int, c_int, c_int, c_int, c_int],
     "mllm_gemm_split_blocks": [c_int, c_int, c_int, c_int],
     "mllm_gemm_split_blocks_anywhere": [c_int, c_int, c_int, c_int],
+    "mllm_gemm_split_blocks_row_major": [c_int, c_int, c_int, c_int],
     "mllm_gemm_qkv_cache": [P, P, c_int, P, P, P, P, P, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, P],
     "mllm_convert": [P, P, c_int, c_int, c_int, c_int, c_int, P],
     "mllm_pack_matrix": [P, P, c_int, c_int, c_int, c_int, c_int, P],

@@ -51,3 +51,20 @@ def test_tiles_of_the_streaming_product_by_measurement(m, n, k, out, tile):
     from mini_llm_amd.ops.library import library
 
     assert library().mllm_gemm_stream_tile(m, n, k, 1, out) == tile
+
+
+@pytest.mark.parametrize("m,n,k,packed,row_major", [
+    # counts within 3 % of the best measured, with the layer norm behind the product
+    (100, 768, 3072, {6, 7, 8}, {6, 7, 8}), (400, 1024, 1024, {2, 3}, {2}), (400, 1280, 1280, {2}, {2, 3}), (528, 1280, 1280, {1, 2}, None), (528, 1280, 5120, {2}, None),
+    (400, 1600, 1600, {2}, {2}), (528, 1600, 1600, {1, 2}, {2}), (400, 2048, 2048, {2}, {2}), (200, 1600, 1600, {3, 4}, None), (1200, 256, 1024, {2, 3}, None),
+    (1000, 1600, 6400, None, {1, 2}), (257, 1280, 1280, None, {2}), (2048, 768, 3072, {1}, {1}), (2048, 1600, 1600, {1}, {1})])
+def test_cuts_along_k_of_bfloat16_products_of_many_rows(m, n, k, packed, row_major):
+    from mini_llm_amd.ops.library import library
+
+    lib = library()
+    assert packed is None or lib.mllm_gemm_split_blocks_anywhere(m, n, k, 1) in packed
+    assert row_major is None or lib.mllm_gemm_split_blocks_row_major(m, n, k, 1) in row_major
+    # the same for all counts of rows that need the same number of 128-row tiles, and never an answer of 0 or beyond 8
+    for rows in (-(-m // 128) * 128, (m - 1) // 128 * 128 + 1):
+        assert rows <= 64 or lib.mllm_gemm_split_blocks_anywhere(rows, n, k, 1) == lib.mllm_gemm_split_blocks_anywhere(m, n, k, 1)
+        assert rows <= 64 or lib.mllm_gemm_split_blocks_row_major(rows, n, k, 1) == lib.mllm_gemm_split_blocks_row_major(m, n, k, 1)
