@@ -770,17 +770,21 @@ __global__ __launch_bounds__(64 * LATENT_WAVES, 2) void latent_attention_mfma_ke
 // with a pair a lane and keys 8 g + 4 half + e in the registers, which is what the weighted sum O^T = C_latent^T P^T takes as its other operand if its step
 // (g, e) means key 8 g + e in one half of the lanes and 8 g + 4 + e in the other: weights never leave their registers. A key's latent is read four elements a
 // lane, an element for each of four output tiles (tile e of four: elements 128 j + 4 i + e).
+// The grid: more than eight requests lie side by side, and one that is none where their number is even, tile after tile. Blocks go to the eight XCDs in turn, so that
+// a request's tiles and the single tiles of many requests both lie on all of them then. With a request's tiles side by side 64 decoding requests beside prompts of 240
+// pairs, eight tiles, had theirs on one XCD: 64 tokens over 600 keys and 13 prompts of 20 130 -> 58 us, 100 prompts of 20 beside one of 600 280 -> 140. Few
+// requests stay request after request (six of 19 to 640, the longest first, 78 us and 84 tile after tile; six of 300 84 and 76).
 // Keys are asked for a chunk ahead of the products, behind scheduling borders: moved up further they would not fit 256 registers, which two waves a SIMD leave
 // each (one covers the other's softmax).
 // Rows of 288 floats, 12 heads, a wave a row (or shared) -> here: six prompts of 19 to 640 304 -> 119 us, one of 1,024 401 -> 87 (79 TFLOP/s of the instruction's 157).
-constexpr int LATENT_F32_KEYS = 32, LATENT_F32_WAVES = 8;
+constexpr int LATENT_F32_KEYS = 32, LATENT_F32_WAVES = 8, LATENT_F32_FEW_REQUESTS = 8;
 
 template <int DK>
 __global__ __launch_bounds__(64 * LATENT_F32_WAVES) void latent_attention_f32_mfma_kernel(
     const float* __restrict__ q, const float* __restrict__ pages, const float* __restrict__ sinks, float* __restrict__ out, float* __restrict__ parts,
     const int* __restrict__ token_request, int n_rows,
     const int* __restrict__ q_starts, const int* __restrict__ context_lens, const int* __restrict__ block_tables, int max_blocks,
-    int n_heads, int R, int page_size, float scale, int run_length) {
+    int n_heads, int R, int page_size, float scale, int run_length, int n_requests) {
     constexpr int D = 16 * DK, GROUPS = D / 8, CHUNK = GROUPS % 6 == 0 ? 6 : 4, CHUNKS = GROUPS / CHUNK;   // a group: a piece of four numbers in either half
     constexpr int FOURS = D > 128 ? 2 : 1;                                                              // times four output tiles of 32 latent elements (R <= 256)
     constexpr int Q_ROW = D + 4, SLOT_ROW = WAVE * 4 + 4;                                               // floats; padded by a piece
@@ -790,9 +794,17 @@ __global__ __launch_bounds__(64 * LATENT_F32_WAVES) void latent_attention_f32_mf
     __shared__ float wave_top[LATENT_F32_WAVES][32], wave_weight[LATENT_F32_WAVES][32];
     __shared__ int wave_endless[LATENT_F32_WAVES];
     const int lane = threadIdx.x % WAVE, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE), lane32 = lane % 32, half = lane / 32;
-    const int request = blockIdx.y, run = blockIdx.z, n_runs = gridDim.z;
+    const int run = blockIdx.z, n_runs = gridDim.z;
+    int request = blockIdx.y, tile = blockIdx.x, n_tiles = gridDim.x;
+    if (n_requests > LATENT_F32_FEW_REQUESTS) {
+        const int side_by_side = n_requests | 1, folds = gridDim.x / side_by_side;
+        request = blockIdx.x % side_by_side;
+        tile = blockIdx.y * folds + blockIdx.x / side_by_side;
+        n_tiles = gridDim.y * folds;
+        if (request >= n_requests) return;
+    }
     if (n_runs == 1 && request == 0) {   // rows of no request are zero, as above
-        for (int row0 = (blockIdx.x * LATENT_F32_WAVES + wave) * WAVE; row0 < n_rows; row0 += gridDim.x * LATENT_F32_WAVES * WAVE) {
+        for (int row0 = (tile * LATENT_F32_WAVES + wave) * WAVE; row0 < n_rows; row0 += n_tiles * LATENT_F32_WAVES * WAVE) {
             unsigned long long nobodys = __ballot(row0 + lane < n_rows && token_request[min(row0 + lane, n_rows - 1)] < 0);
             for (; nobodys; nobodys &= nobodys - 1) {
                 float* row = out + (size_t)(row0 + __builtin_ctzll(nobodys)) * n_heads * R;
@@ -803,7 +815,7 @@ __global__ __launch_bounds__(64 * LATENT_F32_WAVES) void latent_attention_f32_mf
     const int context = context_lens[request];
     if (context < 0) return;   // a padding request
     const int q_first = q_starts[request], q_len = q_starts[request + 1] - q_first;
-    const int pair0 = (gridDim.x - 1 - blockIdx.x) * 32, n_pairs = q_len * n_heads;   // (a portion's last pairs, which have the most keys, go first)
+    const int pair0 = (n_tiles - 1 - tile) * 32, n_pairs = q_len * n_heads;   // (a portion's last pairs, which have the most keys, go first)
     if (pair0 >= n_pairs) return;
     const int position = context + min((pair0 + lane32) / n_heads, q_len - 1);   // of this lane's pair
     const int* table = block_tables + (size_t)request * max_blocks;
@@ -998,17 +1010,23 @@ __global__ __launch_bounds__(64 * LATENT_F32_WAVES) void latent_attention_f32_mf
 
 struct LatentMfmaArgs {
     const float* q; const void* pages; const float* sinks; float* out; float* parts; const int* token_request; int n_rows;
-    const int* q_starts; const int* context_lens; const int* block_tables; int max_blocks, n_heads, R, page_size; float scale; int run_length; dim3 grid; hipStream_t stream;
+    const int* q_starts; const int* context_lens; const int* block_tables; int max_blocks, n_heads, R, page_size; float scale; int run_length, max_tiles, n_requests, n_runs; hipStream_t stream;
 };
 
 template <int DK>
 void launch_latent_mfma(const LatentMfmaArgs& a, int dtype) {
-    auto go = [&](auto kernel, auto pages, int waves) {
-        kernel<<<a.grid, 64 * waves, 0, a.stream>>>(a.q, pages, a.sinks, a.out, a.parts, a.token_request, a.n_rows, a.q_starts, a.context_lens, a.block_tables,
-                                                           a.max_blocks, a.n_heads, a.R, a.page_size, a.scale, a.run_length);
+    auto go = [&](auto kernel, auto pages, int waves, dim3 grid, auto... requests) {
+        kernel<<<grid, 64 * waves, 0, a.stream>>>(a.q, pages, a.sinks, a.out, a.parts, a.token_request, a.n_rows, a.q_starts, a.context_lens, a.block_tables,
+                                                  a.max_blocks, a.n_heads, a.R, a.page_size, a.scale, a.run_length, requests...);
     };
-    if (dtype == MLLM_F32) go(latent_attention_f32_mfma_kernel<DK>, (const float*)a.pages, LATENT_F32_WAVES);
-    else go(latent_attention_mfma_kernel<DK>, (const bf16_t*)a.pages, LATENT_WAVES);
+    if (dtype == MLLM_F32) {
+        // (where requests lie in the first dimension, tiles beyond what the second holds lie beside them)
+        const int folds = ceil_div(a.max_tiles, 65535);
+        const dim3 grid = a.n_requests > LATENT_F32_FEW_REQUESTS ? dim3((a.n_requests | 1) * folds, ceil_div(a.max_tiles, folds), a.n_runs) : dim3(a.max_tiles, a.n_requests, a.n_runs);
+        go(latent_attention_f32_mfma_kernel<DK>, (const float*)a.pages, LATENT_F32_WAVES, grid, a.n_requests);
+    } else {
+        go(latent_attention_mfma_kernel<DK>, (const bf16_t*)a.pages, LATENT_WAVES, dim3(a.max_tiles, a.n_requests, a.n_runs));
+    }
 }
 
 template <typename KernelT>
@@ -1185,7 +1203,7 @@ MLLM_API int mllm_latent_attention_mfma(const float* q, const void* pages, const
     if (n_rows == 0 || n_requests == 0) return 0;
     if (n_runs == 1) run_length = 1 << 30;
     LatentMfmaArgs a{q, pages, sinks, out, parts, token_request, n_rows, q_starts, context_lens, block_tables, max_blocks, n_heads, R, page_size, scale, run_length,
-                     dim3(ceil_div(max_pairs, 32), n_requests, n_runs), stream};
+                     ceil_div(max_pairs, 32), n_requests, n_runs, stream};
     mllm_count_kernel(MLLM_K_LATENT_ATTENTION);
     switch (D / 16) {
         case 2: launch_latent_mfma<2>(a, dtype); break;

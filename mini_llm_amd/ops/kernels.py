@@ -1069,15 +1069,18 @@ def heads_linear(x, weight, out, *, n_heads, k, x_head_stride, n_out=None, gate=
 
 
 LATENT_RUN_MIN = 64        # cached rows a run of a token's keys should at least hold: a tile of the kernel
-LATENT_TARGET_BLOCKS = 256   # blocks (four waves that share the keys of 32 pairs) the matrix-core kernel's launch should have before keys are left whole
-LATENT_BLOCK_RUN_MIN = 128   # and the cached rows its runs are multiples of there: what a block takes at a time
-# A 32-bit cache runs through the matrix-core kernel from so many (token, head) pairs on, if a sequence may be longer than so many keys. The kernel of a wave (or
-# block) a row / it, us, rows of 288 floats, 12 heads: a prompt of 128 19.0 / 19.5, of 260 39.0 / 37.0, of 640 136 / 57, of 1,024 401 / 87, six prompts of 19 to
-# 640 304 / 119; 6 heads over rows of 192: 260 (1,560 pairs) 24.7 / 30.1, 508 (3,048) 45 / 48, 640 62 / 41; 64 single tokens over 600 keys 37.5 / 32.7, 256 of
-# them 124 / 60. Short sequences leave seven of a block's eight waves without a tile: 100 prompts of 20 35 / 75, 256 single tokens over 60 keys 14.9 / 19.7, 64
-# portions of 8 over 60 37 / 20.
+LATENT_TARGET_BLOCKS = 256   # blocks (whose waves share the keys of 32 pairs) the matrix-core kernels' launch should have before keys are left whole
+LATENT_BLOCK_RUN_MIN = 128   # and the cached rows its runs are multiples of there: what a block of four waves takes at a time. (A 32-bit cache's has eight, but
+                             # from LATENT_F32_PAIRS pairs on there are two runs at the most, for sequences of 256 keys or more.)
+# A 32-bit cache runs through the matrix-core kernel from so many (token, head) pairs on, if a sequence may be longer than so many keys, and where none is twice as
+# long, portions of more than a few tokens bring so many rows a request. The kernel of a wave (or block) a row / it, us, rows of 288 floats, 12 heads: a prompt of 128
+# 19.0 / 19.5, of 260 38 / 37, of 640 136 / 57, of 1,024 401 / 87, six prompts of 19 to 640 304 / 119, 64 tokens over 600 keys beside 13 prompts of 20 65 / 58; 6
+# heads over rows of 192: 260 (1,560 pairs) 24.7 / 30.1, 508 (3,048) 45 / 48, 640 62 / 41; 64 single tokens over 600 keys 37.5 / 32.7, 256 of them 124 / 60, over
+# 200 49 / 31, 64 portions of 8 over 100 44 / 21. Short sequences leave seven of a block's eight waves without a tile: 100 prompts of 20 35 / 75, 256 single tokens
+# over 60 keys 14.9 / 19.7, 100 prompts of 20 beside one of 100 58 / 80, 30 of 10 to 60 beside one of 70 46 / 56 (rows of 192 22 / 33); 16 of 16 to 128 50 / 39 (30 / 34).
 LATENT_F32_PAIRS = 3072
 LATENT_F32_KEYS = 64
+LATENT_F32_ROWS = 48
 LATENT_TARGET_WAVES = 2048   # waves a launch should have before a token's keys are left whole (eight to a compute unit)
 
 
@@ -1092,6 +1095,13 @@ def latent_row_size(needed: int) -> int:
     return size if size else -(-int(needed) // 8) * 8
 
 
+def latent_f32_by_matrix(rows: int, n_heads: int, requests: int, max_q_len: int, longest: int) -> bool:
+    """Whether the latent attention over a 32-bit cache runs through the matrix-core kernel, if the row size does: what was measured stands at the constants."""
+    if rows * n_heads < LATENT_F32_PAIRS or longest <= LATENT_F32_KEYS:
+        return False
+    return longest > 2 * LATENT_F32_KEYS or max_q_len <= DECODE_MAX_Q_LEN or rows >= LATENT_F32_ROWS * requests
+
+
 def latent_attention(q_full, pages, sinks, token_request, positions, block_tables, rank, scale, max_len=None, q_starts=None, context_lens=None,
                      max_q_len=None):
     """Causal attention of each row's heads over its request's cached rows: score = scale * q_full[row, h] . cached row, softmax
@@ -1100,7 +1110,7 @@ def latent_attention(q_full, pages, sinks, token_request, positions, block_table
     rank]. Few rows with many keys are cut into runs of keys (``max_len``: the longest sequence of the batch).
     With ``q_starts`` ([requests + 1]: each request's rows are consecutive), ``context_lens`` ([requests]: the position of a
     request's first row; negative: a padding request) and ``max_q_len``, a cache of a row size the matrix-core kernels
-    take runs through them (32 (token, head) pairs of a request to a block; a 32-bit cache where LATENT_F32_PAIRS and LATENT_F32_KEYS say so)."""
+    take runs through them (32 (token, head) pairs of a request to a block; a 32-bit cache where ``latent_f32_by_matrix`` says so)."""
     _device_tensor(q_full, "q_full", torch.float32, 3)
     _device_tensor(pages, "pages", dim=4)
     n, n_heads, row_size = q_full.shape
@@ -1120,7 +1130,7 @@ def latent_attention(q_full, pages, sinks, token_request, positions, block_table
     reach = block_tables.shape[1] * page_size
     longest = reach if max_len is None else max(1, min(int(max_len), reach))
     if (q_starts is not None and context_lens is not None and max_q_len is not None
-            and (pages.dtype != torch.float32 or (n * n_heads >= LATENT_F32_PAIRS and longest > LATENT_F32_KEYS))
+            and (pages.dtype != torch.float32 or latent_f32_by_matrix(n, n_heads, context_lens.shape[0], int(max_q_len), longest))
             and lib.mllm_latent_attention_mfma_supported(int(rank), row_size, _code(pages.dtype))):
         _device_tensor(q_starts, "q_starts", torch.int32, 1)
         _device_tensor(context_lens, "context_lens", torch.int32, 1)

@@ -68,3 +68,13 @@ def test_cuts_along_k_of_bfloat16_products_of_many_rows(m, n, k, packed, row_maj
     for rows in (-(-m // 128) * 128, (m - 1) // 128 * 128 + 1):
         assert rows <= 64 or lib.mllm_gemm_split_blocks_anywhere(rows, n, k, 1) == lib.mllm_gemm_split_blocks_anywhere(m, n, k, 1)
         assert rows <= 64 or lib.mllm_gemm_split_blocks_row_major(rows, n, k, 1) == lib.mllm_gemm_split_blocks_row_major(m, n, k, 1)
+
+
+@pytest.mark.parametrize("rows,heads,requests,max_q_len,longest,by_matrix", [
+    (255, 12, 1, 255, 255, False), (256, 12, 1, 256, 256, True), (1024, 12, 1, 1024, 1024, True), (2000, 12, 100, 20, 20, False), (256, 12, 256, 1, 60, False),
+    (256, 12, 256, 1, 100, True), (512, 12, 64, 8, 100, True), (2100, 12, 101, 100, 100, False), (1154, 12, 30, 70, 70, False), (2600, 12, 101, 600, 600, True),
+    (324, 12, 77, 20, 600, True), (960, 12, 16, 128, 128, True)])
+def test_32_bit_latent_attention_by_matrix_instructions(rows, heads, requests, max_q_len, longest, by_matrix):
+    from mini_llm_amd.ops import kernels as K
+
+    assert K.latent_f32_by_matrix(rows, heads, requests, max_q_len, longest) == by_matrix

@@ -78,3 +78,36 @@ def test_32_bit_latent_attention_on_the_matrix_cores(monkeypatch, heads, rank, r
     assert got[first : first + place].isfinite().all()
     assert not got[first + place : first + portions[0], :, 5].isfinite().any()
     assert got[first + portions[0] : sum(portions)].isfinite().all()
+
+
+# one request, an even and an odd number of them, eight (the most of which a request's tiles lie side by side) and more, a padding one at the end and rows of no request; portions of one tile beside ones of several
+@pytest.mark.parametrize("contexts,portions", [([0], [70]), ([5], [1]), ([300, 0], [1, 40]), ([0, 90, 300], [33, 1, 2]), ([40, 0, 200, 7, 0, 150, 31, 9], [1, 30, 1, 1, 12, 1, 1, 1]),
+                                               ([130] * 10 + [0], [1] * 10 + [60])])
+@pytest.mark.parametrize("padding", [0, 1])
+def test_32_bit_latent_attention_finds_every_tile_of_every_request(monkeypatch, contexts, portions, padding):
+    from mini_llm_amd.ops import kernels as k
+
+    monkeypatch.setattr(k, "LATENT_F32_PAIRS", 1)
+    monkeypatch.setattr(k, "LATENT_F32_KEYS", 1)
+    heads, rank, size, page_size, scale = 6, 160, 192, 16, 0.1
+    generator = torch.Generator().manual_seed(len(contexts))
+    blocks = [-(-(c + p) // page_size) for c, p in zip(contexts, portions)]
+    pages = torch.randn(sum(blocks) + 1, 1, page_size, size, generator=generator)
+    order = torch.randperm(sum(blocks) + 1, generator=generator)
+    tables = torch.full((len(contexts) + padding, max(blocks)), -1, dtype=torch.int32)
+    for r, n in enumerate(blocks):
+        tables[r, :n] = order[sum(blocks[:r]) : sum(blocks[: r + 1])]
+    rows, spare = sum(portions), 5 * padding
+    owner = torch.cat([torch.full((p,), i) for i, p in enumerate(portions)] + [torch.full((spare,), -1)])
+    positions = torch.cat([torch.arange(c, c + p) for c, p in zip(contexts, portions)] + [torch.zeros(spare, dtype=torch.long)])
+    starts = torch.tensor([0] + [sum(portions[: i + 1]) for i in range(len(portions))] + [rows + spare] * padding)
+    q = torch.randn(rows + spare, heads, size, generator=generator)
+    ints = lambda t: t.int().cuda()
+    got = k.latent_attention(q.cuda(), pages.cuda(), None, ints(owner), ints(positions), ints(tables), rank, scale, max_len=max(c + p for c, p in zip(contexts, portions)),
+                             q_starts=ints(starts), context_lens=ints(torch.tensor(contexts + [-1] * padding)), max_q_len=max(portions)).cpu().double()
+    assert (got[rows:] == 0).all()
+    for r in range(len(contexts)):
+        mine = slice(int(starts[r]), int(starts[r + 1]))
+        cached = pages[tables[r, : blocks[r]].long()].reshape(-1, size)[: contexts[r] + portions[r]].double()
+        want = attend(q[mine].double(), cached, positions[mine], rank, scale, None)
+        assert (got[mine] - want).norm() / want.norm() < 1e-5   # (the bound above, for shorter rows)
