@@ -132,7 +132,7 @@ __global__ __launch_bounds__(256) void rms_norm_kernel(const float* __restrict__
 // lane before it can add anything up. A wave a row / a block a row, us, in 32-bit with a residual and a second norm: rows of 768, 8 of them 4.1 / 2.7 (two partial
 // products 4.2 / 3.0, five 5.1 / 3.1), 256 4.4 / 2.9, 2,048 6.3 / 5.9; rows of 1,600, 8 of them 6.2 / 2.9, 2,048 14.2 / 10.1; without either, rows of 768, 8 of
 // them 3.8 / 2.4, 2,048 4.8 / 4.1. What stays with a wave a row (block_a_row below): rows of up to 256, of which a wave asks for four numbers a lane and most of a block
-// has nothing to do (8 rows of 64 with five partial products 2.9 / 3.2, 64 of 256 with an addend 3.0 / 3.1); of up to 512, its eight numbers a lane, from some 512 rows on
+// has nothing to do (8 rows of 64 with five partial products 2.9 / 3.2, 64 of 256 with an addend 3.0 / 3.1; few of more than 128 without one do not: 2.8 / 2.5); of up to 512, its eight numbers a lane, from some 512 rows on
 // (512 of 512 with four 4.1 / 3.7, 768 with nine 4.6 / 5.1, 2,048 with one 4.6 / 5.7; behind 512 it asks for sixteen: 2,048 of 576 with four 0.87 of its time); and
 // thousands of rows with many partial products, which are bound by their bytes (32,768 rows of 768 with five 141 / 147; of 1,024, whose blocks are as large as 768's
 // and hold a third more, 2,048 with sixteen 24.4 / 27.0, 8,192 with eight 54.4 / 56.7; of 1,600, 8,192 with eight 124 / 103 the other way).
@@ -426,10 +426,12 @@ __global__ __launch_bounds__(256) void silu_mul_kernel(const T* __restrict__ bot
 
 }  // namespace
 
-// Whether so many rows take the kernel with a block a row, if their operands lie on their borders: the lines and what was measured are named there.
+// Whether so many rows, with so many partial products added (0: none), take the kernel with a block a row, if their operands lie on their borders: the lines and
+// what was measured are named there.
 MLLM_API int mllm_rms_norm_block_a_row(int n_rows, int width, int n_partials) {
     if (width % 4 != 0 || width > 2048 || n_rows > 16384) return 0;
-    if (width <= 512) return width > 256 && n_rows <= 512;
+    if (width <= 256) return width > 128 && n_partials == 0 && n_rows <= 256;
+    if (width <= 512) return n_rows <= 512;
     return width <= 768 || width > 1024 || n_partials < 8 || (long long)n_rows * n_partials < 32768;
 }
 
@@ -449,7 +451,7 @@ MLLM_API int mllm_rms_norm(const float* x, const void* y, int y_dtype, float alp
     mllm_count_kernel(MLLM_K_RMS_NORM);
     const size_t wide = (size_t)x | (size_t)weight | (size_t)residual | (size_t)next_weight | (size_t)stream_out | (y_dtype == MLLM_F32 ? (size_t)y : 0) |
                         (rows_dtype == MLLM_F32 ? (size_t)rows_out : 0) | (size_t)(partial_stride * (n_partials > 1 ? 4 : 0));
-    if (mllm_rms_norm_block_a_row(n_rows, width, n_partials) && wide % 16 == 0 && (((size_t)y | (size_t)rows_out) & 7) == 0) {
+    if (mllm_rms_norm_block_a_row(n_rows, width, y ? n_partials : 0) && wide % 16 == 0 && (((size_t)y | (size_t)rows_out) & 7) == 0) {
 #define LAUNCH(THREADS) rms_norm_row_kernel<THREADS><<<n_rows, THREADS, 0, stream>>>(x, y, y_dtype, alpha, row_index, weight, one_plus, eps, stream_out, rows_out, rows_dtype, width, n_partials, partial_stride, residual, next_weight)
         if (width <= 1024) LAUNCH(256);
         else LAUNCH(512);

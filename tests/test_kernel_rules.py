@@ -18,7 +18,7 @@ def test_waves_of_the_decode_attention(rows, heads, keys, key_bytes, best):
 
 @pytest.mark.parametrize("rows,width,partials,block", [
     # measured: which is faster, a block or a wave a row
-    (8, 64, 5, 0), (256, 60, 1, 0), (64, 256, 1, 0), (64, 320, 1, 1), (256, 384, 9, 1), (512, 512, 4, 1), (768, 512, 9, 0), (2048, 512, 1, 0), (8192, 512, 8, 0),
+    (8, 64, 5, 0), (256, 60, 1, 0), (64, 256, 1, 0), (64, 256, 0, 1), (257, 256, 0, 0), (8, 64, 0, 0), (8, 768, 0, 1), (64, 320, 1, 1), (256, 384, 9, 1), (512, 512, 4, 1), (768, 512, 9, 0), (2048, 512, 1, 0), (8192, 512, 8, 0),
     (2048, 576, 4, 1), (8, 768, 1, 1), (8192, 768, 16, 1), (32768, 768, 5, 0), (8192, 1024, 5, 1), (8192, 1024, 8, 0), (2048, 1024, 9, 1), (2048, 1024, 16, 0),
     (8192, 1600, 16, 1), (8192, 2048, 8, 1),
     # what the kernel does not take

@@ -6,7 +6,7 @@ import torch
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("rows,width", [(1, 4), (3, 60), (257, 512), (5, 1024), (300, 1028), (2, 2048), (9, 2052), (7, 770)])
+@pytest.mark.parametrize("rows,width", [(1, 4), (3, 60), (9, 132), (64, 256), (257, 512), (5, 1024), (300, 1028), (2, 2048), (9, 2052), (7, 770)])
 @pytest.mark.parametrize("partials", [0, 1, 2, 4, 5, 9])
 @pytest.mark.parametrize("out_dtype", [torch.float32, torch.bfloat16])
 def test_norm_of_a_row_by_a_block(rows, width, partials, out_dtype):
