@@ -60,9 +60,11 @@ class BranchProduct:
     or, where few rows meet few output columns and a long K (the library says: ``kernels.split_blocks``), cut along K into
     partial products [n, rows, out] that the norm adds up on its way in. With a residual the sum is taken inside the product, and
     so is a bias's.
-    Up to FEW_ROWS rows only a long K is cut (``cut_few_rows``): a short one loses more to the norm's further loads than the product saves. With the norm
+    Up to FEW_ROWS rows only a long K is cut (``cut_few_rows``), where the product saves more than the norm's further loads cost in either precision. With the norm
     behind it, whole / cut, us: 8 rows in 32-bit 768 x 768 7.3 / 6.8, 1,600 x 1,024 8.0 / 8.1, 768 x 2,048 10.0 / 8.1, 1,600 x 2,048 10.7 / 9.2; in bfloat16
-    768 x 768 5.5 / 5.9, 768 x 2,048 7.1 / 6.5, 1,600 x 2,048 7.3 / 7.5, 1,600 x 3,072 8.1 / 7.7; a single row 0.2 to 0.5 less of a gain."""
+    768 x 768 5.5 / 5.9, 768 x 2,048 7.1 / 6.5, 1,600 x 2,048 7.3 / 7.5, 1,600 x 3,072 8.1 / 7.7; a single row 0.2 to 0.5 less of a gain. (The first of these, a
+    short K in 32-bit over few columns, would gain too and stays whole.) Callers that add the partial products up themselves (``later``, and whoever
+    asks ``blocks``) leave up to FEW_ROWS rows whole: measured with the norm alone."""
 
     FEW_ROWS = 16
 
@@ -77,7 +79,7 @@ class BranchProduct:
         return k >= 1536 if dtype == torch.float32 else k >= (2048 if n <= 1024 else 3072)
 
     def blocks(self, x, weight) -> int:
-        """Into how many partial products the product of these rows is cut (1: it stays whole, as all of up to FEW_ROWS rows do)."""
+        """Into how many partial products a caller that adds them up itself should cut the product of these rows (1: it stays whole, as up to FEW_ROWS rows do)."""
         return 1 if x.shape[0] <= self.FEW_ROWS else self._blocks(x, weight)
 
     def _blocks(self, x, weight) -> int:
