@@ -424,8 +424,11 @@ DECODE_TARGET_WAVES = 4096  # the most waves a launch should have: 16 to each of
 # 8 rows of 64 keys 4.1 / 4.3 / 4.9 / 4.9 / 6.2, of 128 5.3 / 4.6 / 5.1 / 5.1 / 6.3, of 200 8.6 / 6.6 / 6.0 / 6.0 / 7.1, of 300 10.2 / 8.1 / 7.4 / 6.8 / 7.9, of 500
 # 14.3 / 9.9 / 8.1 / 7.2 / 8.4, of 900 23.1 / 15.6 / 11.4 / 9.1 / 10.1, of 1,500 41.5 / 26.1 / 18.3 / 14.3 / 15.2, of 3,000 78.5 / 49.8 / 32.3 / 25.1 / 24.8; one
 # row of 128 5.1 / 4.4 / 4.8 / 4.9 / 6.0, of 500 11.9 / 8.1 / 6.6 / 5.9 / 7.0; in 32-bit 8 rows of 900 44.8 / 27.4 / 23.7 / 19.6 / 18.0. (A captured step's run is
-# as long as the cache may become, and its waves the same however few keys there are yet.)
+# as long as the cache may become, and its waves the same however few keys there are yet.) Keys that are cut into runs are many or may become so: a wave takes 16 KiB of
+# a run at least, four of 512 keys. One row in two runs of 512, 12 heads, us with 4 / 8 waves: 128 keys 6.6 / 6.9, 300 6.8 / 7.1, 900 8.5 / 8.1; in eight, 500 keys 8.6 /
+# 9.0, 1,500 9.3 / 9.5; in two of 750 11.0 / 10.2 (eight).
 DECODE_MIN_SPLIT = 64
+DECODE_MIN_CUT_BYTES = 16 * 1024
 DECODE_WIDE_BYTES = 192 * 1024
 DECODE_MAX_SPLITS = 16      # waves per block
 DECODE_COMMON_SPLITS = 8    # and of a run that holds less than DECODE_WIDE_BYTES
@@ -459,11 +462,12 @@ def _arrivals(k_pages, rows: int, n_heads: int):
     return counters
 
 
-def decode_waves(blocks: int, keys: int, key_bytes: int) -> int:
-    """Waves a block of the decode attention for so many blocks, each with up to ``keys`` keys of ``key_bytes`` bytes."""
+def decode_waves(blocks: int, keys: int, key_bytes: int, cut: bool = False) -> int:
+    """Waves a block of the decode attention for so many blocks, each with up to ``keys`` keys of ``key_bytes`` bytes (``cut``: a run of a token's)."""
+    least = max(DECODE_MIN_SPLIT, DECODE_MIN_CUT_BYTES // key_bytes) if cut else DECODE_MIN_SPLIT
     most = DECODE_MAX_SPLITS if keys * key_bytes >= DECODE_WIDE_BYTES else DECODE_COMMON_SPLITS
     waves = 1
-    while waves < most and 2 * blocks * waves <= DECODE_TARGET_WAVES and waves * DECODE_MIN_SPLIT < keys:
+    while waves < most and 2 * blocks * waves <= DECODE_TARGET_WAVES and waves * least < keys:
         waves *= 2
     return waves
 
@@ -550,7 +554,7 @@ def paged_attention(q, k_pages, v_pages, token_request, positions, block_tables,
         while n_parts < DECODE_MAX_PARTS and 2 * n * n_heads * n_parts <= units and 2 * n_parts * min_part <= reach:
             n_parts *= 2
         part_reach = -(-reach // n_parts)
-        n_splits = decode_waves(n * n_heads * n_parts, part_reach, head_size * q.element_size())
+        n_splits = decode_waves(n * n_heads * n_parts, part_reach, head_size * q.element_size(), cut=n_parts > 1)
         result = out
         if packed_out:
             result = empty_packed_rows(n, width, q.dtype, q.device)

@@ -16,6 +16,13 @@ def test_waves_of_the_decode_attention(rows, heads, keys, key_bytes, best):
     assert K.decode_waves(rows * heads, keys, key_bytes) in best
 
 
+@pytest.mark.parametrize("runs,keys,key_bytes,best", [(2, 512, 128, {4, 8}), (8, 512, 128, {4}), (2, 750, 128, {8}), (4, 750, 128, {8}), (2, 512, 256, {8})])
+def test_waves_of_the_decode_attention_of_one_row_in_runs(runs, keys, key_bytes, best):
+    from mini_llm_amd.ops import kernels as K
+
+    assert K.decode_waves(12 * runs, keys, key_bytes, cut=True) in best
+
+
 @pytest.mark.parametrize("rows,width,partials,block", [
     # measured: which is faster, a block or a wave a row
     (8, 64, 5, 0), (256, 60, 1, 0), (64, 256, 1, 0), (64, 256, 0, 1), (257, 256, 0, 0), (8, 64, 0, 0), (8, 768, 0, 1), (64, 320, 1, 1), (256, 384, 9, 1), (512, 512, 4, 1), (768, 512, 9, 0), (2048, 512, 1, 0), (8192, 512, 8, 0),
