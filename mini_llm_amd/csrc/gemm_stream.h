@@ -670,11 +670,13 @@ inline Shape choose(int M, int N, int K, int k_blocks, bool bf16_out) {
     // each 64 x 64 tile along K have half the reads of A's rows under way at a time: the better for a long K whose rows lie whole multiples of 8 KiB apart, where the
     // rows of a load meet in the same channels of memory (K of 4,096, us, four stages / shared: 65 rows of 1,024 20.0 / 19.0, 300 20.6 / 20.0, 1,500 22.4 / 22.0; K of
     // 8,192 0.95 of its time; of 3,072, 3,584, 5,632 and 6,400 from 128 rows on 1.01 to 1.02), or of little more than half a tile of rows (65 rows, K of 3,072 to 6,400:
-    // 0.97 to 0.92); short ones lose by it (K of 768 1.08, of 1,600 1.02, of 2,560 1.03).
+    // 0.97 to 0.92); short ones lose by it (K of 768 1.08, of 1,600 1.02, of 2,560 1.03), and a round that is nearly full has its memory busy as it is (2,048 x 1,024 x
+    // 4,096, 256 blocks, 25.4 / 25.2 alone, and a pass of the medium shape's prompts, which takes it 24 times a step, 0.1 % longer).
     // In more rounds, which take outputs of up to 64 columns and many thousand rows, three stages leave room for two blocks a compute unit (65,536 x 64 x 768 20.3 us,
     // with four stages 23.7; x 2,048 44.6, 46.2, shared 47.6).
-    if ((long)ceil_div(M, 128) * ceil_div(N, 64) * k_blocks > 256) return S128x64_ROUNDS;
-    return ceil_div(K, k_blocks) >= 3072 && (K % 4096 == 0 || M <= 96) ? S128x64_SHARED : S128x64;
+    const long blocks = (long)ceil_div(M, 128) * ceil_div(N, 64) * k_blocks;
+    if (blocks > 256) return S128x64_ROUNDS;
+    return ceil_div(K, k_blocks) >= 3072 && ((K % 4096 == 0 && blocks <= 192) || M <= 96) ? S128x64_SHARED : S128x64;
 }
 
 template <typename OutT>

@@ -50,7 +50,7 @@ def test_every_tile_of_the_streaming_product_has_a_shape_in_its_test():
 
 @pytest.mark.parametrize("m,n,k,out,tile", [
     # a long K in one round of narrow tiles: shared where measured faster (see the kernel's rule)
-    (65, 1024, 4096, 0, 1280641), (1500, 1024, 4096, 0, 1280641), (300, 2048, 8192, 1, 1280641), (65, 1600, 6400, 1, 1280641), (128, 1600, 6400, 0, 1280640),
+    (65, 1024, 4096, 0, 1280641), (1500, 1024, 4096, 0, 1280641), (300, 2048, 8192, 1, 1280641), (2048, 1024, 4096, 0, 1280640), (65, 1600, 6400, 1, 1280641), (128, 1600, 6400, 0, 1280640),
     (2048, 768, 3072, 0, 1280640), (300, 768, 2048, 0, 1280640), (65, 768, 2048, 0, 1280640),
     # many rounds
     (16384, 1600, 6400, 0, 2561280), (65536, 64, 768, 0, 1280642)])
