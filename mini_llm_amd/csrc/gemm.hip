@@ -863,6 +863,14 @@ MLLM_API int mllm_gemm_stream_tile(int M, int N, int K, int k_blocks, int out_dt
     return tiles[stream::choose(M, N, K, k_blocks, out_dtype == MLLM_BF16)];
 }
 
+// The tile of outputs with which a 32-bit product of M rows and a W packed with its pieces runs, in k_blocks parts along K: 1,000 times its rows and its columns. 0: another kernel.
+MLLM_API int mllm_gemm_pieces_tile(int M, int N, int K, int k_blocks) {
+    if (M <= 0 || N <= 0 || K <= 0 || k_blocks < 1 || !pieces::takes_sizes(M, N, K, ceil_div(N, 16), PACKED_WITH_PIECES)) return 0;
+    int best = 0;
+    pieces::cost(M, N, K, k_blocks, best);
+    return pieces::CHOICES[best].bm * 1000 + pieces::CHOICES[best].bn;
+}
+
 // x_packed: A is in the packed layout of an [M, K] matrix; out_packed: out is written in the packed
 // layout of an [M, N] matrix (no residual then). Both only where mllm_gemm_takes_packed_rows says so.
 MLLM_API int mllm_gemm(const void* A, const void* W, int w_packed, const float* bias, const float* residual,

@@ -13,10 +13,15 @@
 //
 // W's pieces are laid out once, when the matrix is packed (common.h: packed_pieces): the chunks of the packed layout for bfloat16, the three of a k-step
 // behind each other. A's rows come as they are, and a wave splits the fragments it has read.
-// A block of four waves owns BM x BN outputs and walks K in tiles of 32: rows of A and chunks of W go from memory straight into LDS
-// (global_load_lds_dwordx4), one tile ahead of the products, in two stages. The stages leave room for two blocks a compute unit: one's splitting,
-// fragment reads and barriers run under the other's products. Fragment reads are inline assembly with waits of their own: through the compiler each
-// would wait for the loads into LDS that are under way.
+// A block of four waves owns BM x BN outputs and walks K in tiles of 32, two steps of 16: rows of A and chunks of W go from memory straight into LDS
+// (global_load_lds_dwordx4), one tile ahead of the products, in two stages, which leave room for two blocks a compute unit (a third stage and one block: 2,048 x 2,304 x 768
+// with 128 x 128 58 -> 69 us). What bounds it: the matrix cores, and beside them the chip's power. A SIMD runs a wave's vector instructions under its own matrix instructions
+// only where they stand between them: 24 products behind the splitting of their rows take 2,101 cycles a tile, with the splitting of the next step's rows between them
+// 1,609, and two waves a SIMD, each in two such halves, 1,860 each. So a step's products carry the splitting of the next step's rows, its fragment reads, and one by one
+// the loads of the tile after the next (a compute unit takes a load of 1 KiB every 16 cycles, and a wave that asks for all at once waits).
+// With the loads at a tile's start and the splitting in front of its products (us -> now): 2,048 x 2,304 x 768 56.2 -> 48.4 (128 x 96), 2,048 x 3,072 x 768 65.9 -> 60,
+// 2,670 x 768 x 3,072 in two 81.8 -> 70.5, 8,192 x 3,072 x 768 212 -> 203.
+// Fragment reads are inline assembly with waits of their own: through the compiler each would wait for the loads into LDS that are under way.
 #pragma once
 
 namespace pieces {
@@ -37,28 +42,31 @@ __device__ __forceinline__ void ask(i32x4& to, unsigned address) {
 __device__ __forceinline__ void landed(i32x4& first) { asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(first)); }
 __device__ __forceinline__ void this_too(i32x4& fragment) { asm volatile("" : "+v"(fragment)); }
 
-// Eight numbers -> three operands of pieces. (A number that the first rounding makes infinite leaves sums that are not finite, as an infinity does.)
-__device__ __forceinline__ void split(const i32x4 (&raw)[2], bf16x8 (&out)[3]) {
+// until at most LEFT of the wave's LDS reads, the newest, are under way
+template <int LEFT>
+__device__ __forceinline__ void landed_but(i32x4& first) { asm volatile("s_waitcnt lgkmcnt(%1)" : "+v"(first) : "n"(LEFT)); }
+// until at most LEFT of its loads from memory are
+template <int LEFT>
+__device__ __forceinline__ void wait_but() {
+    static_assert(LEFT < 64, "the loads in flight fit the counter");
+    __builtin_amdgcn_s_waitcnt((LEFT & 0xF) | ((LEFT >> 4) << 14) | (0x7 << 4) | (0xF << 8));
+}
+
+// Numbers 2 e and 2 e + 1 of a lane's eight -> their places in three operands of pieces. (A number that the first rounding makes infinite leaves sums that are not finite, as an infinity does.)
+__device__ __forceinline__ void split_pair(const i32x4 (&raw)[2], int e, bf16x8 (&out)[3]) {
     typedef float f32x2 __attribute__((ext_vector_type(2)));
     typedef bf16_t bf16x2 __attribute__((ext_vector_type(2)));
-    float rest[8];
-#pragma unroll
-    for (int e = 0; e < 8; e++) {
-        const int bits = raw[e / 4][e % 4];
-        rest[e] = __builtin_bit_cast(float, bits);
-    }
+    const int first = raw[e / 2][e % 2 * 2], second = raw[e / 2][e % 2 * 2 + 1];
+    float rest[2] = {__builtin_bit_cast(float, first), __builtin_bit_cast(float, second)};
 #pragma unroll
     for (int p = 0; p < 3; p++) {
-        uint32_t pairs[4];
-#pragma unroll
-        for (int e = 0; e < 4; e++) {
-            pairs[e] = __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2{rest[2 * e], rest[2 * e + 1]}), bf16x2));
-            if (p < 2) {
-                rest[2 * e] -= __builtin_bit_cast(float, pairs[e] << 16);
-                rest[2 * e + 1] -= __builtin_bit_cast(float, pairs[e] & 0xffff0000u);
-            }
+        const bf16x2 pair = __builtin_convertvector((f32x2{rest[0], rest[1]}), bf16x2);
+        out[p][2 * e] = pair[0], out[p][2 * e + 1] = pair[1];
+        if (p < 2) {
+            const uint32_t bits = __builtin_bit_cast(uint32_t, pair);
+            rest[0] -= __builtin_bit_cast(float, bits << 16);
+            rest[1] -= __builtin_bit_cast(float, bits & 0xffff0000u);
         }
-        out[p] = *reinterpret_cast<bf16x8*>(pairs);
     }
 }
 
@@ -72,8 +80,8 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N, 2) void gemm_pieces_kernel(
                                                                                int epilogue, CacheScatter scatter, int k_per_block, Group group) {
     constexpr int WAVES = WAVES_M * WAVES_N, STAGE = stage_bytes<BM, BN>(), A_BYTES = BM * BK * 4;
     constexpr int WM = BM / WAVES_M, WN = BN / WAVES_N, TM = WM / 32, TN = WN / 32;
-    constexpr int A_LOADS = BM / 8 / WAVES, W_CHUNKS = BN / 16 * 3, W_LOADS = W_CHUNKS / WAVES;
-    static_assert(TM >= 1 && TN >= 1 && BM / 8 % WAVES == 0 && W_CHUNKS % WAVES == 0, "every wave asks for as much");
+    constexpr int A_LOADS = BM / 8 / WAVES, W_CHUNKS = BN / 16 * 3, W_LOADS = (W_CHUNKS + WAVES - 1) / WAVES;
+    static_assert(TM >= 1 && TN >= 1 && BM / 8 % WAVES == 0, "every wave asks for as much");   // (of W's chunks the last may be asked for twice)
     extern __shared__ __attribute__((aligned(16))) unsigned char piece_lds[];
     const int lane = threadIdx.x % WAVE, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
     const int wave_m = wave / WAVES_N, wave_n = wave % WAVES_N, half = lane / 32, lane32 = lane % 32;
@@ -104,20 +112,22 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N, 2) void gemm_pieces_kernel(
     }
 #pragma unroll
     for (int l = 0; l < W_LOADS; l++) {
-        const int chunk = wave + l * WAVES, row_tile = first_tile + min(n0 / 16 + chunk / 3, row_tiles - 1);
+        const int chunk = min(wave + l * WAVES, W_CHUNKS - 1), row_tile = first_tile + min(n0 / 16 + chunk / 3, row_tiles - 1);
         w_from[l] = ((unsigned)row_tile * (unsigned)k_steps * 3u + (unsigned)(chunk % 3)) * 1024u + lane * 16u;
     }
+    const int tiles = (k_end - k_begin + BK - 1) / BK;
     const unsigned char *a_tile = reinterpret_cast<const unsigned char*>(A + k_begin), *w_tile = w_pieces + (size_t)(k_begin / BK) * 3072;
-    auto issue = [&](int stage) {   // the next tile
-        unsigned char* place = piece_lds + stage * STAGE;
-#pragma unroll
-        for (int l = 0; l < A_LOADS; l++)
+    constexpr int LOADS = A_LOADS + W_LOADS;
+    // load `l` of the tile a_tile and w_tile stand at, into the stage that begins at `stage`
+    auto issue_load = [&](int l, unsigned stage) {
+        if (l < A_LOADS)
             __builtin_amdgcn_global_load_lds((const void __attribute__((address_space(1)))*)(a_tile + a_from[l]),
-                                             (void __attribute__((address_space(3)))*)(place + (wave + l * WAVES) * 1024), 16, 0, 0);
-#pragma unroll
-        for (int l = 0; l < W_LOADS; l++)
-            __builtin_amdgcn_global_load_lds((const void __attribute__((address_space(1)))*)(w_tile + w_from[l]),
-                                             (void __attribute__((address_space(3)))*)(place + A_BYTES + (wave + l * WAVES) * 1024), 16, 0, 0);
+                                             (void __attribute__((address_space(3)))*)(piece_lds + stage + (wave + l * WAVES) * 1024), 16, 0, 0);
+        else
+            __builtin_amdgcn_global_load_lds((const void __attribute__((address_space(1)))*)(w_tile + w_from[l - A_LOADS]),
+                                             (void __attribute__((address_space(3)))*)(piece_lds + stage + A_BYTES + min(wave + (l - A_LOADS) * WAVES, W_CHUNKS - 1) * 1024), 16, 0, 0);
+    };
+    auto next_tile = [&] {
         a_tile += BK * 4;
         w_tile += 3072;
     };
@@ -138,63 +148,128 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N, 2) void gemm_pieces_kernel(
         const TileRows rows = reinterpret_cast<const TileRows*>(w_pieces + packed_pieces_bytes(matrix_tiles, K))[first_tile + min((n0 + wave_n * WN) / 16 + t, row_tiles - 1)];
         w_tiny |= rows.tiny, w_largest = max(w_largest, rows.largest);
     }
-    const int tiles = (k_end - k_begin + BK - 1) / BK;
 #pragma unroll
     for (int j = 0; j < TN; j++)
 #pragma unroll
         for (int i = 0; i < TM; i++)
 #pragma unroll
             for (int v = 0; v < 16; v++) acc[j][i][v] = low[j][i][v] = 0.0f;
-    if (tiles > 0) issue(0);
-    for (int t = 0; t < tiles; t++) {
-        // this wave's loads of the tile have landed; behind the barrier everybody's have, and nobody reads the other stage any more
-        __builtin_amdgcn_s_waitcnt(0);
-        __builtin_amdgcn_s_barrier();
-        __builtin_amdgcn_sched_barrier(0);
-        if (t + 1 < tiles) issue((t + 1) & 1);
-        const unsigned stage = (t & 1) * STAGE;
-        i32x4 raw[2][TM][2], w[2][3][TN];
-        auto ask_step = [&](auto step) {
+    if (tiles > 0) {
+        i32x4 raw[TM][2], w_high[2][TN], w_low[2][TN];   // the next step's rows; W's first pieces of this step and the next; its second and third pieces
+        bf16x8 a[2][TM][3];                              // the pieces of this step's rows, and of the next one's
+        using std::integral_constant;
+        // reads of a step (kk: the first or second sixteen numbers of K of the tile in the stage)
+        auto ask_rows = [&](auto step, unsigned stage) {
             constexpr int kk = decltype(step)::value;
             stream::static_for<TM>([&](auto i) {
-                ask<i * 32 * 128>(raw[kk][i][0], a_at[kk][0] + stage);
-                ask<i * 32 * 128>(raw[kk][i][1], a_at[kk][1] + stage);
+                ask<i * 32 * 128>(raw[i][0], a_at[kk][0] + stage);
+                ask<i * 32 * 128>(raw[i][1], a_at[kk][1] + stage);
             });
-            stream::static_for<3>([&](auto p) { stream::static_for<TN>([&](auto j) { ask<j * 2 * 3072 + p * 1024 + kk * 512>(w[kk][p][j], w_at + stage); }); });
         };
-        auto wait_step = [&](int kk) {
-            landed(raw[kk][0][0]);
-#pragma unroll
-            for (int i = 0; i < TM; i++) this_too(raw[kk][i][0]), this_too(raw[kk][i][1]);
-#pragma unroll
-            for (int p = 0; p < 3; p++)
-#pragma unroll
-                for (int j = 0; j < TN; j++) this_too(w[kk][p][j]);
+        auto ask_columns = [&](auto step, auto piece, unsigned stage) {
+            constexpr int kk = decltype(step)::value, p = decltype(piece)::value;
+            stream::static_for<TN>([&](auto j) { ask<j * 2 * 3072 + p * 1024 + kk * 512>(p == 0 ? w_high[kk][j] : w_low[p - 1][j], w_at + stage); });
         };
-        bf16x8 a[2][TM][3];
-        auto multiply = [&](int kk) {
-            constexpr int OF_A[6] = {2, 0, 1, 1, 0, 0}, OF_W[6] = {0, 2, 1, 0, 1, 0};   // the smallest products first
+        auto rows_here = [&] {
 #pragma unroll
-            for (int c = 0; c < 6; c++)
-#pragma unroll
-                for (int i = 0; i < TM; i++)
-#pragma unroll
-                    for (int j = 0; j < TN; j++) {
-                        f32x16& to = c < 5 ? low[j][i] : acc[j][i];
-                        to = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*reinterpret_cast<const bf16x8*>(&w[kk][OF_W[c]][j]), a[kk][i][OF_A[c]], to, 0, 0, 0);
-                    }
+            for (int i = 0; i < TM; i++) this_too(raw[i][0]), this_too(raw[i][1]);
         };
-        ask_step(std::integral_constant<int, 0>{});
-        wait_step(0);
-        ask_step(std::integral_constant<int, 1>{});
+        auto columns_here = [&](i32x4 (&columns)[TN]) {
+#pragma unroll
+            for (int j = 0; j < TN; j++) this_too(columns[j]);
+        };
+        constexpr integral_constant<int, 0> zero;
+        constexpr integral_constant<int, 1> one;
+        constexpr integral_constant<int, 2> two;
+
+        // The products of two pieces in a step: those of W's third and second piece first, whose registers are then free for the next step's.
+        constexpr int OF_A[6] = {0, 1, 0, 2, 1, 0}, OF_W[6] = {2, 1, 1, 0, 0, 0}, EACH = TM * TN, PAIRS = TM * 4;
+        auto products = [&](auto step, auto from, auto count, auto&& behind) {   // `count` of them from the one numbered `from`; behind(n): what goes behind product n
+            constexpr int kk = decltype(step)::value;
+            stream::static_for<decltype(count)::value>([&](auto n) {
+                constexpr int at = decltype(from)::value + decltype(n)::value, c = at / EACH, i = at % EACH / TN, j = at % TN, p = OF_W[c];
+                const i32x4& columns = p == 0 ? w_high[kk][j] : w_low[p == 0 ? 0 : p - 1][j];
+                f32x16& to = c < 5 ? low[j][i] : acc[j][i];
+                to = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*reinterpret_cast<const bf16x8*>(&columns), a[kk][i][OF_A[c]], to, 0, 0, 0);
+                behind(integral_constant<int, at>{});
+                __builtin_amdgcn_sched_barrier(0);
+            });
+        };
+        // 64 x 64: few products to put a tile's loads between, and few loads: they go out together, and the blocks that are alone on a unit wait less for them
+        constexpr bool AT_ONCE = EACH == 1;
+        // One step: its products, and under them the reads of the next step, the splitting of its rows and, in a tile's second step, the loads of a tile further on.
+        auto step = [&](auto which, auto with_loads, unsigned here, unsigned behind) {   // where this tile's stage begins, and the next one's
+            constexpr int kk = decltype(which)::value;
+            constexpr bool loads = kk == 1 && decltype(with_loads)::value;
+            constexpr integral_constant<int, 1 - kk> next;
+            const unsigned stage = kk == 0 ? here : behind;   // of the next step
+            landed(w_high[kk][0]);
+            columns_here(w_high[kk]), columns_here(w_low[0]), columns_here(w_low[1]);
+            if constexpr (kk == 1) {
+                // every read of this tile has landed, and this wave's loads of the next one: behind the barrier everybody's have, and this tile's stage is free
+                wait_but<0>();
+                __builtin_amdgcn_s_barrier();
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            ask_rows(next, stage);
+            ask_columns(next, zero, stage);
+            if constexpr (loads && AT_ONCE) stream::static_for<LOADS>([&](auto l) { issue_load(decltype(l)::value, here); });
+            __builtin_amdgcn_sched_barrier(0);
+            products(which, integral_constant<int, 0>{}, integral_constant<int, EACH>{}, [](auto) {});
+            ask_columns(next, two, stage);
+            landed_but<2 * TN>(raw[0][0]);
+            rows_here();
+            __builtin_amdgcn_sched_barrier(0);
+            auto under = [&](auto n) {   // the share of product n of the 5 EACH that are left
+                constexpr int at = decltype(n)::value - EACH, OF = 5 * EACH;
+                stream::static_for<(at + 1) * PAIRS / OF - at * PAIRS / OF>([&](auto p) {
+                    constexpr int pair = at * PAIRS / OF + decltype(p)::value, i = pair / 4, e = pair % 4;
+                    split_pair(raw[i], e, a[1 - kk][i]);
+                });
+                if constexpr (loads && !AT_ONCE)
+                    stream::static_for<(at + 1) * LOADS / OF - at * LOADS / OF>([&](auto l) { issue_load(at * LOADS / OF + decltype(l)::value, here); });
+            };
+            products(which, integral_constant<int, EACH>{}, integral_constant<int, 2 * EACH>{}, under);
+            ask_columns(next, one, stage);
+            __builtin_amdgcn_sched_barrier(0);
+            products(which, integral_constant<int, 3 * EACH>{}, integral_constant<int, 3 * EACH>{}, under);
+            if constexpr (loads) next_tile();
+        };
+        auto issue = [&](unsigned stage) {
+#pragma unroll
+            for (int l = 0; l < LOADS; l++) issue_load(l, stage);
+            next_tile();
+        };
+        issue(0);
+        wait_but<0>();
+        stream::wait_lgkmcnt<0>();   // (kernel arguments: a scalar load under way would count among the reads below)
+        __builtin_amdgcn_s_barrier();
         __builtin_amdgcn_sched_barrier(0);
+        ask_rows(zero, 0);
+        ask_columns(zero, zero, 0);
+        ask_columns(zero, one, 0);
+        ask_columns(zero, two, 0);
+        if (tiles > 1) issue(STAGE);
+        landed_but<3 * TN>(raw[0][0]);
+        rows_here();
 #pragma unroll
-        for (int i = 0; i < TM; i++) split(raw[0][i], a[0][i]);
-        multiply(0);
-        wait_step(1);
+        for (int i = 0; i < TM; i++)
 #pragma unroll
-        for (int i = 0; i < TM; i++) split(raw[1][i], a[1][i]);
-        multiply(1);
+            for (int e = 0; e < 4; e++) split_pair(raw[i], e, a[0][i]);
+        __builtin_amdgcn_sched_barrier(0);
+        unsigned here = 0;
+        auto tile = [&](auto with_loads) {
+            step(zero, with_loads, here, STAGE - here);
+            step(one, with_loads, here, STAGE - here);
+            here = STAGE - here;
+        };
+        int t = 0;
+        for (; t + 2 < tiles; t++) tile(std::true_type{});
+        for (; t < tiles; t++) tile(std::false_type{});
+        // what was asked for last, from a stage that holds no further tile, is never used, but on its way into registers that must not be given away yet
+        landed(w_high[0][0]);
+        columns_here(w_high[0]), columns_here(w_low[0]), columns_here(w_low[1]);
+        rows_here();
     }
 
 #pragma unroll
@@ -320,9 +395,9 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N, 2) void gemm_pieces_kernel(
             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
 #pragma unroll
             for (int r = 0; r < 32 / ROWS; r++) {
-                const int in_slab = r * ROWS + lane / LANES_A_ROW, row = row0 + i * 32 + in_slab;
+                const int in_slab = r * ROWS + min(lane / LANES_A_ROW, ROWS - 1), row = row0 + i * 32 + in_slab;
                 f32x4 value = *reinterpret_cast<const f32x4*>(slab + in_slab * SLAB_ROW + (lane % LANES_A_ROW) * 4);
-                if (row >= m_end || out_col >= out_cols || ((unsigned)(bad >> (i * 32)) >> in_slab & 1)) continue;
+                if (lane >= ROWS * LANES_A_ROW || row >= m_end || out_col >= out_cols || ((unsigned)(bad >> (i * 32)) >> in_slab & 1)) continue;
                 put(row, out_col, place, value);
             }
             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
@@ -421,24 +496,29 @@ void launch_whole(const float* a, const float* w, const float* bias, const float
     launch<BM, BN, WAVES_M, WAVES_N>(a, w, bias, residual, o, M, N, K, ceil_div(N, 16), epilogue, stream, scatter, k_blocks, dim3(ceil_div(N, BN), ceil_div(M, BM), k_blocks), stream::Whole{});
 }
 
-// The tiles, and what a tile of K costs a block in microseconds: alone on its compute unit, and beside others (a round of 256 blocks). Measured over
-// 130 to 8,192 rows at GPT-2's widths. A compute unit brings most out of 128 x 128; narrow outputs and few rows fill the chip with smaller ones.
+// The tiles, and what they cost in microseconds: what lies in front of and behind a block's loop, and a tile of K for each block of a compute unit, alone there or not, and
+// more the nearer a round of blocks is to all 256 units (they share the chip's power: products of numbers that are all zero take three quarters of the time).
+// Fitted to 900 products of 66 to 6,000 rows, 512 to 4,096 columns, K of 768 to 4,096, whole and cut, to 3 to 6 %. A compute unit brings most out of 128 x 128; 128 x 96
+// where its blocks are two rounds and 128 x 128's more than one; narrow outputs and few rows fill the chip with smaller ones.
+// 128 x 128 / 128 x 64 / 64 x 64 / 128 x 96, us: 2,048 x 2,304 x 768 58.0 / 53.5 / 53.6 / 48.4, 2,670 x 768 x 3,072 in two 70.5 / 71.5 / 84.2 / 83.5,
+// 2,048 x 768 x 3,072 in two 64.9 / 62.9 / 65.9 / 55.5, 8,192 x 3,072 x 768 217 / 228 / 258 / 214, 130 x 768 x 768 in six 10.9 / 7.7 / 6.2 / 9.7.
 struct Choice {
     int bm, bn;
-    float alone, shared;
+    float start, alone, tile, full;
 };
-constexpr Choice CHOICES[3] = {{128, 128, 1.27f, 1.28f}, {128, 64, 0.83f, 0.72f}, {64, 64, 0.50f, 0.41f}};
+constexpr int CHOICES_COUNT = 4;
+constexpr Choice CHOICES[CHOICES_COUNT] = {{128, 128, 7.5f, 0.07f, 0.83f, 0.30f}, {128, 64, 5.6f, 0.065f, 0.44f, 0.20f}, {64, 64, 4.9f, 0.09f, 0.29f, 0.09f}, {128, 96, 7.25f, 0.025f, 0.64f, 0.25f}};
 
 // Microseconds of a product cut into k_blocks along K with the best of the tiles (`best`): the rounds of blocks, the start and end of a block, and the sums
-// that are written (6 TB/s). Within a sixth of what was measured from 2,048 x 768 x 768 (21.4 us whole, 19.8 in two) to 2,048 x 768 x 3,072 (72 whole,
-// 62 in four, 63 in eight) and 130 x 768 x 768 (15.0 whole, 5.2 in six). With each tile in turn, 128 x 128 / 128 x 64 / 64 x 64: 2,048 x 2,304 x 768 58.8 /
-// 57.0 / 53.8 us, 8,192 x 3,072 x 768 213 / 237 / 253, 130 x 768 x 768 35.6 / 21.4 / 14.9; the rule's is the best of the three or within 3 % of it, but for
-// 1,500 x 2,304 x 768 (39.5 / 34.9 / 41.4, it takes the first).
+// that are written (6 TB/s). Its choice is within 1 % of the best of the four on average over the products above, and at most a fifth longer (2,670 x 512 x 768 in six).
 inline float cost(int M, int N, int K, int k_blocks, int& best) {
     float best_cost = 0.0f;
-    for (int c = 0; c < 3; c++) {
-        const int rounds = (int)(((long long)ceil_div(M, CHOICES[c].bm) * ceil_div(N, CHOICES[c].bn) * k_blocks + 255) / 256), tiles = ceil_div(ceil_div(K, k_blocks), BK);
-        const float us = tiles * (rounds == 1 ? CHOICES[c].alone : rounds * CHOICES[c].shared) + 3.0f + (float)M * N * k_blocks * (4.0f / 6e6f);
+    for (int c = 0; c < CHOICES_COUNT; c++) {
+        const Choice& with = CHOICES[c];
+        const long long blocks = (long long)ceil_div(M, with.bm) * ceil_div(N, with.bn) * k_blocks;
+        const int rounds = (int)((blocks + 255) / 256), tiles = ceil_div(ceil_div(K, k_blocks), BK);
+        const float a_tile = rounds * with.tile + (float)blocks / 256.0f * with.full + (rounds == 1 ? with.alone : 0.0f);
+        const float us = with.start + tiles * a_tile + (float)M * N * k_blocks * (4.0f / 6e6f);
         if (c == 0 || us < best_cost) best = c, best_cost = us;
     }
     return best_cost;
@@ -450,7 +530,8 @@ inline void dispatch(const float* a, const float* w, const float* bias, const fl
     cost(M, N, K, k_blocks, best);
     if (best == 0) launch_whole<128, 128, 2, 2>(a, w, bias, residual, o, M, N, K, epilogue, stream, scatter, k_blocks);
     else if (best == 1) launch_whole<128, 64, 4, 1>(a, w, bias, residual, o, M, N, K, epilogue, stream, scatter, k_blocks);
-    else launch_whole<64, 64, 2, 2>(a, w, bias, residual, o, M, N, K, epilogue, stream, scatter, k_blocks);
+    else if (best == 2) launch_whole<64, 64, 2, 2>(a, w, bias, residual, o, M, N, K, epilogue, stream, scatter, k_blocks);
+    else launch_whole<128, 96, 4, 1>(a, w, bias, residual, o, M, N, K, epilogue, stream, scatter, k_blocks);
 }
 
 // Into how many partial products a product with sums to be taken by whoever reads them is cut, `most` at most: they are read once more there.

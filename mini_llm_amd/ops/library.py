@@ -22,6 +22,7 @@ _SIGNATURES = {
     "mllm_gemm_takes_packed_rows": [c_int, c_int, c_int, c_int],
     "mllm_gemm_split": [P, P, c_int, P, c_int, c_int, c_int, c_int, c_int, c_int, P],
     "mllm_gemm_stream_tile": [c_int, c_int, c_int, c_int, c_int],
+    "mllm_gemm_pieces_tile": [c_int, c_int, c_int, c_int],
     "mllm_gemm_split_blocks": [c_int, c_int, c_int, c_int],
     "mllm_gemm_split_blocks_anywhere": [c_int, c_int, c_int, c_int],
     "mllm_gemm_split_blocks_row_major": [c_int, c_int, c_int, c_int],

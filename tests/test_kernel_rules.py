@@ -85,3 +85,19 @@ def test_32_bit_latent_attention_by_matrix_instructions(rows, heads, requests, m
     from mini_llm_amd.ops import kernels as K
 
     assert K.latent_f32_by_matrix(rows, heads, requests, max_q_len, longest) == by_matrix
+
+
+@pytest.mark.parametrize("m,n,k,cuts,tile", [
+    # the best tile as measured, or within 3 % of it; and what another kernel takes
+    (2048, 2304, 768, 1, 128096), (2670, 2304, 768, 1, 128096), (2048, 768, 3072, 2, 128096), (2670, 768, 3072, 2, 128128), (2048, 4096, 768, 1, 128128), (130, 768, 768, 6, 64064),
+    (300, 768, 3072, 8, 64064), (1024, 768, 3072, 2, 128064), (64, 768, 768, 1, 0), (65, 768, 760, 1, 0), (65, 770, 768, 1, 0)])
+def test_tiles_of_the_product_in_pieces_by_measurement(m, n, k, cuts, tile):
+    from mini_llm_amd.ops.library import library
+
+    assert library().mllm_gemm_pieces_tile(m, n, k, cuts) == tile
+
+
+def test_every_tile_of_the_product_in_pieces_has_a_shape_in_its_test():
+    from test_pieces_tiles_gpu import SHAPES
+
+    assert {shape[3] for shape in SHAPES} == {64064, 128064, 128096, 128128}
