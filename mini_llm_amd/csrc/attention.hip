@@ -73,33 +73,16 @@ __device__ __forceinline__ float capped_score(float s, float cap) {
     return cap * (1.0f - 2.0f * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(x * 2.8853900817779268f)));
 }
 
+// One row of one head by the wave that calls it; my_q: MAX_HEAD floats of LDS that no other wave touches.
 template <typename T>
-__global__ __launch_bounds__(256) void attention_general_kernel(
-    const T* __restrict__ q, int q_stride, const T* __restrict__ k_pages,
-    const T* __restrict__ v_pages, T* __restrict__ out, int out_stride,
-    const int* __restrict__ token_request, const int* __restrict__ positions,
-    const int* __restrict__ block_tables, int max_blocks, int n_heads, int n_kv_heads,
-    int head_size, int page_size, int window, float scale, ScoreOptions options) {
-    __shared__ float q_shared[4][MAX_HEAD];
-    const int lane = threadIdx.x % WAVE, wave = threadIdx.x / WAVE;
-    const int token = blockIdx.x;
-    const int head = blockIdx.y * 4 + wave;
-    if (head >= n_heads) return;  // no block-wide barrier below
-    const int request = token_request[token];
-    const size_t out_row = (size_t)token * out_stride + head * head_size;
-    if (request < 0) {
-        for (int d = lane; d < head_size; d += WAVE) store_result(out, out_row + d, 0.0f, options.wide_out);
-        return;
-    }
-    const int kv_head = head / (n_heads / n_kv_heads);
-    const int position = positions[token];
+__device__ __forceinline__ void general_row(const T* __restrict__ q_row, const T* __restrict__ k_pages, const T* __restrict__ v_pages, T* __restrict__ out, size_t out_row,
+                                            const int* __restrict__ table, int position, int kv_head, int head, int n_kv_heads, int head_size, int page_size, int window,
+                                            float scale, const ScoreOptions& options, float* my_q) {
+    const int lane = threadIdx.x % WAVE;
     const int first_key = first_visible_key(position, window, options.chunk);
     const int keep = min(options.keep, first_key);   // keys 0 .. keep - 1 count beside first_key .. position
-    const int* table = block_tables + (size_t)request * max_blocks;
 
-    float* my_q = q_shared[wave];
-    for (int d = lane; d < head_size; d += WAVE)
-        my_q[d] = to_float(q[(size_t)token * q_stride + head * head_size + d]) * scale;
+    for (int d = lane; d < head_size; d += WAVE) my_q[d] = to_float(q_row[d]) * scale;
     __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
     __builtin_amdgcn_wave_barrier();
 
@@ -124,8 +107,9 @@ __global__ __launch_bounds__(256) void attention_general_kernel(
             score = options.softcap > 0.0f ? capped_score<true>(dot, options.softcap) : dot;
         }
         float new_max = fmaxf(running_max, wave_max(score));
-        float p = valid ? expf(score - new_max) : 0.0f;
-        float rescale = expf(running_max - new_max);
+        const float reference = new_max == -INFINITY ? 0.0f : new_max;   // (only scores of minus infinity so far)
+        float p = valid ? expf(score - reference) : 0.0f;
+        float rescale = expf(running_max - reference);
         running_sum = running_sum * rescale + wave_sum(p);
         running_max = new_max;
 #pragma unroll
@@ -153,6 +137,28 @@ __global__ __launch_bounds__(256) void attention_general_kernel(
         int d = lane + r * WAVE;
         if (d < head_size) store_result(out, out_row + d, o[r] * inverse, options.wide_out);
     }
+}
+
+template <typename T>
+__global__ __launch_bounds__(256) void attention_general_kernel(
+    const T* __restrict__ q, int q_stride, const T* __restrict__ k_pages,
+    const T* __restrict__ v_pages, T* __restrict__ out, int out_stride,
+    const int* __restrict__ token_request, const int* __restrict__ positions,
+    const int* __restrict__ block_tables, int max_blocks, int n_heads, int n_kv_heads,
+    int head_size, int page_size, int window, float scale, ScoreOptions options) {
+    __shared__ float q_shared[4][MAX_HEAD];
+    const int lane = threadIdx.x % WAVE, wave = threadIdx.x / WAVE;
+    const int token = blockIdx.x;
+    const int head = blockIdx.y * 4 + wave;
+    if (head >= n_heads) return;  // no block-wide barrier below
+    const int request = token_request[token];
+    const size_t out_row = (size_t)token * out_stride + head * head_size;
+    if (request < 0) {
+        for (int d = lane; d < head_size; d += WAVE) store_result(out, out_row + d, 0.0f, options.wide_out);
+        return;
+    }
+    general_row<T>(q + (size_t)token * q_stride + head * head_size, k_pages, v_pages, out, out_row, block_tables + (size_t)request * max_blocks, positions[token],
+                   head / (n_heads / n_kv_heads), head, n_kv_heads, head_size, page_size, window, scale, options, q_shared[wave]);
 }
 
 }  // namespace
@@ -871,6 +877,7 @@ void launch_prefill(const void* q, int q_stride, const void* k_pages, const void
 }  // namespace
 
 #include "attention_stream.h"
+#include "attention_pieces.h"
 
 // 1 if the matrix-core prefill kernel takes this head size and page size.
 MLLM_API int mllm_attention_prefill_supported(int head_size, int page_size) {
@@ -914,12 +921,13 @@ MLLM_API int mllm_attention_prefill(const void* q, int q_stride, const void* k_p
         else MLLM_STREAM_CASE(bf16_t, 128);
         return mllm_check_launch("attention_prefill");
     }
+#undef MLLM_STREAM_CASE
     if (dtype == MLLM_F32 && prefill_stream::takes<float>(head_size, page_size, max_q_len, scale, q_stride, out_stride, q, out)) {
-        if (head_size == 32) MLLM_STREAM_CASE(float, 32);
-        else MLLM_STREAM_CASE(float, 64);
+        (head_size == 32 ? prefill_pieces::launch<32> : prefill_pieces::launch<64>)(
+            (const float*)q, q_stride, (const float*)k_pages, (const float*)v_pages, (float*)out, out_stride, q_starts, context_lens, block_tables, max_blocks, n_requests, rows,
+            max_q_len, n_heads, n_kv_heads, page_shift, window, scale, options, stream);
         return mllm_check_launch("attention_prefill");
     }
-#undef MLLM_STREAM_CASE
     if (dtype == MLLM_F32) {
         if (padded == 32) MLLM_PREFILL_CASE(float, 32);
         else if (padded == 64) MLLM_PREFILL_CASE(float, 64);

@@ -1,9 +1,6 @@
-// Prompt attention for rows of 64, 128 or 256 bytes (bfloat16 heads of 32, 64 or 128; 32-bit heads of 32 or 64)
+// Prompt attention for rows of 64, 128 or 256 bytes (bfloat16 heads of 32, 64 or 128; what of it serves 32-bit heads of 32 or 64 too: attention_pieces.h)
 // over pages of at least 32 keys: key and value tiles stream from the cache pages straight into LDS
 // (global_load_lds_dwordx4), and a block's keys are divided among its waves. Included by attention.hip.
-// The text below describes the bfloat16 kernel; what the 32-bit one does differently stands where it does it: the
-// 32-bit matrix instruction (32 x 32 x 2, four to a 16-byte piece of a key), the library's expf, and values read as
-// they are stored (the instruction takes single elements, so nothing has to be transposed).
 //
 // A block owns 64 queries of one (request, head). Each of its four waves holds all 64 queries and walks every fourth
 // tile of 32 keys with softmax statistics of its own; at the end the four partial results are combined through LDS.
@@ -116,27 +113,6 @@ __device__ __forceinline__ void read_transposed<4, 256>(const unsigned (&address
         : "memory");
 }
 
-// Eight 4-byte LDS reads from one address with the offsets the 32-bit value product needs (keys 0-3 and 8-11 of a
-// lane's sixteen, ROW_BYTES apart; `FROM` 0: those, 1: keys 16-19 and 24-27), as instructions, for the reason above.
-// Returns when the values are in registers.
-template <int ROW_BYTES, int FROM>
-__device__ __forceinline__ void read_eight(unsigned address, float (&out)[8]) {
-    asm volatile(
-        "ds_read_b32 %0, %8 offset:%9\n\t"
-        "ds_read_b32 %1, %8 offset:%10\n\t"
-        "ds_read_b32 %2, %8 offset:%11\n\t"
-        "ds_read_b32 %3, %8 offset:%12\n\t"
-        "ds_read_b32 %4, %8 offset:%13\n\t"
-        "ds_read_b32 %5, %8 offset:%14\n\t"
-        "ds_read_b32 %6, %8 offset:%15\n\t"
-        "ds_read_b32 %7, %8 offset:%16\n\t"
-        "s_waitcnt lgkmcnt(0)"
-        : "=&v"(out[0]), "=&v"(out[1]), "=&v"(out[2]), "=&v"(out[3]), "=&v"(out[4]), "=&v"(out[5]), "=&v"(out[6]), "=&v"(out[7])
-        : "v"(address), "n"((16 * FROM + 0) * ROW_BYTES), "n"((16 * FROM + 1) * ROW_BYTES), "n"((16 * FROM + 2) * ROW_BYTES), "n"((16 * FROM + 3) * ROW_BYTES),
-          "n"((16 * FROM + 8) * ROW_BYTES), "n"((16 * FROM + 9) * ROW_BYTES), "n"((16 * FROM + 10) * ROW_BYTES), "n"((16 * FROM + 11) * ROW_BYTES)
-        : "memory");
-}
-
 template <typename T, int HD, int SPLITS>
 struct Layout {
     static constexpr bool FP32 = sizeof(T) == 4;
@@ -232,7 +208,6 @@ __global__ __launch_bounds__(64 * SPLITS, (HD * sizeof(T) <= 128 && SPLITS == 4)
     const int* __restrict__ block_tables, int max_blocks, int n_requests, int n_heads, int n_kv_heads, int page_shift, int given_window, float scale, ScoreOptions options) {
     typedef Layout<T, HD, SPLITS> L;
     const int window = FORM == CAUSAL ? 0 : given_window, chunk = FORM == CAUSAL ? 0 : options.chunk;
-    constexpr bool FP32 = L::FP32;
     constexpr int QSUB = QUERIES / 32;
     static_assert(QUERIES == 32 || QUERIES == 64, "one or two sub-tiles of queries");
     static_assert(HD % 32 == 0, "the output is written in tiles of 32 head dimensions");
@@ -330,21 +305,12 @@ __global__ __launch_bounds__(64 * SPLITS, (HD * sizeof(T) <= 128 && SPLITS == 4)
 #pragma unroll
             for (int v = 0; v < 16; v++) acc_o[qs][i2][v] = 0.0f;
     }
-    // bfloat16: 2^x of a score prescaled by log2(e); 32-bit: the library's e^x of the scaled score. Positive either way, so
-    // the scaling commutes with the maximum.
-    const float score_scale = FP32 ? scale : scale * 1.4426950408889634f;
-    auto weight_of = [](float x) { return FP32 ? expf(x) : __builtin_amdgcn_exp2f(x); };
-    // one 16-byte piece of a key against the same piece of the queries: one product in bfloat16 (32 x 32 x 16), four in
-    // 32-bit (32 x 32 x 2: component c of every lane forms the pair of one product, the same pairing on both operands)
+    // 2^x of a score prescaled by log2(e), which is positive, so the scaling commutes with the maximum
+    const float score_scale = scale * 1.4426950408889634f;
+    auto weight_of = [](float x) { return __builtin_amdgcn_exp2f(x); };
+    // one 16-byte piece of a key against the same piece of the queries
     auto piece_product = [](const Vec16& k_piece, const Vec16& q_piece, f32x16 sums) {
-        if constexpr (FP32) {
-            const f32x4 k4 = *reinterpret_cast<const f32x4*>(&k_piece), q4 = *reinterpret_cast<const f32x4*>(&q_piece);
-#pragma unroll
-            for (int c = 0; c < 4; c++) sums = __builtin_amdgcn_mfma_f32_32x32x2f32(k4[c], q4[c], sums, 0, 0, 0);
-            return sums;
-        } else {
-            return __builtin_amdgcn_mfma_f32_32x32x16_bf16(*reinterpret_cast<const bf16x8*>(&k_piece), *reinterpret_cast<const bf16x8*>(&q_piece), sums, 0, 0, 0);
-        }
+        return __builtin_amdgcn_mfma_f32_32x32x16_bf16(*reinterpret_cast<const bf16x8*>(&k_piece), *reinterpret_cast<const bf16x8*>(&q_piece), sums, 0, 0, 0);
     };
 
     // K fragment (32 keys x 16 columns): lane l holds key l % 32, columns 16 s + 8 (l / 32) .. + 8
@@ -407,11 +373,8 @@ __global__ __launch_bounds__(64 * SPLITS, (HD * sizeof(T) <= 128 && SPLITS == 4)
             if ((FORM == CAPPED || FORM == KEPT) && options.softcap > 0.0f) {   // a capped score, left divided by the scale as the plain ones are: cap tanh(scale s / cap) / scale
                 const float back = options.softcap / scale, into = scale / options.softcap;
 #pragma unroll
-                for (int v = 0; v < 16; v++) {
-                    if constexpr (FP32) s_acc[qs][v] = back * tanhf(s_acc[qs][v] * into);
-                    else   // tanh x = 1 - 2 / (1 + e^(2x)), the hardware's 2^x and reciprocal: five instructions a score
-                        s_acc[qs][v] = __builtin_fmaf(-2.0f * back, __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(s_acc[qs][v] * (into * 2.8853900817779268f))), back);
-                }
+                for (int v = 0; v < 16; v++)   // tanh x = 1 - 2 / (1 + e^(2x)), the hardware's 2^x and reciprocal: five instructions a score
+                    s_acc[qs][v] = __builtin_fmaf(-2.0f * back, __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(s_acc[qs][v] * (into * 2.8853900817779268f))), back);
             }
             if (interior) {
 #pragma unroll
@@ -445,12 +408,10 @@ __global__ __launch_bounds__(64 * SPLITS, (HD * sizeof(T) <= 128 && SPLITS == 4)
                 s_acc[qs][v] = p;
                 running_sum[qs] += p;
             }
-            if constexpr (!FP32) {
 #pragma unroll
-                for (int slab = 0; slab < 2; slab++)
+            for (int slab = 0; slab < 2; slab++)
 #pragma unroll
-                    for (int e = 0; e < 8; e++) p[qs][slab][e] = static_cast<bf16_t>(s_acc[qs][8 * slab + e]);
-            }
+                for (int e = 0; e < 8; e++) p[qs][slab][e] = static_cast<bf16_t>(s_acc[qs][8 * slab + e]);
         };
         softmax(0);
         __builtin_amdgcn_sched_barrier(0);
@@ -476,26 +437,6 @@ __global__ __launch_bounds__(64 * SPLITS, (HD * sizeof(T) <= 128 && SPLITS == 4)
 
         // ---- O^T += V^T . P^T : two slabs of 16 keys; a lane's eight are keys 4 half .. + 4 and 8 + 4 half .. + 4 of the slab ----
         wait_vmcnt<3 * L::LOADS>();  // the newest three are K(i+2) V(i+1) K(i+3): V(i) has landed
-        if constexpr (FP32) {
-            // 32-bit: O^T += V^T . P^T by products of two keys: register v of the scores holds, in the lanes of half h, key
-            // 8 (v / 4) + 4 h + v % 4 of the tile, so product v takes that key's values (column 32 i2 + lane % 32, read as
-            // stored) against the register itself. Eight values a read, for each 32 columns.
-#pragma unroll
-            for (int i2 = 0; i2 < DT; i2++) {
-                const unsigned address = lds_address(v_tile + (4 * half) * L::ROW_BYTES + (i2 * 32 + lane32) * 4);
-                float values[8];
-                read_eight<L::ROW_BYTES, 0>(address, values);
-#pragma unroll
-                for (int e = 0; e < 8; e++)
-#pragma unroll
-                    for (int qs = 0; qs < QSUB; qs++) acc_o[qs][i2] = __builtin_amdgcn_mfma_f32_32x32x2f32(values[e], s_acc[qs][e], acc_o[qs][i2], 0, 0, 0);
-                read_eight<L::ROW_BYTES, 1>(address, values);
-#pragma unroll
-                for (int e = 0; e < 8; e++)
-#pragma unroll
-                    for (int qs = 0; qs < QSUB; qs++) acc_o[qs][i2] = __builtin_amdgcn_mfma_f32_32x32x2f32(values[e], s_acc[qs][8 + e], acc_o[qs][i2], 0, 0, 0);
-            }
-        } else {
         short4_t v_frag[DT][4];      // per 32 columns: slab 0 low keys, slab 0 high keys, slab 1 low, slab 1 high
         {
             unsigned address[DT];
@@ -518,7 +459,6 @@ __global__ __launch_bounds__(64 * SPLITS, (HD * sizeof(T) <= 128 && SPLITS == 4)
 #pragma unroll
                 for (int qs = 0; qs < QSUB; qs++) acc_o[qs][i2] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fragment, p[qs][slab], acc_o[qs][i2], 0, 0, 0);
             }
-        }
         }
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         issue(i + 2, page_v, true);
@@ -560,7 +500,7 @@ __global__ __launch_bounds__(64 * SPLITS, (HD * sizeof(T) <= 128 && SPLITS == 4)
             weight[w] = weight_of(stats_lds[w][qs * 32 + lane32][0] - best);  // a wave that saw no key: a weight of 0
             total += weight[w] * stats_lds[w][qs * 32 + lane32][1];
         }
-        if (options.sinks) total += weight_of(options.sinks[head] * (FP32 ? 1.0f : 1.4426950408889634f) - best);   // the sink: once, with no value
+        if (options.sinks) total += weight_of(options.sinks[head] * 1.4426950408889634f - best);   // the sink: once, with no value
         const float inverse = 1.0f / total;
         const size_t out_row = (size_t)(q_first + q_local) * out_stride + head * HD + i2 * 32;
 #pragma unroll
@@ -575,7 +515,7 @@ __global__ __launch_bounds__(64 * SPLITS, (HD * sizeof(T) <= 128 && SPLITS == 4)
                 o[e] = sum * inverse;
             }
             const size_t at = out_row + 8 * g + 4 * half;
-            if (FP32 || options.wide_out) *reinterpret_cast<f32x4*>(reinterpret_cast<float*>(out) + at) = f32x4{o[0], o[1], o[2], o[3]};
+            if (options.wide_out) *reinterpret_cast<f32x4*>(reinterpret_cast<float*>(out) + at) = f32x4{o[0], o[1], o[2], o[3]};
             else *reinterpret_cast<bf16x4*>(out + at) = bf16x4{static_cast<bf16_t>(o[0]), static_cast<bf16_t>(o[1]), static_cast<bf16_t>(o[2]), static_cast<bf16_t>(o[3])};
         }
     }
@@ -639,32 +579,25 @@ void launch(const void* q, int q_stride, const void* k_pages, const void* v_page
 #define MLLM_STREAM_LAUNCH(QUERIES, SPLITS)                                                                                                 \
     launch_queries<T, HD, QUERIES, SPLITS>(q, q_stride, k_pages, v_pages, out, out_stride, q_starts, context_lens, block_tables, max_blocks, \
                                            n_requests, rows, max_q_len, n_heads, n_kv_heads, page_shift, window, scale, options, stream)
-    if constexpr (sizeof(T) == 4) {
-        // 32-bit: the matrix cores are what a wave waits for (a tile of 32 keys is 96 products of 64 cycles for 32 queries),
-        // so blocks of 32 queries, which the compute units take in turn, the ones with the most keys first
-        // (blocks of 64 queries: 59.2 against 62.1 us for two prompts of 1,024 tokens x 12 heads of 64, 35.0 against 32.2 us for eight of 256)
-        MLLM_STREAM_LAUNCH(32, 4);
-    } else {
-        // blocks of 64 queries where they give every compute unit a block (measured: 2 x 1,024 tokens x 12 heads 15.9 against 17.2 us; 16.8 with the walk
-        // over the portions in front),
-        // else of 32 (4 x 128 tokens on 896 cached: 9.7 against 13.0 us; 512 on 7,680: 46.7 against 66.0 us)
-        const bool wide = (long)n_heads * most_tiles(64, n_requests, rows, max_q_len) >= 256;
-        // Eight waves a block where the block of the last queries has sixteen tiles of keys or more to walk (max_len: the longest
-        // sequence after this step, or what bounds it; a window bounds the keys too) AND every block still finds a compute
-        // unit of its own at once (eight waves' tiles leave room for one block a unit): a long context with few queries.
-        // Measured, heads of 64: 512 queries on 7,680 cached keys 38.2 against 46.7 us with four waves; but two prompts of 1,024
-        // tokens (384 blocks: a second round) 19.1 against 15.9 us, one of 4,096 64.8 against 57 us.
-        const int reach = options.chunk > 0 ? min(max_len, options.chunk + 64) : (window > 0 ? min(max_len, window + options.keep + 64) : max_len);
-        const long blocks = (long)n_heads * most_tiles(wide ? 64 : 32, n_requests, rows, max_q_len);
-        bool eight = false;
-        if constexpr (HD * sizeof(T) <= 128) {  // (eight waves' tiles of rows of 256 bytes do not fit a compute unit's LDS)
-            eight = reach >= 16 * KEYS && blocks <= 256;
-            if (wide && eight) MLLM_STREAM_LAUNCH(64, 8);
-            else if (eight) MLLM_STREAM_LAUNCH(32, 8);
-        }
-        if (wide && !eight) MLLM_STREAM_LAUNCH(64, 4);
-        else if (!eight) MLLM_STREAM_LAUNCH(32, 4);
+    // blocks of 64 queries where they give every compute unit a block (measured: 2 x 1,024 tokens x 12 heads 15.9 against 17.2 us; 16.8 with the walk
+    // over the portions in front),
+    // else of 32 (4 x 128 tokens on 896 cached: 9.7 against 13.0 us; 512 on 7,680: 46.7 against 66.0 us)
+    const bool wide = (long)n_heads * most_tiles(64, n_requests, rows, max_q_len) >= 256;
+    // Eight waves a block where the block of the last queries has sixteen tiles of keys or more to walk (max_len: the longest
+    // sequence after this step, or what bounds it; a window bounds the keys too) AND every block still finds a compute
+    // unit of its own at once (eight waves' tiles leave room for one block a unit): a long context with few queries.
+    // Measured, heads of 64: 512 queries on 7,680 cached keys 38.2 against 46.7 us with four waves; but two prompts of 1,024
+    // tokens (384 blocks: a second round) 19.1 against 15.9 us, one of 4,096 64.8 against 57 us.
+    const int reach = options.chunk > 0 ? min(max_len, options.chunk + 64) : (window > 0 ? min(max_len, window + options.keep + 64) : max_len);
+    const long blocks = (long)n_heads * most_tiles(wide ? 64 : 32, n_requests, rows, max_q_len);
+    bool eight = false;
+    if constexpr (HD * sizeof(T) <= 128) {  // (eight waves' tiles of rows of 256 bytes do not fit a compute unit's LDS)
+        eight = reach >= 16 * KEYS && blocks <= 256;
+        if (wide && eight) MLLM_STREAM_LAUNCH(64, 8);
+        else if (eight) MLLM_STREAM_LAUNCH(32, 8);
     }
+    if (wide && !eight) MLLM_STREAM_LAUNCH(64, 4);
+    else if (!eight) MLLM_STREAM_LAUNCH(32, 4);
 #undef MLLM_STREAM_LAUNCH
 }
 

@@ -24,9 +24,9 @@
 // Fragment reads are inline assembly with waits of their own: through the compiler each would wait for the loads into LDS that are under way.
 #pragma once
 
-namespace pieces {
+#include "number_pieces.h"
 
-typedef int i32x4 __attribute__((ext_vector_type(4)));
+namespace pieces {
 
 constexpr int BK = 32;   // numbers of K in a tile
 
@@ -50,24 +50,6 @@ template <int LEFT>
 __device__ __forceinline__ void wait_but() {
     static_assert(LEFT < 64, "the loads in flight fit the counter");
     __builtin_amdgcn_s_waitcnt((LEFT & 0xF) | ((LEFT >> 4) << 14) | (0x7 << 4) | (0xF << 8));
-}
-
-// Numbers 2 e and 2 e + 1 of a lane's eight -> their places in three operands of pieces. (A number that the first rounding makes infinite leaves sums that are not finite, as an infinity does.)
-__device__ __forceinline__ void split_pair(const i32x4 (&raw)[2], int e, bf16x8 (&out)[3]) {
-    typedef float f32x2 __attribute__((ext_vector_type(2)));
-    typedef bf16_t bf16x2 __attribute__((ext_vector_type(2)));
-    const int first = raw[e / 2][e % 2 * 2], second = raw[e / 2][e % 2 * 2 + 1];
-    float rest[2] = {__builtin_bit_cast(float, first), __builtin_bit_cast(float, second)};
-#pragma unroll
-    for (int p = 0; p < 3; p++) {
-        const bf16x2 pair = __builtin_convertvector((f32x2{rest[0], rest[1]}), bf16x2);
-        out[p][2 * e] = pair[0], out[p][2 * e + 1] = pair[1];
-        if (p < 2) {
-            const uint32_t bits = __builtin_bit_cast(uint32_t, pair);
-            rest[0] -= __builtin_bit_cast(float, bits << 16);
-            rest[1] -= __builtin_bit_cast(float, bits & 0xffff0000u);
-        }
-    }
 }
 
 // The whole product (Group: stream::Whole) or one over rows grouped by expert (stream::ExpertTiles, a one-dimensional grid). W: packed, its pieces behind its

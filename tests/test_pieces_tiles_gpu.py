@@ -32,3 +32,95 @@ def test_tiles_of_the_product_in_pieces(m, n, k, tile):
     infinite = ~ref.isfinite()
     assert bool((got.double()[infinite] == ref[infinite]).all()) and int(infinite.sum()) == 3 * n
     assert bool(((got.double() - ref).abs() <= bound)[~infinite].all())
+
+
+def _prompt(lengths, contexts, heads, head_size, page_size=32):
+    """Queries, pages and the batch's arrays of prompts on cached keys: (q, k_pages, v_pages, requests, positions, tables, starts, contexts), float32."""
+    generator = torch.Generator(device="cuda").manual_seed(sum(lengths) + head_size)
+    pages = [-(-(n + c) // page_size) for n, c in zip(lengths, contexts)]
+    tables = torch.zeros(len(lengths), max(pages), dtype=torch.int32)
+    for r, count in enumerate(pages):
+        tables[r, :count] = torch.arange(sum(pages[:r]), sum(pages[:r]) + count).flip(0)
+    k_pages, v_pages = (torch.randn(sum(pages), heads, page_size, head_size, generator=generator, device="cuda") for _ in range(2))
+    q = torch.randn(sum(lengths), heads * head_size, generator=generator, device="cuda")
+    requests = torch.cat([torch.full((n,), r) for r, n in enumerate(lengths)]).int().cuda()
+    positions = torch.cat([torch.arange(c, c + n) for n, c in zip(lengths, contexts)]).int().cuda()
+    starts = torch.tensor([0, *lengths]).cumsum(0).int().cuda()
+    return q, k_pages, v_pages, requests, positions, tables.cuda(), starts, torch.tensor(contexts).int().cuda()
+
+
+def _attention(q, k_pages, v_pages, requests, positions, tables, starts, contexts, lengths, heads, head_size, **options):
+    from mini_llm_amd.ops import kernels as K
+
+    before = K.launch_counts()
+    out = K.paged_attention(q, k_pages, v_pages, requests, positions, tables, heads, heads, head_size, head_size**-0.5, max_q_len=max(lengths),
+                            max_len=int(positions.max()) + 1, q_starts=starts, context_lens=contexts, **options)
+    assert list(K.launches_since(before)) == ["attention_prefill_stream"]
+    return out
+
+
+def _exact(q, k_pages, v_pages, tables, starts, contexts, heads, head_size, window=0, keep_first=0, one_by_one=False):
+    """The same in 64 bits."""
+    out = torch.empty(q.shape, dtype=torch.float64, device="cuda")
+    for r in range(len(contexts)):
+        lo, hi, context = int(starts[r]), int(starts[r + 1]), int(contexts[r])
+        keys, values = (pages[tables[r].long()].permute(1, 0, 2, 3).reshape(heads, -1, head_size)[:, : context + hi - lo].double() for pages in (k_pages, v_pages))
+        scores = torch.matmul(q[lo:hi].view(-1, heads, head_size).permute(1, 0, 2).double(), keys.transpose(1, 2).contiguous()) * head_size**-0.5
+        at, key = torch.arange(context, context + hi - lo, device="cuda")[:, None], torch.arange(context + hi - lo, device="cuda")[None]
+        seen = (key <= at) & ((key > at - window) | (key < keep_first) if window else key >= 0)
+        weights = scores.masked_fill(~seen, -torch.inf).softmax(-1)
+        # (a key that a row does not see adds nothing to it, whatever its value)
+        mixed = torch.where(seen[None, :, :, None], weights[..., None] * values[:, None], 0.0).sum(2) if one_by_one else torch.matmul(weights, values)
+        out[lo:hi] = mixed.permute(1, 0, 2).reshape(hi - lo, -1)
+    return out
+
+
+@pytest.mark.parametrize("head_size", [32, 64])
+@pytest.mark.parametrize("lengths,contexts,options", [
+    ([65], [0], {}), ([66, 129, 97], [0, 31, 32], {}), ([128, 300], [700, 0], {}),   # tiles of 32 queries and keys, a row more or less; waves without a tile, with one and with many
+    ([90, 300], [100, 0], dict(window=28)), ([200], [0], dict(window=33)),            # rows whose only keys of a tile are its last four
+    ([90, 300], [100, 0], dict(window=40, keep_first=5))])
+def test_prompt_attention_in_pieces(head_size, lengths, contexts, options):
+    heads = 3
+    arrays = _prompt(lengths, contexts, heads, head_size)
+    out = _attention(*arrays, lengths, heads, head_size, **options)
+    ref = _exact(*(arrays[n] for n in (0, 1, 2, 5, 6, 7)), heads, head_size, **options)
+    # scores of head_size products, each 2^-24 off at the most, with as many roundings as there are instructions; the weights' and the values' sums alike, over up to 1,000 keys whose
+    # values are of order one: some 2^-24 (head_size + 60) of the largest value
+    assert float((out.double() - ref).abs().max()) < 2**-24 * (head_size + 60) * 4
+
+
+@pytest.mark.parametrize("what", ["infinite key", "infinite value", "largest value", "no number", "tiny values", "tiny queries", "large queries"])
+def test_prompt_attention_of_numbers_that_have_no_pieces(what):
+    heads, head_size, lengths, contexts = 2, 64, [100, 70], [0, 40]
+    arrays = _prompt(lengths, contexts, heads, head_size)
+    q, k_pages, v_pages, tables = arrays[0], arrays[1], arrays[2], arrays[5]
+    page = int(tables[0, 1])   # keys 32 to 63 of the first request
+    if what == "infinite key":      # a score of minus infinity for queries on its other side, no number for those on its own
+        k_pages[page, 0, 3, 5] = torch.inf
+    elif what == "infinite value":
+        v_pages[page, 1, 4, 7] = -torch.inf
+    elif what == "largest value":   # rounds to infinity as a bfloat16 number
+        v_pages[page, 1, 4, 7] = torch.finfo(torch.float32).max
+    elif what == "no number":
+        v_pages[page, 0, 9, 0] = torch.nan
+    elif what == "tiny values":
+        v_pages[:, 1] *= 2.0**-118
+    elif what == "tiny queries":    # times keys that make up for it
+        q *= 2.0**-100
+        k_pages *= 2.0**100
+        q[3, 4] = 2.0**-126
+    else:
+        q *= 2.0**100
+        k_pages *= 2.0**-112
+        q *= 2.0**12
+    out = _attention(*arrays, lengths, heads, head_size)
+    ref = _exact(*(arrays[n] for n in (0, 1, 2, 5, 6, 7)), heads, head_size, one_by_one=True)
+    # a product with an infinity in 64 bits is that in 32: what is no number there is none here, infinities are the same, and so is the rest
+    assert bool((out.isnan() == ref.isnan()).all())
+    plain = ref.isfinite() & out.isfinite()
+    assert bool((out.double() == ref)[~plain & ~ref.isnan() & ref.isinf()].all())
+    # errors beside a head's common size: 2^-24 of it (or of a number below the smallest normal one) for each of some hundred roundings
+    size = torch.tensor([1.0, 2.0**-118 if what == "tiny values" else 1.0], device="cuda", dtype=torch.float64).repeat_interleave(head_size)
+    error = ((out.double() - ref).abs() / torch.maximum(ref.abs(), size))[plain]
+    assert float(error.max()) < 2**-24 * 300
