@@ -16,8 +16,8 @@
 // A block of four waves owns BM x BN outputs and walks K in tiles of 32, two steps of 16: rows of A and chunks of W go from memory straight into LDS
 // (global_load_lds_dwordx4), one tile ahead of the products, in two stages, which leave room for two blocks a compute unit (a third stage and one block: 2,048 x 2,304 x 768
 // with 128 x 128 58 -> 69 us). What bounds it: the matrix cores, and beside them the chip's power. A SIMD runs a wave's vector instructions under its own matrix instructions
-// only where they stand between them: 24 products behind the splitting of their rows take 2,101 cycles a tile, with the splitting of the next step's rows between them
-// 1,609, and two waves a SIMD, each in two such halves, 1,860 each. So a step's products carry the splitting of the next step's rows, its fragment reads, and one by one
+// only where they stand between them: a tile's 48 products behind the splitting of their rows, step by step, take 2,101 cycles, with the splitting of the next step's rows between
+// them 1,609, and of two waves a SIMD that split first and multiply then each 1,860. So a step's products carry the splitting of the next step's rows, its fragment reads, and one by one
 // the loads of the tile after the next (a compute unit takes a load of 1 KiB every 16 cycles, and a wave that asks for all at once waits).
 // With the loads at a tile's start and the splitting in front of its products (us -> now): 2,048 x 2,304 x 768 56.2 -> 48.4 (128 x 96), 2,048 x 3,072 x 768 65.9 -> 60,
 // 2,670 x 768 x 3,072 in two 81.8 -> 70.5, 8,192 x 3,072 x 768 212 -> 203.
