@@ -14,8 +14,10 @@
 // In a sum of six products the five small ones come first, so that the large sum is rounded once for sixteen numbers (the 32-bit instruction: eight times). Against 64 bits, normally
 // distributed numbers: 2.6e-7 -> 1.5e-7 for the first of these, 8.7e-7 -> 7.4e-7 over 8,192 keys.
 // What pieces cannot hold: a number that is not finite or rounds to infinity has no pieces, and whatever it meets comes out as no number; numbers below 2^-110 lose
-// their third piece. A block whose results are not finite or smaller than 2^-90, or whose queries hold numbers beyond 2^64 or below 2^-90 (which could make up for keys that lost
-// theirs), takes its rows again one by one in 32-bit (general_row).
+// their third piece, below 2^-134 all of them, and weights below 2^-126 are 0. So a weighted sum of values may be off by 2^-126 for each key, times the largest value of its
+// column, or by 2^-134 for each, times its weight. A block with results that are not finite, with weighted sums below 2^-90 or below 2^-90 times the largest value of their column
+// (zeros among them, unless every value of the column is zero), or whose queries hold numbers beyond 2^64 or below 2^-90 (which could make up for keys that lost their pieces), takes
+// its rows again one by one in 32-bit (general_row).
 #pragma once
 
 #include "number_pieces.h"
@@ -45,10 +47,11 @@ constexpr int wave_bytes() {
     return 2 * Layout<float, HD, WAVES>::TILE_BYTES;
 }
 
-// e^x for x <= 0 (0 for minus infinity and whatever is below e^-128; no number stays one): 2^t of the rounded t = x log2(e), and what the rounding left by the first two terms of
-// its series, x - t ln 2 in two parts. Within 2 units in the last place. Six instructions, the library's expf some fourteen.
+// e^x for x <= 0 (0 for minus infinity and whatever is below 2^-126, x < -87.3: the hardware's 2^x has no subnormal results; no number stays one): 2^t of the rounded
+// t = x log2(e), and what the rounding left by the first two terms of its series, x - t ln 2 in two parts. With an exact 2^t within one unit in the last place, 0.33 of it on
+// average (the library's expf: 0.64 and 0.25). Six instructions, the library's expf some fourteen.
 __device__ __forceinline__ float exp_below(float x) {
-    x = __builtin_elementwise_maximum(x, -128.0f);   // (keeps what is no number)
+    x = __builtin_elementwise_maximum(x, -128.0f);   // (keeps what is no number, and minus infinity from becoming that below)
     const float t = x * 1.44269504f;
     float left = __builtin_fmaf(-t, 0.693147182f, x);   // ln 2 = 0.693147182 - 1.90465421e-9
     left = __builtin_fmaf(t, 1.90465421e-9f, left);
@@ -146,6 +149,7 @@ __global__ __launch_bounds__(64 * WAVES, 2) void attention_prefill_pieces_kernel
     static_assert(WAVE_BYTES >= QUERIES * HD * 4 && WAVE_BYTES >= MAX_HEAD * 4, "what a wave leaves takes the place of its tiles");
     extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
     __shared__ float stats_lds[WAVES][QUERIES][2];
+    __shared__ __attribute__((aligned(16))) float largest_lds[WAVES][HD];
     __shared__ int again;   // whether the block's rows are taken once more
 
     const int tid = threadIdx.x, lane = tid % WAVE;
@@ -226,6 +230,14 @@ __global__ __launch_bounds__(64 * WAVES, 2) void attention_prefill_pieces_kernel
 
     f32x16 acc_o[DT];
     float running_max = -INFINITY, running_sum = 0.0f;
+    float largest[DT];   // magnitude of the values this lane has split, of its column of every 32 (no number if one of them is)
+#pragma unroll
+    for (int i2 = 0; i2 < DT; i2++) largest[i2] = 0.0f;
+    auto split_values = [&](const i32x4 (&raw)[2], int e, bf16x8 (&out)[3], float& so_far) {   // pieces of pair e
+        pieces::split_pair(raw, e, out);
+        const int first = raw[e / 2][e % 2 * 2], second = raw[e / 2][e % 2 * 2 + 1];
+        so_far = __builtin_elementwise_maximum(__builtin_elementwise_maximum(so_far, fabsf(__builtin_bit_cast(float, first))), fabsf(__builtin_bit_cast(float, second)));
+    };
 #pragma unroll
     for (int i2 = 0; i2 < DT; i2++)
 #pragma unroll
@@ -359,7 +371,7 @@ __global__ __launch_bounds__(64 * WAVES, 2) void attention_prefill_pieces_kernel
         constexpr int FRAGMENTS = 2 * DT, EACH = 6, VALUES = FRAGMENTS * EACH, OTHERS = 2 * L::LOADS + 4 * KS;
         bf16x8 v_piece[FRAGMENTS][3];
 #pragma unroll
-        for (int e = 0; e < 4; e++) pieces::split_pair(v_raw[0][0], e, v_piece[0]);
+        for (int e = 0; e < 4; e++) split_values(v_raw[0][0], e, v_piece[0], largest[0]);
         stream_for<VALUES / AT_ONCE>([&](auto group) {
             constexpr int G = decltype(group)::value * AT_ONCE, F = G / EACH;
             stream_for<AT_ONCE>([&](auto n) {
@@ -368,7 +380,7 @@ __global__ __launch_bounds__(64 * WAVES, 2) void attention_prefill_pieces_kernel
             });
             if constexpr (F + 1 < FRAGMENTS) {
                 constexpr int FROM = G % EACH * 4 / EACH, TO = (G % EACH + AT_ONCE) * 4 / EACH;
-                stream_for<TO - FROM>([&](auto n) { pieces::split_pair(v_raw[(F + 1) / DT][(F + 1) % DT], FROM + decltype(n)::value, v_piece[F + 1]); });
+                stream_for<TO - FROM>([&](auto n) { split_values(v_raw[(F + 1) / DT][(F + 1) % DT], FROM + decltype(n)::value, v_piece[F + 1], largest[(F + 1) % DT]); });
             }
             constexpr int FROM = G * OTHERS / VALUES, TO = (G + AT_ONCE) * OTHERS / VALUES;
             stream_for<TO - FROM>([&](auto n) {
@@ -393,6 +405,11 @@ __global__ __launch_bounds__(64 * WAVES, 2) void attention_prefill_pieces_kernel
         stats_lds[wave][lane32][1] = running_sum;
     }
 #pragma unroll
+    for (int i2 = 0; i2 < DT; i2++) {
+        const float of_column = larger_of_halves(largest[i2]);
+        if (half == 0) largest_lds[wave][i2 * 32 + lane32] = of_column;
+    }
+#pragma unroll
     for (int i2 = 0; i2 < DT; i2++)
 #pragma unroll
         for (int v = 0; v < 16; v++) partial[(i2 * 16 + v) * WAVE + lane] = acc_o[i2][v];
@@ -413,15 +430,21 @@ __global__ __launch_bounds__(64 * WAVES, 2) void attention_prefill_pieces_kernel
         float* const out_row = out + (size_t)(q_first + own_query) * out_stride + head * HD + 8 * wave + 4 * half;
 #pragma unroll
         for (int i2 = 0; i2 < DT; i2++) {
-            f32x4 o;
+            f32x4 o, most = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+            for (int w = 0; w < WAVES; w++) {
+                const f32x4 here = *reinterpret_cast<const f32x4*>(&largest_lds[w][i2 * 32 + 8 * wave + 4 * half]);
+#pragma unroll
+                for (int e = 0; e < 4; e++) most[e] = fmaxf(most[e], here[e]);
+            }
 #pragma unroll
             for (int e = 0; e < 4; e++) {
                 float sum = 0.0f;
 #pragma unroll
                 for (int w = 0; w < WAVES; w++) sum += weight[w] * reinterpret_cast<const float*>(lds + w * WAVE_BYTES)[(i2 * 16 + 4 * wave + e) * WAVE + lane];
-                sum *= inverse;
-                o[e] = sum;
-                odd |= !(fabsf(sum) < INFINITY) || (sum != 0.0f && fabsf(sum) < 0x1p-90f);
+                odd |= (most[e] > 0.0f) & (fabsf(sum) < fmaxf(most[e], 1.0f) * 0x1p-90f);
+                o[e] = sum * inverse;
+                odd |= !(fabsf(o[e]) < INFINITY);
             }
             *reinterpret_cast<f32x4*>(out_row + i2 * 32) = o;
         }

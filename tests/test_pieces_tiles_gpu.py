@@ -124,3 +124,27 @@ def test_prompt_attention_of_numbers_that_have_no_pieces(what):
     size = torch.tensor([1.0, 2.0**-118 if what == "tiny values" else 1.0], device="cuda", dtype=torch.float64).repeat_interleave(head_size)
     error = ((out.double() - ref).abs() / torch.maximum(ref.abs(), size))[plain]
     assert float(error.max()) < 2**-24 * 300
+
+
+@pytest.mark.parametrize("head_size", [32, 64])
+@pytest.mark.parametrize("what", ["a large value at a small weight", "a column of tiny values"])
+def test_prompt_attention_whose_pieces_are_lost(head_size, what):
+    """Finite results of ordinary size (or exact zeros) to which numbers belong that leave no pieces: they are taken again in 32-bit."""
+    heads, lengths, contexts = 2, [100, 70], [0, 40]
+    arrays = _prompt(lengths, contexts, heads, head_size)
+    q, k_pages, v_pages, tables = arrays[0], arrays[1], arrays[2], arrays[5]
+    page = int(tables[0, 1])   # keys 32 to 63 of the first request
+    if what == "a column of tiny values":
+        v_pages[:, 1, :, 9] = 2.0**-136 * (1 + torch.rand(v_pages.shape[0], v_pages.shape[2], device="cuda"))
+    else:   # all scores 0, but -88 for key 35, whose weight is e^-88 = 6e-39 and whose value is 1.3e38
+        k_pages.zero_(), q.zero_()
+        k_pages[page, 0, 3, 0], q[:, 0] = -1.0, 88.0 * head_size**0.5
+        v_pages[page, 0, 3, 7] = 1.5 * 2.0**126
+    out = _attention(*arrays, lengths, heads, head_size)
+    ref = _exact(*(arrays[n] for n in (0, 1, 2, 5, 6, 7)), heads, head_size)
+    if what == "a column of tiny values":   # subnormal sums of at most 110 products over a total of at least 1, each a part of 2^-149 off: the weights add up to the total
+        at = head_size + 9
+        assert float((out[:, at].double() - ref[:, at]).abs().max()) <= 2**-149 * 4
+    else:   # the weight is subnormal, 2^-22 off itself, and so is its share of 0.8 / n; the rest as ever
+        assert float((out[:100, 7].double() - ref[:100, 7]).abs().max()) < 2**-20
+        assert float((ref[40:100, 7] - _exact(q, k_pages, v_pages.clamp(max=1e30), *(arrays[n] for n in (5, 6, 7)), heads, head_size)[40:100, 7]).abs().min()) > 1e-3   # (it counts)
