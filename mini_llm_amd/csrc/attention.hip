@@ -106,6 +106,11 @@ __device__ __forceinline__ void general_row(const T* __restrict__ q_row, const T
             for (int d = 0; d < head_size; d++) dot += my_q[d] * to_float(k_row[d]);
             score = options.softcap > 0.0f ? capped_score<true>(dot, options.softcap) : dot;
         }
+        if (__any(score != score)) {   // no number: nor is anything that comes of it
+            running_sum = score != score ? score : running_sum;
+            running_sum = wave_sum(running_sum);
+            break;
+        }
         float new_max = fmaxf(running_max, wave_max(score));
         const float reference = new_max == -INFINITY ? 0.0f : new_max;   // (only scores of minus infinity so far)
         float p = valid ? expf(score - reference) : 0.0f;

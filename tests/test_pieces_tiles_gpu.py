@@ -148,3 +148,17 @@ def test_prompt_attention_whose_pieces_are_lost(head_size, what):
     else:   # the weight is subnormal, 2^-22 off itself, and so is its share of 0.8 / n; the rest as ever
         assert float((out[:100, 7].double() - ref[:100, 7]).abs().max()) < 2**-20
         assert float((ref[40:100, 7] - _exact(q, k_pages, v_pages.clamp(max=1e30), *(arrays[n] for n in (5, 6, 7)), heads, head_size)[40:100, 7]).abs().min()) > 1e-3   # (it counts)
+
+
+@pytest.mark.parametrize("what", ["a tiny number", "a large number", "no number"])
+def test_a_query_taken_again_leaves_the_others_alone(what):
+    """Rows of a query tile that need no second way keep their results, bit for bit, beside one that does (and what is no number needs none)."""
+    heads, head_size, lengths, contexts = 2, 64, [100, 70], [0, 40]
+    arrays = _prompt(lengths, contexts, heads, head_size)
+    q, row = arrays[0], 40
+    plain = _attention(*arrays, lengths, heads, head_size)
+    q[row, 5] = {"a tiny number": 2.0**-100, "a large number": 2.0**70, "no number": torch.nan}[what]
+    out = _attention(*arrays, lengths, heads, head_size)
+    others = torch.arange(q.shape[0], device="cuda") != row
+    assert bool((out[others] == plain[others]).all()) and bool((out[row, head_size:] == plain[row, head_size:]).all())
+    assert bool(out[row, :head_size].isnan().all()) == (what == "no number")
