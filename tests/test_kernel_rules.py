@@ -101,3 +101,10 @@ def test_every_tile_of_the_product_in_pieces_has_a_shape_in_its_test():
     from test_pieces_tiles_gpu import SHAPES
 
     assert {shape[3] for shape in SHAPES} == {64064, 128064, 128096, 128128}
+
+
+def test_every_tile_of_the_product_in_pieces_is_compared_with_the_32_bit_instruction():
+    from mini_llm_amd.ops.library import library
+    from test_kernels_gpu import NEARER_SHAPES
+
+    assert {library().mllm_gemm_pieces_tile(*shape, 1) for shape in NEARER_SHAPES} == {64064, 128064, 128096, 128128}

@@ -882,6 +882,37 @@ def test_attention_picks_out_single_keys(K, path, dtype, page_size, window):
             assert np.abs(last - v[hot]).max() > 0.2, f"key {hot} lies outside the window and must not count"
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("sinks", [False, True])
+@pytest.mark.parametrize("key", [-np.inf, np.nan])
+def test_the_general_attention_over_keys_that_are_infinite_or_no_numbers(K, dtype, sinks, key):
+    # keys 0 to 69, more than the kernel takes at a time, score minus infinity: they add nothing, and rows that see no others have no result but a sink's; or key 3 is no
+    # number: nor are the rows behind it
+    rng = np.random.default_rng(9)
+    heads, size, total = 2, 40, 200
+    q, k, v = (bf16_round(rng.standard_normal((total, heads * size))) for _ in range(3))
+    q[:, 0] = 1.0
+    k[slice(0, 70) if key == -np.inf else 3, 0] = key
+    pages = [torch.zeros((7, heads, 32, size), device=DEV).to(dtype) for _ in range(2)]
+    K.cache_write(dev(k, dtype), dev(v, dtype), *pages, dev(np.arange(total), torch.int32), heads, size)
+    sink = dev([0.5, -0.5]) if sinks else None
+    out = host(K.paged_attention(dev(q, dtype), *pages, dev(np.zeros(total), torch.int32), dev(np.arange(total), torch.int32), dev(np.arange(7)[None], torch.int32), heads, heads, size,
+                                 size**-0.5, sinks=sink))
+    for h in range(heads):
+        at = slice(h * size, (h + 1) * size)
+        scores = q[:, at] @ np.where(np.isfinite(k[:, at]), k[:, at], 0.0).T * size**-0.5
+        if h == 0:
+            scores[:, slice(0, 70) if key == -np.inf else 3] = key
+        scores[~np.tri(total, dtype=bool)] = -np.inf
+        top = np.maximum(np.nanmax(scores, axis=1), -1e30)
+        weights = np.exp(scores - top[:, None])
+        with np.errstate(invalid="ignore"):
+            ref = weights @ v[:, at] / (weights.sum(1) + (np.exp(float(sink[h]) - top) if sinks else 0.0))[:, None]
+        if h == 0 and key == -np.inf:
+            ref[:70] = 0.0 if sinks else np.nan   # no key: the sink's share of nothing, or none
+        np.testing.assert_allclose(out[:, at], ref, atol=2e-5 if dtype == torch.float32 else 2e-2, rtol=2e-5)
+
+
 @pytest.mark.parametrize("rows,cols", [(1, 1), (33, 65), (96, 288), (1000, 96), (31, 32)])
 @pytest.mark.parametrize("src,dst", [(torch.float32, torch.bfloat16), (torch.bfloat16, torch.float32), (torch.float32, torch.float32)])
 def test_convert_and_transpose(K, rows, cols, src, dst):
@@ -1145,7 +1176,10 @@ def test_32_bit_products_in_pieces_lean_to_no_side(K):
     assert np.abs(host(K.linear(dev(x), K.pack_matrix(dev(w)))) / ref - 1).max() < 2**-24 + 2 * 2**-24
 
 
-@pytest.mark.parametrize("m,n,k", [(130, 768, 768), (520, 260, 3072), (2048, 200, 320)])   # tiles of each size
+NEARER_SHAPES = [(130, 768, 768), (520, 260, 3072), (2048, 200, 320), (1281, 772, 384), (897, 2180, 384), (2690, 2308, 288)]   # tiles of each size (test_kernel_rules.py sees to it)
+
+
+@pytest.mark.parametrize("m,n,k", NEARER_SHAPES)
 @pytest.mark.parametrize("kind", ["normal", "relu", "one sign"])
 def test_32_bit_products_in_pieces_are_nearer_than_32_bit_ones(K, m, n, k, kind):
     # the small products have a running sum of their own, so the large one is rounded once for sixteen numbers of K, where the 32-bit instruction rounds
