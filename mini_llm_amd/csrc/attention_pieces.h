@@ -9,10 +9,13 @@
 // after the next. A tile's numbers go from LDS into registers a tile before they are used, so that one place for keys and one for values is enough, and two blocks share
 // a compute unit: one's waits run under the other's instructions (blocks of 64 queries, which split a tile's keys and values for twice the products but leave room for one
 // block alone, us: two prompts of 1,024 tokens x 12 heads of 64 46 and 42 so, eight of 256 30 and 24, one of 4,096 217 and 204).
-// With the 32-bit instruction, a quarter of the pieces' rate, one block a unit and the library's expf -> now, us: those 64.6 -> 42.2, 34.3 -> 24.4 and 331 -> 204, five prompts of 67
-// to 1,001 77.4 -> 46.6, 512 queries on 7,680 cached keys 193 -> 132, 32 prompts of 70 44.8 -> 29.0, one of 128 10.1 -> 9.7; four of 512 over a window with a cap 52.3 -> 37.1.
-// In a sum of six products the five small ones come first, so that the large sum is rounded once for sixteen numbers (the 32-bit instruction: eight times). Against 64 bits, normally
-// distributed numbers: 2.6e-7 -> 1.5e-7 for the first of these, 8.7e-7 -> 7.4e-7 over 8,192 keys.
+// With the 32-bit instruction, a quarter of the pieces' rate, one block a unit and the library's expf -> now, alone in a loop, us: those 58.8 -> 39.2, 32.3 -> 21.6 and 329 -> 197, five
+// prompts of 67 to 1,001 70.3 -> 39.7, 512 queries on 7,680 cached keys 192 -> 120, 32 prompts of 70 43.7 -> 25.3, one of 66 9.2 -> 8.4, of 128 9.4 -> 8.4; four of 512 over a window of 128
+// with a cap 41.0 -> 24.6. (The blocks' shapes above were compared before the queries' check lost its branches, 0.8 to 1.4 us a block.)
+// In a sum of six products the five small ones come first. A score's sum starts at zero, so the large one is rounded once for sixteen numbers (the 32-bit instruction: eight times);
+// the values' sum runs over all tiles and takes all six, six roundings for sixteen keys, in which the small ones are lost once it is long (a second sum for them, as gemm_pieces.h
+// has it, would take 32 registers that are not there). Against 64 bits, normally distributed numbers: 2.6e-7 -> 1.5e-7 for the first of these, 8.7e-7 -> 7.3e-7 over 8,192 keys.
+// (The instruction cuts its sums off downwards: errors lie 2e-8 to 7e-8 of the results' mean magnitude below zero on average, with the 32-bit instruction 1e-8 or less.)
 // What pieces cannot hold: a number that is not finite or rounds to infinity has no pieces, and whatever it meets comes out as no number; numbers below 2^-110 lose
 // their third piece, below 2^-134 all of them, and weights below 2^-126 are 0. So a weighted sum of values may be off by 2^-126 for each key, times the largest value of its
 // column, or by 2^-134 for each, times its weight. Rows with results that are not finite, with weighted sums below 2^-90 or below 2^-90 times the largest value of their column
@@ -146,7 +149,7 @@ __global__ __launch_bounds__(64 * WAVES, 2) void attention_prefill_pieces_kernel
     int n_kv_heads, int page_shift, int given_window, float scale, ScoreOptions options) {
     typedef Layout<float, HD, WAVES> L;
     const int window = FORM == CAUSAL ? 0 : given_window, chunk = FORM == CAUSAL ? 0 : options.chunk;
-    constexpr int QUERIES = 32, KS = HD / 16, DT = HD / 32, WAVE_BYTES = wave_bytes<HD>();
+    constexpr int KS = HD / 16, DT = HD / 32, WAVE_BYTES = wave_bytes<HD>();
     static_assert(WAVE_BYTES >= QUERIES * HD * 4 && WAVE_BYTES >= MAX_HEAD * 4, "what a wave leaves takes the place of its tiles");
     extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
     __shared__ float stats_lds[WAVES][QUERIES][2];
@@ -174,7 +177,7 @@ __global__ __launch_bounds__(64 * WAVES, 2) void attention_prefill_pieces_kernel
     const int n_tiles = kept_tiles + (block_last_position - first_base) / KEYS + 1;
     const int n_mine = n_tiles > wave ? (n_tiles - wave + WAVES - 1) / WAVES : 0;  // tiles wave, wave + WAVES, ...
 
-    // One half (keys or values) of this wave's i-th tile, into place i % 2; beyond the wave's last tile that one again, never used (the count of loads in flight is then the
+    // One half (keys or values) of this wave's i-th tile, into the one place there is for each; beyond the wave's last tile that one again, never used (the count of loads in flight is then the
     // same in every step), and behind the last stored key that key's row again, masked by position.
     unsigned char* const wave_lds = lds + wave * WAVE_BYTES;
     auto tile_base = [&](int i) {

@@ -115,7 +115,7 @@ __device__ __forceinline__ void read_transposed<4, 256>(const unsigned (&address
 
 template <typename T, int HD, int SPLITS>
 struct Layout {
-    static constexpr bool FP32 = sizeof(T) == 4;
+    static constexpr bool FP32 = sizeof(T) == 4;   // attention_pieces.h, which loads tiles as this file does
     static constexpr int ROW_BYTES = HD * (int)sizeof(T);
     static constexpr int PPR = ROW_BYTES / 16;      // 16-byte pieces per row
     static constexpr int ROWS_PER_LOAD = 1024 / ROW_BYTES;  // rows a wave's 1 KiB load covers

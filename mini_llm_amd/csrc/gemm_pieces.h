@@ -8,8 +8,8 @@
 // smaller products have a running sum of their own, added to the large one at the end: in one sum they are lost to its rounding once it is long, and it is
 // rounded six times for sixteen numbers of K instead of once (the 32-bit instruction: eight times). Measured against 64-bit sums over rows of 768 and 3,072
 // normally distributed numbers: 1.6e-7 and 3.4e-7 of the result's norm, in one sum 4.2e-7 and 8.6e-7, with the 32-bit instruction 5.0e-7 and 9.9e-7; over
-// rows of which half are zero, as behind a clamp, 1.2e-7 and 2.7e-7, 4.0e-7 and 8.2e-7, 3.5e-7 and 7.1e-7. It is the 64 registers that the 128 x 128 tile
-// has left (188 -> 252, none spilled), and little time: 2,048 x 3,072 x 768 60.6 us, 63.2 in one sum, on another machine 64.4 and 63.3.
+// rows of which half are zero, as behind a clamp, 1.2e-7 and 2.7e-7, 4.0e-7 and 8.2e-7, 3.5e-7 and 7.1e-7. It is 64 registers that the 128 x 128 tile
+// has left (238 in all, none spilled), and little time: with the loop before the present one 2,048 x 3,072 x 768 60.6 us, 63.2 in one sum, on another machine 64.4 and 63.3.
 //
 // W's pieces are laid out once, when the matrix is packed (common.h: packed_pieces): the chunks of the packed layout for bfloat16, the three of a k-step
 // behind each other. A's rows come as they are, and a wave splits the fragments it has read.
@@ -19,8 +19,9 @@
 // only where they stand between them: a tile's 48 products behind the splitting of their rows, step by step, take 2,101 cycles, with the splitting of the next step's rows between
 // them 1,609, and of two waves a SIMD that split first and multiply then each 1,860. So a step's products carry the splitting of the next step's rows, its fragment reads, and one by one
 // the loads of the tile after the next (a compute unit takes a load of 1 KiB every 16 cycles, and a wave that asks for all at once waits).
-// With the loads at a tile's start and the splitting in front of its products (us -> now): 2,048 x 2,304 x 768 56.2 -> 48.4 (128 x 96), 2,048 x 3,072 x 768 65.9 -> 60,
-// 2,670 x 768 x 3,072 in two 81.8 -> 70.5, 8,192 x 3,072 x 768 212 -> 203.
+// With the loads at a tile's start and the splitting in front of its products -> now, alone in a loop, on one machine in turn, us: 2,048 x 2,304 x 768 53.5 -> 44.4 (64 x 64, 128 x 96),
+// 2,048 x 3,072 x 768 58.3 -> 51.5 (128 x 64, 128 x 96), 2,670 x 768 x 3,072 in two 79.2 -> 67.6; on one that gives less power 69.8 -> 58.3, 71.1 -> 60.2, 90.1 -> 81.4 and
+// 8,192 x 3,072 x 768 217 -> 211; in a prompt step of 2,048 rows the first two take 52 and 63 us.
 // Fragment reads are inline assembly with waits of their own: through the compiler each would wait for the loads into LDS that are under way.
 #pragma once
 
@@ -482,10 +483,10 @@ void launch_whole(const float* a, const float* w, const float* bias, const float
 
 // The tiles, and what they cost in microseconds: what lies in front of and behind a block's loop, and a tile of K for each block of a compute unit, alone there or not, and
 // more the nearer a round of blocks is to all 256 units (they share the chip's power: products of numbers that are all zero take three quarters of the time).
-// Fitted to 900 products of 66 to 6,000 rows, 512 to 4,096 columns, K of 768 to 4,096, whole and cut, to 3 to 6 %. A compute unit brings most out of 128 x 128; 128 x 96
+// Fitted to 900 products of 66 to 6,000 rows, 512 to 4,096 columns, K of 768 to 4,096, whole and cut. A compute unit brings most out of 128 x 128; 128 x 96
 // where its blocks are two rounds and 128 x 128's more than one; narrow outputs and few rows fill the chip with smaller ones.
-// 128 x 128 / 128 x 64 / 64 x 64 / 128 x 96, us: 2,048 x 2,304 x 768 58.0 / 53.5 / 53.6 / 48.4, 2,670 x 768 x 3,072 in two 70.5 / 71.5 / 84.2 / 83.5,
-// 2,048 x 768 x 3,072 in two 64.9 / 62.9 / 65.9 / 55.5, 8,192 x 3,072 x 768 217 / 228 / 258 / 214, 130 x 768 x 768 in six 10.9 / 7.7 / 6.2 / 9.7.
+// 128 x 128 / 128 x 64 / 64 x 64 / 128 x 96, us (more sizes: profiles/pieces_tiles_f32.md): 2,048 x 2,304 x 768 53.7 / 49.0 / 49.9 / 44.4, 2,670 x 768 x 3,072 in two 67.6 / 67.6 /
+// 79.9 / 82.4, 2,048 x 768 x 3,072 in two 58.6 / 59.0 / 61.6 / 52.9, 130 x 2,304 x 768 28.6 / 18.5 / 14.9 / 22.8.
 struct Choice {
     int bm, bn;
     float start, alone, tile, full;
@@ -494,7 +495,9 @@ constexpr int CHOICES_COUNT = 4;
 constexpr Choice CHOICES[CHOICES_COUNT] = {{128, 128, 7.5f, 0.07f, 0.83f, 0.30f}, {128, 64, 5.6f, 0.065f, 0.44f, 0.20f}, {64, 64, 4.9f, 0.09f, 0.29f, 0.09f}, {128, 96, 7.25f, 0.025f, 0.64f, 0.25f}};
 
 // Microseconds of a product cut into k_blocks along K with the best of the tiles (`best`): the rounds of blocks, the start and end of a block, and the sums
-// that are written (6 TB/s). Its choice is within 1 % of the best of the four on average over the products above, and at most a fifth longer (2,670 x 512 x 768 in six).
+// that are written (6 TB/s). Measured at 440 sizes that it was not fitted to: whole products of as many columns as K or more 0.4 % behind the best of the four on average and 15 % at
+// most, cut ones of as many at most 1.6 % behind the best tile and count, and 18 % at most (130 and 170 rows: the count is that of 256). Fitted to those instead it came to
+// 0.3 and 1.0 % there, and at 559 further sizes was 0.3 % faster on average and up to a quarter slower (550 x 896 x 1,792 19.0 -> 23.8 us): left as it is.
 inline float cost(int M, int N, int K, int k_blocks, int& best) {
     float best_cost = 0.0f;
     for (int c = 0; c < CHOICES_COUNT; c++) {

@@ -906,7 +906,7 @@ def test_the_general_attention_over_keys_that_are_infinite_or_no_numbers(K, dtyp
         scores[~np.tri(total, dtype=bool)] = -np.inf
         top = np.maximum(np.nanmax(scores, axis=1), -1e30)
         weights = np.exp(scores - top[:, None])
-        with np.errstate(invalid="ignore"):
+        with np.errstate(invalid="ignore", over="ignore"):
             ref = weights @ v[:, at] / (weights.sum(1) + (np.exp(float(sink[h]) - top) if sinks else 0.0))[:, None]
         if h == 0 and key == -np.inf:
             ref[:70] = 0.0 if sinks else np.nan   # no key: the sink's share of nothing, or none
