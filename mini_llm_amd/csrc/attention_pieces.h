@@ -9,9 +9,9 @@
 // after the next. A tile's numbers go from LDS into registers a tile before they are used, so that one place for keys and one for values is enough, and two blocks share
 // a compute unit: one's waits run under the other's instructions (blocks of 64 queries, which split a tile's keys and values for twice the products but leave room for one
 // block alone, us: two prompts of 1,024 tokens x 12 heads of 64 46 and 42 so, eight of 256 30 and 24, one of 4,096 217 and 204).
-// With the 32-bit instruction, a quarter of the pieces' rate, one block a unit and the library's expf -> now, alone in a loop, us: those 58.8 -> 39.2, 32.3 -> 21.6 and 329 -> 197, five
-// prompts of 67 to 1,001 70.3 -> 39.7, 512 queries on 7,680 cached keys 192 -> 120, 32 prompts of 70 43.7 -> 25.3, one of 66 9.2 -> 8.4, of 128 9.4 -> 8.4; four of 512 over a window of 128
-// with a cap 41.0 -> 24.6. (The blocks' shapes above were compared before the queries' check lost its branches, 0.8 to 1.4 us a block.)
+// With the 32-bit instruction, a quarter of the pieces' rate, one block a unit and the library's expf -> now, alone in a loop, us: those 58.8 -> 39.6, 32.3 -> 21.9 and 329 -> 194, five
+// prompts of 67 to 1,001 70.3 -> 39.8, 512 queries on 7,680 cached keys 192 -> 120, 32 prompts of 70 43.7 -> 25.7, one of 66 9.2 -> 8.5, of 128 9.4 -> 8.6; four of 512 over a window of 128
+// with a cap 41.0 -> 24.7. (The blocks' shapes above were compared before the queries' check lost its branches, 0.8 to 1.4 us a block.)
 // In a sum of six products the five small ones come first. A score's sum starts at zero, so the large one is rounded once for sixteen numbers (the 32-bit instruction: eight times);
 // the values' sum runs over all tiles and takes all six, six roundings for sixteen keys, in which the small ones are lost once it is long (a second sum for them, as gemm_pieces.h
 // has it, would take 32 registers that are not there). Against 64 bits, normally distributed numbers: 2.6e-7 -> 1.5e-7 for the first of these, 8.7e-7 -> 7.3e-7 over 8,192 keys.
@@ -21,7 +21,7 @@
 // column, or by 2^-134 for each, times its weight. Rows with results that are not finite, with weighted sums below 2^-90 or below 2^-90 times the largest value of their column
 // (zeros among them, unless every value of the column is zero), or whose queries hold numbers beyond 2^64 or below 2^-90 (which could make up for keys that lost their pieces), are
 // taken again one by one in 32-bit (general_row), but for queries that hold what is no number: nothing else can come of them. (General_row ends at the first key whose score is none, so
-// that a key which is no number costs the rows behind it a few steps and not a walk: two prompts of 1,024 tokens x 12 heads, of which key 3 is none, 1,484 -> 71 us.)
+// that a key which is no number costs the rows behind it a few steps and not a walk: two prompts of 1,024 tokens x 12 heads, of which key 3 is none, 1,484 -> 72 us.)
 #pragma once
 
 #include "number_pieces.h"
@@ -427,7 +427,8 @@ __global__ __launch_bounds__(64 * WAVES, 2) void attention_prefill_pieces_kernel
     if (tid == 0) again = 0;
     __syncthreads();
     bool odd = odd_queries >> lane32 & 1;
-    if (own_query < q_len) {   // of every 32 columns wave w finishes 8 w .. + 8
+    f32x4 o[DT];   // of every 32 columns wave w finishes 8 w .. + 8
+    if (own_query < q_len) {
         float best = -INFINITY;
 #pragma unroll
         for (int w = 0; w < WAVES; w++) best = fmaxf(best, stats_lds[w][lane32][0]);
@@ -439,10 +440,9 @@ __global__ __launch_bounds__(64 * WAVES, 2) void attention_prefill_pieces_kernel
         }
         if (options.sinks) total += expf(options.sinks[head] - best);   // the sink: once, with no value
         const float inverse = 1.0f / total;
-        float* const out_row = out + (size_t)(q_first + own_query) * out_stride + head * HD + 8 * wave + 4 * half;
 #pragma unroll
         for (int i2 = 0; i2 < DT; i2++) {
-            f32x4 o, most = {0.0f, 0.0f, 0.0f, 0.0f};
+            f32x4 most = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
             for (int w = 0; w < WAVES; w++) {
                 const f32x4 here = *reinterpret_cast<const f32x4*>(&largest_lds[w][i2 * 32 + 8 * wave + 4 * half]);
@@ -455,16 +455,20 @@ __global__ __launch_bounds__(64 * WAVES, 2) void attention_prefill_pieces_kernel
 #pragma unroll
                 for (int w = 0; w < WAVES; w++) sum += weight[w] * reinterpret_cast<const float*>(lds + w * WAVE_BYTES)[(i2 * 16 + 4 * wave + e) * WAVE + lane];
                 odd |= (most[e] > 0.0f) & (fabsf(sum) < fmaxf(most[e], 1.0f) * 0x1p-90f);
-                o[e] = sum * inverse;
-                odd |= !(fabsf(o[e]) < INFINITY);
+                o[i2][e] = sum * inverse;
+                odd |= !(fabsf(o[i2][e]) < INFINITY);
             }
-            *reinterpret_cast<f32x4*>(out_row + i2 * 32) = o;
         }
     }
     const unsigned odd_rows = rows_of(odd & (own_query < q_len)) & ~none_rows;
     if (odd_rows != 0 && lane == 0) atomicOr(&again, odd_rows);
     __syncthreads();
     unsigned rows = __builtin_amdgcn_readfirstlane(again);
+    if (own_query < q_len && !(rows >> lane32 & 1)) {   // (not the others: they are read once more below, and the output may lie where they do)
+        float* const out_row = out + (size_t)(q_first + own_query) * out_stride + head * HD + 8 * wave + 4 * half;
+#pragma unroll
+        for (int i2 = 0; i2 < DT; i2++) *reinterpret_cast<f32x4*>(out_row + i2 * 32) = o[i2];
+    }
     float* my_q = reinterpret_cast<float*>(lds + wave * WAVE_BYTES);
     for (int n = 0; rows != 0; rows &= rows - 1, n++) {   // by the waves in turn
         if (n % WAVES != wave) continue;

@@ -225,3 +225,15 @@ def test_a_query_taken_again_leaves_the_others_alone(what):
     others = torch.arange(q.shape[0], device="cuda") != row
     assert bool((out[others] == plain[others]).all()) and bool((out[row, head_size:] == plain[row, head_size:]).all())
     assert bool(out[row, :head_size].isnan().all()) == (what == "no number")
+
+
+def test_prompt_attention_over_its_own_queries():
+    """Results may take the queries' place: what is taken again reads them before anything is stored over them."""
+    heads, head_size, lengths, contexts = 2, 64, [100, 70], [0, 40]
+    arrays = _prompt(lengths, contexts, heads, head_size)
+    arrays[2][int(arrays[5][0, 1]), 1, 4, 7] = -torch.inf
+    arrays[0][50, 3] = 2.0**-100
+    want = _attention(*arrays, lengths, heads, head_size)
+    got = _attention(*arrays, lengths, heads, head_size, out=arrays[0])
+    assert got.data_ptr() == arrays[0].data_ptr() and bool(got.isfinite().any())
+    torch.testing.assert_close(got, want, rtol=0, atol=0, equal_nan=True)
