@@ -308,6 +308,9 @@ def measure_kernels(engine, batch: int = 8, context: int = 776, decode: bool = T
         layer_us = sum(us for _, us in cut[1])
         note("decode_layer", layer_us, (4.0 * d * d + 2.0 * d * ff) * e + cache_bytes, hbm, "HBM peak")
         out["decode_layer"]["by_entry_point"] = _by_entry_point([name for name, _ in cut[1]], [us for _, us in cut[1]])
+    if len(names) == 5 and names[1] == "decode_stack":   # all layers in one kernel
+        note("decode_stack", each[1], n_layer * ((4.0 * d * d + 2.0 * d * ff) * e + cache_bytes), hbm, "HBM peak")
+        cut = (names[0], each[0]), None, list(zip(names[-3:], each[-3:]))
     if cut is not None:
         out["decode_embed"] = {"us": round(cut[0][1], 2), "holds": "what a replay costs by itself"}
         (_, final_norm), (_, head), (_, choice) = cut[2]
@@ -343,7 +346,7 @@ _KERNEL_CLASSES = {
                  "projection_rows", "head_gate", "gated_norm", "short_conv", "map_rows", "map_difference", "turn_heads", "gate_unit", "route", "route_rows", "expert_unit", "expert_lists",
                  "branch_join", "join_norms", "soft_cap"),
     "recurrence": ("recurrence", "recurrence_chunked", "gated_scan", "channel_memory"),
-    "layer kernels": ("decode_attention_half", "decode_mlp_half"),
+    "layer kernels": ("decode_attention_half", "decode_mlp_half", "decode_stack"),
     "choice": ("choose", "sample"),
 }
 

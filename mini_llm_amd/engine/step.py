@@ -174,9 +174,15 @@ class _DecodeGraph:
         batch = self.static_batch
         batch.request_ids = [e.request_id for e in entries]
         if self.graph is None:
+            self._take_stack(batch)
             self.graph, self.logits = _capture(runner, batch, lanes=self.lanes)
         self.graph.replay()
         return batch, self.logits[: len(entries)]
+
+    def _take_stack(self, batch) -> None:
+        """One kernel for all layers, where the model has one for steps like this one (it lives as long as the graph that launches it)."""
+        if self.lanes is None:
+            batch.stack = self.runner.model.decode_stack(batch, self.runner.cache)
 
     def _run_choosing(self, entries, sampling=None):
         import torch
@@ -208,6 +214,7 @@ class _DecodeGraph:
         batch = self.static_batch
         batch.request_ids = [e.request_id for e in entries]
         if self.graph is None:
+            self._take_stack(batch)
             draws = DrawParameters(*self.builder.draw_views(self.buffer)) if self.draws else None
             choice = TokenChoice(cache.last_token, host_ring=self.ring, cursor=self.builder.cursor_view(self.buffer), advance=True, draws=draws)
             self.graph, self.logits = _capture(runner, batch, choice, self.lanes)

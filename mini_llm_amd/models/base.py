@@ -178,10 +178,27 @@ class Model(Part):
             out[EMBEDDING_STATE] = need
         return out
 
+    def decode_stack(self, batch, cache):
+        """One kernel for all layers of a step of single tokens like ``batch`` (kernels.DecodeStack), or None where the model, its sizes or the batch's
+        have none. It holds the addresses of the model's tensors and of the cache's pages, as a captured step does, and belongs to one."""
+        if self.step_vectors is not None or [call.block for call in self.schedule] != list(range(len(self.blocks))) or len(cache.groups) != 1:
+            return None
+        layers = [getattr(self.blocks[call.block], "stack_layer", lambda ctx: None)(cache.layer_context(batch, call)) for call in self.schedule]
+        if not layers or None in layers or any(shared != layers[0][1] for _, shared in layers):
+            return None
+        width, inner, n_heads, head_size, page_size, eps_1, eps_2, scale, activation = layers[0][1]
+        if not kernels.decode_stack_pays(batch.n_tokens, batch.max_total_len, len(layers), width, inner, n_heads, head_size, page_size, layers[0][0].w_qkv.dtype):
+            return None
+        if any(pages.numel() * pages.element_size() >= 2**32 for layer, _ in layers for pages in (layer.k_pages, layer.v_pages)):   # what the kernel's offsets reach
+            return None
+        return kernels.DecodeStack([layer for layer, _ in layers], batch.n_tokens, n_heads, eps_1, eps_2, scale, activation)
+
     def _layers(self, hidden, batch, cache, observer=None):
         """The schedule over the rows of ``batch``; the stream comes back as the last layer leaves it. A layer is told what comes ahead of
         the next one (``Ahead``) and may do it in its own last kernel; it is not told of a vector that joins the stream behind it while an
         observer looks on, which is shown the stream as the layer alone leaves it."""
+        if getattr(batch, "stack", None) is not None and observer is None:
+            return batch.stack.run(kernels.settle(hidden), batch.token_request, batch.positions, batch.groups[0].slots, batch.groups[0].block_tables)
         told = None
         for index, call in enumerate(self.schedule):
             block = self.blocks[call.block]

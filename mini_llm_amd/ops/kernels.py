@@ -935,6 +935,93 @@ def decode_mlp_half(hidden, gamma, beta, eps, w_up, b_up, w_down, b_down, activa
     return PendingRows(summed, out, b_down)
 
 
+@dataclass
+class StackLayer:
+    """One pre-norm layer as the kernel for whole stacks takes it: two layer norms with their eps, the four products with biases
+    (PackedMatrix and float32 vector), the layer's cache pages."""
+
+    gain_1: torch.Tensor
+    offset_1: torch.Tensor
+    w_qkv: "PackedMatrix"
+    b_qkv: torch.Tensor
+    w_out: "PackedMatrix"
+    b_out: torch.Tensor
+    gain_2: torch.Tensor
+    offset_2: torch.Tensor
+    w_up: "PackedMatrix"
+    b_up: torch.Tensor
+    w_down: "PackedMatrix"
+    b_down: torch.Tensor
+    k_pages: torch.Tensor
+    v_pages: torch.Tensor
+
+
+def decode_stack_supported(rows, n_layers, width, inner, n_heads, head_size, page_size, dtype) -> bool:
+    """Whether one kernel decodes all layers of such a model for so many rows (``decode_stack``)."""
+    return bool(library().mllm_decode_stack_supported(int(rows), int(n_layers), int(width), int(inner), int(n_heads), int(head_size), int(page_size), _code(dtype)))
+
+
+def decode_stack_pays(rows, reach, n_layers, width, inner, n_heads, head_size, page_size, dtype) -> bool:
+    """Whether a step of so many rows, of sequences up to ``reach`` tokens, is faster as one kernel than layer by layer (the library's own answer, where
+    the measurements behind it are written down)."""
+    return (decode_stack_supported(rows, n_layers, width, inner, n_heads, head_size, page_size, dtype)
+            and bool(library().mllm_decode_stack_pays(int(rows), int(reach), int(width))))
+
+
+class DecodeStack:
+    """All layers of a pre-norm model for up to ``rows`` rows that bring one token each, in one kernel. Holds what the launches of one captured step
+    share: the layers' tensors (and their addresses on the device), the words that the blocks of a launch hand to each other and the launch's control words.
+    Launches of one DecodeStack follow each other on a stream; steps that may run side by side have one each."""
+
+    def __init__(self, layers, rows: int, n_heads: int, eps_1: float, eps_2: float, scale: float, activation: str, blocks: int | None = None):
+        """``blocks``: blocks of a launch (None: one for each compute unit)."""
+        first = layers[0]
+        self.layers, self.rows, self.n_heads = list(layers), int(rows), int(n_heads)
+        self.eps_1, self.eps_2, self.scale, self.activation = float(eps_1), float(eps_2), float(scale), activation
+        self.width, self.inner = first.w_up.cols, first.w_up.rows
+        self.dtype, device = first.w_qkv.dtype, first.k_pages.device
+        head_size = self.width // self.n_heads
+        _, self.page_size = _check_pages(first.k_pages, first.v_pages, n_heads, head_size)
+        _require(activation in ("gelu_new", "gelu"), f"unknown activation {activation!r}")
+        _require(decode_stack_supported(rows, len(layers), self.width, self.inner, n_heads, head_size, self.page_size, self.dtype), "no kernel for a stack of these sizes")
+        width, inner = self.width, self.inner
+        for i, layer in enumerate(layers):
+            for w, name, shape in ((layer.w_qkv, "w_qkv", (3 * width, width)), (layer.w_out, "w_out", (width, width)),
+                                   (layer.w_up, "w_up", (inner, width)), (layer.w_down, "w_down", (width, inner))):
+                _require(isinstance(w, PackedMatrix) and w.dtype == self.dtype and w.shape == shape, f"layer {i}: {name} is no packed matrix {shape} of {self.dtype}")
+                _device_tensor(w.data, name, self.dtype, 1)
+            for v, name, n in ((layer.gain_1, "gain_1", width), (layer.offset_1, "offset_1", width), (layer.b_qkv, "b_qkv", 3 * width), (layer.b_out, "b_out", width),
+                               (layer.gain_2, "gain_2", width), (layer.offset_2, "offset_2", width), (layer.b_up, "b_up", inner), (layer.b_down, "b_down", width)):
+                _device_tensor(v, name, torch.float32, 1)
+                _require(v.shape[0] == n, f"layer {i}: {name} does not match its matrix")
+            _check_pages(layer.k_pages, layer.v_pages, n_heads, head_size)
+            _require(layer.k_pages.dtype == self.dtype and layer.k_pages.shape[2] == self.page_size, f"layer {i}: pages of another kind")
+            _require(layer.k_pages.numel() * layer.k_pages.element_size() < 2**32, f"layer {i}: more keys than 32-bit offsets reach")
+        names = StackLayer.__dataclass_fields__
+        _require(library().mllm_decode_stack_layer_pointers() == len(names), "a layer's pointers do not match the library's")
+        addresses = [[_ptr(getattr(layer, name).data if isinstance(getattr(layer, name), PackedMatrix) else getattr(layer, name)) for name in names] for layer in layers]
+        self.addresses = torch.tensor(addresses, dtype=torch.int64, device=device)
+        self.words = torch.zeros(int(library().mllm_decode_stack_word_bytes(self.rows, width, inner, _code(self.dtype))) // 4, dtype=torch.int32, device=device)
+        self.control = torch.zeros(int(library().mllm_decode_stack_control_ints()), dtype=torch.int32, device=device)
+        self.blocks = torch.cuda.get_device_properties(device).multi_processor_count if blocks is None else int(blocks)
+
+    def run(self, hidden, token_request, positions, slots, block_tables):
+        """hidden: float32 [rows, width], each row the newest token of its request -> the stream behind the last layer. Keys and values
+        go into the cache."""
+        _device_tensor(hidden, "hidden", torch.float32, 2)
+        _require(tuple(hidden.shape) == (self.rows, self.width), f"the rows are not [{self.rows}, {self.width}]")
+        for t, name in ((slots, "slots"), (token_request, "token_request"), (positions, "positions")):
+            _device_tensor(t, name, torch.int32, 1)
+            _require(t.shape[0] >= self.rows, f"{name} has fewer entries than rows")
+        _device_tensor(block_tables, "block_tables", torch.int32, 2)
+        out = torch.empty_like(hidden)
+        check(library().mllm_decode_stack(
+            _ptr(self.addresses), len(self.layers), _ptr(hidden), _ptr(out), _ptr(token_request), _ptr(positions), _ptr(slots), _ptr(block_tables), block_tables.shape[1],
+            _ptr(self.words), _ptr(self.control), self.rows, self.width, self.inner, self.n_heads, self.page_size, self.eps_1, self.eps_2, self.scale,
+            EPILOGUES[self.activation], _code(self.dtype), self.blocks, _stream()))
+        return out
+
+
 # -- layers that norm after the sum, norm their heads, gate their feed-forward, or keep a latent -----------------
 RMS_NORM_TWICE_WIDTH = 2048   # the widest rows that one launch norms twice (they stay in a wave's registers between the two)
 

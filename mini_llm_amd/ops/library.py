@@ -49,6 +49,12 @@ _SIGNATURES = {
     "mllm_decode_attention_half": [P, P, P, c_int, P, P, P, c_float, P, P, P, P, P, P, P, P, P, c_int, P,
                                    c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_float, c_int, P],
     "mllm_decode_mlp_half": [P, P, P, c_int, P, P, P, c_float, P, P, P, P, c_int, c_int, c_int, c_int, c_int, P],
+    "mllm_decode_stack_supported": [c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int],
+    "mllm_decode_stack_pays": [c_int, c_int, c_int],
+    "mllm_decode_stack_word_bytes": [c_int, c_int, c_int, c_int],
+    "mllm_decode_stack_control_ints": [],
+    "mllm_decode_stack_layer_pointers": [],
+    "mllm_decode_stack": [P, c_int, P, P, P, P, P, P, c_int, P, P, c_int, c_int, c_int, c_int, c_int, c_float, c_float, c_float, c_int, c_int, c_int, P],
     "mllm_pending_sum": [P, P, P, c_int, P, c_int, c_int, P],
     "mllm_linear_split_static": [P, P, c_int, P, P, P, c_int, c_int, c_int, c_int, c_int, P],
     "mllm_static_scratch_prepare": [],
@@ -130,7 +136,7 @@ def library() -> ctypes.CDLL:
             fn = getattr(lib, name)
             fn.argtypes = argtypes
             fn.restype = c_int
-        lib.mllm_packed_elements.restype = lib.mllm_pieces_bytes.restype = c_longlong
+        lib.mllm_packed_elements.restype = lib.mllm_pieces_bytes.restype = lib.mllm_decode_stack_word_bytes.restype = c_longlong
         lib.mllm_static_scratch_bytes.restype = c_longlong
         lib.mllm_static_scratch_bytes.argtypes = []
         lib.mllm_last_error.restype = ctypes.c_char_p

@@ -22,6 +22,25 @@ class PreNormBlock(Block):
 
     takes_pending = True
 
+    def stack_layer(self, ctx: LayerContext):
+        """The layer as the kernel for whole stacks takes it, (kernels.StackLayer, the numbers that all layers of a stack share), or None where
+        it does not: layer norms around plain causal attention over a whole cache and a dense feed-forward, every matrix packed, every product with a bias."""
+        from ..ops import kernels
+        from .attention import CausalSelfAttention
+        from .feedforward import DenseMLP
+        from .norms import LayerNorm
+
+        mixer, mlp = self.mixer, self.feed_forward
+        if not (type(mixer) is CausalSelfAttention and type(mlp) is DenseMLP and type(self.norm_1) is LayerNorm and type(self.norm_2) is LayerNorm):
+            return None
+        products = (mixer.qkv, mixer.out, mlp.up, mlp.down)
+        if (mixer.window is not None or mixer.n_kv_heads != mixer.n_heads or mixer.q_width != mixer.width or not ctx.write_cache or ctx.k_pages is None
+                or any(not isinstance(p.weight, kernels.PackedMatrix) or p.bias is None or p.weight.dtype != ctx.k_pages.dtype for p in products)):
+            return None
+        layer = kernels.StackLayer(self.norm_1.weight, self.norm_1.bias, mixer.qkv.weight, mixer.qkv.bias, mixer.out.weight, mixer.out.bias,
+                                   self.norm_2.weight, self.norm_2.bias, mlp.up.weight, mlp.up.bias, mlp.down.weight, mlp.down.bias, ctx.k_pages, ctx.v_pages)
+        return layer, (mixer.width, mlp.inner, mixer.n_heads, mixer.head_size, ctx.k_pages.shape[2], self.norm_1.eps, self.norm_2.eps, mixer.scale, mlp.activation)
+
     def forward(self, hidden, ctx: LayerContext):
         hidden = self.mixer.forward_normed(hidden, self.norm_1, self.compute_dtype, ctx)
         return self.feed_forward.forward_normed(hidden, self.norm_2, self.compute_dtype, ctx)

@@ -1,0 +1,164 @@
+"""The kernel that decodes all layers of a pre-norm model at once, against the same layers one by one in float64 with numbers kept in the kernel's
+precision where it keeps them: sizes at the edges of its tiles, steps and key rounds, few and many blocks, padding rows."""
+
+import math
+
+import numpy as np
+import pytest
+import torch
+
+import plain_gpt2 as P
+
+DEV = "cuda:0"
+
+
+@pytest.mark.parametrize("rows,reach,width,pays", [(1, 1024, 768, True), (8, 1792, 768, True), (8, 1793, 768, False), (9, 1024, 768, True), (16, 1025, 768, False),
+                                                   (17, 64, 768, False), (2, 1792, 1600, True), (4, 1024, 1600, True), (4, 1792, 1600, False), (5, 64, 1600, False)])
+def test_where_one_kernel_for_all_layers_pays(rows, reach, width, pays):
+    from mini_llm_amd.ops.library import library
+
+    assert bool(library().mllm_decode_stack_pays(rows, reach, width)) == pays
+
+
+@pytest.mark.parametrize("rows,layers,width,inner,heads,head,page,dtype,supported", [
+    (1, 12, 768, 3072, 12, 64, 64, torch.bfloat16, True), (16, 64, 768, 3072, 12, 64, 1, torch.float32, True), (16, 48, 1600, 6400, 25, 64, 64, torch.bfloat16, True),
+    (17, 12, 768, 3072, 12, 64, 64, torch.bfloat16, False), (1, 65, 768, 3072, 12, 64, 64, torch.bfloat16, False), (1, 12, 768, 3072, 24, 32, 64, torch.bfloat16, False),
+    (1, 12, 768, 3088, 12, 64, 64, torch.bfloat16, False), (1, 12, 768, 3104, 12, 64, 64, torch.bfloat16, True), (1, 12, 1600, 6400, 25, 64, 64, torch.float32, False),
+    (1, 12, 768, 3072, 12, 64, 48, torch.bfloat16, False), (1, 12, 768, 3072, 11, 64, 64, torch.bfloat16, False), (1, 12, 1856, 1024, 29, 64, 64, torch.bfloat16, False)])
+def test_what_one_kernel_for_all_layers_takes(rows, layers, width, inner, heads, head, page, dtype, supported):
+    from mini_llm_amd.ops import kernels as K
+
+    assert K.decode_stack_supported(rows, layers, width, inner, heads, head, page, dtype) == supported
+
+
+def _stack(rng, layers, width, inner, contexts, page_size, dtype, activation, blocks):
+    """A DecodeStack over random layers and a cache that holds ``contexts`` keys a row (-1: a padding row), what it is run on, and what the layers give in float64."""
+    from test_kernels_gpu import as_weight, bf16_round, dev, plain_paged_attention
+
+    from mini_llm_amd.ops import kernels as K
+
+    kept = bf16_round if dtype == torch.bfloat16 else (lambda a: np.asarray(a, dtype=np.float32).astype(np.float64))
+    heads, rows, eps = width // 64, len(contexts), 2e-5
+    blocks_of = [(c + 1 + page_size - 1) // page_size if c >= 0 else 0 for c in contexts]
+    num_pages, max_blocks = sum(blocks_of) + 2, max(blocks_of)
+    order = rng.permutation(num_pages).tolist()
+    tables, slots = np.full((rows, max_blocks), -1, dtype=np.int32), np.full(rows, -1, dtype=np.int32)
+    for r, n in enumerate(blocks_of):
+        tables[r, :n] = [order.pop() for _ in range(n)]
+        if n:
+            slots[r] = tables[r, contexts[r] // page_size] * page_size + contexts[r] % page_size
+    stream = rng.standard_normal((rows, width)).astype(np.float32)
+    x, made, expected_rows = stream.astype(np.float64), [], []
+    for _ in range(layers):
+        vector = lambda n, mean=0.0: (mean + 0.1 * rng.standard_normal(n)).astype(np.float32)
+        matrix = lambda n, k, scale: kept(rng.standard_normal((n, k)) * (scale / math.sqrt(k)))
+        g1, o1, g2, o2 = vector(width, 1.0), vector(width), vector(width, 1.0), vector(width)
+        w_qkv, w_out, w_up, w_down = matrix(3 * width, width, 2.0), matrix(width, width, 0.5), matrix(inner, width, 1.0), matrix(width, inner, 0.5)
+        b_qkv, b_out, b_up, b_down = vector(3 * width), vector(width), vector(inner), vector(width)
+        k_pages = torch.full((num_pages, heads, page_size, 64), float("nan"), device=DEV, dtype=dtype)
+        v_pages = torch.full_like(k_pages, float("nan"))
+        qkv = kept(kept(P.layernorm(x, g1, o1, eps)) @ w_qkv.T + b_qkv)
+        mixed, here = np.zeros((rows, width)), []
+        for r, context in enumerate(contexts):
+            if context < 0:
+                continue
+            keys, values = kept(rng.standard_normal((context + 1, width))), kept(rng.standard_normal((context + 1, width)))
+            if context:
+                at = np.array([tables[r, p // page_size] * page_size + p % page_size for p in range(context)], dtype=np.int32)
+                K.cache_write(dev(keys[:context], dtype), dev(values[:context], dtype), k_pages, v_pages, dev(at, torch.int32), heads, 64)
+            keys[context], values[context] = qkv[r, width : 2 * width], qkv[r, 2 * width :]
+            here.append((int(slots[r]), keys[context], values[context]))
+            mixed[r] = kept(plain_paged_attention(qkv[r : r + 1, :width], keys, values, heads, heads, None))[0]
+        x = x + mixed @ w_out.T + b_out
+        up = kept(P.layernorm(x, g2, o2, eps)) @ w_up.T + b_up
+        gelu = 0.5 * up * (1.0 + np.tanh(0.7978845608 * (up + 0.044715 * up**3))) if activation == "gelu_new" else \
+            0.5 * up * (1.0 + torch.erf(torch.as_tensor(up / math.sqrt(2.0))).numpy())
+        x = x + kept(gelu) @ w_down.T + b_down
+        weight = lambda w: as_weight(K, w, dtype, True)
+        made.append(K.StackLayer(dev(g1), dev(o1), weight(w_qkv), dev(b_qkv), weight(w_out), dev(b_out), dev(g2), dev(o2), weight(w_up), dev(b_up), weight(w_down), dev(b_down),
+                                 k_pages, v_pages))
+        expected_rows.append(here)
+    request = np.array([r if c >= 0 else -1 for r, c in enumerate(contexts)], dtype=np.int32)
+    stack = K.DecodeStack(made, rows, heads, eps, eps, 0.125, activation, blocks=blocks)
+    given = (dev(stream), dev(request, torch.int32), dev(np.maximum(contexts, 0), torch.int32), dev(slots, torch.int32), dev(tables, torch.int32))
+    return stack, given, x, expected_rows
+
+
+B, F = torch.bfloat16, torch.float32
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype,layers,width,inner,contexts,page_size,activation,blocks", [
+    (B, 1, 64, 32, [0], 64, "gelu_new", None),                              # the smallest: one head, one step of K for a wave or none
+    (B, 2, 128, 512, [5, 0, 64], 16, "gelu", None),
+    (B, 3, 768, 3072, [0, 1, 7, 8, 9, 63, 512, 700], 64, "gelu_new", None),  # key shares of a wave at the edges of a load of eight keys
+    (B, 2, 768, 3072, [1023, 1024, -1, 1030], 64, "gelu_new", None),         # 128 keys a wave in registers, and more; a padding row
+    (B, 2, 768, 3104, [100] * 5, 1, "gelu_new", None),                       # pages of one key; hidden units beyond whole rounds of steps
+    (B, 2, 832, 1056, [33, 600], 32, "gelu", None),                          # 26 steps of K for eight waves
+    (B, 2, 1024, 4096, [40] * 16, 64, "gelu_new", None),                     # two pairs a block
+    (B, 2, 1600, 6400, [20, 129], 64, "gelu_new", None),                     # norm pieces that end inside a row of lanes
+    (B, 1, 1600, 6400, [70, -1, 300] + [9] * 13, 64, "gelu_new", None),      # four pairs a block, tiles not asked for ahead
+    (F, 2, 64, 32, [3, 0], 64, "gelu_new", None),
+    (F, 2, 768, 3072, [0, 3, 4, 5, 511, 512, 600, -1], 64, "gelu_new", None),
+    (F, 1, 768, 3072, [77] * 16, 16, "gelu", None),
+    (F, 2, 1024, 4096, [1, 200, 30], 64, "gelu_new", None),
+    (F, 2, 832, 1056, [33], 64, "gelu", None),
+    # work divided among fewer blocks: several groups of pairs a block, several tiles of the rows, rounds of tiles
+    (B, 2, 192, 768, [10, 3, 100], 16, "gelu_new", 3), (B, 2, 768, 3072, [10, 65], 64, "gelu_new", 7), (F, 2, 192, 768, [10, 3, 100], 16, "gelu_new", 4),
+    (B, 2, 768, 3072, [300] * 8, 64, "gelu_new", 40),
+    (B, 2, 768, 3072, [30] * 8, 64, "gelu_new", 300),                        # more blocks than find a compute unit at once: the late ones are not members
+])
+def test_all_layers_in_one_kernel(dtype, layers, width, inner, contexts, page_size, activation, blocks):
+    from test_kernels_gpu import host
+
+    rng = np.random.default_rng(width + inner + len(contexts))
+    stack, given, expected, new_rows = _stack(rng, layers, width, inner, contexts, page_size, dtype, activation, blocks)
+    before = [(layer.k_pages.clone(), layer.v_pages.clone()) for layer in stack.layers]
+    live = [r for r, c in enumerate(contexts) if c >= 0]
+    # The bounds of the kernels for half a layer (5e-3: what roundings to bfloat16 that fall the other way come to) for each half; in 32-bit
+    # sums of up to 4,096 products of numbers around 1 in another order, 2^-24 sqrt(4,096) each, a few times over a layer.
+    bound = 1e-2 * layers if dtype == B else 2e-5 * layers
+    out = stack.run(*given)
+    np.testing.assert_allclose(host(out)[live], expected[live], rtol=bound, atol=bound)
+    assert torch.isfinite(out).all()   # the padding row too
+    for layer, (k_before, v_before), here in zip(stack.layers, before, new_rows):
+        for pages, was, which in ((layer.k_pages, k_before, 1), (layer.v_pages, v_before, 2)):
+            flat, flat_was = (t.permute(0, 2, 1, 3).reshape(-1, width) for t in (pages, was))
+            for row in here:
+                np.testing.assert_allclose(host(flat[row[0]]), row[which], rtol=bound, atol=bound)
+                flat_was[row[0]] = flat[row[0]]
+            raw = torch.int16 if dtype == B else torch.int32
+            assert torch.equal(flat.view(raw), flat_was.view(raw))   # nothing else was written
+    # launch after launch the same bits (the words of the last launch lie where this one's will), and the control words ready for the next
+    for _ in range(3):
+        assert torch.equal(stack.run(*given), out)
+    control = stack.control.cpu()
+    assert control[96] == 4 and int(control.count_nonzero()) == 1
+
+
+@pytest.mark.gpu
+def test_all_layers_in_one_kernel_replayed_and_beside_another_stream():
+    # a captured launch replayed with other work between the replays, and two stacks at once on two streams: each takes the units it finds
+    rng = np.random.default_rng(5)
+    first, given, expected, _ = _stack(rng, 2, 768, 3072, [50] * 8, 64, B, "gelu_new", None)
+    second, given_2, expected_2, _ = _stack(rng, 2, 768, 3072, [80] * 4, 64, B, "gelu_new", None)
+    out, out_2 = first.run(*given), second.run(*given_2)
+    graph = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph):
+        replayed = first.run(*given)
+    for _ in range(4):
+        replayed.zero_()
+        graph.replay()
+        assert torch.equal(replayed, out)
+        assert torch.equal(first.run(*given), out)
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    outs = [[], []]
+    torch.cuda.synchronize()
+    for _ in range(20):
+        for stream, stack, args, into in ((streams[0], first, given, outs[0]), (streams[1], second, given_2, outs[1])):
+            with torch.cuda.stream(stream):
+                into.append(stack.run(*args))
+    torch.cuda.synchronize()
+    # with fewer members a block has more tiles and pairs, each summed in the same order: the same bits
+    assert all(torch.equal(o, out) for o in outs[0]) and all(torch.equal(o, out_2) for o in outs[1])
