@@ -247,19 +247,19 @@ constexpr int DECODE_MAX_SPLITS = 16;
 // weight in `parts_out` ([token, head, part, HD + 2] floats) and counts itself in arrivals[token, head] (zero before the
 // launch); the block that is through last puts the runs together, out = sum_p o_p e^(m_p - M) / sum_p l_p e^(m_p - M),
 // and the count is zero again behind it (it wraps), so the same counters serve the next launch.
+// The work of a block: part `part` of `n_parts` of one (token, head), by the block's n_splits waves.
 template <typename T, int HD, bool TOGETHER, bool KEPT = false>
-__global__ __launch_bounds__(1024) void attention_decode_kernel(
-    const T* __restrict__ q, int q_stride, const T* __restrict__ k_pages,
+__device__ __forceinline__ void decode_block(
+    int head, int token, int part, int n_parts, int n_splits, const T* __restrict__ q, int q_stride, const T* __restrict__ k_pages,
     const T* __restrict__ v_pages, T* __restrict__ out, int out_stride,
     const int* __restrict__ token_request, const int* __restrict__ positions,
     const int* __restrict__ block_tables, int max_blocks, int n_heads, int n_kv_heads,
-    int page_shift, int window, float scale, int out_packed, float* parts_out, int* __restrict__ arrivals, ScoreOptions options) {
-    constexpr int VEC = KeySweep<T, HD>::VEC, LPR = KeySweep<T, HD>::LPR, RPI = KeySweep<T, HD>::RPI;
+    int page_shift, int window, float scale, int out_packed, float* parts_out, int* __restrict__ arrivals, const ScoreOptions& options) {
+    constexpr int VEC = KeySweep<T, HD>::VEC, LPR = KeySweep<T, HD>::LPR;
     __shared__ float partial[DECODE_MAX_SPLITS][HD + 2];
     __shared__ int through_last;
 
-    const int lane = threadIdx.x % WAVE, split = threadIdx.x / WAVE, n_splits = blockDim.x / WAVE;
-    const int head = blockIdx.x, token = blockIdx.y;
+    const int lane = threadIdx.x % WAVE, split = threadIdx.x / WAVE;
     const int request = token_request[token];
     // out_packed: the rows go out in the packed layout of a [tokens, n_heads * HD] matrix, for the
     // output product of few rows that reads them next
@@ -267,7 +267,6 @@ __global__ __launch_bounds__(1024) void attention_decode_kernel(
         store_result(out, out_packed ? packed_element<T>(token, head * HD + d, n_heads * HD) : (size_t)token * out_stride + head * HD + d, value,
                      options.wide_out);
     };
-    const int n_parts = gridDim.z, part = blockIdx.z;
     if (request < 0) {  // a padding row; the whole block leaves together (its zeros come from the block of the first run)
         if (part == 0)
             for (int d = threadIdx.x; d < HD; d += blockDim.x) put_out(d, 0.0f);
@@ -408,6 +407,17 @@ __global__ __launch_bounds__(1024) void attention_decode_kernel(
         for (int s = 0; s < n_splits; s++) value += partial[s][d] * expf(partial[s][HD] - total_max);
         put_out(d, value * inverse);
     }
+}
+
+template <typename T, int HD, bool TOGETHER, bool KEPT = false>
+__global__ __launch_bounds__(1024) void attention_decode_kernel(
+    const T* __restrict__ q, int q_stride, const T* __restrict__ k_pages,
+    const T* __restrict__ v_pages, T* __restrict__ out, int out_stride,
+    const int* __restrict__ token_request, const int* __restrict__ positions,
+    const int* __restrict__ block_tables, int max_blocks, int n_heads, int n_kv_heads,
+    int page_shift, int window, float scale, int out_packed, float* parts_out, int* __restrict__ arrivals, ScoreOptions options) {
+    decode_block<T, HD, TOGETHER, KEPT>(blockIdx.x, blockIdx.y, blockIdx.z, gridDim.z, blockDim.x / WAVE, q, q_stride, k_pages, v_pages, out, out_stride, token_request,
+                                        positions, block_tables, max_blocks, n_heads, n_kv_heads, page_shift, window, scale, out_packed, parts_out, arrivals, options);
 }
 
 template <typename T>
@@ -948,4 +958,93 @@ MLLM_API int mllm_attention_prefill(const void* q, int q_stride, const void* k_p
     }
 #undef MLLM_PREFILL_CASE
     return mllm_check_launch("attention_prefill");
+}
+
+// ------------------------------------------------------------------------------------------------
+// A step of both kinds, decoding rows (or portions as short) beside prompt portions, in one launch: the blocks of the two kernels side by side.
+// Behind one another they cost a step of continuous batching two kernels' starts and each the wait for its longest block on a chip that the other's
+// blocks would have filled. A block takes either part whole; the decoding rows' blocks, each as long as its row's keys are many, come first, and the
+// prompts' behind them in their order, the longest first. Blocks of four waves, two to a compute unit (the prompts' tiles in LDS), for both.
+// Measured in replayed graphs, two launches -> one, us: bfloat16, 16 heads, 10 rows of 700 keys (6 padding rows) beside a prompt of 480 19.0 -> 11.0, beside 250
+// on 512 20.2 -> 13.0, 24 rows of 500 beside 480 21.9 -> 14.8, of 900 31.5 -> 22.1; 25 heads, 48 rows of 500 beside 480 42.6 -> 34.1; one row beside 80 tokens
+// 11.8 -> 5.9. In 32-bit, 12 heads, 10 rows of 700 beside 480 29.4 -> 17.8. What is left is the longer of the two parts.
+// ------------------------------------------------------------------------------------------------
+namespace {
+
+// The longest sequence, after the step, that one launch takes: a row's keys are divided among four waves here, where a launch of decoding rows alone gives
+// it eight or sixteen, or several blocks. Two launches / one, us, 16 heads, the prompt of 512 new tokens or 400 on 1,500: bfloat16, one row of 1,900 keys 18.3 / 15.3 and
+// 24.2 / 16.9, eight 25.0 / 17.9 and 32.6 / 25.0; one of 3,500 19.5 / 23.6 and 26.2 / 24.4, of 7,500 24.4 / 45.4; in 32-bit one of 1,900 27.2 / 22.7, of 3,500 29.6 / 37.8.
+constexpr int MIXED_REACH = 2048;
+
+template <typename T, int HD, int QUERIES>
+__global__ __launch_bounds__(256, 2) void attention_mixed_kernel(
+    const T* __restrict__ q, int q_stride, const T* __restrict__ k_pages, const T* __restrict__ v_pages, T* __restrict__ out, int out_stride,
+    const int* __restrict__ token_request, const int* __restrict__ positions, const int* __restrict__ q_starts, const int* __restrict__ context_lens,
+    const int* __restrict__ block_tables, int max_blocks, int short_rows, int short_requests, int long_requests, int short_blocks, int n_heads, int n_kv_heads,
+    int page_shift, float scale) {
+    const ScoreOptions plain = {0.0f, nullptr, 0, 0, 0};
+    const int block = blockIdx.x;
+    if (block < short_blocks) {
+        const int token = block / n_heads;
+        if (token >= short_rows) return;   // (short_blocks: a multiple of eight, so that a head of the prompts keeps to its XCD)
+        decode_block<T, HD, true>(block % n_heads, token, 0, 1, 4, q, q_stride, k_pages, v_pages, out, out_stride, token_request, positions, block_tables, max_blocks,
+                                  n_heads, n_kv_heads, page_shift, 0, scale, 0, nullptr, nullptr, plain);
+        return;
+    }
+    const int place = block - short_blocks;
+    const int* tables = block_tables + (size_t)short_requests * max_blocks;
+    if constexpr (sizeof(T) == 2)
+        prefill_stream::stream_block<T, HD, QUERIES, 4, prefill_stream::CAUSAL>(place, q, q_stride, k_pages, v_pages, out, out_stride, q_starts + short_requests,
+                                                                                context_lens + short_requests, tables, max_blocks, long_requests, n_heads, n_kv_heads, page_shift, 0,
+                                                                                scale, plain);
+    else
+        prefill_pieces::pieces_block<HD, prefill_stream::CAUSAL>(place, q, q_stride, k_pages, v_pages, out, out_stride, q_starts + short_requests, context_lens + short_requests,
+                                                                 tables, max_blocks, long_requests, n_heads, n_kv_heads, page_shift, 0, scale, plain);
+}
+
+template <typename T, int QUERIES>
+void launch_mixed(const void* q, int q_stride, const void* k_pages, const void* v_pages, void* out, int out_stride, const int* token_request, const int* positions,
+                  const int* q_starts, const int* context_lens, const int* block_tables, int max_blocks, int short_rows, int short_requests, int long_requests, int rows,
+                  int max_q_len, int n_heads, int n_kv_heads, int page_shift, float scale, hipStream_t stream) {
+    constexpr int LDS_BYTES = sizeof(T) == 2 ? prefill_stream::Layout<bf16_t, 64, 4>::LDS_BYTES : prefill_pieces::WAVES * prefill_pieces::wave_bytes<64>();
+    static bool raised = false;   // (as for the prompts' own kernels)
+    if (!raised && LDS_BYTES > 60 * 1024)
+        raised = hipFuncSetAttribute((const void*)attention_mixed_kernel<T, 64, QUERIES>, hipFuncAttributeMaxDynamicSharedMemorySize, LDS_BYTES) == hipSuccess;
+    const int short_blocks = (short_rows * n_heads + 7) & ~7;
+    const int grid = short_blocks + n_heads * prefill_stream::most_tiles(QUERIES, long_requests, rows - short_rows, max_q_len);
+    mllm_count_kernel(MLLM_K_ATTENTION_MIXED);
+    attention_mixed_kernel<T, 64, QUERIES><<<grid, 256, LDS_BYTES, stream>>>(
+        (const T*)q, q_stride, (const T*)k_pages, (const T*)v_pages, (T*)out, out_stride, token_request, positions, q_starts, context_lens, block_tables, max_blocks, short_rows,
+        short_requests, long_requests, short_blocks, n_heads, n_kv_heads, page_shift, scale);
+}
+
+}  // namespace
+
+// Whether a step of both kinds takes one launch: heads of 64 without a mask of their own, pages and portions as the prompts' kernels for such rows take them.
+MLLM_API int mllm_attention_mixed_takes(const void* q, int q_stride, const void* out, int out_stride, int head_size, int page_size, int max_q_len, int reach, float scale, int dtype) {
+    if (head_size != 64 || (dtype != MLLM_F32 && dtype != MLLM_BF16) || !mllm_attention_decode_supported(head_size, page_size, dtype)) return 0;
+    if (reach < 1 || reach > MIXED_REACH) return 0;
+    return dtype == MLLM_BF16 ? prefill_stream::takes<bf16_t>(head_size, page_size, max_q_len, scale, q_stride, out_stride, q, out)
+                              : prefill_stream::takes<float>(head_size, page_size, max_q_len, scale, q_stride, out_stride, q, out);
+}
+
+// rows: all rows, the short portions' first; token_request and positions: for these; q_starts, context_lens, block_tables: of all requests, the short portions' first.
+MLLM_API int mllm_attention_mixed(const void* q, int q_stride, const void* k_pages, const void* v_pages, void* out, int out_stride, const int* token_request, const int* positions,
+                                  const int* q_starts, const int* context_lens, const int* block_tables, int max_blocks, int rows, int n_requests, int short_rows, int short_requests,
+                                  int max_q_len, int reach, int n_heads, int n_kv_heads, int head_size, int page_size, float scale, int dtype, hipStream_t stream) {
+    MLLM_REQUIRE(n_heads > 0 && n_kv_heads > 0 && max_blocks > 0 && n_heads % n_kv_heads == 0, "attention_mixed: bad sizes");
+    MLLM_REQUIRE(short_rows > 0 && short_rows < rows && short_requests > 0 && short_requests < n_requests, "attention_mixed: no step of both kinds");
+    MLLM_REQUIRE(n_requests <= 65535 && n_heads <= 65535 && short_rows <= 65535, "attention_mixed: too many rows, requests or heads for one launch");
+    MLLM_REQUIRE(q_stride >= n_heads * head_size && out_stride >= n_heads * head_size, "attention_mixed: rows are too short for the heads");
+    MLLM_REQUIRE(mllm_attention_mixed_takes(q, q_stride, out, out_stride, head_size, page_size, max_q_len, reach, scale, dtype), "attention_mixed: no kernel for these rows");
+    int page_shift = 0;
+    while ((1 << page_shift) < page_size) page_shift++;
+#define MLLM_MIXED(T, QUERIES)                                                                                                                                             \
+    launch_mixed<T, QUERIES>(q, q_stride, k_pages, v_pages, out, out_stride, token_request, positions, q_starts, context_lens, block_tables, max_blocks, short_rows,       \
+                             short_requests, n_requests - short_requests, rows, max_q_len, n_heads, n_kv_heads, page_shift, scale, stream)
+    if (dtype == MLLM_F32) MLLM_MIXED(float, 32);
+    else if ((long)n_heads * prefill_stream::most_tiles(64, n_requests - short_requests, rows - short_rows, max_q_len) >= 256) MLLM_MIXED(bf16_t, 64);   // (as without decoding rows)
+    else MLLM_MIXED(bf16_t, 32);
+#undef MLLM_MIXED
+    return mllm_check_launch("attention_mixed");
 }

@@ -143,8 +143,8 @@ __device__ __forceinline__ void stream_for(F&& f) {   // a loop whose index is a
 
 // FORM: attention_stream.h.
 template <int HD, int FORM>
-__global__ __launch_bounds__(64 * WAVES, 2) void attention_prefill_pieces_kernel(
-    const float* __restrict__ q, int q_stride, const float* __restrict__ k_pages, const float* __restrict__ v_pages, float* __restrict__ out, int out_stride,
+__device__ __forceinline__ void pieces_block(
+    int place, const float* __restrict__ q, int q_stride, const float* __restrict__ k_pages, const float* __restrict__ v_pages, float* __restrict__ out, int out_stride,
     const int* __restrict__ q_starts, const int* __restrict__ context_lens, const int* __restrict__ block_tables, int max_blocks, int n_requests, int n_heads,
     int n_kv_heads, int page_shift, int given_window, float scale, ScoreOptions options) {
     typedef Layout<float, HD, WAVES> L;
@@ -160,8 +160,8 @@ __global__ __launch_bounds__(64 * WAVES, 2) void attention_prefill_pieces_kernel
     const int wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
     const int lane32 = lane % 32, half = lane / 32;
     // (places and heads: attention_stream.h)
-    const int slot = blockIdx.x / n_heads, at = blockIdx.x % n_heads;
-    const int head = at < (n_heads & ~7) ? (at & ~7) | (blockIdx.x & 7) : at;
+    const int slot = place / n_heads, at = place % n_heads;
+    const int head = at < (n_heads & ~7) ? (at & ~7) | (place & 7) : at;
     int request, q_first, q_len, context, query_tile;
     if (!tile_of_slot<QUERIES>(slot, n_requests, q_starts, context_lens, request, q_first, q_len, context, query_tile)) return;
     const int tile_q0 = query_tile * QUERIES;
@@ -476,6 +476,15 @@ __global__ __launch_bounds__(64 * WAVES, 2) void attention_prefill_pieces_kernel
         general_row<float>(q + (size_t)(q_first + row) * q_stride + head * HD, k_pages, v_pages, out, (size_t)(q_first + row) * out_stride + head * HD, table, context + row, kv_head,
                            head, n_kv_heads, HD, 1 << page_shift, given_window, scale, options, my_q);
     }
+}
+
+template <int HD, int FORM>
+__global__ __launch_bounds__(64 * WAVES, 2) void attention_prefill_pieces_kernel(
+    const float* __restrict__ q, int q_stride, const float* __restrict__ k_pages, const float* __restrict__ v_pages, float* __restrict__ out, int out_stride,
+    const int* __restrict__ q_starts, const int* __restrict__ context_lens, const int* __restrict__ block_tables, int max_blocks, int n_requests, int n_heads,
+    int n_kv_heads, int page_shift, int given_window, float scale, ScoreOptions options) {
+    pieces_block<HD, FORM>(blockIdx.x, q, q_stride, k_pages, v_pages, out, out_stride, q_starts, context_lens, block_tables, max_blocks, n_requests, n_heads, n_kv_heads, page_shift,
+                           given_window, scale, options);
 }
 
 template <int HD, int FORM>

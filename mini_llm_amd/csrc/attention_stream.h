@@ -201,9 +201,10 @@ enum Form : int {
     KEPT = 3,     // a window with kept first keys, with or without a cap
 };
 
+// `place`: the block's own place among a launch's (tile, head) blocks.
 template <typename T, int HD, int QUERIES, int SPLITS, int FORM>
-__global__ __launch_bounds__(64 * SPLITS, (HD * sizeof(T) <= 128 && SPLITS == 4) ? 2 : 1) void attention_prefill_stream_kernel(
-    const T* __restrict__ q, int q_stride, const T* __restrict__ k_pages, const T* __restrict__ v_pages,
+__device__ __forceinline__ void stream_block(
+    int place, const T* __restrict__ q, int q_stride, const T* __restrict__ k_pages, const T* __restrict__ v_pages,
     T* __restrict__ out, int out_stride, const int* __restrict__ q_starts, const int* __restrict__ context_lens,
     const int* __restrict__ block_tables, int max_blocks, int n_requests, int n_heads, int n_kv_heads, int page_shift, int given_window, float scale, ScoreOptions options) {
     typedef Layout<T, HD, SPLITS> L;
@@ -223,8 +224,8 @@ __global__ __launch_bounds__(64 * SPLITS, (HD * sizeof(T) <= 128 && SPLITS == 4)
     // places one after the other, the heads of a place side by side: the blocks with the most keys start first, whatever their head. Of each eight
     // heads one belongs to an XCD (which has every eighth block), so that its keys and values are read through one L2; the heads beyond a multiple of
     // eight are where they fall.
-    const int slot = blockIdx.x / n_heads, at = blockIdx.x % n_heads;
-    const int head = at < (n_heads & ~7) ? (at & ~7) | (blockIdx.x & 7) : at;
+    const int slot = place / n_heads, at = place % n_heads;
+    const int head = at < (n_heads & ~7) ? (at & ~7) | (place & 7) : at;
     int request, q_first, q_len, context, query_tile;
     if (!tile_of_slot<QUERIES>(slot, n_requests, q_starts, context_lens, request, q_first, q_len, context, query_tile)) return;
     const int tile_q0 = query_tile * QUERIES;
@@ -519,6 +520,15 @@ __global__ __launch_bounds__(64 * SPLITS, (HD * sizeof(T) <= 128 && SPLITS == 4)
             else *reinterpret_cast<bf16x4*>(out + at) = bf16x4{static_cast<bf16_t>(o[0]), static_cast<bf16_t>(o[1]), static_cast<bf16_t>(o[2]), static_cast<bf16_t>(o[3])};
         }
     }
+}
+
+template <typename T, int HD, int QUERIES, int SPLITS, int FORM>
+__global__ __launch_bounds__(64 * SPLITS, (HD * sizeof(T) <= 128 && SPLITS == 4) ? 2 : 1) void attention_prefill_stream_kernel(
+    const T* __restrict__ q, int q_stride, const T* __restrict__ k_pages, const T* __restrict__ v_pages,
+    T* __restrict__ out, int out_stride, const int* __restrict__ q_starts, const int* __restrict__ context_lens,
+    const int* __restrict__ block_tables, int max_blocks, int n_requests, int n_heads, int n_kv_heads, int page_shift, int given_window, float scale, ScoreOptions options) {
+    stream_block<T, HD, QUERIES, SPLITS, FORM>(blockIdx.x, q, q_stride, k_pages, v_pages, out, out_stride, q_starts, context_lens, block_tables, max_blocks, n_requests, n_heads,
+                                               n_kv_heads, page_shift, given_window, scale, options);
 }
 
 // Whether prompt portions with these sizes take this kernel.

@@ -490,8 +490,9 @@ def paged_attention(q, k_pages, v_pages, token_request, positions, block_tables,
     matrix-core kernel, which walks tiles of one request's queries. ``short_rows`` and
     ``short_requests``: the first so many rows are the portions of the first so many requests and
     none of them is longer than DECODE_MAX_Q_LEN, while the rest are longer portions; a batch of
-    both kinds then runs as two launches, each kind in its own kernel (a single decoded token with
-    a long context would otherwise walk all its keys in one wave of the kernel for portions).
+    both kinds then runs as one launch with blocks of both kinds, where it takes the sizes, or as two launches,
+    each kind in its own kernel (a single decoded token with a long context would otherwise walk all its
+    keys in one wave of the kernel for portions).
     ``packed_out``: where the kernel for decoding and short portions runs, the rows come as
     PackedRows (for the output product of few rows that reads them next); elsewhere as ever.
     ``first_row``: where the rows are a part of a step's batch whose other parts may run at the same time on other
@@ -530,6 +531,15 @@ def paged_attention(q, k_pages, v_pages, token_request, positions, block_tables,
             and lib.mllm_attention_decode_supported(head_size, page_size, _code(q.dtype))
             and lib.mllm_attention_prefill_supported(head_size, page_size)):
         _require(0 < short_requests < context_lens.shape[0], "short_requests does not cut the batch in two")
+        reach = block_tables.shape[1] * page_size if max_len is None else max(1, min(max_len, block_tables.shape[1] * page_size))
+        if (not (window or chunk or softcap or wide_out) and sinks is None and q_starts.shape[0] == context_lens.shape[0] + 1 and block_tables.shape[0] >= context_lens.shape[0]
+                and lib.mllm_attention_mixed_takes(_ptr(q), q.stride(0), _ptr(out), out.stride(0), head_size, page_size, int(max_q_len), reach, float(scale), _code(q.dtype))):
+            _device_tensor(q_starts, "q_starts", torch.int32, 1)
+            _device_tensor(context_lens, "context_lens", torch.int32, 1)
+            check(lib.mllm_attention_mixed(_ptr(q), q.stride(0), _ptr(k_pages), _ptr(v_pages), _ptr(out), out.stride(0), _ptr(token_request), _ptr(positions), _ptr(q_starts),
+                                           _ptr(context_lens), _ptr(block_tables), block_tables.shape[1], n, context_lens.shape[0], int(short_rows), int(short_requests),
+                                           int(max_q_len), reach, n_heads, n_kv_heads, head_size, page_size, float(scale), _code(q.dtype), _stream()))
+            return out
         common = dict(n_heads=n_heads, n_kv_heads=n_kv_heads, head_size=head_size, scale=scale, window=window, max_len=max_len, first_row=first_row,
                       softcap=softcap, sinks=sinks, chunk=chunk, keep_first=keep_first, wide_out=wide_out)
         paged_attention(q[:short_rows], k_pages, v_pages, token_request, positions, block_tables, max_q_len=DECODE_MAX_Q_LEN,
