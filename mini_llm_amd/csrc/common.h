@@ -17,6 +17,7 @@ enum MllmEpilogue : int {
     MLLM_EPI_GELU_TANH = 1,  // gelu_new(+ bias)
     MLLM_EPI_GELU_ERF = 2,   // gelu(+ bias)
     MLLM_EPI_SQUARED_RELU = 3,   // max(+ bias, 0)^2
+    MLLM_EPI_GATED_SILU = 4,     // W's rows are eight gate and eight up rows in turn: silu(gate) * up, half as many columns
 };
 
 typedef __bf16 bf16_t;
@@ -212,6 +213,12 @@ __device__ __forceinline__ float gelu_tanh(float x) {
 // exact GELU (engine/src/gelu.c:5-9).
 __device__ __forceinline__ float gelu_erf(float x) {
     return 0.5f * x * (1.0f + erff(x * 0.70710678118654752440f));
+}
+
+__device__ __forceinline__ float gated_silu(float gate, float up) { return gate / (1.0f + expf(-gate)) * up; }
+// for results that are rounded to bfloat16 right after, as below
+__device__ __forceinline__ float gated_silu_for_bf16(float gate, float up) {
+    return gate * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.4426950408889634f * gate)) * up;
 }
 
 // The same two functions for results that are rounded to bfloat16 (eight bits of fraction) right

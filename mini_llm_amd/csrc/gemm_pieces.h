@@ -352,6 +352,7 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N, 2) void gemm_pieces_kernel(
     const Place place = place_of(out_col);   // a lane's columns are the same in every row
     auto leave = [&](auto kind) {
         constexpr int KIND = decltype(kind)::value;
+        constexpr bool UNITS = KIND == MLLM_EPI_GATED_SILU;   // two groups of eight columns become eight
 #pragma unroll
         for (int i = 0; i < TM; i++) {
             float in_weight = 1.0f, out_weight = 1.0f;
@@ -362,8 +363,14 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N, 2) void gemm_pieces_kernel(
 #pragma unroll
             for (int j = 0; j < TN; j += Group::GATED ? 2 : 1)
 #pragma unroll
-                for (int g = 0; g < 4; g++) {
+                for (int g = 0; g < 4; g += UNITS ? 2 : 1) {
                     f32x4 value;
+                    if constexpr (UNITS) {
+#pragma unroll
+                        for (int e = 0; e < 4; e++) value[e] = gated_silu(acc[j][i][4 * g + e], acc[j][i][4 * g + 4 + e]);
+                        *reinterpret_cast<f32x4*>(slab + lane32 * SLAB_ROW + j * 16 + 4 * g + 4 * half) = value;
+                        continue;
+                    }
                     if constexpr (Group::GATED) {
 #pragma unroll
                         for (int e = 0; e < 4; e++)
@@ -383,13 +390,19 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N, 2) void gemm_pieces_kernel(
                 const int in_slab = r * ROWS + min(lane / LANES_A_ROW, ROWS - 1), row = row0 + i * 32 + in_slab;
                 f32x4 value = *reinterpret_cast<const f32x4*>(slab + in_slab * SLAB_ROW + (lane % LANES_A_ROW) * 4);
                 if (lane >= ROWS * LANES_A_ROW || row >= m_end || out_col >= out_cols || ((unsigned)(bad >> (i * 32)) >> in_slab & 1)) continue;
+                if constexpr (UNITS) {
+                    const int unit = col0 / 2 + (lane % LANES_A_ROW) * 4;
+                    if (lane % LANES_A_ROW < LANES_A_ROW / 2 && unit < N / 2) *reinterpret_cast<f32x4*>(out + (size_t)row * (N / 2) + unit) = value;
+                    continue;
+                }
                 put(row, out_col, place, value);
             }
             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         }
     };
     using std::integral_constant;
-    if (Group::GROUPED || epilogue == MLLM_EPI_NONE) leave(integral_constant<int, MLLM_EPI_NONE>{});
+    if constexpr (Group::UNITS) leave(integral_constant<int, MLLM_EPI_GATED_SILU>{});
+    else if (Group::GROUPED || epilogue == MLLM_EPI_NONE) leave(integral_constant<int, MLLM_EPI_NONE>{});
     else if (epilogue == MLLM_EPI_GELU_TANH) leave(integral_constant<int, MLLM_EPI_GELU_TANH>{});
     else if (epilogue == MLLM_EPI_GELU_ERF) leave(integral_constant<int, MLLM_EPI_GELU_ERF>{});
     else leave(integral_constant<int, MLLM_EPI_SQUARED_RELU>{});
@@ -434,6 +447,13 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N, 2) void gemm_pieces_kernel(
 #pragma unroll
             for (int t = 0; t < TILES; t++) {
                 const int col = col0 + t * 16 + 4 * quad;
+                if constexpr (Group::UNITS) {   // a tile's gate columns in the first 32 lanes, its up columns in the others (of the same rows)
+                    f32x4 unit;
+#pragma unroll
+                    for (int e = 0; e < 4; e++) unit[e] = gated_silu(sum[t][e], __shfl_xor(sum[t][e], 32, WAVE));
+                    if (quad < 2 && col < out_cols) *reinterpret_cast<f32x4*>(out + (size_t)row * (N / 2) + col0 / 2 + t * 8 + 4 * quad) = unit;
+                    continue;
+                }
                 if (col >= out_cols) continue;
                 f32x4 value = sum[t];
                 if (!Group::GROUPED && bias) value += *reinterpret_cast<const f32x4*>(bias + col);
@@ -475,10 +495,10 @@ void launch(const float* a, const float* w, const float* bias, const float* resi
                                                                                                           k_per_block, group);
 }
 
-template <int BM, int BN, int WAVES_M, int WAVES_N>
+template <int BM, int BN, int WAVES_M, int WAVES_N, typename Group>
 void launch_whole(const float* a, const float* w, const float* bias, const float* residual, float* o, int M, int N, int K, int epilogue, hipStream_t stream, const CacheScatter& scatter,
                   int k_blocks) {
-    launch<BM, BN, WAVES_M, WAVES_N>(a, w, bias, residual, o, M, N, K, ceil_div(N, 16), epilogue, stream, scatter, k_blocks, dim3(ceil_div(N, BN), ceil_div(M, BM), k_blocks), stream::Whole{});
+    launch<BM, BN, WAVES_M, WAVES_N>(a, w, bias, residual, o, M, N, K, ceil_div(N, 16), epilogue, stream, scatter, k_blocks, dim3(ceil_div(N, BN), ceil_div(M, BM), k_blocks), Group{});
 }
 
 // The tiles, and what they cost in microseconds: what lies in front of and behind a block's loop, and a tile of K for each block of a compute unit, alone there or not, and
@@ -511,14 +531,15 @@ inline float cost(int M, int N, int K, int k_blocks, int& best) {
     return best_cost;
 }
 
-inline void dispatch(const float* a, const float* w, const float* bias, const float* residual, float* o, int M, int N, int K, int epilogue, hipStream_t stream,
+template <typename Group = stream::Whole>
+void dispatch(const float* a, const float* w, const float* bias, const float* residual, float* o, int M, int N, int K, int epilogue, hipStream_t stream,
                      const CacheScatter& scatter, int k_blocks) {
     int best = 0;
     cost(M, N, K, k_blocks, best);
-    if (best == 0) launch_whole<128, 128, 2, 2>(a, w, bias, residual, o, M, N, K, epilogue, stream, scatter, k_blocks);
-    else if (best == 1) launch_whole<128, 64, 4, 1>(a, w, bias, residual, o, M, N, K, epilogue, stream, scatter, k_blocks);
-    else if (best == 2) launch_whole<64, 64, 2, 2>(a, w, bias, residual, o, M, N, K, epilogue, stream, scatter, k_blocks);
-    else launch_whole<128, 96, 4, 1>(a, w, bias, residual, o, M, N, K, epilogue, stream, scatter, k_blocks);
+    if (best == 0) launch_whole<128, 128, 2, 2, Group>(a, w, bias, residual, o, M, N, K, epilogue, stream, scatter, k_blocks);
+    else if (best == 1) launch_whole<128, 64, 4, 1, Group>(a, w, bias, residual, o, M, N, K, epilogue, stream, scatter, k_blocks);
+    else if (best == 2) launch_whole<64, 64, 2, 2, Group>(a, w, bias, residual, o, M, N, K, epilogue, stream, scatter, k_blocks);
+    else launch_whole<128, 96, 4, 1, Group>(a, w, bias, residual, o, M, N, K, epilogue, stream, scatter, k_blocks);
 }
 
 // Into how many partial products a product with sums to be taken by whoever reads them is cut, `most` at most: they are read once more there.

@@ -128,7 +128,12 @@ __device__ __forceinline__ void put4<bf16_t>(bf16_t* at, f32x4 v) {
 
 // Which rows and which matrix a block's tile takes. The whole product: rows of A in order, one matrix.
 struct Whole {
-    static constexpr bool GROUPED = false, GATED = false;
+    static constexpr bool GROUPED = false, GATED = false, UNITS = false;
+};
+// The same over a W of eight gate and eight up rows in turn, whose result is the gate units (MLLM_EPI_GATED_SILU): kernels of their own, since the registers that one more
+// end takes are not there in the others (256 x 256: 48 -> 496 bytes of spilled ones).
+struct Units {
+    static constexpr bool GROUPED = false, GATED = false, UNITS = true;
 };
 // A product over rows grouped by expert, each group with a matrix of its own: the groups' entries lie behind each other in one list, and
 // `tiles` names the tiles of it that hold an expert's entries: (expert, first entry, the end of the expert's entries, unused). Entry i
@@ -137,7 +142,7 @@ struct Whole {
 // weight[i] multiplying the sums (weigh_input) or the unit.
 template <bool GATED_>
 struct ExpertTiles {
-    static constexpr bool GROUPED = true, GATED = GATED_;
+    static constexpr bool GROUPED = true, GATED = GATED_, UNITS = false;
     const int4* tiles;
     const int* n_tiles;
     const int* a_row;
@@ -274,7 +279,7 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N * WAVES_K) void gemm_stream_
             const int n = n_wave + j * 32 + 8 * g + 4 * (lane / 32);  // N is a multiple of 8: four columns are inside or outside together
             early_bias[j][g] = bias && n < N ? *reinterpret_cast<const f32x4*>(bias + n) : f32x4{0.0f, 0.0f, 0.0f, 0.0f};
         }
-    constexpr bool WITH_RESIDUAL = sizeof(OutT) == 4 && !GROUPED, CAN_SCATTER = sizeof(OutT) == 2 && !GROUPED;
+    constexpr bool WITH_RESIDUAL = sizeof(OutT) == 4 && !GROUPED, CAN_SCATTER = sizeof(OutT) == 2 && !GROUPED && !Group::UNITS;
     f32x4 early_residual[WITH_RESIDUAL ? OWN : 1][WITH_RESIDUAL ? ROW_STEPS : 1];
     if constexpr (WITH_RESIDUAL) {
         const float* residual_lane = residual + (size_t)m_lane * N + n_lane;
@@ -460,11 +465,11 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N * WAVES_K) void gemm_stream_
     // [M, q_width]), 2 all of them key columns or all of them value columns (into the cache pages), 3 some of each.
     auto leave = [&](auto kind, auto where) {
         constexpr int KIND = decltype(kind)::value, WHERE = decltype(where)::value;
-        constexpr bool SCATTERED = WHERE != 0;
+        constexpr bool SCATTERED = WHERE != 0, UNITS = KIND == MLLM_EPI_GATED_SILU;   // (UNITS: two groups of eight columns become eight)
         // where a lane's piece goes: q columns to out [M, q_width], key and value columns into the cache page at the
         // row's slot (a piece lies inside one head: the head size is a multiple of 8)
-        const int row_stride = SCATTERED ? scatter.q_width : n_out;
-        OutT* out_lane = out + (size_t)m_lane * row_stride + n_lane;
+        const int row_stride = SCATTERED ? scatter.q_width : UNITS ? N / 2 : n_out;
+        OutT* out_lane = out + (size_t)m_lane * row_stride + (UNITS ? n_wave / 2 + lane_piece * OUT_VEC : n_lane);
         // A piece in the cache lies at page * (bytes of a page) + ((head << page_shift) + offset) * (bytes of a row) + the
         // piece's place in the row: all but page and offset is the lane's own constant.
         bool to_cache = false;
@@ -491,6 +496,16 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N * WAVES_K) void gemm_stream_
 #pragma unroll
                         for (int e = 0; e < 4; e++) value[e] = gated(acc[j][i][4 * g + e] * in_weight, acc[j + 1][i][4 * g + e] * in_weight, group.unit) * out_weight;
                         put4<OutT>(reinterpret_cast<OutT*>(slab_write) + (j / 2) * 32 + 8 * g, value);
+                    }
+            } else if constexpr (UNITS) {
+#pragma unroll
+                for (int j = 0; j < FN; j++)
+#pragma unroll
+                    for (int g = 0; g < 4; g += 2) {
+                        f32x4 value;
+#pragma unroll
+                        for (int e = 0; e < 4; e++) value[e] = gated_silu_for_bf16(acc[j][i][4 * g + e], acc[j][i][4 * g + 4 + e]);
+                        put4<OutT>(reinterpret_cast<OutT*>(slab_write) + j * 16 + 4 * g, value);
                     }
             } else {
 #pragma unroll
@@ -520,6 +535,7 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N * WAVES_K) void gemm_stream_
                 const int row = i * 32 + r * ROWS_A_STEP;
                 Vec16 v = *reinterpret_cast<const Vec16*>(slab_read + r * ROWS_A_STEP * SLAB_ROW);
                 if (row >= rows_left) continue;
+                if (UNITS && (lane_piece >= PIECES / 2 || n_wave / 2 + lane_piece * OUT_VEC >= N / 2)) continue;
                 if constexpr (WHERE >= 2) {
                     if (WHERE == 2 || to_cache) {
                         const int slot = early_slot[i][r];
@@ -550,13 +566,17 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N * WAVES_K) void gemm_stream_
             return;
         }
     }
+    if constexpr (Group::UNITS) {
+        leave(integral_constant<int, MLLM_EPI_GATED_SILU>{}, integral_constant<int, 0>{});
+        return;
+    }
     if (epilogue == MLLM_EPI_GELU_TANH) leave(integral_constant<int, MLLM_EPI_GELU_TANH>{}, integral_constant<int, 0>{});
     else if (epilogue == MLLM_EPI_GELU_ERF) leave(integral_constant<int, MLLM_EPI_GELU_ERF>{}, integral_constant<int, 0>{});
     else if (epilogue == MLLM_EPI_SQUARED_RELU) leave(integral_constant<int, MLLM_EPI_SQUARED_RELU>{}, integral_constant<int, 0>{});
     else leave(integral_constant<int, MLLM_EPI_NONE>{}, integral_constant<int, 0>{});
 }
 
-template <typename OutT, int BM, int BN, int WAVES_M, int WAVES_N, int WAVES_K, int STAGES>
+template <typename OutT, int BM, int BN, int WAVES_M, int WAVES_N, int WAVES_K, int STAGES, typename Group>
 void launch(const bf16_t* a, const bf16_t* w, const float* bias, const float* residual, OutT* o, int M, int N, int K, int epilogue,
            hipStream_t stream, CacheScatter scatter, int k_blocks) {
     // the stages of the loop, or what the epilogue passes through LDS (the sums that waves sharing a tile hand each other,
@@ -569,14 +589,14 @@ void launch(const bf16_t* a, const bf16_t* w, const float* bias, const float* re
     static bool raised = false;  // per instantiation: the limit on dynamic LDS is a property of the kernel
     if (!raised && LDS_BYTES > 64 * 1024) {
         // (if this fails the launch below fails too, and the entry point reports that)
-        raised = hipFuncSetAttribute((const void*)gemm_stream_kernel<OutT, BM, BN, WAVES_M, WAVES_N, WAVES_K, STAGES, Whole>,
+        raised = hipFuncSetAttribute((const void*)gemm_stream_kernel<OutT, BM, BN, WAVES_M, WAVES_N, WAVES_K, STAGES, Group>,
                                      hipFuncAttributeMaxDynamicSharedMemorySize, LDS_BYTES) == hipSuccess;
     }
     const int k_per_block = k_blocks == 1 ? K : ceil_div(ceil_div(K, k_blocks), 64) * 64;
     const XcdTiles places = place_tiles(ceil_div(M, BM), ceil_div(N, BN), BM, BN, k_blocks);
     mllm_count_kernel(MLLM_K_GEMM_STREAM);
-    gemm_stream_kernel<OutT, BM, BN, WAVES_M, WAVES_N, WAVES_K, STAGES, Whole><<<8 * places.per_xcd, 64 * NW, LDS_BYTES, stream>>>(
-        a, w, bias, residual, o, M, N, K, epilogue, scatter, k_per_block, places, Whole{});
+    gemm_stream_kernel<OutT, BM, BN, WAVES_M, WAVES_N, WAVES_K, STAGES, Group><<<8 * places.per_xcd, 64 * NW, LDS_BYTES, stream>>>(
+        a, w, bias, residual, o, M, N, K, epilogue, scatter, k_per_block, places, Group{});
 }
 
 // The same loop over rows grouped by expert. entries: how many there are; max_tiles: how many tiles of BM they can make at most.
@@ -679,11 +699,11 @@ inline Shape choose(int M, int N, int K, int k_blocks, bool bf16_out) {
     return ceil_div(K, k_blocks) >= 3072 && ((K % 4096 == 0 && blocks <= 192) || M <= 96) ? S128x64_SHARED : S128x64;
 }
 
-template <typename OutT>
+template <typename OutT, typename Group = Whole>
 void dispatch(const bf16_t* a, const bf16_t* w, const float* bias, const float* residual, OutT* o, int M, int N, int K, int epilogue,
               hipStream_t stream, CacheScatter scatter, int k_blocks) {
-#define MLLM_STREAM(BM, BN, WM_, WN_, WK_, ST) launch<OutT, BM, BN, WM_, WN_, WK_, ST>(a, w, bias, residual, o, M, N, K, epilogue, stream, scatter, k_blocks)
-    switch (choose(M, N, K, k_blocks, sizeof(OutT) == 2)) {
+#define MLLM_STREAM(BM, BN, WM_, WN_, WK_, ST) launch<OutT, BM, BN, WM_, WN_, WK_, ST, Group>(a, w, bias, residual, o, M, N, K, epilogue, stream, scatter, k_blocks)
+    switch (choose(M, N, K, k_blocks, sizeof(OutT) == 2 && !Group::UNITS)) {
         case S128x192: MLLM_STREAM(128, 192, 2, 2, 1, 3); break;
         case S192x128: MLLM_STREAM(192, 128, 2, 2, 1, 3); break;
         case S256x128: MLLM_STREAM(256, 128, 4, 2, 1, 3); break;
@@ -694,7 +714,7 @@ void dispatch(const bf16_t* a, const bf16_t* w, const float* bias, const float* 
         case S128x64_SHARED: MLLM_STREAM(128, 64, 2, 1, 2, 4); break;
         case S128x64_ROUNDS: MLLM_STREAM(128, 64, 2, 2, 1, 3); break;
         case S256x256:
-            if constexpr (sizeof(OutT) == 2) MLLM_STREAM(256, 256, 2, 2, 1, 2);
+            if constexpr (sizeof(OutT) == 2 && !Group::UNITS) MLLM_STREAM(256, 256, 2, 2, 1, 2);
             break;
     }
 #undef MLLM_STREAM

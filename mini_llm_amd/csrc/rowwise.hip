@@ -395,16 +395,16 @@ __global__ __launch_bounds__(256) void latent_rows_kernel(const T* __restrict__ 
     for (int i = 2 * half + lane; i < row_size - rank; i += WAVE) out[rank + i] = i < rot ? in[rank + i] : from_float<T>(0.0f);
 }
 
-// out[row, j] = silu(both[row, j]) * both[row, inner + j]: the two halves of a fused gate / up product. A thread takes a
-// 16-byte piece of each half where the rows are whole pieces (PIECES), else an element.
+// out[row, j] = silu(gate[row, j]) * up[row, j] over a fused gate / up product, whose columns are `turn` gate and `turn` up columns in turn (inner: the two
+// halves). A thread takes a 16-byte piece of each where they are whole pieces (PIECES), else an element.
 template <typename T, bool PIECES>
-__global__ __launch_bounds__(256) void silu_mul_kernel(const T* __restrict__ both, T* __restrict__ out, int inner) {
+__global__ __launch_bounds__(256) void silu_mul_kernel(const T* __restrict__ both, T* __restrict__ out, int inner, int turn) {
     constexpr int VEC = PIECES ? 16 / (int)sizeof(T) : 1;
     const int j = (blockIdx.x * blockDim.x + threadIdx.x) * VEC;
     if (j >= inner) return;
     const size_t row = blockIdx.y;
-    const T* a_at = both + row * 2 * inner + j;
-    const T* b_at = a_at + inner;
+    const T* a_at = both + row * 2 * inner + j + j / turn * turn;
+    const T* b_at = a_at + turn;
     T* out_at = out + row * inner + j;
     if constexpr (PIECES) {
         const Vec16 a = *reinterpret_cast<const Vec16*>(a_at), b = *reinterpret_cast<const Vec16*>(b_at);
@@ -539,19 +539,19 @@ MLLM_API int mllm_latent_rows(const void* q, int q_stride, const void* dkv, int 
 }
 
 template <typename T>
-void launch_silu_mul(const void* both, void* out, int n_rows, int inner, hipStream_t stream) {
+void launch_silu_mul(const void* both, void* out, int n_rows, int inner, int turn, hipStream_t stream) {
     constexpr int VEC = 16 / (int)sizeof(T);
-    if (inner % VEC == 0) {
+    if (turn % VEC == 0) {
         dim3 grid(ceil_div(inner / VEC, 256), n_rows);
-        silu_mul_kernel<T, true><<<grid, 256, 0, stream>>>((const T*)both, (T*)out, inner);
+        silu_mul_kernel<T, true><<<grid, 256, 0, stream>>>((const T*)both, (T*)out, inner, turn);
     } else {
         dim3 grid(ceil_div(inner, 256), n_rows);
-        silu_mul_kernel<T, false><<<grid, 256, 0, stream>>>((const T*)both, (T*)out, inner);
+        silu_mul_kernel<T, false><<<grid, 256, 0, stream>>>((const T*)both, (T*)out, inner, turn);
     }
 }
 
-MLLM_API int mllm_silu_mul(const void* both, void* out, int n_rows, int inner, int dtype, hipStream_t stream) {
-    MLLM_REQUIRE(n_rows >= 0 && n_rows <= 65535 * 64 && inner > 0, "silu_mul: bad sizes");
+MLLM_API int mllm_silu_mul(const void* both, void* out, int n_rows, int inner, int turn, int dtype, hipStream_t stream) {
+    MLLM_REQUIRE(n_rows >= 0 && n_rows <= 65535 * 64 && inner > 0 && turn > 0 && inner % turn == 0, "silu_mul: bad sizes");
     MLLM_REQUIRE(dtype == MLLM_F32 || dtype == MLLM_BF16, "silu_mul: unknown dtype %d", dtype);
     if (n_rows == 0) return 0;
     mllm_count_kernel(MLLM_K_SILU_MUL);
@@ -560,8 +560,8 @@ MLLM_API int mllm_silu_mul(const void* both, void* out, int n_rows, int inner, i
         const size_t element = dtype == MLLM_F32 ? 4 : 2;
         const char* in_at = (const char*)both + (size_t)row0 * 2 * inner * element;
         char* out_at = (char*)out + (size_t)row0 * inner * element;
-        if (dtype == MLLM_F32) launch_silu_mul<float>(in_at, out_at, rows, inner, stream);
-        else launch_silu_mul<bf16_t>(in_at, out_at, rows, inner, stream);
+        if (dtype == MLLM_F32) launch_silu_mul<float>(in_at, out_at, rows, inner, turn, stream);
+        else launch_silu_mul<bf16_t>(in_at, out_at, rows, inner, turn, stream);
     }
     return mllm_check_launch("silu_mul");
 }

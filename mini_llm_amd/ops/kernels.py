@@ -1107,13 +1107,39 @@ def head_norm(qkv, q_gain, k_gain, eps, positions, slots, k_pages, v_pages, n_he
     return q
 
 
-def silu_mul(both):
-    """silu(a) * b for rows [a | b] of a fused gate / up product: [rows, 2 * inner] -> [rows, inner]."""
+def silu_mul(both, turn: int | None = None):
+    """silu(a) * b for rows [a | b] of a fused gate / up product: [rows, 2 * inner] -> [rows, inner]. ``turn``: the rows hold so many columns of
+    a and as many of b in turn (None: one turn, the two halves)."""
     _device_tensor(both, "both", dim=2)
     _require(both.shape[1] % 2 == 0, "the rows do not hold two halves")
     n, inner = both.shape[0], both.shape[1] // 2
+    turn = inner if turn is None else int(turn)
+    _require(turn > 0 and inner % turn == 0, "the halves are no whole turns")
     out = torch.empty((n, inner), dtype=both.dtype, device=both.device)
-    check(library().mllm_silu_mul(_ptr(both), _ptr(out), n, inner, _code(both.dtype), _stream()))
+    check(library().mllm_silu_mul(_ptr(both), _ptr(out), n, inner, turn, _code(both.dtype), _stream()))
+    return out
+
+
+GATE_TURN = 8   # gate rows and up rows in turn of a matrix for ``gated_linear``
+
+
+def gate_up_rows(gate, up):
+    """Two matrices [inner, width], inner a multiple of GATE_TURN, as the one that ``gated_linear`` takes: GATE_TURN rows of either in turn."""
+    inner, width = gate.shape
+    return torch.stack([gate.reshape(-1, GATE_TURN, width), up.reshape(-1, GATE_TURN, width)], dim=1).reshape(2 * inner, width)
+
+
+def gated_linear(x, weight: PackedMatrix):
+    """silu(x gate^T) * (x up^T), [rows, inner] of x's type, from ``weight`` = ``gate_up_rows`` packed: the unit inside the product where one of
+    its kernels takes the sizes, else (rounded to x's type in between) in a kernel of its own."""
+    _device_tensor(x, "x", dim=2)
+    w_ptr, w_packed, n, k = _matrix(weight, "weight", x.dtype)
+    _require(w_packed and n % (2 * GATE_TURN) == 0 and x.shape[1] == k, "x and the packed gate and up rows do not match")
+    m, lib = x.shape[0], library()
+    out = torch.empty((m, n // 2), dtype=x.dtype, device=x.device)
+    if not lib.mllm_gemm_gated_takes(_ptr(x), _ptr(out), m, n, k, w_packed, _code(x.dtype)):
+        return silu_mul(linear(x, weight), turn=GATE_TURN)
+    check(lib.mllm_gemm_gated(_ptr(x), w_ptr, w_packed, _ptr(out), m, n, k, _code(x.dtype), _stream()))
     return out
 
 

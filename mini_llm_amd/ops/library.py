@@ -65,7 +65,9 @@ _SIGNATURES = {
     "mllm_rms_norm": [P, P, c_int, c_float, P, P, c_int, c_float, P, P, c_int, c_int, c_int, c_int, c_longlong, P, P, P],
     "mllm_head_norm": [P, c_int, P, P, c_float, c_float, c_int, P, P, P, P, P, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, P],
     "mllm_latent_rows": [P, c_int, P, c_int, P, c_float, P, c_float, c_int, c_int, P, P, P, P, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, P],
-    "mllm_silu_mul": [P, P, c_int, c_int, c_int, P],
+    "mllm_silu_mul": [P, P, c_int, c_int, c_int, c_int, P],
+    "mllm_gemm_gated_takes": [P, P, c_int, c_int, c_int, c_int, c_int],
+    "mllm_gemm_gated": [P, P, c_int, P, c_int, c_int, c_int, c_int, P],
     "mllm_map_rows": [P, c_int, c_int, c_int, c_int, P, P, c_float, P, c_int, P, P, P, P, P, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int,
                       c_int, P, c_int, c_int, c_int, P],
     "mllm_turn_heads": [P, c_int, P, c_int, P, c_int, c_int, c_float, P, c_int, c_int, c_int, c_int, c_int, P],

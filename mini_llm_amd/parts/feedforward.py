@@ -49,8 +49,9 @@ class DenseMLP(FeedForward):
 
 class GatedMLP(FeedForward):
     """down(silu(gate x) * (up x)), no biases; the three matrices are stored [out, in] under their bare names. Gate and up run
-    as one product over the two matrices laid behind each other, the activation and the multiplication as one kernel over its
-    halves, and the residual sum (if a residual is given) inside the down product."""
+    as one product over rows of the two matrices in turn, the activation and the multiplication in its end (of widths that are no
+    multiple of eight: over the two laid behind each other, and a kernel over its halves), and the residual sum (if a residual is
+    given) inside the down product."""
 
     def __init__(self, width: int, inner: int, names=("gate", "up", "down")):
         self.width, self.inner = width, inner
@@ -68,11 +69,13 @@ class GatedMLP(FeedForward):
 
     def bind(self, tensors):
         gate, up, down = (tensors[name] for name in self._names)
-        self.gate_up = kernels.pack_matrix(torch.cat([gate, up], dim=0).contiguous()) if gate.is_cuda else torch.cat([gate, up], dim=0)
+        self._in_turn = self.inner % kernels.GATE_TURN == 0
+        both = kernels.gate_up_rows(gate, up) if self._in_turn else torch.cat([gate, up], dim=0)
+        self.gate_up = kernels.pack_matrix(both.contiguous()) if both.is_cuda else both
         self.down = down
 
     def forward(self, x, residual):
-        inner = kernels.silu_mul(kernels.linear(x, self.gate_up))
+        inner = kernels.gated_linear(x, self.gate_up) if self._in_turn else kernels.silu_mul(kernels.linear(x, self.gate_up))
         return self._down_product(inner, self.down, residual)
 
 
