@@ -308,13 +308,14 @@ def measure_kernels(engine, batch: int = 8, context: int = 776, decode: bool = T
         layer_us = sum(us for _, us in cut[1])
         note("decode_layer", layer_us, (4.0 * d * d + 2.0 * d * ff) * e + cache_bytes, hbm, "HBM peak")
         out["decode_layer"]["by_entry_point"] = _by_entry_point([name for name, _ in cut[1]], [us for _, us in cut[1]])
-    if len(names) == 5 and names[1] == "decode_stack":   # all layers in one kernel
+    if len(names) == 4 and names[1] == "decode_stack":   # all layers and the norm behind them in one kernel
         note("decode_stack", each[1], n_layer * ((4.0 * d * d + 2.0 * d * ff) * e + cache_bytes), hbm, "HBM peak")
-        cut = (names[0], each[0]), None, list(zip(names[-3:], each[-3:]))
+        cut = (names[0], each[0]), None, [(None, None), *zip(names[-2:], each[-2:])]
     if cut is not None:
         out["decode_embed"] = {"us": round(cut[0][1], 2), "holds": "what a replay costs by itself"}
         (_, final_norm), (_, head), (_, choice) = cut[2]
-        out["decode_final_norm"] = {"us": round(final_norm, 2)}
+        if final_norm is not None:
+            out["decode_final_norm"] = {"us": round(final_norm, 2)}
         note("decode_head", head, float(vocab) * d * e, hbm, "HBM peak")
         out["decode_choice"] = {"us": round(choice, 2)}
     else:

@@ -11,6 +11,7 @@ from dataclasses import dataclass
 from ..ops import kernels
 from ..parts.base import Ahead, Norm, Part, PositionEncoding
 from ..parts.embedding import TokenEmbedding
+from ..parts.norms import LayerNorm
 from ..weights.spec import VECTOR, Normal, TensorSpec
 
 
@@ -191,7 +192,10 @@ class Model(Part):
             return None
         if any(pages.numel() * pages.element_size() >= 2**32 for layer, _ in layers for pages in (layer.k_pages, layer.v_pages)):   # what the kernel's offsets reach
             return None
-        return kernels.DecodeStack([layer for layer, _ in layers], batch.n_tokens, n_heads, eps_1, eps_2, scale, activation)
+        # a decode step wants the logits of all its rows, in their order: the norm in front of the head belongs to the kernel too
+        norm = self.final_norm
+        final = (norm.weight, norm.bias, norm.eps) if type(norm) is LayerNorm and batch.n_logit_rows == batch.n_tokens else None
+        return kernels.DecodeStack([layer for layer, _ in layers], batch.n_tokens, n_heads, eps_1, eps_2, scale, activation, final=final)
 
     def _layers(self, hidden, batch, cache, observer=None):
         """The schedule over the rows of ``batch``; the stream comes back as the last layer leaves it. A layer is told what comes ahead of
@@ -267,10 +271,13 @@ class Model(Part):
             hidden = self._layers(hidden, batch, cache, observer)
             if batch.n_logit_rows == 0:
                 return None
-            if not self.final_norm.takes_pending:
-                hidden = kernels.settle(hidden)
-            # the final norm runs on the wanted rows only (engine/src/gpt2_gpu.cu:254-258)
-            normed = self.final_norm.forward(hidden, self.precision.compute, row_index=batch.logit_rows)
+            if observer is None and batch.stack is not None and batch.stack.final is not None:
+                normed = hidden
+            else:
+                if not self.final_norm.takes_pending:
+                    hidden = kernels.settle(hidden)
+                # the final norm runs on the wanted rows only (engine/src/gpt2_gpu.cu:254-258)
+                normed = self.final_norm.forward(hidden, self.precision.compute, row_index=batch.logit_rows)
         if choice is None:
             return self.head.forward(normed)
         # Greedy tokens on the device. A head that can leave the best of its columns instead of all of them does (the

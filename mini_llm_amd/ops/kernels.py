@@ -983,8 +983,8 @@ class DecodeStack:
     share: the layers' tensors (and their addresses on the device), the words that the blocks of a launch hand to each other and the launch's control words.
     Launches of one DecodeStack follow each other on a stream; steps that may run side by side have one each."""
 
-    def __init__(self, layers, rows: int, n_heads: int, eps_1: float, eps_2: float, scale: float, activation: str, blocks: int | None = None):
-        """``blocks``: blocks of a launch (None: one for each compute unit)."""
+    def __init__(self, layers, rows: int, n_heads: int, eps_1: float, eps_2: float, scale: float, activation: str, blocks: int | None = None, final=None):
+        """``blocks``: blocks of a launch (None: one for each compute unit). ``final``: (gain, offset, eps) of a layer norm behind the last layer."""
         first = layers[0]
         self.layers, self.rows, self.n_heads = list(layers), int(rows), int(n_heads)
         self.eps_1, self.eps_2, self.scale, self.activation = float(eps_1), float(eps_2), float(scale), activation
@@ -1007,6 +1007,11 @@ class DecodeStack:
             _check_pages(layer.k_pages, layer.v_pages, n_heads, head_size)
             _require(layer.k_pages.dtype == self.dtype and layer.k_pages.shape[2] == self.page_size, f"layer {i}: pages of another kind")
             _require(layer.k_pages.numel() * layer.k_pages.element_size() < 2**32, f"layer {i}: more keys than 32-bit offsets reach")
+        self.final = final
+        if final is not None:
+            for v, name in zip(final, ("the final gain", "the final offset")):
+                _device_tensor(v, name, torch.float32, 1)
+                _require(v.shape[0] == width, f"{name} does not match the rows")
         names = StackLayer.__dataclass_fields__
         _require(library().mllm_decode_stack_layer_pointers() == len(names), "a layer's pointers do not match the library's")
         addresses = [[_ptr(getattr(layer, name).data if isinstance(getattr(layer, name), PackedMatrix) else getattr(layer, name)) for name in names] for layer in layers]
@@ -1016,17 +1021,19 @@ class DecodeStack:
         self.blocks = torch.cuda.get_device_properties(device).multi_processor_count if blocks is None else int(blocks)
 
     def run(self, hidden, token_request, positions, slots, block_tables):
-        """hidden: float32 [rows, width], each row the newest token of its request -> the stream behind the last layer. Keys and values
-        go into the cache."""
+        """hidden: float32 [rows, width], each row the newest token of its request -> the stream behind the last layer, or its rows normed
+        (of the matrices' type). Keys and values go into the cache."""
         _device_tensor(hidden, "hidden", torch.float32, 2)
         _require(tuple(hidden.shape) == (self.rows, self.width), f"the rows are not [{self.rows}, {self.width}]")
         for t, name in ((slots, "slots"), (token_request, "token_request"), (positions, "positions")):
             _device_tensor(t, name, torch.int32, 1)
             _require(t.shape[0] >= self.rows, f"{name} has fewer entries than rows")
         _device_tensor(block_tables, "block_tables", torch.int32, 2)
-        out = torch.empty_like(hidden)
+        gain, offset, eps = self.final if self.final is not None else (None, None, 0.0)
+        out = torch.empty_like(hidden, dtype=torch.float32 if gain is None else self.dtype)
         check(library().mllm_decode_stack(
-            _ptr(self.addresses), len(self.layers), _ptr(hidden), _ptr(out), _ptr(token_request), _ptr(positions), _ptr(slots), _ptr(block_tables), block_tables.shape[1],
+            _ptr(self.addresses), len(self.layers), _ptr(hidden), _ptr(out if gain is None else None), _ptr(token_request), _ptr(positions), _ptr(gain), _ptr(offset), float(eps),
+            _ptr(None if gain is None else out), _ptr(slots), _ptr(block_tables), block_tables.shape[1],
             _ptr(self.words), _ptr(self.control), self.rows, self.width, self.inner, self.n_heads, self.page_size, self.eps_1, self.eps_2, self.scale,
             EPILOGUES[self.activation], _code(self.dtype), self.blocks, _stream()))
         return out

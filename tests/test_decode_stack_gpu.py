@@ -137,6 +137,25 @@ def test_all_layers_in_one_kernel(dtype, layers, width, inner, contexts, page_si
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("dtype,width,contexts,blocks", [(B, 64, [3], None), (B, 768, [5] * 8, None), (B, 832, [9] * 16, None), (F, 768, [4, -1, 70], None), (F, 192, [10, 3, 8, 2], 4)])
+def test_the_norm_behind_the_last_layer(dtype, width, contexts, blocks):
+    # one block that norms and several rows; more rows than waves; a padding row
+    from mini_llm_amd.ops import kernels as K
+
+    rng = np.random.default_rng(width)
+    stack, given, _, _ = _stack(rng, 2, width, 2 * width, contexts, 64, dtype, "gelu_new", blocks)
+    stream = stack.run(*given)
+    gain, offset = (torch.as_tensor(rng.standard_normal(width).astype(np.float32), device=DEV) for _ in range(2))
+    normed = K.DecodeStack(stack.layers, len(contexts), width // 64, 2e-5, 2e-5, 0.125, "gelu_new", blocks=blocks, final=(gain, offset, 3e-5))
+    out = normed.run(*given)
+    # the norm's sums in another order: a few 2^-24 of numbers around 1; in bfloat16 a rounding that falls the other way, 2^-8 of them
+    bound = 2.0 ** -7 if dtype == B else 1e-5
+    torch.testing.assert_close(out.float(), K.layernorm(stream, gain, offset, 3e-5, out_dtype=dtype).float(), rtol=bound, atol=bound)
+    for _ in range(3):
+        assert out.dtype == dtype and torch.equal(normed.run(*given), out)
+
+
+@pytest.mark.gpu
 def test_all_layers_in_one_kernel_replayed_and_beside_another_stream():
     # a captured launch replayed with other work between the replays, and two stacks at once on two streams: each takes the units it finds
     rng = np.random.default_rng(5)
