@@ -73,7 +73,9 @@ def main(argv=None, steps=None, out=None) -> int:
                 observer = lambda name, rows: rows.cpu().numpy().astype("<f4", copy=False).tofile(hidden_dir / f"{step}.{name}.f32")
             logits = runner.step(entries, observer=observer)
             if logits is not None:
-                logits.cpu().numpy().astype("<f4", copy=False).tofile(out_dir / f"{step}.f32")
+                rows = logits.cpu().numpy()
+                runner.check()
+                rows.astype("<f4", copy=False).tofile(out_dir / f"{step}.f32")
         for request_id in record.get("end", []):
             if cache.has(request_id):
                 cache.close(request_id)

@@ -18,7 +18,8 @@
 // members is closed once, by whoever enters last or by a block that has waited CLOSE_AFTER for the rest (another stream's kernels may hold
 // the compute units), and blocks that start later leave at once. Work is divided among the members, however many they are. Phases
 // follow each other in one order in every block, and a block's waits are for earlier phases only, so the earliest phase that is
-// not done can always go on.
+// not done can always go on. A wave that has looked for its words very many times takes the device for broken: it goes on without numbers (NaN), so that
+// the launch ends, says so in memory that the host reads, and from there on no block keeps keys or values in the cache.
 //
 // Measured (replayed steps of GPT-2 small in bfloat16 with 512 keys a row; the two layer kernels a layer before): 8 rows 353 -> 206 us a step, 14.4 us a layer, 1 row
 // 296 -> 158; in 32-bit (seven kernels a layer before) 8 rows 496 -> 344. A layer's 14.4 us, from one hand to the next: stream to normed rows 1.7 and to q/k/v 1.1, to the
@@ -42,9 +43,10 @@ constexpr int ST_KEY_LOADS = 16;     // loads of keys, and of values, that a wav
 constexpr int ST_MIN_MEMBERS = 3;   // a block of each part
 constexpr int ST_MAX_PAIRS = 4;     // (row, head) pairs of an attending block: its waves are divided among them
 constexpr long long CLOSE_AFTER = 2000;   // ticks of 10 ns
-constexpr int PATIENCE = 1 << 22;         // looks at a word, each a trip to memory, before a wave takes the device for broken
-// control words, each on a cache line of its own
-constexpr int ARRIVED = 0, MEMBERS = 32, LEFT = 64, EPOCH = 96, CONTROL_INTS = 128;
+// control words, each on a cache line of its own; the last line holds what the host leaves there: PATIENCE, looks at a word, each a trip to memory, before a wave
+// takes the device for broken, and GAVE_UP, the address of the word on the host that becomes 1 then (two ints)
+constexpr int ARRIVED = 0, MEMBERS = 32, LEFT = 64, EPOCH = 96, PATIENCE = 128, GAVE_UP = 130, CONTROL_INTS = 160;
+constexpr unsigned BROKEN = 0, FIRST_REGION = 128;   // bytes among the words: what is not zero once a wave has given up a wait; where the words to hand on begin
 
 struct StackLayer {
     const float *gain_1, *offset_1;
@@ -108,10 +110,23 @@ __device__ __forceinline__ V load16(const void* uniform_base, unsigned byte_offs
 }
 __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
+// Looks that a wave has left, and the block's word for whether any wave of it has given up a wait.
+struct Patience {
+    int left;
+    int* block_gave_up;
+    // Whoever reads a word that the block hands on behind this finds BROKEN set.
+    __device__ __forceinline__ void give_up(const Words& words) {
+        left = 0;
+        *static_cast<volatile int*>(block_gave_up) = 1;
+        __builtin_amdgcn_raw_buffer_store_b32(1u, words.all, BROKEN, 0, DEVICE_WIDE);
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    }
+};
+
 // Loads N pieces of 16 bytes (two words each), piece i `further(i)` bytes behind the lane's `at`, until all of them, in every lane of the wave
 // and as far as they count, carry the tag.
 template <int N, typename Further, typename Counts>
-__device__ __forceinline__ void await_words(u32x4 (&got)[N], const Words& from, uint32_t tag, int& patience, unsigned at, Further further, Counts counts) {
+__device__ __forceinline__ void await_words(u32x4 (&got)[N], const Words& from, uint32_t tag, Patience& patience, unsigned at, Further further, Counts counts) {
     for (;;) {
         asm volatile("" ::: "memory");   // look again, and not at what an earlier look found
 #pragma unroll
@@ -120,19 +135,19 @@ __device__ __forceinline__ void await_words(u32x4 (&got)[N], const Words& from, 
 #pragma unroll
         for (int i = 0; i < N; i++) there = there && ((got[i][1] == tag && got[i][3] == tag) || !counts(i));
         if (__builtin_amdgcn_ballot_w64(!there) == 0) return;
-        if (patience-- <= 0) break;
+        if (patience.left-- <= 0) break;
     }
-    patience = 0;   // no number at all, here and in all that is computed from it
+    patience.give_up(from);   // no number at all, here and in all that is computed from it
 #pragma unroll
     for (int i = 0; i < N; i++) got[i] = u32x4{~0u, tag, ~0u, tag};
 }
 template <int N, typename Further>
-__device__ __forceinline__ void await_words(u32x4 (&got)[N], const Words& from, uint32_t tag, int& patience, unsigned at, Further further) {
+__device__ __forceinline__ void await_words(u32x4 (&got)[N], const Words& from, uint32_t tag, Patience& patience, unsigned at, Further further) {
     await_words(got, from, tag, patience, at, further, [](int) { return true; });
 }
 // The same with a place of its own for every piece, in every lane.
 template <int N, typename At>
-__device__ __forceinline__ void await_words_at(u32x4 (&got)[N], const Words& from, uint32_t tag, int& patience, At at) {
+__device__ __forceinline__ void await_words_at(u32x4 (&got)[N], const Words& from, uint32_t tag, Patience& patience, At at) {
     unsigned place[N];
 #pragma unroll
     for (int i = 0; i < N; i++) place[i] = at(i);
@@ -144,9 +159,9 @@ __device__ __forceinline__ void await_words_at(u32x4 (&got)[N], const Words& fro
 #pragma unroll
         for (int i = 0; i < N; i++) there = there && got[i][1] == tag && got[i][3] == tag;
         if (__builtin_amdgcn_ballot_w64(!there) == 0) return;
-        if (patience-- <= 0) break;
+        if (patience.left-- <= 0) break;
     }
-    patience = 0;
+    patience.give_up(from);
 #pragma unroll
     for (int i = 0; i < N; i++) got[i] = u32x4{~0u, tag, ~0u, tag};
 }
@@ -226,7 +241,7 @@ __global__ __launch_bounds__(ST_THREADS) void decode_stack_kernel(StackArgs a) {
     constexpr int NORM_ROWS = ROWS > ST_WAVES ? 2 : 1;   // rows a wave norms
     extern __shared__ __attribute__((aligned(16))) char lds[];
     __shared__ StackLayer layer_at[ST_MAX_LAYERS];
-    __shared__ int shared_rank, shared_members, shared_epoch;
+    __shared__ int shared_rank, shared_members, shared_epoch, shared_patience, shared_gave_up;
 
     // each on its own: kept together, as they arrive, sixteen scalar registers are brought back for one
     anew(a.words), anew(a.rows_in), anew(a.rows_out), anew(a.block_tables), anew(a.token_request), anew(a.positions), anew(a.slots), anew(a.layers), anew(a.control);
@@ -235,6 +250,7 @@ __global__ __launch_bounds__(ST_THREADS) void decode_stack_kernel(StackArgs a) {
     int wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
     int M = a.rows, width = a.width, inner = a.inner;
     if (tid == 0) {
+        shared_patience = a.control[PATIENCE], shared_gave_up = 0;
         shared_epoch = __hip_atomic_load(a.control + EPOCH, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         const int blocks = (int)gridDim.x;
         const int rank = __hip_atomic_fetch_add(a.control + ARRIVED, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -262,10 +278,10 @@ __global__ __launch_bounds__(ST_THREADS) void decode_stack_kernel(StackArgs a) {
 
     // the regions of words: a layer's input rows, the rows behind its attention, q/k/v, the heads' outputs, the hidden units
     const unsigned row_bytes = (unsigned)(M * width) * 8u, mixed_bytes = row_bytes / EPW, unit_bytes = (unsigned)(M * inner) * 8u / EPW;
-    const unsigned region_ends = 2 * row_bytes + 4 * mixed_bytes;
+    const unsigned region_ends = FIRST_REGION + 2 * row_bytes + 4 * mixed_bytes;
     const __amdgpu_buffer_rsrc_t all_words = __builtin_amdgcn_make_buffer_rsrc(a.words, 0, region_ends + unit_bytes, 0x00020000);
-    const Words rows_words{all_words, 0}, later_words{all_words, row_bytes}, qkv_words{all_words, 2 * row_bytes};
-    const Words mixed_words{all_words, 2 * row_bytes + 3 * mixed_bytes}, unit_words{all_words, region_ends};
+    const Words rows_words{all_words, FIRST_REGION}, later_words{all_words, FIRST_REGION + row_bytes}, qkv_words{all_words, FIRST_REGION + 2 * row_bytes};
+    const Words mixed_words{all_words, FIRST_REGION + 2 * row_bytes + 3 * mixed_bytes}, unit_words{all_words, region_ends};
 
     const Operands mixed_lie{128u, (unsigned)(width / KC) * 128u}, unit_lie{(unsigned)M * 128u, 16u};
     // a tile's 16 columns of q, k or v lie together, row behind row
@@ -277,7 +293,7 @@ __global__ __launch_bounds__(ST_THREADS) void decode_stack_kernel(StackArgs a) {
     const int row_tiles = width / 16;
     const int attending = min(groups, max(members / 2, 1)), summing = min(row_tiles, max((members - attending) / 2, 1));
     const int norming = members - attending - summing;
-    int patience = PATIENCE;
+    Patience patience{__builtin_amdgcn_readfirstlane(shared_patience), &shared_gave_up};
     auto pointer = [&](auto StackLayer::*which, int layer) {   // a pointer of a layer, in scalar registers
         const unsigned long long held = (unsigned long long)(layer_at[layer].*which);
         const unsigned lo = (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)held), hi = (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)(held >> 32));
@@ -308,6 +324,7 @@ __global__ __launch_bounds__(ST_THREADS) void decode_stack_kernel(StackArgs a) {
         // ---- attending: the block's waves are divided among its pairs, and a pair's waves share its keys, the token's own (the newest) among them
         constexpr int LPR = Sweep::LPR, RPI = Sweep::RPI;   // lanes that share a key, keys a load of the wave covers
         float (*merged)[ST_HEAD + 4] = reinterpret_cast<float (*)[ST_HEAD + 4]>(lds);   // [waves]: output, maximum, sum
+        Vec16 (*own_rows)[2][LPR] = reinterpret_cast<Vec16 (*)[2][LPR]>(lds + sizeof(float) * ST_WAVES * (ST_HEAD + 4));   // [waves]: the token's own key and value
         const int pair_waves = ST_WAVES / per_block, wave_in_pair = wave % pair_waves;
         const int sub = lane % LPR, group_in_wave = lane / LPR, page_mask = (1 << a.page_shift) - 1;
         int token, head, slot, far, begin, end, own;   // the wave's keys: far .. begin-1 from memory, begin .. end-1 in registers; the own key's place among these (or none: < 0)
@@ -362,14 +379,10 @@ __global__ __launch_bounds__(ST_THREADS) void decode_stack_kernel(StackArgs a) {
                     await_words(six, qkv_words, tag, patience, q_at, [&](int i) { return (unsigned)(i / 2) * step + (unsigned)(i % 2) * 16u; });
                     q_words[0] = six[0], q_words[1] = six[1];
                     const Vec16 key{{six[2][0], six[2][2], six[3][0], six[3][2]}}, value{{six[4][0], six[4][2], six[5][0], six[5][2]}};
+                    if (lane < LPR) own_rows[wave][0][sub] = key, own_rows[wave][1][sub] = value;
 #pragma unroll
                     for (int u = 0; u < ST_KEY_LOADS; u++)
                         if (u == own / RPI && group_in_wave >= own % RPI) keys[u] = __builtin_bit_cast(Raw, key), values[u] = __builtin_bit_cast(Raw, value);
-                    if (slot >= 0 && lane < LPR) {   // into the cache, for later steps
-                        const size_t row = ((((size_t)(slot >> a.page_shift) * a.n_heads + head) << a.page_shift) + (slot & page_mask)) * ST_HEAD + sub * VEC;
-                        *reinterpret_cast<Vec16*>(reinterpret_cast<T*>(pointer(&StackLayer::k_pages, layer)) + row) = key;
-                        *reinterpret_cast<Vec16*>(reinterpret_cast<T*>(pointer(&StackLayer::v_pages, layer)) + row) = value;
-                    }
                 } else {
                     await_words(q_words, qkv_words, tag, patience, q_at, [&](int i) { return (unsigned)i * 16u; });
                 }
@@ -446,6 +459,12 @@ __global__ __launch_bounds__(ST_THREADS) void decode_stack_kernel(StackArgs a) {
                     if (lane % OWN == 0 && live) store_operand<T>(mixed_words, mixed_lie, token, head * ST_HEAD + lane, piece, tag);
                 }
                 lds_barrier();   // what this layer has to say is on its way before the next keys are asked for: a unit's memory pipeline is one queue
+                // Into the cache, for later steps, once all else is done that others wait for: behind a look at whether these are numbers.
+                if (own >= 0 && slot >= 0 && __builtin_amdgcn_raw_buffer_load_b32(all_words, BROKEN, 0, DEVICE_WIDE) == 0u && lane < LPR) {
+                    const size_t row = ((((size_t)(slot >> a.page_shift) * a.n_heads + head) << a.page_shift) + (slot & page_mask)) * ST_HEAD + sub * VEC;
+                    *reinterpret_cast<Vec16*>(reinterpret_cast<T*>(pointer(&StackLayer::k_pages, layer)) + row) = own_rows[wave][0][sub];
+                    *reinterpret_cast<Vec16*>(reinterpret_cast<T*>(pointer(&StackLayer::v_pages, layer)) + row) = own_rows[wave][1][sub];
+                }
             }
         }
     } else if (rank < attending + summing) {
@@ -724,6 +743,7 @@ __global__ __launch_bounds__(ST_THREADS) void decode_stack_kernel(StackArgs a) {
     // the block that leaves last makes the control words ready for the next launch, which begins behind this one's end
     __syncthreads();
     if (tid == 0) {
+        if (shared_gave_up) __hip_atomic_store(*reinterpret_cast<int* const*>(a.control + GAVE_UP), 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
         const int left = __hip_atomic_fetch_add(a.control + LEFT, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         if (left == (int)gridDim.x - 1) {
             __hip_atomic_store(a.control + ARRIVED, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -771,9 +791,10 @@ MLLM_API int mllm_decode_stack_pays(int rows, int reach, int width) {
 
 MLLM_API long long mllm_decode_stack_word_bytes(int rows, int width, int inner, int dtype) {
     const long long row = (long long)rows * width * 8, per = dtype == MLLM_BF16 ? 2 : 1;
-    return 2 * row + 4 * row / per + (long long)rows * inner * 8 / per;
+    return FIRST_REGION + 2 * row + 4 * row / per + (long long)rows * inner * 8 / per;
 }
 MLLM_API int mllm_decode_stack_control_ints() { return CONTROL_INTS; }
+MLLM_API int mllm_decode_stack_patience_at() { return PATIENCE; }   // where among the control words the host leaves the patience, and two ints on the word that says of a wait given up
 MLLM_API int mllm_decode_stack_layer_pointers() { return LAYER_POINTERS; }
 
 MLLM_API int mllm_decode_stack(const void* layers, int n_layers, const float* rows_in, float* rows_out, const int* token_request, const int* positions,
@@ -793,7 +814,7 @@ MLLM_API int mllm_decode_stack(const void* layers, int n_layers, const float* ro
     StackArgs a{(const StackLayer*)layers, rows_in, rows_out, final_gain, final_offset, normed_out, token_request, positions, slots, block_tables, (char*)words, control,
                 n_layers, rows, width, inner, n_heads, max_blocks, page_shift, pairs_a_block, activation, eps_1, eps_2, eps_final, scale};
     const int element = dtype == MLLM_BF16 ? 2 : 4, steps = stack_steps(rows, width, inner, n_heads, element);
-    const size_t normed = (size_t)rows * normed_stride(width, element) * element, attend = ST_WAVES * (ST_HEAD + 4) * 4;
+    const size_t normed = (size_t)rows * normed_stride(width, element) * element, attend = ST_WAVES * ((ST_HEAD + 4) * 4 + 2 * ST_HEAD * element);
 #define MLLM_STACK_LAUNCH(T, STEPS, TILES, ROWS)                                                                                     \
     case ROWS: {                                                                                                                     \
         auto kernel = decode_stack_kernel<T, STEPS, TILES, ROWS>;                                                                    \

@@ -113,8 +113,10 @@ class Session:
 
     def prefill(self, token_ids) -> np.ndarray:
         tokens = [int(t) for t in token_ids]
-        logits = self._active().runner.step([StepEntry(self._handle, tokens, [len(tokens) - 1])])
-        return logits[0].cpu().numpy()
+        runner = self._active().runner
+        row = runner.step([StepEntry(self._handle, tokens, [len(tokens) - 1])])[0].cpu().numpy()
+        runner.check()
+        return row
 
     def decode(self, token_id: int) -> np.ndarray:
         return self.prefill([token_id])

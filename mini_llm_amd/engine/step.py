@@ -64,13 +64,14 @@ class ChosenTokens:
     """The tokens a step chose on the device: ``device`` (int32, one per wanted row, valid until the next step) and, on
     the host, a row of page-locked memory. The row is complete once ``event`` has passed or, where the step's last
     kernel writes the row itself, once the row's last entry shows the step's ``number`` (``tolist`` waits for either).
-    A row is used again ``TOKEN_RING_ROWS`` steps later."""
+    A row is used again ``TOKEN_RING_ROWS`` steps later. ``check``: called once the row is complete; raises where its tokens
+    are none (a step that was given up on the device)."""
 
-    __slots__ = ("device", "_host", "_n", "_event", "_number", "_flags")
+    __slots__ = ("device", "_host", "_n", "_event", "_number", "_flags", "_check")
     WAIT_SECONDS = 30.0
 
-    def __init__(self, device, host, n, event=None, number=None, flags=1):
-        self.device, self._host, self._n, self._event, self._number, self._flags = device, host, n, event, number, flags
+    def __init__(self, device, host, n, event=None, number=None, flags=1, check=None):
+        self.device, self._host, self._n, self._event, self._number, self._flags, self._check = device, host, n, event, number, flags, check
 
     def __len__(self):
         return self._n
@@ -80,6 +81,8 @@ class ChosenTokens:
             self._event.synchronize()
         else:
             self._await_number()
+        if self._check is not None:
+            self._check()
         return self._host[: self._n].tolist()
 
     def _await_number(self) -> None:
@@ -168,6 +171,8 @@ class _DecodeGraph:
 
     def run(self, entries, sampling=None):
         runner = self.runner
+        if self.static_batch.stack is not None:
+            self.static_batch.stack.check()   # a step that was given up: its sequences have nothing to go on from
         if self.chooses:
             return self._run_choosing(entries, sampling)
         runner.staging.upload(self.builder.fill(entries), into=self.buffer)
@@ -219,7 +224,8 @@ class _DecodeGraph:
             choice = TokenChoice(cache.last_token, host_ring=self.ring, cursor=self.builder.cursor_view(self.buffer), advance=True, draws=draws)
             self.graph, self.logits = _capture(runner, batch, choice, self.lanes)
         self.graph.replay()
-        chosen = ChosenTokens(self.logits[: len(entries)], self.ring_rows[self.ring_at], len(entries), number=self.number, flags=self.flags)
+        chosen = ChosenTokens(self.logits[: len(entries)], self.ring_rows[self.ring_at], len(entries), number=self.number, flags=self.flags,
+                              check=None if batch.stack is None else batch.stack.check)
         self.ring_at = (self.ring_at + 1) % TOKEN_RING_ROWS
         self.number = (self.number + 1) & 0x3FFFFFFF
         self.on_device = [(r, r.table_changes, r.length + 1, how, None if count is None else count + 1) for r, how, count in zip(records, hows, counts)]
@@ -320,6 +326,12 @@ class ModelRunner:
         self._sampler = None
         self.portion_graphs_made = 0      # captures of steps with prompt portions, and those given up for a newer shape
         self.portion_graphs_dropped = 0
+
+    def check(self) -> None:
+        """Raises where the last step, whose results have been waited for, was given up on the device: for whoever reads the
+        logits of ``step`` (chosen tokens are checked as they are read)."""
+        if self.last_batch is not None and self.last_batch.stack is not None:
+            self.last_batch.stack.check()
 
     def drop_graphs(self) -> None:
         """Gives the captured steps back now (they and the runner refer to each other, so otherwise they would lie around

@@ -981,10 +981,15 @@ def decode_stack_pays(rows, reach, n_layers, width, inner, n_heads, head_size, p
 class DecodeStack:
     """All layers of a pre-norm model for up to ``rows`` rows that bring one token each, in one kernel. Holds what the launches of one captured step
     share: the layers' tensors (and their addresses on the device), the words that the blocks of a launch hand to each other and the launch's control words.
-    Launches of one DecodeStack follow each other on a stream; steps that may run side by side have one each."""
+    Launches of one DecodeStack follow each other on a stream; steps that may run side by side have one each. A launch whose blocks have waited for each other
+    in vain (``PATIENCE`` looks: seconds) ends all the same, with no numbers in its rows; whoever reads them calls ``check`` first."""
 
-    def __init__(self, layers, rows: int, n_heads: int, eps_1: float, eps_2: float, scale: float, activation: str, blocks: int | None = None, final=None):
-        """``blocks``: blocks of a launch (None: one for each compute unit). ``final``: (gain, offset, eps) of a layer norm behind the last layer."""
+    PATIENCE = 1 << 22   # looks at a word, each a trip to memory, before a wave takes the device for broken
+
+    def __init__(self, layers, rows: int, n_heads: int, eps_1: float, eps_2: float, scale: float, activation: str, blocks: int | None = None, final=None,
+                 patience: int | None = None):
+        """``blocks``: blocks of a launch (None: one for each compute unit). ``final``: (gain, offset, eps) of a layer norm behind the last layer.
+        ``patience``: instead of PATIENCE."""
         first = layers[0]
         self.layers, self.rows, self.n_heads = list(layers), int(rows), int(n_heads)
         self.eps_1, self.eps_2, self.scale, self.activation = float(eps_1), float(eps_2), float(scale), activation
@@ -1017,8 +1022,20 @@ class DecodeStack:
         addresses = [[_ptr(getattr(layer, name).data if isinstance(getattr(layer, name), PackedMatrix) else getattr(layer, name)) for name in names] for layer in layers]
         self.addresses = torch.tensor(addresses, dtype=torch.int64, device=device)
         self.words = torch.zeros(int(library().mllm_decode_stack_word_bytes(self.rows, width, inner, _code(self.dtype))) // 4, dtype=torch.int32, device=device)
-        self.control = torch.zeros(int(library().mllm_decode_stack_control_ints()), dtype=torch.int32, device=device)
+        self._gave_up = torch.zeros(1, dtype=torch.int32).pin_memory()   # written by a launch that gave up a wait
+        self._gave_up_read = self._gave_up.numpy()                       # the same memory, for the host's looks
+        at = int(library().mllm_decode_stack_patience_at())
+        control = torch.zeros(int(library().mllm_decode_stack_control_ints()), dtype=torch.int32)
+        control[at] = self.PATIENCE if patience is None else int(patience)
+        control[at + 2 : at + 4] = torch.tensor([_ptr(self._gave_up)], dtype=torch.int64).view(torch.int32)
+        self._all_control = control.to(device)
+        self.control = self._all_control[:at]   # the launches' own
         self.blocks = torch.cuda.get_device_properties(device).multi_processor_count if blocks is None else int(blocks)
+
+    def check(self):
+        """Raises where a launch that is over has given up a wait: neither its rows nor what it left in the cache can be used."""
+        if self._gave_up_read[0]:
+            raise RuntimeError("a decode step on the device waited for its own blocks in vain and was given up")
 
     def run(self, hidden, token_request, positions, slots, block_tables):
         """hidden: float32 [rows, width], each row the newest token of its request -> the stream behind the last layer, or its rows normed

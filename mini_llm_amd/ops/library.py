@@ -55,6 +55,7 @@ _SIGNATURES = {
     "mllm_decode_stack_pays": [c_int, c_int, c_int],
     "mllm_decode_stack_word_bytes": [c_int, c_int, c_int, c_int],
     "mllm_decode_stack_control_ints": [],
+    "mllm_decode_stack_patience_at": [],
     "mllm_decode_stack_layer_pointers": [],
     "mllm_decode_stack": [P, c_int, P, P, P, P, P, P, c_float, P, P, P, c_int, P, P, c_int, c_int, c_int, c_int, c_int, c_float, c_float, c_float, c_int, c_int, c_int, P],
     "mllm_pending_sum": [P, P, P, c_int, P, c_int, c_int, P],

@@ -181,3 +181,60 @@ def test_all_layers_in_one_kernel_replayed_and_beside_another_stream():
     torch.cuda.synchronize()
     # with fewer members a block has more tiles and pairs, each summed in the same order: the same bits
     assert all(torch.equal(o, out) for o in outs[0]) and all(torch.equal(o, out_2) for o in outs[1])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype,with_norm", [(B, False), (B, True), (F, False), (F, True)])
+def test_a_wait_that_is_given_up(dtype, with_norm):
+    # Without patience the first look at words that are not there yet is the last one: the launch ends, says so, and neither rows nor cache hold numbers
+    # that were not computed.
+    from mini_llm_amd.ops import kernels as K
+
+    rng = np.random.default_rng(11)
+    contexts = [70, 5, -1]
+    stack, given, _, _ = _stack(rng, 3, 768, 3072, contexts, 64, dtype, "gelu_new", None)
+    good = stack.run(*given).clone()
+    torch.cuda.synchronize()
+    stack.check()
+    kept = [(layer.k_pages.clone(), layer.v_pages.clone()) for layer in stack.layers]
+    vector = lambda: torch.as_tensor(rng.standard_normal(768).astype(np.float32), device=DEV)
+    hasty = K.DecodeStack(stack.layers, len(contexts), 12, 2e-5, 2e-5, 0.125, "gelu_new", final=(vector(), vector(), 2e-5) if with_norm else None, patience=0)
+    out = hasty.run(*given)
+    torch.cuda.synchronize()
+    assert torch.isnan(out).any()
+    with pytest.raises(RuntimeError, match="given up"):
+        hasty.check()
+    for layer, pages in zip(stack.layers, kept):   # (the keys and values of this token, where its launch came so far, are those of the launch before)
+        for here, was in zip((layer.k_pages, layer.v_pages), pages):
+            raw = torch.int16 if dtype == B else torch.int32
+            assert torch.equal(here.view(raw), was.view(raw))
+    control = hasty.control.cpu()
+    assert control[96] == 1 and int(control.count_nonzero()) == 1   # ready for the next launch
+    assert torch.equal(stack.run(*given), good)                     # and others are as they were
+    stack.check()
+
+
+@pytest.mark.gpu
+def test_an_engine_reports_a_step_that_was_given_up(monkeypatch):
+    from mini_llm_amd.config import config_from_dict
+    from mini_llm_amd.engine import StepEntry
+    from mini_llm_amd.engine.engine import Engine, EngineOptions
+    from mini_llm_amd.ops import kernels as K
+
+    monkeypatch.setattr(K.DecodeStack, "PATIENCE", 0)
+    raw = {"architectures": ["GPT2LMHeadModel"], "n_layer": 2, "n_embd": 128, "n_head": 2, "n_inner": 512, "vocab_size": 300, "n_positions": 128,
+           "layer_norm_epsilon": 1e-5, "activation_function": "gelu_new"}
+    engine = Engine.from_random(config_from_dict(raw), 3, EngineOptions(dtype="bfloat16", max_sessions=4))
+    handle = engine.try_take_cache()
+    token = engine.prefill_greedy(handle, [1, 2, 3])
+    with pytest.raises(RuntimeError, match="given up"):
+        engine.decode_batch([handle], [token])                       # chosen tokens: as they are read
+    length = engine.cache.length(handle)
+    with pytest.raises(RuntimeError, match="given up"):
+        engine.runner.step([StepEntry(handle, [4], [0])], choose=True)   # the next step of the kind: before it is launched
+    assert engine.cache.length(handle) == length
+    with engine.open_session() as session:
+        session.prefill([5, 6, 7])
+        with pytest.raises(RuntimeError, match="given up"):
+            session.decode(8)                                        # logits: as they are read
+    engine.close()
