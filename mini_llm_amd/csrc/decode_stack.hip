@@ -15,8 +15,8 @@
 // among the block's waves. The owner of a tile of the output product and of the same tile of the down product keeps its part of the residual stream in registers.
 //
 // Who waits for whom. A wait is only ever for a block that is on the chip. Blocks enter themselves in a count as they start; the set of
-// members is closed once, by whoever enters last or by a block that has waited CLOSE_AFTER for the rest (another stream's kernels may hold
-// the compute units), and blocks that start later leave at once. Work is divided among the members, however many they are. Phases
+// members is closed once, by whoever enters last or by a block that has waited long enough for the rest (another stream's kernels may hold
+// the compute units; LOSS_A_LAYER), and blocks that start later leave at once. Work is divided among the members, however many they are. Phases
 // follow each other in one order in every block, and a block's waits are for earlier phases only, so the earliest phase that is
 // not done can always go on. A wave that has looked for its words very many times takes the device for broken: it goes on without numbers (NaN), so that
 // the launch ends, says so in memory that the host reads, and from there on no block keeps keys or values in the cache.
@@ -42,10 +42,15 @@ constexpr int ST_MAX_LAYERS = 64;   // their pointers lie in LDS
 constexpr int ST_KEY_LOADS = 16;     // loads of keys, and of values, that a wave keeps in registers: 128 keys in bfloat16, 64 in 32-bit
 constexpr int ST_MIN_MEMBERS = 3;   // a block of each part
 constexpr int ST_MAX_PAIRS = 4;     // (row, head) pairs of an attending block: its waves are divided among them
-constexpr long long CLOSE_AFTER = 2000;   // ticks of 10 ns
+// How long (ticks of 10 ns) a launch waits for blocks that have not found a place: CLOSE_AFTER, and what it would lose by going on without them, so that it never
+// takes much longer than twice what is best. A step's time goes with one over the members (12 layers of 768 columns, 8 rows in bfloat16, us with
+// 16 / 64 / 128 / 192 / 256 blocks: 2,597 / 601 / 344 / 217 / 192), about LOSS_A_LAYER for each time that the missing blocks are as many as the members. Such steps one after the
+// other beside another stream's products of 45 us: 200 to 1,080 us each where all that were there after CLOSE_AFTER went on, 220 to 260 now; beside products of
+// 177 us 200 to 3,300, and 220 to 590 now.
+constexpr int CLOSE_AFTER = 2000, LOSS_A_LAYER = 1000;
 // control words, each on a cache line of its own; the last line holds what the host leaves there: PATIENCE, looks at a word, each a trip to memory, before a wave
-// takes the device for broken, and GAVE_UP, the address of the word on the host that becomes 1 then (two ints)
-constexpr int ARRIVED = 0, MEMBERS = 32, LEFT = 64, EPOCH = 96, PATIENCE = 128, GAVE_UP = 130, CONTROL_INTS = 160;
+// takes the device for broken, and GAVE_UP, the address of the word on the host that becomes 1 then (two ints); and for the host TOOK_PART, how many members the last launch had
+constexpr int ARRIVED = 0, MEMBERS = 32, LEFT = 64, EPOCH = 96, PATIENCE = 128, GAVE_UP = 130, TOOK_PART = 132, CONTROL_INTS = 160;
 constexpr unsigned BROKEN = 0, FIRST_REGION = 128;   // bytes among the words: what is not zero once a wave has given up a wait; where the words to hand on begin
 
 struct StackLayer {
@@ -262,9 +267,10 @@ __global__ __launch_bounds__(ST_THREADS) void decode_stack_kernel(StackArgs a) {
         const long long since = wall_clock64();
         int members;
         while ((members = __hip_atomic_load(a.control + MEMBERS, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) == 0) {
-            if (wall_clock64() - since > CLOSE_AFTER) {
-                const int count = __hip_atomic_load(a.control + ARRIVED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                if (count >= ST_MIN_MEMBERS) close(min(count, blocks));
+            const long long waited = wall_clock64() - since;
+            if (waited > CLOSE_AFTER) {
+                const int count = min(__hip_atomic_load(a.control + ARRIVED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT), blocks);
+                if (count >= ST_MIN_MEMBERS && (waited - CLOSE_AFTER) * count > (long long)LOSS_A_LAYER * a.n_layers * (blocks - count)) close(count);
             }
         }
         shared_members = members;
@@ -747,6 +753,7 @@ __global__ __launch_bounds__(ST_THREADS) void decode_stack_kernel(StackArgs a) {
         const int left = __hip_atomic_fetch_add(a.control + LEFT, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         if (left == (int)gridDim.x - 1) {
             __hip_atomic_store(a.control + ARRIVED, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            a.control[TOOK_PART] = members;
             __hip_atomic_store(a.control + MEMBERS, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             __hip_atomic_store(a.control + LEFT, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             __hip_atomic_store(a.control + EPOCH, shared_epoch + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -794,7 +801,7 @@ MLLM_API long long mllm_decode_stack_word_bytes(int rows, int width, int inner, 
     return FIRST_REGION + 2 * row + 4 * row / per + (long long)rows * inner * 8 / per;
 }
 MLLM_API int mllm_decode_stack_control_ints() { return CONTROL_INTS; }
-MLLM_API int mllm_decode_stack_patience_at() { return PATIENCE; }   // where among the control words the host leaves the patience, and two ints on the word that says of a wait given up
+MLLM_API int mllm_decode_stack_patience_at() { return PATIENCE; }   // where among the control words the host leaves the patience, two ints on the address of the word that says of a wait given up, and again two on finds how many blocks took part
 MLLM_API int mllm_decode_stack_layer_pointers() { return LAYER_POINTERS; }
 
 MLLM_API int mllm_decode_stack(const void* layers, int n_layers, const float* rows_in, float* rows_out, const int* token_request, const int* positions,

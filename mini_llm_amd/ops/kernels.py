@@ -1032,6 +1032,10 @@ class DecodeStack:
         self.control = self._all_control[:at]   # the launches' own
         self.blocks = torch.cuda.get_device_properties(device).multi_processor_count if blocks is None else int(blocks)
 
+    def blocks_of_last(self) -> int:
+        """How many blocks shared the work of the last launch (waits for it): fewer than ``blocks`` where other streams' kernels held compute units for long."""
+        return int(self._all_control[self.control.shape[0] + 4])
+
     def check(self):
         """Raises where a launch that is over has given up a wait: neither its rows nor what it left in the cache can be used."""
         if self._gave_up_read[0]:
