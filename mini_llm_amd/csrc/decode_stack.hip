@@ -767,7 +767,6 @@ __global__ __launch_bounds__(ST_THREADS) void decode_stack_kernel(StackArgs a) {
 static int stack_steps(int rows, int width, int inner, int n_heads, int element_size) {
     const int kc = 64 / element_size;
     if (rows < 1 || rows > ST_MAX_ROWS || width < 64 || width % 64 || n_heads * ST_HEAD != width || inner < 32 || inner % 32) return 0;
-    if ((rows * n_heads + ST_MAX_PAIRS - 1) / ST_MAX_PAIRS > 128) return 0;
     const int steps = ceil_div(width / kc, ST_WAVES), long_steps = ceil_div(inner / kc, ST_WAVES);
     for (int built : {3, 4, 6, 7, 8}) {
         if ((element_size == 2) == (built == 6 || built == 8)) continue;   // (those two in 32-bit)

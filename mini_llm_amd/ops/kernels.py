@@ -1050,6 +1050,7 @@ class DecodeStack:
             _device_tensor(t, name, torch.int32, 1)
             _require(t.shape[0] >= self.rows, f"{name} has fewer entries than rows")
         _device_tensor(block_tables, "block_tables", torch.int32, 2)
+        _require(block_tables.shape[0] >= self.rows, "block_tables has fewer lines than rows")
         gain, offset, eps = self.final if self.final is not None else (None, None, 0.0)
         out = torch.empty_like(hidden, dtype=torch.float32 if gain is None else self.dtype)
         check(library().mllm_decode_stack(

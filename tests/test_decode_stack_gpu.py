@@ -266,3 +266,13 @@ def test_a_launch_waits_for_compute_units_that_come_free_soon(rows):
         members.append(stack.blocks_of_last())
         assert torch.equal(here, out)
     assert min(members) >= stack.blocks // 2, members
+
+
+@pytest.mark.gpu
+def test_rows_that_do_not_match_their_tables_are_refused():
+    stack, given, _, _ = _stack(np.random.default_rng(2), 1, 64, 64, [3, 4], 64, B, "gelu_new", None)
+    hidden, request, positions, slots, tables = given
+    for wrong in ((hidden[:1], request, positions, slots, tables), (hidden, request[:1], positions, slots, tables), (hidden, request, positions[:1], slots, tables),
+                  (hidden, request, positions, slots[:1], tables), (hidden, request, positions, slots, tables[:1])):
+        with pytest.raises(ValueError):
+            stack.run(*wrong)
