@@ -782,8 +782,8 @@ MLLM_API int mllm_decode_stack_supported(int rows, int n_layers, int width, int 
     return stack_steps(rows, width, inner, n_heads, dtype == MLLM_BF16 ? 2 : 4) > 0;
 }
 
-// Whether a step of so many rows, none of whose sequences is longer than `reach`, is faster as one kernel than layer by layer. Measured on whole steps of
-// random GPT-2 models (layer by layer / one kernel, us; 24 layers at 1,024 columns, 12 else):
+// Whether a step of so many rows, none of whose sequences is longer than `reach`, is faster as one kernel than layer by layer, of models with many layers and hidden units four times
+// the columns. Measured on whole steps of random GPT-2 models (layer by layer / one kernel, us; 24 layers at 1,024 columns in bfloat16, 12 else):
 //   bfloat16,   768 columns: 1 row 297 / 168 at 500 keys, 327 / 185 at 1,000, 363 / 340 at 1,900; 8 rows 328 / 208, 398 / 281, 476 / 416; 16 rows 365 / 289, 429 / 430, 551 / 696
 //   bfloat16, 1,024 columns: 1 row 752 / 359, 810 / 517, 816 / 766; 8 rows 761 / 447, 872 / 547, 989 / 823; 16 rows 843 / 614, 1,018 / 916, 1,260 / 1,432
 //   bfloat16, 1,600 columns: 1 row 492 / 279, 520 / 289, 528 / 419; 2 rows 486 / 296, 515 / 309, 587 / 442; 4 rows 487 / 436, 521 / 455, 595 / 595; 8 rows 516 / 507, 580 / 652
@@ -793,6 +793,22 @@ MLLM_API int mllm_decode_stack_supported(int rows, int n_layers, int width, int 
 MLLM_API int mllm_decode_stack_pays(int rows, int reach, int width) {
     if (width <= 1024) return rows <= 8 ? reach <= 1792 : rows <= 16 && reach <= 1024;
     return rows <= 2 ? reach <= 1792 : rows <= 4 && reach <= 1024;
+}
+
+// The same for any model. Measured as above with 1, 2, 4 and 12 layers of 64 to 1,792 columns and inner / columns of 1.9 to 16, at 60, 1,000 and 1,780 keys, 1 to 16 rows; where nothing
+// else is said at least as fast as one kernel (us, layer by layer / one kernel):
+//   one layer: 768 columns 38 / 33 (1 row, 60 keys), 44 / 46 (8 rows, 1,000), 48 / 58 (16 rows, 1,000), 40 / 43 (1 row, 1,780): its start costs what a layer gains. Two: 62 / 44, 71 / 62, 71 / 70
+//   more than 8 rows: few layers (16 rows, 1,000 keys in bfloat16: 128 columns, 2 layers 55 / 62, 4 layers 99 / 102, 12 of 64 columns 258 / 240; 768 columns, 2 layers 79 / 86, 4 142 / 153, 12
+//     429 / 430) and many hidden units (60 keys: 512 columns and 7,168 units 372 / 454, 1,024 and 5,632 404 / 520; in 32-bit 256 and 4,096 345 / 387). What is
+//     left is behind at the last of its keys alone (640 columns 289 / 247 at 60 keys, 404 / 425 at 1,000)
+//   more than 2 rows of more than 1,024 columns: 1,600, 4 rows of 60 and of 1,000 keys, 2 layers 87 / 90 and 94 / 96, 4 layers 154 / 153 and 185 / 171
+//   32-bit beyond 1,024 keys (1,780): few layers (1,024 columns, 1 row, 2 layers 89 / 93, 4 174 / 184, 12 518 / 512), few columns (192, 8 rows 416 / 447; 384, 4 rows 426 / 451; 512, 2 rows
+//     430 / 435; 640, 2 rows 488 / 452) and many hidden units (512 and 4,096, 1 row 443 / 485; 768 and 4,096 502 / 503)
+MLLM_API int mllm_decode_stack_pays_for(int rows, int reach, int n_layers, int width, int inner, int dtype) {
+    if (!mllm_decode_stack_pays(rows, reach, width) || n_layers < 2) return 0;
+    if (rows > 8 && (n_layers < 8 || inner > 4 * width)) return 0;
+    if (rows > 2 && width > 1024 && n_layers < 4) return 0;
+    return dtype != MLLM_F32 || reach <= 1024 || (n_layers >= 8 && width >= 640 && inner <= 4 * width);
 }
 
 MLLM_API long long mllm_decode_stack_word_bytes(int rows, int width, int inner, int dtype) {

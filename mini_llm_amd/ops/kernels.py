@@ -975,7 +975,7 @@ def decode_stack_pays(rows, reach, n_layers, width, inner, n_heads, head_size, p
     """Whether a step of so many rows, of sequences up to ``reach`` tokens, is faster as one kernel than layer by layer (the library's own answer, where
     the measurements behind it are written down)."""
     return (decode_stack_supported(rows, n_layers, width, inner, n_heads, head_size, page_size, dtype)
-            and bool(library().mllm_decode_stack_pays(int(rows), int(reach), int(width))))
+            and bool(library().mllm_decode_stack_pays_for(int(rows), int(reach), int(n_layers), int(width), int(inner), _code(dtype))))
 
 
 class DecodeStack:

@@ -53,6 +53,7 @@ _SIGNATURES = {
     "mllm_decode_mlp_half": [P, P, P, c_int, P, P, P, c_float, P, P, P, P, c_int, c_int, c_int, c_int, c_int, P],
     "mllm_decode_stack_supported": [c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int],
     "mllm_decode_stack_pays": [c_int, c_int, c_int],
+    "mllm_decode_stack_pays_for": [c_int, c_int, c_int, c_int, c_int, c_int],
     "mllm_decode_stack_word_bytes": [c_int, c_int, c_int, c_int],
     "mllm_decode_stack_control_ints": [],
     "mllm_decode_stack_patience_at": [],

@@ -20,6 +20,21 @@ def test_where_one_kernel_for_all_layers_pays(rows, reach, width, pays):
     assert bool(library().mllm_decode_stack_pays(rows, reach, width)) == pays
 
 
+@pytest.mark.parametrize("rows,reach,layers,width,inner,dtype,pays", [
+    (8, 1792, 12, 768, 3072, torch.bfloat16, True), (16, 1024, 12, 768, 3072, torch.bfloat16, True), (8, 1793, 12, 768, 3072, torch.bfloat16, False),
+    (1, 64, 1, 768, 3072, torch.bfloat16, False), (1, 64, 2, 768, 3072, torch.bfloat16, True), (1, 64, 1, 768, 3072, torch.float32, False),          # one layer
+    (16, 64, 7, 768, 3072, torch.bfloat16, False), (16, 64, 8, 768, 3072, torch.bfloat16, True), (8, 64, 2, 768, 3072, torch.bfloat16, True),       # more than 8 rows: few layers,
+    (16, 64, 12, 768, 3104, torch.bfloat16, False), (8, 64, 12, 768, 3104, torch.bfloat16, True), (16, 64, 12, 1024, 5632, torch.bfloat16, False),   # many hidden units
+    (4, 64, 3, 1600, 6400, torch.bfloat16, False), (4, 64, 4, 1600, 6400, torch.bfloat16, True), (2, 64, 2, 1600, 6400, torch.bfloat16, True),
+    (1, 1025, 7, 768, 3072, torch.float32, False), (1, 1025, 8, 768, 3072, torch.float32, True), (1, 1024, 2, 768, 3072, torch.float32, True),       # 32-bit and many keys
+    (1, 1025, 12, 576, 2304, torch.float32, False), (1, 1025, 12, 640, 2560, torch.float32, True), (1, 1025, 12, 640, 2592, torch.float32, False),
+    (1, 1025, 2, 128, 4096, torch.bfloat16, True)])
+def test_for_which_models_one_kernel_for_all_layers_pays(rows, reach, layers, width, inner, dtype, pays):
+    from mini_llm_amd.ops import kernels as K
+
+    assert K.decode_stack_pays(rows, reach, layers, width, inner, width // 64, 64, 64, dtype) == pays
+
+
 @pytest.mark.parametrize("rows,layers,width,inner,heads,head,page,dtype,supported", [
     (1, 12, 768, 3072, 12, 64, 64, torch.bfloat16, True), (16, 64, 768, 3072, 12, 64, 1, torch.float32, True), (16, 48, 1600, 6400, 25, 64, 64, torch.bfloat16, True),
     (17, 12, 768, 3072, 12, 64, 64, torch.bfloat16, False), (1, 65, 768, 3072, 12, 64, 64, torch.bfloat16, False), (1, 12, 768, 3072, 24, 32, 64, torch.bfloat16, False),
