@@ -934,10 +934,15 @@ void launch_gated(const T* a, const T* w, T* o, int M, int N, int K, hipStream_t
 }  // namespace
 
 // Whether a product over eight gate and eight up rows in turn ([N, K], packed) leaves silu(gate) * up itself: where it takes the kernel for few rows or one of
-// those for many; the tiled kernel that takes what is left has no such end.
+// those for many; the tiled kernel that takes what is left has no such end. Nor has the tile of 256 x 256, and where the plain product would take that one over a long K, what its loop
+// gains is more than what the unit's own kernel costs: in bfloat16, the product and the unit behind it / the unit inside, us: 1,536 rows, 14,336 units of K 4,096 339 / 351, 13,824 of
+// 5,120 408 / 424; 4,096 rows, 4,096 units of 8,192 437 / 465; with a K below as below: 4,096 rows, 8,192 units of 3,072 380 / 378, 9,472 of 3,584 516 / 517, 8,192 rows 1,021 / 995.
 MLLM_API int mllm_gemm_gated_takes(const void* A, const void* out, int M, int N, int K, int w_packed, int dtype) {
     if (M < 1 || N < 16 || N % 16 != 0 || K < 1 || !w_packed || ((size_t)out & 15) != 0) return 0;
-    if (dtype == MLLM_BF16) return takes_few_row_kernel<bf16_t>(M, N, K) || stream::takes(M, N, K, true, CacheScatter{}, 2);
+    if (dtype == MLLM_BF16) {
+        if (takes_few_row_kernel<bf16_t>(M, N, K)) return 1;
+        return stream::takes(M, N, K, true, CacheScatter{}, 2) && !(K >= 4096 && stream::choose(M, N, K, 1, true) == stream::S256x256);
+    }
     if (dtype == MLLM_F32) return takes_few_row_kernel<float>(M, N, K) || pieces::takes(A, nullptr, nullptr, out, M, N, K, ceil_div(N, 16), w_packed, CacheScatter{});
     return 0;
 }
@@ -945,7 +950,7 @@ MLLM_API int mllm_gemm_gated_takes(const void* A, const void* out, int M, int N,
 // out [M, N / 2] = silu(x gate^T) * (x up^T). The unit in the product's own end, where a lane holds a unit's two sums (or LDS does), instead of a kernel behind it that reads 2 * M * N
 // numbers' worth of sums again, each rounded to the element type before the unit (here the sums go into it as they are). Measured, the product and the unit behind it -> this,
 // us in a replayed graph: bfloat16, 2,048 units of 768 columns, 8 rows 6.0 -> 3.5, 64 8.5 -> 6.1, 300 10.7 -> 7.1, 2,048 25.8 -> 16.7; 4,288 of 1,600, 300 19.2 -> 14.7, 2,048
-// 76.5 -> 65.2 (without the tile of 256 x 256, which the product alone takes there). In 32-bit, 2,048 of 768, 8 rows 7.3 -> 4.7, 64 12.8 -> 10.4, 2,048 75.1 -> 66.6.
+// 76.5 -> 65.2 (without the tile of 256 x 256, which the product alone takes there; above). In 32-bit, 2,048 of 768, 8 rows 7.3 -> 4.7, 64 12.8 -> 10.4, 2,048 75.1 -> 66.6.
 MLLM_API int mllm_gemm_gated(const void* A, const void* W, int w_packed, void* out, int M, int N, int K, int dtype, hipStream_t stream) {
     MLLM_REQUIRE(mllm_gemm_gated_takes(A, out, M, N, K, w_packed, dtype), "gemm_gated: no kernel for M=%d N=%d K=%d dtype %d", M, N, K, dtype);
     MLLM_REQUIRE(ceil_div(M, 32) <= 65535, "gemm_gated: M=%d has too many row tiles", M);

@@ -21,6 +21,19 @@ def _exact(x, gate, up):
     return g / (1.0 + np.exp(-g)) * u
 
 
+@pytest.mark.parametrize("rows,inner,width,dtype,inside", [
+    (1536, 14336, 4096, B, False), (4096, 4096, 8192, B, False), (16384, 11008, 4096, B, False),   # the plain product's tile of 256 x 256, over a long K
+    (4096, 9472, 3584, B, True), (2048, 5632, 2048, B, True),                                     # over a shorter one
+    (1024, 5632, 4096, B, True), (2048, 2048, 8192, B, True), (64, 2048, 8192, B, True),          # another tile, the kernel for few rows
+    (1536, 14336, 4096, F, True)])
+def test_where_the_unit_is_inside(rows, inner, width, dtype, inside):
+    from mini_llm_amd.ops import kernels as K
+    from mini_llm_amd.ops.library import library
+
+    code, address, packed = (1, 256, 1) if dtype == B else (0, 256, K.PACKED_WITH_PIECES)
+    assert bool(library().mllm_gemm_gated_takes(address, address, rows, 2 * inner, width, packed, code)) == inside
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("rows,inner,width,inside", [
     (1, 8, 64, True), (1, 2048, 768, True), (8, 2048, 768, True), (16, 40, 96, True), (17, 1000, 64, True), (33, 2048, 768, True), (64, 2760, 320, True),
