@@ -1160,7 +1160,9 @@ def gate_up_rows(gate, up):
 
 def gated_linear(x, weight: PackedMatrix):
     """silu(x gate^T) * (x up^T), [rows, inner] of x's type, from ``weight`` = ``gate_up_rows`` packed: the unit inside the product where one of
-    its kernels takes the sizes, else (rounded to x's type in between) in a kernel of its own."""
+    its kernels takes the sizes, else (rounded to x's type in between; x as PackedRows too) in a kernel of its own."""
+    if isinstance(x, PackedRows):
+        return silu_mul(linear(x, weight), turn=GATE_TURN)
     _device_tensor(x, "x", dim=2)
     w_ptr, w_packed, n, k = _matrix(weight, "weight", x.dtype)
     _require(w_packed and n % (2 * GATE_TURN) == 0 and x.shape[1] == k, "x and the packed gate and up rows do not match")

@@ -87,3 +87,18 @@ def test_silu_mul_of_columns_in_turn(dtype, inner, turn):
     want = (torch.nn.functional.silu(parts[:, :, 0]) * parts[:, :, 1]).reshape(5, inner)
     got = K.silu_mul(both.to(DEV), turn=turn).cpu().double()
     torch.testing.assert_close(got, want, rtol=2.0 ** -8 if dtype == B else 1e-6, atol=1e-6)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [B, F])
+def test_rows_in_the_packed_layout(dtype):
+    from mini_llm_amd.ops import kernels as K
+
+    _, gate, up = _sides(np.random.default_rng(9), 1, 200, 96, dtype)
+    weight = K.pack_matrix(K.gate_up_rows(gate, up).contiguous().to(DEV))
+    stream, gain, offset = (torch.randn(shape, generator=torch.Generator().manual_seed(i)).to(DEV) for i, shape in enumerate(((20, 96), (96,), (96,))))
+    plain, packed = (K.layernorm(stream, gain, offset, 1e-5, out_dtype=dtype, packed_out=packed) for packed in (False, True))
+    assert isinstance(packed, K.PackedRows)
+    out = K.gated_linear(packed, weight).float().cpu().numpy()
+    tolerance = dict(rtol=2e-5, atol=2e-5) if dtype == F else dict(rtol=2.0 ** -6, atol=2e-2)   # (as above, the unit in a kernel of its own)
+    np.testing.assert_allclose(out, _exact(plain.cpu(), gate, up), **tolerance)
