@@ -975,6 +975,11 @@ namespace {
 // it eight or sixteen, or several blocks. Two launches / one, us, 16 heads, the prompt of 512 new tokens or 400 on 1,500: bfloat16, one row of 1,900 keys 18.3 / 15.3 and
 // 24.2 / 16.9, eight 25.0 / 17.9 and 32.6 / 25.0; one of 3,500 19.5 / 23.6 and 26.2 / 24.4, of 7,500 24.4 / 45.4; in 32-bit one of 1,900 27.2 / 22.7, of 3,500 29.6 / 37.8.
 constexpr int MIXED_REACH = 2048;
+// The most blocks of decoding rows, a row and head each, that one launch takes: they come first, four waves each where a launch of their own has as many waves on a compute unit as it
+// holds, and a prompt's blocks wait for them. Two launches / one, us, rows of 60 keys beside 400 new tokens on 1,500: bfloat16, 8 heads, 112 rows 20.9 / 20.7, 128 21.2 / 22.9, 160 21.1 /
+// 23.8; 16 heads, 64 rows 21.5 / 23.8; 40 heads, 48 rows 37.4 / 40.9; 64 heads, 64 rows 45.9 / 56.0, beside 80 tokens 20.8 / 32.0; in 32-bit, 12 heads, 80 rows 46.9 / 59.1. (With 300
+// keys a row one launch is ahead there too, 34.6 / 33.6 at 16 heads, 64 rows; a captured step does not know how many its rows will have.)
+constexpr int MIXED_SHORT_BLOCKS = 896;
 
 template <typename T, int HD, int QUERIES>
 __global__ __launch_bounds__(256, 2) void attention_mixed_kernel(
@@ -1021,9 +1026,9 @@ void launch_mixed(const void* q, int q_stride, const void* k_pages, const void* 
 }  // namespace
 
 // Whether a step of both kinds takes one launch: heads of 64 without a mask of their own, pages and portions as the prompts' kernels for such rows take them.
-MLLM_API int mllm_attention_mixed_takes(const void* q, int q_stride, const void* out, int out_stride, int head_size, int page_size, int max_q_len, int reach, float scale, int dtype) {
+MLLM_API int mllm_attention_mixed_takes(const void* q, int q_stride, const void* out, int out_stride, int short_rows, int n_heads, int head_size, int page_size, int max_q_len, int reach, float scale, int dtype) {
     if (head_size != 64 || (dtype != MLLM_F32 && dtype != MLLM_BF16) || !mllm_attention_decode_supported(head_size, page_size, dtype)) return 0;
-    if (reach < 1 || reach > MIXED_REACH) return 0;
+    if (reach < 1 || reach > MIXED_REACH || (long long)short_rows * n_heads > MIXED_SHORT_BLOCKS) return 0;
     return dtype == MLLM_BF16 ? prefill_stream::takes<bf16_t>(head_size, page_size, max_q_len, scale, q_stride, out_stride, q, out)
                               : prefill_stream::takes<float>(head_size, page_size, max_q_len, scale, q_stride, out_stride, q, out);
 }
@@ -1034,9 +1039,9 @@ MLLM_API int mllm_attention_mixed(const void* q, int q_stride, const void* k_pag
                                   int max_q_len, int reach, int n_heads, int n_kv_heads, int head_size, int page_size, float scale, int dtype, hipStream_t stream) {
     MLLM_REQUIRE(n_heads > 0 && n_kv_heads > 0 && max_blocks > 0 && n_heads % n_kv_heads == 0, "attention_mixed: bad sizes");
     MLLM_REQUIRE(short_rows > 0 && short_rows < rows && short_requests > 0 && short_requests < n_requests, "attention_mixed: no step of both kinds");
-    MLLM_REQUIRE(n_requests <= 65535 && n_heads <= 65535 && short_rows <= 65535, "attention_mixed: too many rows, requests or heads for one launch");
+    MLLM_REQUIRE(n_requests - short_requests <= 65535 && n_heads <= 65535, "attention_mixed: too many requests or heads for one launch");   // (as for the prompts alone)
     MLLM_REQUIRE(q_stride >= n_heads * head_size && out_stride >= n_heads * head_size, "attention_mixed: rows are too short for the heads");
-    MLLM_REQUIRE(mllm_attention_mixed_takes(q, q_stride, out, out_stride, head_size, page_size, max_q_len, reach, scale, dtype), "attention_mixed: no kernel for these rows");
+    MLLM_REQUIRE(mllm_attention_mixed_takes(q, q_stride, out, out_stride, short_rows, n_heads, head_size, page_size, max_q_len, reach, scale, dtype), "attention_mixed: no kernel for these rows");
     int page_shift = 0;
     while ((1 << page_shift) < page_size) page_shift++;
 #define MLLM_MIXED(T, QUERIES)                                                                                                                                             \

@@ -533,7 +533,7 @@ def paged_attention(q, k_pages, v_pages, token_request, positions, block_tables,
         _require(0 < short_requests < context_lens.shape[0], "short_requests does not cut the batch in two")
         reach = block_tables.shape[1] * page_size if max_len is None else max(1, min(max_len, block_tables.shape[1] * page_size))
         if (not (window or chunk or softcap or wide_out) and sinks is None and q_starts.shape[0] == context_lens.shape[0] + 1 and block_tables.shape[0] >= context_lens.shape[0]
-                and lib.mllm_attention_mixed_takes(_ptr(q), q.stride(0), _ptr(out), out.stride(0), head_size, page_size, int(max_q_len), reach, float(scale), _code(q.dtype))):
+                and lib.mllm_attention_mixed_takes(_ptr(q), q.stride(0), _ptr(out), out.stride(0), int(short_rows), n_heads, head_size, page_size, int(max_q_len), reach, float(scale), _code(q.dtype))):
             _device_tensor(q_starts, "q_starts", torch.int32, 1)
             _device_tensor(context_lens, "context_lens", torch.int32, 1)
             check(lib.mllm_attention_mixed(_ptr(q), q.stride(0), _ptr(k_pages), _ptr(v_pages), _ptr(out), out.stride(0), _ptr(token_request), _ptr(positions), _ptr(q_starts),

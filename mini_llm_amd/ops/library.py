@@ -38,7 +38,7 @@ _SIGNATURES = {
     "mllm_attention": [P, c_int, P, P, P, c_int, P, P, P, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_float, c_int, c_float, P, c_int, c_int, c_int, P],
     "mllm_attention_decode": [P, c_int, P, P, P, c_int, P, P, P, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_float, c_int, c_int, c_int, c_int, P, P, c_float, P, c_int, c_int, c_int, P],
     "mllm_attention_decode_supported": [c_int, c_int, c_int],
-    "mllm_attention_mixed_takes": [P, c_int, P, c_int, c_int, c_int, c_int, c_int, c_float, c_int],
+    "mllm_attention_mixed_takes": [P, c_int, P, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_float, c_int],
     "mllm_attention_mixed": [P, c_int, P, P, P, c_int, P, P, P, P, P, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_float, c_int, P],
     "mllm_attention_prefill": [P, c_int, P, P, P, c_int, P, P, P, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_float, c_int, c_float, P, c_int, c_int, c_int, P],
     "mllm_attention_prefill_supported": [c_int, c_int],

@@ -9,6 +9,17 @@ DEV = "cuda:0"
 B, F = torch.bfloat16, torch.float32
 
 
+@pytest.mark.parametrize("short_rows,heads,reach,longest,takes", [
+    (112, 8, 2048, 65, True), (113, 8, 2048, 65, False), (896, 1, 64, 512, True), (32, 28, 2048, 512, True), (64, 16, 2048, 512, False), (65535, 65535, 64, 512, False),
+    (16, 16, 2049, 512, False), (16, 16, 2048, 64, False)])
+@pytest.mark.parametrize("dtype", [B, F])
+def test_where_both_kinds_take_one_launch(dtype, short_rows, heads, reach, longest, takes):
+    from mini_llm_amd.ops.library import library
+
+    stride = min(heads, 1024) * 64
+    assert bool(library().mllm_attention_mixed_takes(256, stride, 256, stride, short_rows, heads, 64, 64, longest, reach, 0.125, 1 if dtype == B else 0)) == takes
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [B, F])
 @pytest.mark.parametrize("heads,kv_heads,page_size,max_blocks,stored,portions,one_launch", [
