@@ -223,6 +223,15 @@ struct Tile {
 // Elements from one normed row in LDS to the next: whole rounds of the 64 banks and a quarter round, so that four rows' pieces of a step (64 bytes each) share no bank.
 __host__ __device__ __forceinline__ int normed_stride(int width, int element) { return ((width * element + 255) / 256 * 256 + 64) / element; }
 
+// Sums that a wave's steps of K take in turn, of the products that the rows' blocks and that the norming blocks do. In 32-bit a product's error is that of its sums' roundings in a row: the
+// relative error of a step's logits against 64 bits, three layers, with one sum each / two and one / four and two / layer by layer, in 1e-7: 768 columns, 8 rows 5.7 / 5.0 / 4.2 / 5.1,
+// 1,024 columns, 2 rows 6.6 / 5.6 / 4.7 / 5.0, 16 rows 6.3 / 5.4 / 4.6 / 5.1. (A step of 12 layers, 8 rows: 768 columns 318 / 312 / 313 us, products of one sum wait for each other; 1,024
+// 405 / 403 / 400, of fewer loads at a time.) In bfloat16 the operands' own rounding is all there is to see.
+template <typename T>
+constexpr int SUMS_OVER_UNITS = sizeof(T) == 4 ? 4 : 1;
+template <typename T>
+constexpr int SUMS_OVER_WIDTH = sizeof(T) == 4 ? 2 : 1;
+
 constexpr int PART_STRIDE = 20;   // floats a row of a tile's partial sums: 16, and 4 that spread the rows over the LDS banks
 typedef float PartRows[ST_WAVES][ST_MAX_ROWS][PART_STRIDE];
 
@@ -483,10 +492,14 @@ __global__ __launch_bounds__(ST_THREADS) void decode_stack_kernel(StackArgs a) {
         // (what the rows beyond hold meanwhile goes into sums that nobody takes).
         constexpr int FOLD = ST_MAX_ROWS / ROWS;
         auto operand_sum = [&](const auto& w, const Words& from, const Operands& lie, int n_steps, uint32_t tag) {
-            constexpr int ALL = (int)(sizeof(w.w) / sizeof(Vec16)), LOADS = (ALL + FOLD - 1) / FOLD, CHUNK = LOADS <= 12 ? LOADS : LOADS % 8 == 0 ? 8 : 7;
+            constexpr int ALL = (int)(sizeof(w.w) / sizeof(Vec16)), LOADS = (ALL + FOLD - 1) / FOLD;
+            constexpr int CHUNK = LOADS <= 12 ? LOADS : LOADS == 16 && sizeof(T) == 4 ? 4 : LOADS % 8 == 0 ? 8 : 7;   // (1,024 columns, 8 rows in 32-bit: eight at a time spill 39 registers, 424 us a step for 399)
             static_assert(LOADS % CHUNK == 0, "whole chunks");
             const int folded = row16 / ROWS, folded_row = min(row16 % ROWS, M - 1);
-            f32x4 sum = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+            constexpr int SUMS = SUMS_OVER_UNITS<T>;
+            f32x4 sum[SUMS];
+#pragma unroll
+            for (int i = 0; i < SUMS; i++) sum[i] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
             auto turned = [&](auto amount, u32x4 a, u32x4 b) {
                 constexpr int N = decltype(amount)::value;
                 Vec16 x{{a[0], a[2], b[0], b[2]}};
@@ -518,7 +531,10 @@ __global__ __launch_bounds__(ST_THREADS) void decode_stack_kernel(StackArgs a) {
                     auto step = [&](auto fold) {
                         constexpr int F = decltype(fold)::value;
                         if constexpr (F < FOLD) {
-                            if ((c + j) * FOLD + F < ALL) sum = multiply<T>(w.w[(c + j) * FOLD + F < ALL ? (c + j) * FOLD + F : 0], turned(std::integral_constant<int, F * ROWS % 16>{}, got[2 * j], got[2 * j + 1]), sum);
+                            if ((c + j) * FOLD + F < ALL) {
+                                f32x4& into = sum[((c + j) * FOLD + F) % SUMS];
+                                into = multiply<T>(w.w[(c + j) * FOLD + F < ALL ? (c + j) * FOLD + F : 0], turned(std::integral_constant<int, F * ROWS % 16>{}, got[2 * j], got[2 * j + 1]), into);
+                            }
                         }
                     };
                     step(std::integral_constant<int, 0>{}), step(std::integral_constant<int, 1>{}), step(std::integral_constant<int, 2>{}), step(std::integral_constant<int, 3>{});
@@ -527,7 +543,11 @@ __global__ __launch_bounds__(ST_THREADS) void decode_stack_kernel(StackArgs a) {
                     step(std::integral_constant<int, 12>{}), step(std::integral_constant<int, 13>{}), step(std::integral_constant<int, 14>{}), step(std::integral_constant<int, 15>{});
                 }
             }
-            return sum;
+#pragma unroll
+            for (int apart = 1; apart < SUMS; apart *= 2)
+#pragma unroll
+                for (int i = 0; i + apart < SUMS; i += 2 * apart) sum[i] += sum[i + apart];
+            return sum[0];
         };
         const int sum_row = tid / 8, sum_column = tid % 8 * 2;   // two columns of a row to a thread: the stream goes on in 32-bit
         const bool sums = sum_row < M;
@@ -691,20 +711,27 @@ __global__ __launch_bounds__(ST_THREADS) void decode_stack_kernel(StackArgs a) {
                 }
                 PartRows* part = parts + turn * TILES;
                 turn ^= 1;
-                f32x4 sum[TILES];
+                constexpr int SUMS = SUMS_OVER_WIDTH<T>;
+                f32x4 sum[TILES][SUMS];
 #pragma unroll
-                for (int t = 0; t < TILES; t++) sum[t] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+                for (int t = 0; t < TILES; t++)
+#pragma unroll
+                    for (int i = 0; i < SUMS; i++) sum[t][i] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
                 for (int j = 0; j < STEPS; j++) {
                     const int step = min(wave + ST_WAVES * j, width_steps - 1);
                     const Vec16 x = *reinterpret_cast<const Vec16*>(normed + own_row * stride + step * KC + quad * VEC);
 #pragma unroll
                     for (int t = 0; t < TILES; t++)
-                        if (t == 0 || first + t * norming < tiles) sum[t] = multiply<T>(w[t].w[j], x, sum[t]);
+                        if (t == 0 || first + t * norming < tiles) sum[t][j % SUMS] = multiply<T>(w[t].w[j], x, sum[t][j % SUMS]);
                 }
 #pragma unroll
                 for (int t = 0; t < TILES; t++)
-                    if (t == 0 || first + t * norming < tiles) leave_part(part[t], sum[t]);
+                    if (t == 0 || first + t * norming < tiles) {
+#pragma unroll
+                        for (int i = 1; i < SUMS; i++) sum[t][0] += sum[t][i];
+                        leave_part(part[t], sum[t][0]);
+                    }
                 lds_barrier();
                 const int tile = first + sum_tile * norming;
                 if (sum_tile < TILES && tile < tiles && sum_row < M) finish(tile, whole_sum(part[sum_tile], sum_row, sum_column, Own{}) + add);

@@ -291,3 +291,39 @@ def test_rows_that_do_not_match_their_tables_are_refused():
                   (hidden, request, positions, slots[:1], tables), (hidden, request, positions, slots, tables[:1])):
         with pytest.raises(ValueError):
             stack.run(*wrong)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("width,rows", [(768, 8), (1024, 2), (1024, 16), (512, 4), (192, 16)])
+def test_32_bit_sums_are_no_further_off_than_layer_by_layer(tmp_path, monkeypatch, width, rows):
+    # The relative error (2-norm) of a decode step's logits against 64 bits, over all rows of a few models: one kernel's sums run over as many products as the
+    # separate kernels', in an order of their own, so that neither should be the further off.
+    from mini_llm_amd.config import config_from_dict
+    from mini_llm_amd.engine import StepEntry
+    from mini_llm_amd.engine.engine import Engine, EngineOptions
+    from mini_llm_amd.ops import kernels as K
+    from mini_llm_amd.weights import write_model_dir
+
+    raw = {"architectures": ["GPT2LMHeadModel"], "n_layer": 3, "n_embd": width, "n_head": width // 64, "n_inner": 4 * width, "vocab_size": 600, "n_positions": 64,
+           "layer_norm_epsilon": 1e-5, "activation_function": "gelu_new"}
+    errors = {True: [], False: []}
+    for seed in range(3):
+        folder = tmp_path / str(seed)
+        write_model_dir(config_from_dict(raw), seed, folder)
+        config, weights = P.load_model_dir(folder)
+        rng = np.random.default_rng(seed)
+        sequences = [rng.integers(0, 600, 24).tolist() for _ in range(rows)]
+        want = np.stack([P.forward(config, weights, tokens)[-1] for tokens in sequences]).astype(np.float64)
+        for one_kernel in (True, False):
+            with monkeypatch.context() as patch:
+                patch.setattr(K, "decode_stack_pays", lambda *sizes: one_kernel)
+                engine = Engine(folder, EngineOptions(dtype="float32", max_sessions=rows))
+                handles = [engine.try_take_cache() for _ in sequences]
+                engine.runner.step([StepEntry(h, tokens[:-1], []) for h, tokens in zip(handles, sequences)])
+                before = K.launch_counts()
+                got = engine.runner.step([StepEntry(h, tokens[-1:], [0]) for h, tokens in zip(handles, sequences)]).double().cpu().numpy()
+                assert ("decode_stack" in K.launches_since(before)) == one_kernel
+                engine.close()
+            errors[one_kernel].append(np.linalg.norm(got - want) / np.linalg.norm(want))
+    assert np.mean(errors[True]) <= np.mean(errors[False]), errors
+    assert np.mean(errors[True]) > 0.0
