@@ -248,7 +248,7 @@ constexpr int DECODE_MAX_SPLITS = 16;
 // launch); the block that is through last puts the runs together, out = sum_p o_p e^(m_p - M) / sum_p l_p e^(m_p - M),
 // and the count is zero again behind it (it wraps), so the same counters serve the next launch.
 // The work of a block: part `part` of `n_parts` of one (token, head), by the block's n_splits waves.
-template <typename T, int HD, bool TOGETHER, bool KEPT = false>
+template <typename T, int HD, bool TOGETHER, bool KEPT = false, bool ROUNDS_APART = false>
 __device__ __forceinline__ void decode_block(
     int head, int token, int part, int n_parts, int n_splits, const T* __restrict__ q, int q_stride, const T* __restrict__ k_pages,
     const T* __restrict__ v_pages, T* __restrict__ out, int out_stride,
@@ -298,7 +298,8 @@ __device__ __forceinline__ void decode_block(
     const int kv_head = head / (n_heads / n_kv_heads);
     const int* table = block_tables + (size_t)request * max_blocks;
 
-    KeySweep<T, HD, KEPT> sweep;
+    typedef KeySweep<T, HD, KEPT, ROUNDS_APART> Sweep;
+    Sweep sweep;
     sweep.init();
     sweep.cap = options.softcap;
     if constexpr (KEPT) sweep.gap_from = kept, sweep.gap = gap;
@@ -322,7 +323,7 @@ __device__ __forceinline__ void decode_block(
         const typename Chunk<T>::Raw raw = *reinterpret_cast<const typename Chunk<T>::Raw*>(q + (size_t)token * q_stride + head * HD + sub * VEC);
         int page[UNROLL];
         sweep.look_up(page, table, page_shift, begin, end, spare_key, lane);
-        typename KeySweep<T, HD, KEPT>::Fetched f;
+        typename Sweep::Fetched f;
         sweep.fetch_rows(f, page, k_pages, v_pages, kv_head, n_kv_heads, page_shift, begin, end, spare_key, lane);
         float qf[VEC];
 #pragma unroll
@@ -968,6 +969,8 @@ MLLM_API int mllm_attention_prefill(const void* q, int q_stride, const void* k_p
 // Measured in replayed graphs, two launches -> one, us: bfloat16, 16 heads, 10 rows of 700 keys (6 padding rows) beside a prompt of 480 19.0 -> 11.0, beside 250
 // on 512 20.2 -> 13.0, 24 rows of 500 beside 480 21.9 -> 14.8, of 900 31.5 -> 22.1; 25 heads, 48 rows of 500 beside 480 42.6 -> 34.1; one row beside 80 tokens
 // 11.8 -> 5.9. In 32-bit, 12 heads, 10 rows of 700 beside 480 29.4 -> 17.8. What is left is the longer of the two parts.
+// Four waves have more keys each than the waves of a launch for decoding rows alone: in 32-bit they add up each round of keys by itself, and their error against 64 bits is no larger
+// (a launch alone / four waves with one sum / with rounds apart, in 1e-7: 8 rows of 100 keys 1.4 / 1.4 / 1.4, of 700 1.6 / 1.8 / 1.5, 16 rows of 2,000 2.0 / 2.6 / 1.8).
 // ------------------------------------------------------------------------------------------------
 namespace {
 
@@ -992,7 +995,7 @@ __global__ __launch_bounds__(256, 2) void attention_mixed_kernel(
     if (block < short_blocks) {
         const int token = block / n_heads;
         if (token >= short_rows) return;   // (short_blocks: a multiple of eight, so that a head of the prompts keeps to its XCD)
-        decode_block<T, HD, true>(block % n_heads, token, 0, 1, 4, q, q_stride, k_pages, v_pages, out, out_stride, token_request, positions, block_tables, max_blocks,
+        decode_block<T, HD, true, false, sizeof(T) == 4>(block % n_heads, token, 0, 1, 4, q, q_stride, k_pages, v_pages, out, out_stride, token_request, positions, block_tables, max_blocks,
                                   n_heads, n_kv_heads, page_shift, 0, scale, 0, nullptr, nullptr, plain);
         return;
     }

@@ -35,7 +35,9 @@ __device__ __forceinline__ float sweep_exp(float x) {
 }
 
 // GAPS: keys are numbered without a stretch the request does not look at: number n from `gap_from` on is key n + gap.
-template <typename T, int HD, bool GAPS = false>
+// ROUNDS_APART: the keys of a round are added up by themselves, in pairs, before they join the sums: a rounding in a row for a round instead of one for each of its
+// loads, for a wave that has many 32-bit keys.
+template <typename T, int HD, bool GAPS = false, bool ROUNDS_APART = false>
 struct KeySweep {
     static constexpr int VEC = Chunk<T>::VEC;
     static constexpr int LPR = HD / VEC;      // lanes that share a row
@@ -171,6 +173,27 @@ struct KeySweep {
         running_sum *= rescale;
 #pragma unroll
         for (int i = 0; i < VEC; i++) o[i] *= rescale;
+        if constexpr (ROUNDS_APART) {
+            float p[UNROLL], term[UNROLL];
+            auto in_pairs = [&]() {
+#pragma unroll
+                for (int apart = 1; apart < UNROLL; apart *= 2)
+#pragma unroll
+                    for (int u = 0; u < UNROLL; u += 2 * apart) term[u] += term[u + apart];
+                return term[0];
+            };
+#pragma unroll
+            for (int u = 0; u < UNROLL; u++) term[u] = p[u] = base + u * RPI + group < end ? sweep_exp<T>(score[u] - reference) : 0.0f;
+            running_sum += in_pairs();
+#pragma unroll
+            for (int i = 0; i < VEC; i++) {
+#pragma unroll
+                for (int u = 0; u < UNROLL; u++) term[u] = CLEAN_VALUES && base + u * RPI + group >= end ? 0.0f : p[u] * Chunk<T>::get(f.vf[u], i);
+                o[i] += in_pairs();
+            }
+            running_max = new_max;
+            return;
+        }
 #pragma unroll
         for (int u = 0; u < UNROLL; u++) {
             const bool counts = base + u * RPI + group < end;

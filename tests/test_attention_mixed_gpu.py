@@ -20,6 +20,26 @@ def test_where_both_kinds_take_one_launch(dtype, short_rows, heads, reach, longe
     assert bool(library().mllm_attention_mixed_takes(256, stride, 256, stride, short_rows, heads, 64, 64, longest, reach, 0.125, 1 if dtype == B else 0)) == takes
 
 
+def _step(seed, dtype, heads, kv_heads, page_size, max_blocks, stored, portions):
+    """Queries, pages and tables of a step: rows that decode over ``stored`` keys each (-1: a padding row), then prompt portions (keys stored, new tokens)."""
+    rng = torch.Generator(device=DEV).manual_seed(seed)
+    contexts, news = stored + [c for c, _ in portions], [1] * len(stored) + [n for _, n in portions]
+    needs = [-(-(c + n) // page_size) if c >= 0 else 0 for c, n in zip(contexts, news)]
+    pages = torch.randperm(sum(needs) + 1, generator=torch.Generator().manual_seed(1)).tolist()
+    tables = np.full((len(contexts), max_blocks), -1, dtype=np.int32)
+    for r, need in enumerate(needs):
+        tables[r, :need] = [pages.pop() for _ in range(need)]
+    rand = lambda *shape: torch.randn(shape, generator=rng, device=DEV).to(dtype)
+    k_pages, v_pages = (rand(sum(needs) + 1, kv_heads, page_size, 64) for _ in range(2))
+    q = rand(sum(news), heads * 64)
+    request = np.concatenate([np.full(n, r if c >= 0 else -1) for r, (c, n) in enumerate(zip(contexts, news))])
+    position = np.concatenate([max(c, 0) + np.arange(n) for c, n in zip(contexts, news)])
+    ints = lambda a: torch.as_tensor(np.asarray(a, dtype=np.int32), device=DEV)
+    request, position, starts, lens, tables = ints(request), ints(position), ints(np.cumsum([0] + news)), ints(contexts), ints(tables)
+    shared = dict(n_heads=heads, n_kv_heads=kv_heads, head_size=64, scale=0.125)
+    return q, (k_pages, v_pages), (request, position, tables), (starts, lens), news, shared
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [B, F])
 @pytest.mark.parametrize("heads,kv_heads,page_size,max_blocks,stored,portions,one_launch", [
@@ -34,22 +54,8 @@ def test_where_both_kinds_take_one_launch(dtype, short_rows, heads, reach, longe
 def test_both_kinds_in_one_launch(dtype, heads, kv_heads, page_size, max_blocks, stored, portions, one_launch):
     from mini_llm_amd.ops import kernels as K
 
-    rng = torch.Generator(device=DEV).manual_seed(heads * max_blocks)
-    contexts, news = stored + [c for c, _ in portions], [1] * len(stored) + [n for _, n in portions]
-    needs = [-(-(c + n) // page_size) if c >= 0 else 0 for c, n in zip(contexts, news)]
-    pages = torch.randperm(sum(needs) + 1, generator=torch.Generator().manual_seed(1)).tolist()
-    tables = np.full((len(contexts), max_blocks), -1, dtype=np.int32)
-    for r, need in enumerate(needs):
-        tables[r, :need] = [pages.pop() for _ in range(need)]
-    rand = lambda *shape: torch.randn(shape, generator=rng, device=DEV).to(dtype)
-    k_pages, v_pages = (rand(sum(needs) + 1, kv_heads, page_size, 64) for _ in range(2))
-    q = rand(sum(news), heads * 64)
-    request = np.concatenate([np.full(n, r if c >= 0 else -1) for r, (c, n) in enumerate(zip(contexts, news))])
-    position = np.concatenate([max(c, 0) + np.arange(n) for c, n in zip(contexts, news)])
-    ints = lambda a: torch.as_tensor(np.asarray(a, dtype=np.int32), device=DEV)
-    request, position, starts, lens, tables = ints(request), ints(position), ints(np.cumsum([0] + news)), ints(contexts), ints(tables)
+    q, (k_pages, v_pages), (request, position, tables), (starts, lens), news, shared = _step(heads * max_blocks, dtype, heads, kv_heads, page_size, max_blocks, stored, portions)
     few, longest = len(stored), max(news)
-    shared = dict(n_heads=heads, n_kv_heads=kv_heads, head_size=64, scale=0.125)
     before = K.launch_counts()
     got = K.paged_attention(q, k_pages, v_pages, request, position, tables, max_q_len=longest, q_starts=starts, context_lens=lens, short_rows=few, short_requests=few, **shared)
     assert K.launches_since(before).get("attention_mixed", 0) == int(one_launch)
@@ -60,3 +66,25 @@ def test_both_kinds_in_one_launch(dtype, heads, kv_heads, page_size, max_blocks,
     bound = 2e-5 if dtype == F else 2.0 ** -7
     for here, there in ((got[:few], rows), (got[few:], prompts[few:])):
         torch.testing.assert_close(here.float(), there.float(), rtol=bound, atol=bound)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows,keys", [(8, 700), (16, 2000)])
+def test_32_bit_rows_beside_a_prompt_are_no_further_off_than_alone(rows, keys):
+    # The relative error (2-norm) against 64 bits over a few steps: four waves a row here, sixteen or several blocks in a launch of their own.
+    from mini_llm_amd.ops import kernels as K
+
+    errors = {True: [], False: []}
+    for seed in range(3):
+        q, (k_pages, v_pages), (request, position, tables), (starts, lens), news, shared = _step(seed, F, 12, 12, 64, 32, [keys] * rows, [(0, 480)])
+        want = torch.empty((rows, 12 * 64), dtype=torch.float64, device=DEV)
+        for r in range(rows):
+            pages = tables[r][tables[r] >= 0].long()
+            k, v = (p[pages].double().transpose(0, 1).reshape(12, -1, 64)[:, : keys + 1] for p in (k_pages, v_pages))
+            weights = torch.softmax((q[r].double().view(12, 1, 64) * k).sum(-1) * 0.125, -1)
+            want[r] = (weights[..., None] * v).sum(1).reshape(-1)
+        beside = K.paged_attention(q, k_pages, v_pages, request, position, tables, max_q_len=max(news), q_starts=starts, context_lens=lens, short_rows=rows, short_requests=rows, **shared)
+        alone = K.paged_attention(q[:rows], k_pages, v_pages, request, position, tables, max_q_len=1, **shared)
+        for here, out in ((True, beside[:rows]), (False, alone)):
+            errors[here].append(((out.double() - want).norm() / want.norm()).item())
+    assert np.mean(errors[True]) <= np.mean(errors[False]), errors
