@@ -46,6 +46,86 @@ def test_what_one_kernel_for_all_layers_takes(rows, layers, width, inner, heads,
     assert K.decode_stack_supported(rows, layers, width, inner, heads, head, page, dtype) == supported
 
 
+def _plain_block(width=128, heads=2, kv_heads=None, window=None, inner=256, eps=(1e-5, 1e-5), dtype=torch.bfloat16):
+    """A pre-norm layer as a GPT-2 has it, every matrix packed (their numbers do not matter here)."""
+    from mini_llm_amd.ops import kernels as K
+    from mini_llm_amd.parts.attention import CausalSelfAttention
+    from mini_llm_amd.parts.block import PreNormBlock
+    from mini_llm_amd.parts.feedforward import DenseMLP
+    from mini_llm_amd.parts.norms import LayerNorm
+
+    block = PreNormBlock(LayerNorm(width, eps[0]), CausalSelfAttention(width, heads, kv_heads, window=window), LayerNorm(width, eps[1]), DenseMLP(width, inner, "gelu_new"), dtype)
+    for norm in (block.norm_1, block.norm_2):
+        norm.weight, norm.bias = torch.ones(width), torch.zeros(width)
+    for product in (block.mixer.qkv, block.mixer.out, block.feed_forward.up, block.feed_forward.down):
+        product.weight = K.PackedMatrix(torch.zeros(product.out_features * product.in_features, dtype=dtype), product.out_features, product.in_features)
+        product.bias = torch.zeros(product.out_features)
+    return block
+
+
+def _context(width=128, dtype=torch.bfloat16, write_cache=True, page_size=16):
+    from types import SimpleNamespace
+
+    pages = torch.zeros((3, width // 64, page_size, 64), dtype=dtype)
+    return SimpleNamespace(k_pages=pages, v_pages=pages, write_cache=write_cache)
+
+
+def test_the_layers_that_one_kernel_takes():
+    from mini_llm_amd.ops import kernels as K
+    from mini_llm_amd.parts.feedforward import PlainMLP
+    from mini_llm_amd.parts.norms import LayerNorm, RMSNorm
+
+    layer, shared = _plain_block().stack_layer(_context())
+    assert isinstance(layer, K.StackLayer) and shared == (128, 256, 2, 64, 16, 1e-5, 1e-5, 0.125, "gelu_new")
+
+    def refused(change=lambda block: None, context=None, **how):
+        block = _plain_block(**how)
+        change(block)
+        return block.stack_layer(context or _context()) is None
+
+    row_major = lambda product: setattr(product, "weight", torch.zeros((product.out_features, product.in_features), dtype=torch.bfloat16))
+    assert not refused()
+    assert refused(window=32)
+    assert refused(heads=2, kv_heads=1)
+    assert refused(lambda b: setattr(b, "norm_1", RMSNorm(128, 1e-5))) and refused(lambda b: setattr(b, "norm_2", type("Other", (LayerNorm,), {})(128, 1e-5)))
+    assert refused(lambda b: setattr(b, "feed_forward", PlainMLP(128, 256, "gelu_new")))
+    for product in (lambda b: b.mixer.qkv, lambda b: b.mixer.out, lambda b: b.feed_forward.up, lambda b: b.feed_forward.down):
+        assert refused(lambda b: row_major(product(b)))
+        assert refused(lambda b: setattr(product(b), "bias", None))
+    assert refused(context=_context(dtype=torch.float32))             # pages of another type than the matrices
+    assert refused(context=_context(write_cache=False))               # a layer that reads what another has stored
+    no_pages = _context()
+    no_pages.k_pages = None
+    assert refused(context=no_pages)
+
+
+def test_the_models_and_steps_that_one_kernel_takes(monkeypatch):
+    from types import SimpleNamespace
+
+    from mini_llm_amd.models.base import LayerCall, Model
+    from mini_llm_amd.ops import kernels as K
+    from mini_llm_amd.parts.norms import LayerNorm, RMSNorm
+
+    monkeypatch.setattr(K, "DecodeStack", lambda layers, rows, n_heads, eps_1, eps_2, scale, activation, final: (len(layers), rows, n_heads, eps_1, eps_2, scale, activation, final))
+
+    def made(blocks=None, schedule=None, rows=4, reach=512, wanted=None, groups=1, vectors=None, norm=LayerNorm, page_size=16):
+        blocks = [_plain_block(), _plain_block()] if blocks is None else blocks
+        model = SimpleNamespace(blocks=blocks, schedule=[LayerCall(i, i) for i in range(len(blocks))] if schedule is None else schedule, step_vectors=vectors, final_norm=norm(128, 3e-5))
+        model.final_norm.weight = model.final_norm.bias = torch.ones(128)
+        batch = SimpleNamespace(n_tokens=rows, n_logit_rows=rows if wanted is None else wanted, max_total_len=reach)
+        cache = SimpleNamespace(groups=[None] * groups, layer_context=lambda batch, call: _context(page_size=page_size))
+        return Model.decode_stack(model, batch, cache)
+
+    *sizes, final = made()
+    assert sizes == [2, 4, 2, 1e-5, 1e-5, 0.125, "gelu_new"] and final[2] == 3e-5
+    assert made(norm=RMSNorm)[-1] is None and made(wanted=3)[-1] is None   # the norm in front of the head stays a kernel of its own
+    assert made(blocks=[_plain_block(), _plain_block(eps=(1e-5, 1e-6))]) is None and made(blocks=[_plain_block(), _plain_block(inner=512)]) is None
+    assert made(blocks=[_plain_block(), _plain_block(window=16)]) is None and made(blocks=[]) is None
+    assert made(schedule=[LayerCall(0, 0), LayerCall(0, 1)]) is None      # a block that runs twice
+    assert made(groups=2) is None and made(vectors=object()) is None
+    assert made(reach=1793) is None and made(rows=17) is None and made(blocks=[_plain_block()]) is None and made(page_size=24) is None
+
+
 def _stack(rng, layers, width, inner, contexts, page_size, dtype, activation, blocks):
     """A DecodeStack over random layers and a cache that holds ``contexts`` keys a row (-1: a padding row), what it is run on, and what the layers give in float64."""
     from test_kernels_gpu import as_weight, bf16_round, dev, plain_paged_attention

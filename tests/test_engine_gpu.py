@@ -459,6 +459,50 @@ def test_a_step_takes_the_kernels_it_is_meant_to(tmp_path, dtype):
     engine.close()
 
 
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+def test_a_captured_decode_step_takes_one_kernel_for_all_layers(tmp_path, dtype):
+    # Which kernels a capture holds shows in the launch counts of its two runs (the warm-up's and the recorded one's; replays do not count). Five sequences in
+    # a bucket of eight, so three padding rows, that cross pages of 16 tokens while they are replayed.
+    import plain_gpt2
+    import replay
+    from mini_llm_amd.config import config_from_dict
+    from mini_llm_amd.engine import StepEntry
+    from mini_llm_amd.engine.engine import Engine, EngineOptions
+    from mini_llm_amd.ops import kernels
+    from mini_llm_amd.weights import write_model_dir
+
+    raw = {"architectures": ["GPT2LMHeadModel"], "n_layer": 2, "n_embd": 768, "n_head": 12, "n_inner": 3072, "vocab_size": 9001,
+           "n_positions": 128, "layer_norm_epsilon": 1e-5, "activation_function": "gelu_new"}
+    write_model_dir(config_from_dict(raw), 3, tmp_path)
+    config, weights = plain_gpt2.load_model_dir(tmp_path)
+    bf16 = dtype == "bfloat16"
+    engine = Engine(tmp_path, EngineOptions(dtype=dtype, max_sessions=20, page_size=16))
+    rng = np.random.default_rng(1)
+    sequences = [rng.integers(0, 9001, n).tolist() for n in (20, 30, 17, 21, 36)]
+    handles = [engine.try_take_cache() for _ in sequences]
+    fed = [n - 5 for n in map(len, sequences)]
+    engine.runner.step([StepEntry(h, tokens[:n], []) for h, tokens, n in zip(handles, sequences, fed)])
+    got, whole = [], {"embed": 2, "decode_stack": 2, "gemm_tiled": 2}   # the norm in front of the head in the kernel too
+    for step in range(5):
+        before = kernels.launch_counts()
+        got.append(engine.runner.step([StepEntry(h, [tokens[n + step]], [0]) for h, tokens, n in zip(handles, sequences, fed)]).cpu().numpy())
+        assert kernels.launches_since(before) == (whole if step == 0 else {}), step
+    assert engine.runner.graph_steps == 5
+    stored = [plain_gpt2.forward(config, plain_gpt2.bf16_weights(weights) if bf16 else weights, tokens, stored=plain_gpt2.stored_as_bf16 if bf16 else plain_gpt2._keep)[-5:] for tokens in sequences]
+    np.testing.assert_allclose(np.stack(got, axis=1), np.stack(stored), **replay.tolerance(dtype))
+    # a step that also chooses its tokens; then steps that one kernel does not take: more rows than it has, and few layers for so many
+    before = kernels.launch_counts()
+    engine.runner.step([StepEntry(h, [5], [0]) for h in handles], choose=True).tolist()
+    assert kernels.launches_since(before).get("decode_stack") == 2 and "pending_layernorm" not in kernels.launches_since(before)
+    more = [engine.try_take_cache() for _ in range(12)]
+    engine.runner.step([StepEntry(h, [1, 2, 3], []) for h in more])
+    for rows in (17, 12):
+        before = kernels.launch_counts()
+        engine.runner.step([StepEntry(h, [5], [0]) for h in (more + handles)[:rows]])
+        assert "decode_stack" not in kernels.launches_since(before) and kernels.launches_since(before).get("pending_layernorm"), rows
+    engine.close()
+
+
 @pytest.mark.parametrize("use_graphs", [True, False])
 def test_decoding_changes_kernels_where_the_sequences_grow_long(model_dirs, monkeypatch, use_graphs):
     # Past a length that the mixer names, a decode step runs its attention through the separate kernels instead of the

@@ -116,13 +116,31 @@ def small_shape_dir(real_shape_dirs):
 @pytest.mark.parametrize("shape", ["small", "medium"])
 def test_replay_at_gpt2_small_and_medium_sizes(real_shape_dirs, tmp_path, dtype, shape):
     # mixed: portions beside decoded tokens of up to four requests, then the last tokens one by one
-    # (at small's sizes the bfloat16 decode steps take the layer kernels, at medium's the separate
-    # kernels; the portions take the tiled products and the prompt attention; the head runs over the
-    # whole odd vocabulary)
+    # (the decode steps take one kernel for all layers; the portions take the tiled products and the
+    # prompt attention; the head runs over the whole odd vocabulary)
     folder, config, weights = real_shape_dirs(shape)
     requests = {f"s{i}": random_tokens(200 + i, n, config["vocab_size"]) for i, n in enumerate((40, 70, 130, 23, 65))}
     collector = replay.mixed(requests, seed=1)
     outputs = replay.run_trace(folder, dtype, collector.steps, tmp_path / "out", replay.peak_tokens(collector))
+    ref = replay.plain_logits(config, weights, requests, bf16=(dtype == "bfloat16"))
+    replay.compare(collector.gather(outputs), ref, **replay.tolerance(dtype))
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("shape", ["small", "medium"])
+def test_replay_layer_by_layer_at_gpt2_small_and_medium_sizes(real_shape_dirs, tmp_path, monkeypatch, dtype, shape):
+    # the same with captured decode steps that keep their layers apart, as steps of more rows or longer sequences do: at small's sizes
+    # in bfloat16 the layer kernels, else the separate kernels
+    from mini_llm_amd.ops import kernels
+
+    folder, config, weights = real_shape_dirs(shape)
+    requests = {f"s{i}": random_tokens(200 + i, n, config["vocab_size"]) for i, n in enumerate((40, 70, 130, 23, 65))}
+    collector = replay.mixed(requests, seed=1)
+    monkeypatch.setattr(kernels, "decode_stack_pays", lambda *sizes: False)
+    before = kernels.launch_counts()
+    outputs = replay.run_trace(folder, dtype, collector.steps, tmp_path / "out", replay.peak_tokens(collector))
+    launched = kernels.launches_since(before)
+    assert "decode_stack" not in launched and ("decode_attention_half" in launched) == (dtype == "bfloat16" and shape == "small"), launched
     ref = replay.plain_logits(config, weights, requests, bf16=(dtype == "bfloat16"))
     replay.compare(collector.gather(outputs), ref, **replay.tolerance(dtype))
 
