@@ -1,10 +1,10 @@
 // All layers of a pre-norm model for a few rows that bring one token each (decoding), in one kernel.
 //
 // What bounds a decode step of few rows is not what it reads but how often one part of the chip has to learn what another part has
-// computed: norm, q/k/v, attention, output product, norm, up, down are five handings-on a layer. A kernel boundary hands on in 3.5 to 4 us
+// computed, five times a layer: stream to norms and q/k/v, these to attention, the heads' outputs to the output product, the stream to norms and up, hidden units to down. A kernel boundary hands on in 3.5 to 4 us
 // (the start of a dependent kernel, then its first trip to memory, both for its inputs and for its weights). Inside one kernel whose blocks
-// are all on the chip the same takes 2.1 to 3.1 us for 4 to 100 KB (measured with 256 blocks that each store a share and read everything),
-// and the weights are in registers by then: they do not depend on anything and are asked for a phase earlier.
+// are all on the chip 256 blocks that each store a share and then read everything, and do nothing else, take 2.1 to 3.1 us for 4 to 100 KB. Here, where a block reads what
+// it needs and uses first what is there first, a handing-on takes 1.0 to 2.1, and the weights are in registers by then: they do not depend on anything and are asked for a phase earlier.
 //
 // What is handed on are words of 8 bytes: 4 of numbers and 4 that say of which launch and layer they are (the tag). Who needs the words
 // loads them until all tags are the expected ones: no flags, no barriers across the chip, no memory to clear, and what arrives first is
@@ -22,9 +22,12 @@
 // the launch ends, says so in memory that the host reads, and from there on no block keeps keys or values in the cache.
 //
 // Measured (replayed steps of GPT-2 small in bfloat16 with 512 keys a row; the two layer kernels a layer before): 8 rows 353 -> 206 us a step, 14.4 us a layer, 1 row
-// 296 -> 158; in 32-bit (seven kernels a layer before) 8 rows 496 -> 344. A layer's 14.4 us, from one hand to the next: stream to normed rows 1.7 and to q/k/v 1.1, to the
-// attending blocks 1.0, scores and values 1.3, their sums 1.2, to the output product 1.6 and to the stream 0.7, to normed rows 2.1 and to hidden units 1.0, to the down product
-// 1.8 and to the stream 0.9. Bound by these trips and by the instructions between them (a lone wave's chain, 4 cycles an instruction), not by bytes.
+// 296 -> 158; in 32-bit (seven kernels a layer before) 8 rows 496 -> 344 (of which the layers 325, and 314 since their sums go on side by side). A layer's 14.4 us are five handings-on from block to block (the stream to normed rows 1.7, q/k/v to the
+// attending blocks 1.0, heads' outputs to the output product 1.6, the stream to normed rows 2.1, hidden units to the down product 1.8) and six stretches of a block's own work (q/k/v 1.1,
+// scores and values 1.3, their sums 1.2, the stream behind the output product 0.7, hidden units 1.0, the stream behind the down product 0.9). Bound by these trips and by the instructions
+// between them (a lone wave's chain, 4 cycles an instruction), not by bytes. Part of that chain are scalars that the compiler brings back from vector lanes: three parts with their regions and
+// pointers do not fit 106 scalar registers, 95 of them are spilled where rows have up to 768 columns in bfloat16 (144 for 16 rows), 145 to 236 up to 1,024, 301 to 491 beyond; of vector registers
+// 1, and beyond 1,024 columns 32 (119 for 16 rows, which the rule below never sends here); in 32-bit 120 to 292 scalars and 1 to 8 vector registers.
 #include "common.h"
 #include "key_sweep.h"
 
